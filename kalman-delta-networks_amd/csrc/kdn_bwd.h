@@ -2,9 +2,10 @@
 //
 // Per chunk of C = 64 tokens (h = state entering the chunk, dh = gradient of the state leaving
 // it, delta / d delta = the chunk's delta and its gradient, A = (I + N)^{-1} saved by the forward):
-//   state-gradient products  dQg = dO h^T,  dW = -d delta h^T,  dKf = delta dh^T,
+//   transposed solve         dX = A^T d delta, the gradient of X = V - Kg h (delta = A X), so dV = dX
+//   state-gradient products  dQg = dO h^T,  dKg = -dX h^T,  dKf = delta dh^T,
 //                            dM = lower(dO delta^T),  dgl_i = 2^{G_last,i} sum_v h_iv dh_iv
-//   transposed solves        dV = A^T d delta,  dKg = A^T dW,  dN = -strict_lower(dV U^T + dKg W^T)
+//   inverse                  dN = -strict_lower(A^T (d delta X^T) A^T) = -strict_lower(dX delta^T)
 //   gradients                with block anchors m (below): e = 2^{G_c - m}, Lk = k e, Lq = q e,
 //                            R = kappa / e, eg = 2^{G_c}, f = 2^{G_last - G_c}
 //                            dLk = dN R,  dLq = scale dM R,  dR = dN^T Lk + scale dM^T Lq
@@ -67,31 +68,28 @@ __device__ __forceinline__ void upper_tile(int t, int& I, int& J) {
   J = (0xfb9u >> (2 * t)) & 3;
 }
 
-// index of lower tile (I, J) in the order of lower_tile
-__device__ __forceinline__ int lower_tile_index(int I, int J) {
-  const int d = I - J;
-  return d == 0 ? I : d == 1 ? 4 + J : d == 2 ? 7 + J : 9;
-}
-
 // ---------------------------------------------------------------------------------------------
 // The whole chunk-parallel backward of one chunk in one kernel: the state-gradient products, the
 // transposed solves and the gradients.  dQg, dW, dKf, dM, dKg, dN and the g_last dots never go to
 // HBM: each is produced in the register or LDS layout its consumer takes.
 // One chunk-head task of the order task = (NT - 1 - n) * B*H + bh (last chunks first, the order in
-// which the reverse state pass finishes them); block 512 (8 waves), one workgroup per CU (LDS ~106 KB).
-//  * Staging.  The chunk rows of dO, delta and d delta are split into LDS fragments (rows c,
-//    k = v, natural order), all 64 rows at once.
-//  * Wave w owns channel tile it = w (16 channels of K) and V tile w (16 columns of V).  It loads
-//    its 16 rows of h and of dh straight into split fragments (one layout serves as the A operand
-//    h (rows i, k = v) and as the B operand h^T (k = v, cols i)) and forms
+// which the reverse state pass finishes them); block 512 (8 waves), one workgroup per CU (LDS 157 KB).
+//  * Staging.  The chunk rows of dO and delta are split into LDS fragments (rows c, k = v, natural
+//    order), all 64 rows at once; A^T goes to LDS as fp32.
+//  * Wave w owns V tile w (16 columns of V): its columns of d delta come from the reverse pass as the
+//    accumulator tiles that pass held (dd_off), two stacked tiles being a fragment in permuted k order, and
+//    give dX^T = d delta^T A (D tile: lane -> chunk row, 4 consecutive v), stored as dv and split into the
+//    row fragments of dX in LDS.
+//  * Wave w owns channel tile it = w (16 channels of K).  It loads its 16 rows of h and of dh straight into
+//    split fragments (A operand, rows i, k = v) and forms, beside the solve,
 //      dQg^T = h dO^T,  dKf^T = dh delta^T    (D tile: lane -> chunk row, 4 consecutive channels:
 //                                              the layout of the gradient phase's elementwise terms)
-//      -dW   = d delta h^T                    (D tile: lane -> channel, 4 chunk rows: two stacked
-//                                              tiles are the solve's A operand in permuted k order)
-//      dgl_i = 2^{G_last,i} sum_v h_iv dh_iv,  and dM = lower(dO delta^T) for lower tiles w, w + 8.
-//  * Solve.  Per wave one 32-column block: its V tile of d delta (dv stored) and its K tile of dW
-//    (dKg kept in registers), with A^T read in the same permuted k order; the block's dN^T share
-//    over the 8 waves is summed through LDS in two steps (waves 4..7 into 0..3, then the four).
+//      dgl_i = 2^{G_last,i} sum_v h_iv dh_iv,  and dM = lower(dO delta^T) for lower tiles w, w + 8;
+//    and from dX's fragments  dKg^T = -h dX^T  and  dN = -strict_lower(dX delta^T)  in the same forms.
+//    dX carries everything the inverse's gradient needs, so neither U nor W is read and no partial sum
+//    crosses the waves: as dN = -strict_lower(dV U^T + dKg W^T) the kernel read 1,024 B more per
+//    token-head (302 MB at B4 T4096 H18 d128) and summed eight waves' dN shares through LDS (step there
+//    1538 -> 1474 us isotropic, 2122 -> 2044 us diagonal).
 //  * Gradients.  dN, dM and their transposes are split once into LDS fragments (permuted k order:
 //    slot 4h + j of lane group g <-> k = 32 kb + 16 h + 4 g + j).  Per channel tile the factors R,
 //    Lk, Lq are built per lane for one channel and 16 chunk rows (rows outside the contraction's
@@ -99,39 +97,36 @@ __device__ __forceinline__ int lower_tile_index(int I, int J) {
 //    fragments as B: the D tiles give each lane 4 consecutive channels of one chunk row, the layout
 //    of dQg, dKf and dKg, so the elementwise inputs and outputs move as 16-byte (fp32) and 8-byte
 //    (bf16) vectors.
-// Chunks flagged by the forward store the products (dQg, dW, dKf, dM, dgl) for the exact kernels
-// and stop after them.
+// Chunks flagged by the forward store the products (dQg, dW = -d delta h^T, dKf, dM, dgl) for the exact
+// kernels and stop after them.
 // ---------------------------------------------------------------------------------------------
 template <int K, int V, bool ISO, typename TDO, int HM>
 __device__ __forceinline__ void chunk_bwd_task(
-    int task, const void* __restrict__ hbuf, const void* __restrict__ dhbuf, const void* __restrict__ Dl,
-    const void* __restrict__ dDl, const TDO* __restrict__ dO, const float* __restrict__ At,
-    const float* __restrict__ U, const float* __restrict__ W, const int* __restrict__ flags,
+    int task, const void* __restrict__ hbuf, const void* __restrict__ dhbuf, const float* __restrict__ Dl,
+    const float* __restrict__ dDl, const TDO* __restrict__ dO, const float* __restrict__ At,
+    const int* __restrict__ flags,
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, const float* __restrict__ q_rstd, const float* __restrict__ k_rstd, int T, int H,
     int NT, int BH, float scale, bf16_t* __restrict__ dv, bf16_t* __restrict__ dq, bf16_t* __restrict__ dk,
     float* __restrict__ dkap, float* __restrict__ dbeta, float* __restrict__ dg, float* __restrict__ xQg,
     float* __restrict__ xW, float* __restrict__ xKf, float* __restrict__ xM, float* __restrict__ xgl) {
   constexpr bool DO_BF16 = sizeof(TDO) == 2;
-  // HM: which of h, dh, delta, d delta were stored in bf16 (kdn_state::HB_*; the recurrences ran in
-  // fp32 and rounded those copies once).  A bf16 operand enters a product without a lo half: one
-  // MFMA against another bf16 operand, two against a split fp32 one.
+  // HM: which of h, dh were stored in bf16 (kdn_state::HB_*; the recurrences ran in fp32 and rounded
+  // those copies once).  A bf16 operand enters a product without a lo half: one MFMA against another
+  // bf16 operand, two against a split fp32 one.
   constexpr bool LH = !(HM & kdn_state::HB_H), LDH = !(HM & kdn_state::HB_DH);  // fp32 (split) copies
-  constexpr bool LD = !(HM & kdn_state::HB_D), LDD = !(HM & kdn_state::HB_DD);
   constexpr bool LO_ = !DO_BF16;
-  constexpr int EH = LH ? 4 : 2, EDH = LDH ? 4 : 2, ED = LD ? 4 : 2, EDD = LDD ? 4 : 2;  // bytes per element
+  constexpr int EH = LH ? 4 : 2, EDH = LDH ? 4 : 2;  // bytes per element
   constexpr int NW = 8;
   constexpr int VB = V / 32;        // k-blocks of the V contraction
   constexpr int NIT = K / 16;       // channel tiles (waves 0 .. NIT-1 own one each)
   constexpr int NVT = V / 16;       // V tiles (waves 0 .. NVT-1)
   constexpr int RB = VB * TILE;     // one 16-row block of a [rows][V] operand as fragments
   constexpr int FR = 8 * TILE;      // one 64 x 64 operand as (4 row tiles x 2 k-blocks) fragments
-  constexpr int AP4 = C + 4;        // LDS row stride of A^T (and of dM while it is passed on)
-  constexpr int STAGE_BYTES = 3 * 4 * RB * 2;
-  constexpr int SOLVE_BYTES = (C * AP4 + 2 * 4 * 10 * 256) * 4;
+  constexpr int AP4 = C + 4;        // LDS row stride of A^T
+  constexpr int STAGE_BYTES = 3 * 4 * RB * 2 + C * AP4 * 4;
   constexpr int CONTRIB_BYTES = 4 * FR * 2;
-  constexpr int LDS_A = STAGE_BYTES > SOLVE_BYTES ? STAGE_BYTES : SOLVE_BYTES;
-  constexpr int LDS_BYTES = LDS_A > CONTRIB_BYTES ? LDS_A : CONTRIB_BYTES;
+  constexpr int LDS_BYTES = STAGE_BYTES > CONTRIB_BYTES ? STAGE_BYTES : CONTRIB_BYTES;
   constexpr int SU = C * V / 8 / 512;  // staging units (8 consecutive v of one row) per thread per operand
   static_assert(SU >= 1 && (C * V / 8) % 512 == 0, "staging units per thread");
   static_assert(NIT <= NW && NVT <= NW, "K, V <= 128");
@@ -141,12 +136,10 @@ __device__ __forceinline__ void chunk_bwd_task(
   __shared__ float sDot[2][NW][C];  // in-op L2 norm: per-wave partial row dots y . dy of q and k
   __shared__ float sRs[2][C];       // ... and the rows' rstd of q and k (their raw values in memory)
   __shared__ float sBt[ISO ? C : 1];  // iso: the rows' beta (0 past L), for the gradient phase
-  bf16_t* sO = reinterpret_cast<bf16_t*>(smem);  // phase 1: dO, delta, d delta row fragments
+  bf16_t* sO = reinterpret_cast<bf16_t*>(smem);  // dO, delta, dX row fragments
   bf16_t* sD = sO + 4 * RB;
-  bf16_t* sdD = sD + 4 * RB;
-  float* sAt = reinterpret_cast<float*>(smem);   // solve: A^T [C][AP4]
-  float* sP = sAt + C * AP4;                      // per-wave partial dN^T tiles (4 slots)
-  float* sP2 = sP + 4 * 10 * 256;                 // ... and the same partials transposed (dN tiles)
+  bf16_t* sX = sD + 4 * RB;
+  float* sAt = reinterpret_cast<float*>(sX + 4 * RB);  // A^T [C][AP4]
   bf16_t* sF = reinterpret_cast<bf16_t*>(smem);  // gradients: dN, dM, dN^T, dM^T fragments
   const int n = NT - 1 - task / BH, bh = task % BH, b = bh / H, h = bh % H;
   const int t0 = n * C, L = min(C, T - t0);
@@ -167,28 +160,30 @@ __device__ __forceinline__ void chunk_bwd_task(
 
   // ================================ loads ================================
   const int64_t row0 = ((int64_t)bh * T + t0) * V;
-  const bufrsrc rD = make_buf(reinterpret_cast<const char*>(Dl) + row0 * ED, L * V * ED);  // rows past L read 0
-  const bufrsrc rdD = make_buf(reinterpret_cast<const char*>(dDl) + row0 * EDD, L * V * EDD);
+  const bufrsrc rD = make_buf(Dl + row0, L * V * 4);  // rows past L read 0
   const bufrsrc rO = make_buf(dO + (((int64_t)b * T + t0) * H + h) * V, ((L - 1) * H + 1) * V * sizeof(TDO));
-  float4 sr_D[SU][2], sr_dD[SU][2];
-  u32x4 sr_D16[SU], sr_dD16[SU];
+  // d delta of this wave's V tile: accumulator tiles of 16 chunk rows (rows past L hold 0)
+  const float* dDn = dDl + chunk * C * V;
+  f32x4 xd[4];
+#pragma unroll
+  for (int J = 0; J < 4; ++J)
+    xd[J] = own_v ? *reinterpret_cast<const f32x4*>(dDn + ((w * 4 + J) * 64 + lane) * 4) : zero4();
+  // A^T of the chunk
+  constexpr int AU = C * C / 4 / 512;
+  float4 at_r[AU];
+  if (!flagged) {
+    const bufrsrc rA = make_buf(At + chunk * C * C, C * C * 4);
+#pragma unroll
+    for (int u = 0; u < AU; ++u) at_r[u] = buf_ld4(rA, (tid + 512 * u) * 16);
+  }
+  float4 sr_D[SU][2];
   u32x4 sr_O[SU][DO_BF16 ? 1 : 2];
 #pragma unroll
   for (int u = 0; u < SU; ++u) {  // unit e: 16-row block, k-block, fragment lane
     const int e = tid + 512 * u, blk = e / (VB * 64), kb = (e / 64) % VB, sl = e & 63;
     const uint32_t c = (uint32_t)(16 * blk + (sl & 15)), v0 = (uint32_t)(32 * kb + 8 * (sl >> 4));
-    if constexpr (LD) {
-      sr_D[u][0] = buf_ld4(rD, (c * V + v0) * 4);
-      sr_D[u][1] = buf_ld4(rD, (c * V + v0) * 4 + 16);
-    } else {
-      sr_D16[u] = __builtin_amdgcn_raw_buffer_load_b128(rD, (c * V + v0) * 2, 0, 0);
-    }
-    if constexpr (LDD) {
-      sr_dD[u][0] = buf_ld4(rdD, (c * V + v0) * 4);
-      sr_dD[u][1] = buf_ld4(rdD, (c * V + v0) * 4 + 16);
-    } else {
-      sr_dD16[u] = __builtin_amdgcn_raw_buffer_load_b128(rdD, (c * V + v0) * 2, 0, 0);
-    }
+    sr_D[u][0] = buf_ld4(rD, (c * V + v0) * 4);
+    sr_D[u][1] = buf_ld4(rD, (c * V + v0) * 4 + 16);
     if constexpr (DO_BF16) {
       sr_O[u][0] = __builtin_amdgcn_raw_buffer_load_b128(rO, (c * H * V + v0) * 2, 0, 0);
     } else {
@@ -215,17 +210,9 @@ __device__ __forceinline__ void chunk_bwd_task(
     }
     gl_i = buf_ld(make_buf(gc + (((int64_t)b * T + t0 + L - 1) * H + h) * K, K * 4), i * 4);
   }
-  // A^T of the chunk (staged for the solve once the phase-1 fragments are dead)
-  constexpr int AU = C * C / 4 / 512;
-  float4 at_r[AU];
-  if (!flagged) {
-    const bufrsrc rA = make_buf(At + chunk * C * C, C * C * 4);
-#pragma unroll
-    for (int u = 0; u < AU; ++u) at_r[u] = buf_ld4(rA, (tid + 512 * u) * 16);
-  }
   // Diagonal variant, K = 128: the chunk's k and q rows for the gradient phase go straight from memory
-  // into LDS (buffer loads with the LDS flag: no registers held), issued with the solve's U / W rows,
-  // so they arrive during phase 1 and the solve instead of as per-channel gathers in the gradient
+  // into LDS (buffer loads with the LDS flag: no registers held), issued once phase 1's operands have
+  // arrived, so they land during phase 1 and the solve instead of as per-channel gathers in the gradient
   // phase (diag step -30 us; the isotropic variant, whose gradient phase loads less, measured 7 us
   // slower with it and keeps the gathers).
   // One instruction moves 64 lanes x 16 B = 4 rows of 256 B; row c of tensor x sits at
@@ -294,40 +281,74 @@ __device__ __forceinline__ void chunk_bwd_task(
       *reinterpret_cast<uint4*>(dst + off) = hi;
       *reinterpret_cast<uint4*>(dst + off + 512) = lo;
     };
-    // a bf16 copy is staged as its values alone (the lo half stays unused)
-    if constexpr (LD) put8(sD, sr_D[u][0], sr_D[u][1]);
-    else *reinterpret_cast<uint4*>(sD + off) = __builtin_bit_cast(uint4, sr_D16[u]);
-    if constexpr (LDD) put8(sdD, sr_dD[u][0], sr_dD[u][1]);
-    else *reinterpret_cast<uint4*>(sdD + off) = __builtin_bit_cast(uint4, sr_dD16[u]);
-    if constexpr (DO_BF16)
+    put8(sD, sr_D[u][0], sr_D[u][1]);
+    if constexpr (DO_BF16)  // exact in bf16: the lo half stays unused
       *reinterpret_cast<uint4*>(sO + off) = uint4{sr_O[u][0].x, sr_O[u][0].y, sr_O[u][0].z, sr_O[u][0].w};
     else
       put8(sO, __builtin_bit_cast(float4, sr_O[u][0]), __builtin_bit_cast(float4, sr_O[u][1]));
   }
-  __syncthreads();
-
-  // ================================ phase 1: products with h, dh ================================
-  // the solve's rows of U (V tile w) and W (K tile w), issued once phase 1's operands have arrived so
-  // they load during its products (issued with those operands they delay them; after the solve's
-  // products their latency is exposed).  Zero-size descriptors read 0 for a wave without the tile.
-  float4 uw[4][2];
-  {
-    const bufrsrc rUv = make_buf(U + ((int64_t)bh * T + t0) * V, own_v ? L * V * 4 : 0u);
-    const bufrsrc rWk = make_buf(W + ((int64_t)bh * T + t0) * K, own_k ? L * K * 4 : 0u);
+  if (!flagged) {
 #pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      const uint32_t sr = (uint32_t)(16 * J + r16);
-      uw[J][0] = buf_ld4(rUv, (sr * V + 16 * w + 4 * g4) * 4);
-      uw[J][1] = buf_ld4(rWk, (sr * K + i0) * 4);
+    for (int u = 0; u < AU; ++u) {
+      const int e4 = tid + 512 * u, sr = e4 / (C / 4), c4 = e4 % (C / 4);
+      *reinterpret_cast<float4*>(sAt + sr * AP4 + 4 * c4) = at_r[u];
+    }
+  } else {  // the exact kernels take dW = -d delta h^T: the rows of d delta as fragments in dX's place
+#pragma unroll
+    for (int u = 0; u < SU; ++u) {
+      const int e = tid + 512 * u, blk = e / (VB * 64), kb = (e / 64) % VB, sl = e & 63;
+      const int c = 16 * blk + (sl & 15), v0 = 32 * kb + 8 * (sl >> 4);
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = dDn[kdn_state::dd_off(c, v0 + j)];
+      uint4 hi, lo;
+      split8(x, hi, lo);
+      *reinterpret_cast<uint4*>(sX + blk * RB + kb * TILE + sl * 8) = hi;
+      *reinterpret_cast<uint4*>(sX + blk * RB + kb * TILE + sl * 8 + 512) = lo;
     }
   }
-  issue_qk();  // after phase 1's operands, like the U / W rows
+  __syncthreads();
+
+  // ================================ phase 1: the solve, products with h, dh ================================
+  issue_qk();  // after phase 1's operands
   issue_g();
-  f32x4 aQ[4], aW[4], aK[4];  // dQg^T (rows i, cols c), d delta h^T (rows c, cols i), dKf^T
+  if (!flagged && own_v) {
+    // dX^T = d delta^T A (rows v of this wave's tile, cols s); k = chunk row c in permuted order: slot j of
+    // lane group g4 <-> c = 32 kb + 4 g4 + j (j < 4) or 32 kb + 16 + 4 g4 + (j - 4)
+    const bufrsrc rdv = make_buf(dv + (((int64_t)b * T + t0) * H + h) * V, ((L - 1) * H + 1) * V * 2);
+    f32x4 Y[4];
 #pragma unroll
-  for (int tl = 0; tl < 4; ++tl) aQ[tl] = aW[tl] = aK[tl] = zero4();
+    for (int J = 0; J < 4; ++J) Y[J] = zero4();
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      uint4 xh, xl;
+      kdn_state::bfrag(xd[2 * kb], xd[2 * kb + 1], xh, xl);
+#pragma unroll
+      for (int J = 0; J < 4; ++J) {
+        if (J > 2 * kb + 1) continue;  // A[c][s] = 0 for c < s
+        const float* row = sAt + (16 * J + r16) * AP4 + 32 * kb + 4 * g4;
+        const float4 a0 = *reinterpret_cast<const float4*>(row), a1 = *reinterpret_cast<const float4*>(row + 16);
+        const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        uint4 ah, al;
+        split8(av, ah, al);
+        Y[J] = mma3(xh, xl, ah, al, Y[J]);
+      }
+    }
+    const int v0 = 16 * w + 4 * g4;  // this lane's 4 columns of row s = 16 J + r16
+#pragma unroll
+    for (int J = 0; J < 4; ++J) {
+      const uint32_t lo = (uint32_t)f2bf(Y[J][0]) | ((uint32_t)f2bf(Y[J][1]) << 16);
+      const uint32_t hi = (uint32_t)f2bf(Y[J][2]) | ((uint32_t)f2bf(Y[J][3]) << 16);
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2{lo, hi}, rdv, ((uint32_t)((16 * J + r16) * H) * V + v0) * 2, 0, 0);
+      kdn_state::put_unit(sX, J * RB + (v0 >> 5) * TILE + (r16 + 16 * ((v0 & 31) >> 3)) * 8 + (v0 & 7), Y[J][0], Y[J][1],
+                          Y[J][2], Y[J][3]);
+    }
+  }
+  f32x4 aQ[4], aK[4], kg[4];  // dQg^T, dKf^T, dKg^T (rows i, cols c): lane -> chunk row 16 J + r16, channels i0 ..
+#pragma unroll
+  for (int tl = 0; tl < 4; ++tl) aQ[tl] = aK[tl] = kg[tl] = zero4();
+  uint4 fh[VB], fl[VB];  // h (split, or its bf16 values)
   if (own_k) {
-    uint4 fh[VB], fl[VB];  // h (split, or its bf16 values)
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {
       if constexpr (LH) split8(hv[kb], fh[kb], fl[kb]);
@@ -337,13 +358,12 @@ __device__ __forceinline__ void chunk_bwd_task(
     for (int kb = 0; kb < VB; ++kb)
 #pragma unroll
       for (int tl = 0; tl < 4; ++tl) {
-        uint4 oh, ol, xh, xl;
+        uint4 oh, ol;
         afragx<LO_>(sO + tl * RB, kb, lane, oh, ol);
         aQ[tl] = mmx<LH, LO_>(fh[kb], fl[kb], oh, ol, aQ[tl]);
-        afragx<LDD>(sdD + tl * RB, kb, lane, xh, xl);
-        aW[tl] = mmx<LDD, LH>(xh, xl, fh[kb], fl[kb], aW[tl]);
       }
     float dot = 0.f;
+    uint4 eh[VB], el[VB];  // dh
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {
       float hf[8], df[8];
@@ -353,8 +373,8 @@ __device__ __forceinline__ void chunk_bwd_task(
       if constexpr (!LDH) kdn_intra::unpack8(dhr[kb], df);
 #pragma unroll
       for (int j = 0; j < 8; ++j) dot += hf[j] * df[j];
-      if constexpr (LDH) split8(dhv[kb], fh[kb], fl[kb]);  // fh, fl: dh from here on
-      else fh[kb] = __builtin_bit_cast(uint4, dhr[kb]), fl[kb] = uint4{0u, 0u, 0u, 0u};
+      if constexpr (LDH) split8(dhv[kb], eh[kb], el[kb]);
+      else eh[kb] = __builtin_bit_cast(uint4, dhr[kb]), el[kb] = uint4{0u, 0u, 0u, 0u};
     }
     dot += __shfl_xor(dot, 16, 64);
     dot += __shfl_xor(dot, 32, 64);
@@ -364,8 +384,8 @@ __device__ __forceinline__ void chunk_bwd_task(
 #pragma unroll
       for (int tl = 0; tl < 4; ++tl) {
         uint4 xh, xl;
-        afragx<LD>(sD + tl * RB, kb, lane, xh, xl);
-        aK[tl] = mmx<LDH, LD>(fh[kb], fl[kb], xh, xl, aK[tl]);
+        afrag(sD + tl * RB, kb, lane, xh, xl);
+        aK[tl] = mmx<LDH, true>(eh[kb], el[kb], xh, xl, aK[tl]);
       }
   }
   // dM tiles (c-block I, s-block J) = lower(dO delta^T) for lower tiles w and w + 8: mt lane -> column
@@ -382,10 +402,10 @@ __device__ __forceinline__ void chunk_bwd_task(
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {
       uint4 xh, xl, oh, ol;
-      afragx<LD>(sD + J * RB, kb, lane, xh, xl);
+      afrag(sD + J * RB, kb, lane, xh, xl);
       afragx<LO_>(sO + I * RB, kb, lane, oh, ol);
-      mt[x] = mmx<LO_, LD>(oh, ol, xh, xl, mt[x]);
-      mtT[x] = mmx<LD, LO_>(xh, xl, oh, ol, mtT[x]);
+      mt[x] = mmx<LO_, true>(oh, ol, xh, xl, mt[x]);
+      mtT[x] = mmx<true, LO_>(xh, xl, oh, ol, mtT[x]);
     }
     if (I == J) {
 #pragma unroll
@@ -404,12 +424,17 @@ __device__ __forceinline__ void chunk_bwd_task(
       const bufrsrc rKf = make_buf(xKf + ((int64_t)bh * T + t0) * K, L * K * 4);
 #pragma unroll
       for (int tl = 0; tl < 4; ++tl) {
-        const uint32_t c = (uint32_t)(16 * tl + r16);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, aQ[tl]), rQ, (c * K + i0) * 4, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, aK[tl]), rKf, (c * K + i0) * 4, 0, 0);
+        f32x4 aW = zero4();  // (d delta h^T)^T: rows i, cols c
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          buf_st(rW, ((uint32_t)(16 * tl + 4 * g4 + j) * K + 16 * it + r16) * 4, -aW[tl][j]);
+        for (int kb = 0; kb < VB; ++kb) {
+          uint4 xh, xl;
+          afrag(sX + tl * RB, kb, lane, xh, xl);
+          aW = mmx<LH, true>(fh[kb], fl[kb], xh, xl, aW);
+        }
+        const uint32_t o = ((uint32_t)(16 * tl + r16) * K + i0) * 4;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, aQ[tl]), rQ, o, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, aK[tl]), rKf, o, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, -aW), rW, o, 0, 0);
       }
       if (g4 == 0) xgl[chunk * K + 16 * it + r16] = sDgl[16 * it + r16];
     }
@@ -431,111 +456,45 @@ __device__ __forceinline__ void chunk_bwd_task(
     }
     return;
   }
-  __syncthreads();  // phase-1 fragments dead: A^T may overwrite them
-#pragma unroll
-  for (int u = 0; u < AU; ++u) {
-    const int e4 = tid + 512 * u, sr = e4 / (C / 4), c4 = e4 % (C / 4);
-    *reinterpret_cast<float4*>(sAt + sr * AP4 + 4 * c4) = at_r[u];
-  }
-  __syncthreads();
+  __syncthreads();  // dX's fragments are complete
 
-  // ================================ solve ================================
-  // Yt[0] = d delta^T A (V tile w), Yt[1] = dW^T A (K tile w); k = chunk row c in permuted order:
-  // slot j of lane group g4 <-> c = 32 kb + 4 g4 + j (j < 4) or 32 kb + 16 + 4 g4 + (j - 4)
-  const bufrsrc rdv = make_buf(dv + (((int64_t)b * T + t0) * H + h) * V, ((L - 1) * H + 1) * V * 2);
-  f32x4 Yt[2][4];
+  // ================================ products with dX ================================
+  if (own_k) {
 #pragma unroll
-  for (int ct = 0; ct < 2; ++ct)
+    for (int kb = 0; kb < VB; ++kb)
 #pragma unroll
-    for (int J = 0; J < 4; ++J) Yt[ct][J] = zero4();
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    uint4 xh0, xl0, xh1, xl1;
-    {
-      // d delta from phase 1's staged fragments (still intact: the partials overwrite them only after the barrier
-      // that ends the solve's reads): element (c, v) of the [rows c][k = v] fragments, its bf16 hi and lo halves,
-      // the split of the same value this column needs (a bf16 copy has no lo half)
-      const uint16_t* f16 = reinterpret_cast<const uint16_t*>(sdD);
-      const int v = 16 * w + r16;
-      uint32_t xr[8], xq[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int c = 32 * kb + (j < 4 ? 4 * g4 + j : 16 + 4 * g4 + j - 4);
-        const int off = (c >> 4) * RB + (v >> 5) * TILE + ((c & 15) + 16 * ((v & 31) >> 3)) * 8 + (v & 7);
-        xr[j] = own_v ? (uint32_t)f16[off] : 0u;
-        xq[j] = own_v && LDD ? (uint32_t)f16[off + 512] : 0u;
+      for (int tl = 0; tl < 4; ++tl) {
+        uint4 xh, xl;
+        afrag(sX + tl * RB, kb, lane, xh, xl);
+        kg[tl] = mmx<LH, true>(fh[kb], fl[kb], xh, xl, kg[tl]);
       }
-      xh0 = uint4{xr[0] | (xr[1] << 16), xr[2] | (xr[3] << 16), xr[4] | (xr[5] << 16), xr[6] | (xr[7] << 16)};
-      xl0 = uint4{xq[0] | (xq[1] << 16), xq[2] | (xq[3] << 16), xq[4] | (xq[5] << 16), xq[6] | (xq[7] << 16)};
-    }
-    {
-      const f32x4 t0_ = -aW[2 * kb], t1_ = -aW[2 * kb + 1];  // zero for waves without a channel tile
-      kdn_state::bfrag(t0_, t1_, xh1, xl1);
+#pragma unroll
+    for (int tl = 0; tl < 4; ++tl) kg[tl] = -kg[tl];
+  }
+  // dN tiles = -strict_lower(dX delta^T), both forms as dM's
+  f32x4 nt[2], ntT[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    nt[x] = ntT[x] = zero4();
+    const int t = w + NW * x;
+    if (t >= 10) continue;
+    int I, J;
+    lower_tile(t, I, J);
+#pragma unroll
+    for (int kb = 0; kb < VB; ++kb) {
+      uint4 xh, xl, yh, yl;
+      afrag(sD + J * RB, kb, lane, xh, xl);
+      afrag(sX + I * RB, kb, lane, yh, yl);
+      nt[x] = mma3(yh, yl, xh, xl, nt[x]);
+      ntT[x] = mma3(xh, xl, yh, yl, ntT[x]);
     }
 #pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      if (J > 2 * kb + 1) continue;  // A[c][s] = 0 for c < s
-      const float* row = sAt + (16 * J + r16) * AP4 + 32 * kb + 4 * g4;
-      const float4 a0 = *reinterpret_cast<const float4*>(row), a1 = *reinterpret_cast<const float4*>(row + 16);
-      const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-      uint4 ah, al;
-      split8(av, ah, al);
-      Yt[0][J] = mmx<LDD, true>(xh0, xl0, ah, al, Yt[0][J]);
-      Yt[1][J] = mma3(xh1, xl1, ah, al, Yt[1][J]);
+    for (int j = 0; j < 4; ++j) {
+      nt[x][j] = I == J && r16 >= 4 * g4 + j ? 0.f : -nt[x][j];
+      ntT[x][j] = I == J && 4 * g4 + j >= r16 ? 0.f : -ntT[x][j];
     }
   }
-  if (own_v) {  // dv rows s = 16 J + r16, columns 16 w + 4 g4 .. + 3
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      const uint32_t tr = (uint32_t)(16 * J + r16), x0 = (uint32_t)(16 * w + 4 * g4);
-      const f32x4 y = Yt[0][J];
-      const uint32_t lo = (uint32_t)f2bf(y[0]) | ((uint32_t)f2bf(y[1]) << 16);
-      const uint32_t hi = (uint32_t)f2bf(y[2]) | ((uint32_t)f2bf(y[3]) << 16);
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2{lo, hi}, rdv, ((tr * H) * V + x0) * 2, 0, 0);
-    }
-  }
-  // this block's share of dN^T[s][c] = sum_x (U|W)[s][x] Y[x][c] (part: D tiles rows s, cols c) and the
-  // same products transposed (part2: rows c, cols s), for the two orientations of the dN fragments
-  f32x4 part[10], part2[10];
-  {
-    uint4 uh[4], ul[4], yh[4], yl[4];
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      const float4 a0 = uw[J][0], a1 = uw[J][1];
-      const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-      split8(av, uh[J], ul[J]);
-      kdn_state::bfrag(Yt[0][J], Yt[1][J], yh[J], yl[J]);
-    }
-#pragma unroll
-    for (int t = 0; t < 10; ++t) {
-      int I, J;
-      lower_tile(t, I, J);
-      part[t] = mma3(uh[J], ul[J], yh[I], yl[I], zero4());
-      part2[t] = mma3(yh[I], yl[I], uh[J], ul[J], zero4());
-    }
-  }
-  f32x4 kg[4];  // dKg^T tiles: lane -> chunk row 16 J + r16, channels i0 .. i0 + 3
-#pragma unroll
-  for (int J = 0; J < 4; ++J) kg[J] = Yt[1][J];
-  __syncthreads();  // every A^T read done: the partials may overwrite it
-  if (w >= 4) {
-#pragma unroll
-    for (int t = 0; t < 10; ++t) {
-      *reinterpret_cast<f32x4*>(sP + (((w - 4) * 10 + t) * 64 + lane) * 4) = part[t];
-      *reinterpret_cast<f32x4*>(sP2 + (((w - 4) * 10 + t) * 64 + lane) * 4) = part2[t];
-    }
-  }
-  __syncthreads();
-  if (w < 4) {
-#pragma unroll
-    for (int t = 0; t < 10; ++t) {
-      f32x4* slot = reinterpret_cast<f32x4*>(sP + ((w * 10 + t) * 64 + lane) * 4);
-      *slot = *slot + part[t];
-      f32x4* slot2 = reinterpret_cast<f32x4*>(sP2 + ((w * 10 + t) * 64 + lane) * 4);
-      *slot2 = *slot2 + part2[t];
-    }
-  }
-  __syncthreads();
+  __syncthreads();  // every fragment read: the gradient phase's fragments may overwrite them
 
   // ======================= dN, dM staging (the gradient phase's fragments) =======================
   // fragment offset of 4 consecutive k = k0 .. k0 + 3 (k0 % 4 == 0) of one row: permuted k order, slot
@@ -543,64 +502,18 @@ __device__ __forceinline__ void chunk_bwd_task(
   auto foff = [](int row, int k0) {
     return ((row >> 4) * 2 + (k0 >> 5)) * TILE + ((row & 15) + 16 * ((k0 & 15) >> 2)) * 8 + 4 * ((k0 >> 4) & 1);
   };
-  // dN[c][s] = -(sum of the waves' partials), strictly lower: units (row, k0) of the rows form (row c,
-  // k = s, from the part D tiles) and of the transposed form (row s, k = c, from the part2 D tiles)
-  float4 dNu[2], dNtu[2];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int e = tid + 512 * u, row = e >> 4, kb = (e >> 3) & 1, hh = (e >> 2) & 1, gg = e & 3;
-    const int k0 = 32 * kb + 16 * hh + 4 * gg;
-    float4 acc = float4{0.f, 0.f, 0.f, 0.f}, acct = float4{0.f, 0.f, 0.f, 0.f};
-    if ((k0 >> 4) <= (row >> 4)) {  // rows form: tile (c-block row / 16, s-block k0 / 16)
-      const int t = lower_tile_index(row >> 4, k0 >> 4), ln = (row & 15) + 16 * ((k0 & 15) >> 2);
-#pragma unroll
-      for (int ww = 0; ww < 4; ++ww) {
-        const float4 v = *reinterpret_cast<const float4*>(sP + ((ww * 10 + t) * 64 + ln) * 4);
-        acc.x -= v.x, acc.y -= v.y, acc.z -= v.z, acc.w -= v.w;
-      }
-      if (k0 + 0 >= row) acc.x = 0.f;
-      if (k0 + 1 >= row) acc.y = 0.f;
-      if (k0 + 2 >= row) acc.z = 0.f;
-      if (k0 + 3 >= row) acc.w = 0.f;
-    }
-    if ((k0 >> 4) >= (row >> 4)) {  // transposed form: tile (c-block k0 / 16, s-block row / 16)
-      const int t = lower_tile_index(k0 >> 4, row >> 4), ln = (row & 15) + 16 * ((k0 & 15) >> 2);
-#pragma unroll
-      for (int ww = 0; ww < 4; ++ww) {
-        const float4 v = *reinterpret_cast<const float4*>(sP2 + ((ww * 10 + t) * 64 + ln) * 4);
-        acct.x -= v.x, acct.y -= v.y, acct.z -= v.z, acct.w -= v.w;
-      }
-      if (k0 + 0 <= row) acct.x = 0.f;
-      if (k0 + 1 <= row) acct.y = 0.f;
-      if (k0 + 2 <= row) acct.z = 0.f;
-      if (k0 + 3 <= row) acct.w = 0.f;
-    }
-    dNu[u] = acc;
-    dNtu[u] = acct;
-  }
-  __syncthreads();  // every partial read before the fragments overwrite them
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int e = tid + 512 * u, row = e >> 4, kb = (e >> 3) & 1, hh = (e >> 2) & 1, gg = e & 3;
-    const int off = foff(row, 32 * kb + 16 * hh + 4 * gg);
-    kdn_state::put_unit(sF, off, dNu[u].x, dNu[u].y, dNu[u].z, dNu[u].w);
-    kdn_state::put_unit(sF + 2 * FR, off, dNtu[u].x, dNtu[u].y, dNtu[u].z, dNtu[u].w);
-  }
-#pragma unroll
-  for (int x = 0; x < 2; ++x) {  // dM rows (row c, k = s) from mtT, dM^T rows (row s, k = c) from mt
+  for (int x = 0; x < 2; ++x) {  // rows form (row c, k = s) from the T tiles, transposed form (row s, k = c)
     const int t = w + NW * x;
     if (t >= 16) continue;
-    int I, J;
-    f32x4 a = zero4(), at = zero4();
-    if (t < 10) {
-      lower_tile(t, I, J);
-      a = mtT[x];
-      at = mt[x];
-    } else {
-      upper_tile(t - 10, I, J);  // I < J: zero tiles of both forms
-    }
-    kdn_state::put_unit(sF + FR, foff(16 * I + r16, 16 * J + 4 * g4), a[0], a[1], a[2], a[3]);
-    kdn_state::put_unit(sF + 3 * FR, foff(16 * J + r16, 16 * I + 4 * g4), at[0], at[1], at[2], at[3]);
+    int I, J;  // tiles 10 .. 15: I < J, zero in both forms
+    if (t < 10) lower_tile(t, I, J);
+    else upper_tile(t - 10, I, J);
+    const int fr = foff(16 * I + r16, 16 * J + 4 * g4), ft = foff(16 * J + r16, 16 * I + 4 * g4);
+    kdn_state::put_unit(sF, fr, ntT[x][0], ntT[x][1], ntT[x][2], ntT[x][3]);
+    kdn_state::put_unit(sF + FR, fr, mtT[x][0], mtT[x][1], mtT[x][2], mtT[x][3]);
+    kdn_state::put_unit(sF + 2 * FR, ft, nt[x][0], nt[x][1], nt[x][2], nt[x][3]);
+    kdn_state::put_unit(sF + 3 * FR, ft, mt[x][0], mt[x][1], mt[x][2], mt[x][3]);
   }
   if constexpr (QK_LDS || G_LDS) __builtin_amdgcn_s_waitcnt(0);  // this wave's k, q or G rows have reached LDS
   __syncthreads();
@@ -881,17 +794,16 @@ __device__ __forceinline__ void chunk_bwd_task(
 // One workgroup per task: tasks task0 .. task0 + gridDim.x - 1.
 template <int K, int V, bool ISO, typename TDO, int HM>
 __global__ __launch_bounds__(512, 1) void chunk_bwd_kernel(
-    const void* __restrict__ hbuf, const void* __restrict__ dhbuf, const void* __restrict__ Dl,
-    const void* __restrict__ dDl, const TDO* __restrict__ dO, const float* __restrict__ At,
-    const float* __restrict__ U, const float* __restrict__ W, const int* __restrict__ flags,
+    const void* __restrict__ hbuf, const void* __restrict__ dhbuf, const float* __restrict__ Dl,
+    const float* __restrict__ dDl, const TDO* __restrict__ dO, const float* __restrict__ At,
+    const int* __restrict__ flags,
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, const float* __restrict__ q_rstd, const float* __restrict__ k_rstd, int T, int H,
     int NT, int BH, int task0, float scale, bf16_t* __restrict__ dv, bf16_t* __restrict__ dq, bf16_t* __restrict__ dk,
     float* __restrict__ dkap, float* __restrict__ dbeta, float* __restrict__ dg, float* __restrict__ xQg,
     float* __restrict__ xW, float* __restrict__ xKf, float* __restrict__ xM, float* __restrict__ xgl) {
-  chunk_bwd_task<K, V, ISO, TDO, HM>(task0 + (int)blockIdx.x, hbuf, dhbuf, Dl, dDl, dO, At, U, W, flags, q, k, kap, gc,
-                                 q_rstd, k_rstd, T, H, NT, BH, scale, dv, dq, dk, dkap, dbeta, dg, xQg, xW, xKf, xM,
-                                 xgl);
+  chunk_bwd_task<K, V, ISO, TDO, HM>(task0 + (int)blockIdx.x, hbuf, dhbuf, Dl, dDl, dO, At, flags, q, k, kap, gc, q_rstd,
+                                 k_rstd, T, H, NT, BH, scale, dv, dq, dk, dkap, dbeta, dg, xQg, xW, xKf, xM, xgl);
 }
 
 }  // namespace kdn_bwd

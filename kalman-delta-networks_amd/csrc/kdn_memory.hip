@@ -18,10 +18,9 @@
 //   state_fwd    serial over chunks, one workgroup per (V-slice, b, h): h per chunk, delta
 //   readout      chunk-parallel O = Qg h + M delta (kdn_state.h)
 //   state_bwd    serial reverse (kdn_state.h): d delta = M^T dO + Kf dS;  dS <- e dS + Qg^T dO - W^T d delta
-//   chunk_bwd    (kdn_bwd.h, 512 threads) per chunk: dQg = dO h^T, dW = -d delta h^T, dKf = delta dh^T,
-//                dM = dO delta^T, g_last terms; dV = (I+N)^-T d delta, dKg = (I+N)^-T dW,
-//                dN = -(dV U^T + dKg W^T); dq, dk, dkappa (or dbeta), dg from dN, dM and the
-//                elementwise factors
+//   chunk_bwd    (kdn_bwd.h, 512 threads) per chunk: dV = (I+N)^-T d delta, dQg = dO h^T, dKg = -dV h^T,
+//                dKf = delta dh^T, dM = dO delta^T, dN = -dV delta^T, g_last terms; dq, dk, dkappa
+//                (or dbeta), dg from dN, dM and the elementwise factors
 //   *_exact      the chunks the forward flagged: the same backward by per-block anchors and scalar
 //                substitution (the products above come from chunk_bwd through HBM)
 //
@@ -436,7 +435,7 @@ __device__ void bwd_solve_exact_chunk(
     const bf16_t* __restrict__ k, const float* __restrict__ kap, const float* __restrict__ gc,
     const float* __restrict__ dDl, const float* __restrict__ dWg, const float* __restrict__ U,
     const float* __restrict__ W, int T, int H, int NT, bf16_t* __restrict__ dv, float* __restrict__ dKg,
-    float* __restrict__ dNg, int n, int bh, const float* __restrict__ k_rstd, bool dd16, unsigned char* lds) {
+    float* __restrict__ dNg, int n, int bh, const float* __restrict__ k_rstd, unsigned char* lds) {
   constexpr int KP = K + 4;
   constexpr int XP = V + K + 4;
   // phase 1: sK | sA | sG (3 x C x KP); phase 2 (after the solve) reuses it as sX | sUW (2 x C x XP)
@@ -469,9 +468,7 @@ __device__ void bwd_solve_exact_chunk(
         const int c = 16 * I + r;
         float x = 0.f;
         if (c < L)
-          x = !isV ? dWg[bht(bh, t0 + c, T, K) + col]
-              : dd16 ? bf2f(reinterpret_cast<const bf16_t*>(dDl)[bht(bh, t0 + c, T, V) + col])
-                     : dDl[bht(bh, t0 + c, T, V) + col];
+          x = isV ? dDl[((int64_t)bh * NT + n) * C * V + kdn_state::dd_off(c, col)] : dWg[bht(bh, t0 + c, T, K) + col];
         acc[r] = x;
       }
 #pragma unroll 1
@@ -533,14 +530,14 @@ __global__ __launch_bounds__(256) void mem_bwd_solve_exact_kernel(
     const bf16_t* __restrict__ k, const float* __restrict__ kap, const float* __restrict__ gc,
     const float* __restrict__ dDl, const float* __restrict__ dWg, const float* __restrict__ U,
     const float* __restrict__ W, int T, int H, int NT, int NB, const int* __restrict__ flags, bf16_t* __restrict__ dv,
-    float* __restrict__ dKg, float* __restrict__ dNg, const float* __restrict__ k_rstd, bool dd16) {
+    float* __restrict__ dKg, float* __restrict__ dNg, const float* __restrict__ k_rstd) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[ExactLds<K, V>::solve];
   if (!any_flagged(flags, NB)) return;
   for (int lin = blockIdx.x; lin < NB; lin += gridDim.x) {
     if (flags[lin] == 0) continue;
     __syncthreads();
     bwd_solve_exact_chunk<K, V, ISO>(k, kap, gc, dDl, dWg, U, W, T, H, NT, dv, dKg, dNg, lin % NT, lin / NT, k_rstd,
-                                     dd16, lds);
+                                     lds);
   }
 }
 
@@ -795,14 +792,14 @@ __global__ __launch_bounds__(256) void mem_bwd_exact_kernel(
     int NB, const int* __restrict__ flags, float scale, bf16_t* __restrict__ dv, float* __restrict__ dKg,
     float* __restrict__ dNg, bf16_t* __restrict__ dq, bf16_t* __restrict__ dk, float* __restrict__ dkap,
     float* __restrict__ dbeta, float* __restrict__ dg, const float* __restrict__ q_rstd,
-    const float* __restrict__ k_rstd, bool dd16) {
+    const float* __restrict__ k_rstd) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[ExactLds<K, V>::both];
   if (!any_flagged(flags, NB)) return;
   for (int lin = blockIdx.x; lin < NB; lin += gridDim.x) {
     if (flags[lin] == 0) continue;
     const int n = lin % NT, bh = lin / NT;
     __syncthreads();
-    bwd_solve_exact_chunk<K, V, ISO>(k, kap, gc, dDl, dWg, U, W, T, H, NT, dv, dKg, dNg, n, bh, k_rstd, dd16, lds);
+    bwd_solve_exact_chunk<K, V, ISO>(k, kap, gc, dDl, dWg, U, W, T, H, NT, dv, dKg, dNg, n, bh, k_rstd, lds);
     __syncthreads();
     bwd_contrib_exact_chunk<K, V, ISO>(q, k, kap, gc, dNg, dMg, dQg, dKg, dKf, dgl, T, H, NT, scale, dq, dk, dkap,
                                        dbeta, dg, n, bh, q_rstd, k_rstd, lds);
@@ -853,9 +850,8 @@ inline int64_t group_floats(int64_t BH, GroupCount gc, int K, int V) {
 }
 inline int64_t round64(int64_t x) { return (x + 63) / 64 * 64; }
 
-// Precision of the per-chunk copies only the backward reads (the forward pass's h and delta, the
-// reverse pass's dh and d delta; kdn_state::HB_* bits, set = bf16).  The isotropic scan stores h and dh
-// in bf16 (its reference's backward keeps all four in the input dtype: FLA's chunk_gated_delta_rule
+// Precision of the per-chunk state copies only the backward reads (the forward pass's h, the reverse
+// pass's dh; kdn_state::HB_* bits, set = bf16).  The isotropic scan stores h and dh in bf16 (its reference's backward keeps all four in the input dtype: FLA's chunk_gated_delta_rule
 // allocates h, v_new, dh and dv2 like k): half the bytes of the two largest copies, written by the
 // state passes and read by the chunk backward, whose products with them take one or two bf16 MFMAs
 // instead of three.  delta and d delta stay fp32: in bf16 they moved the parameter gradients that sum
@@ -903,7 +899,7 @@ struct BwdLayout {
     gc = plan_groups(B * H, cdiv(T, C), K, V);
     dh = 0;
     dD = dh + NB * K * V;
-    dQg = dD + TT * V;
+    dQg = dD + NB * C * V;  // whole accumulator tiles (kdn_state::dd_off)
     dW = dQg + TT * K;
     dKf = dW + TT * K;
     dM = dKf + TT * K;
@@ -1205,8 +1201,8 @@ int mem_bwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
   auto launch_chunk = [&](int task0, int task_end, hipStream_t st) {
 #define KDN_CHUNK_BWD(ISO_, HB_)                                                                                    \
   hipLaunchKernelGGL((kdn_bwd::chunk_bwd_kernel<K, V, ISO_, TDO, HB_>), dim3(task_end - task0), dim3(512), 0, st, hb, \
-                     dh, D, dD, dO, A, U, W, flags, q, k, kap, gc, q_rstd, k_rstd, T, H, NT, B * H, task0, scale, dv, \
-                     dq, dk, dkap, dbeta, dg, dQg, dW, dKf, dM, dgl)
+                     dh, D, dD, dO, A, flags, q, k, kap, gc, q_rstd, k_rstd, T, H, NT, B * H, task0, scale, dv, dq, dk, \
+                     dkap, dbeta, dg, dQg, dW, dKf, dM, dgl)
     if (iso && hm == kIsoHalfCopies) KDN_CHUNK_BWD(true, kIsoHalfCopies);
     else if (iso) KDN_CHUNK_BWD(true, 0);
     else KDN_CHUNK_BWD(false, 0);
@@ -1260,7 +1256,7 @@ int mem_bwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
 #define KDN_EXACT(ISO_)                                                                                               \
   hipLaunchKernelGGL((mem_bwd_exact_kernel<K, V, ISO_>), dim3(gx), dim3(256), 0, stream, q, k, kap, gc, dD, dW, U, W, \
                      dM, dQg, dKf, dgl, T, H, NT, NB, flags, scale, dv, dKg, dN, dq, dk, dkap, dbeta, dg, q_rstd,      \
-                     k_rstd, (hm & kdn_state::HB_DD) != 0)
+                     k_rstd)
     if (iso) KDN_EXACT(true);
     else KDN_EXACT(false);
 #undef KDN_EXACT
@@ -1271,10 +1267,10 @@ int mem_bwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
     const int NB = B * H * NT, gx = min(NB, 512);
     if (iso)
       hipLaunchKernelGGL((mem_bwd_solve_exact_kernel<K, V, true>), dim3(gx), dim3(256), 0, stream, k, kap, gc, dD, dW,
-                         U, W, T, H, NT, NB, flags, dv, dKg, dN, k_rstd, (hm & kdn_state::HB_DD) != 0);
+                         U, W, T, H, NT, NB, flags, dv, dKg, dN, k_rstd);
     else
       hipLaunchKernelGGL((mem_bwd_solve_exact_kernel<K, V, false>), dim3(gx), dim3(256), 0, stream, k, kap, gc, dD,
-                         dW, U, W, T, H, NT, NB, flags, dv, dKg, dN, k_rstd, (hm & kdn_state::HB_DD) != 0);
+                         dW, U, W, T, H, NT, NB, flags, dv, dKg, dN, k_rstd);
     KDN_CHECK_LAUNCH();
   }
   if (stages & 8) {  // the exact path's gradients

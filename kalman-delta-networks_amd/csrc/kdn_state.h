@@ -156,14 +156,6 @@ __device__ __forceinline__ void st_rows4(bufrsrc r, uint32_t vbase, uint32_t row
 __device__ __forceinline__ bufrsrc rows_from(const float* p, int r0, int L, int D) {
   return make_buf(p + (int64_t)r0 * D, (uint32_t)(L > r0 ? (L - r0) * D * 4 : 0));
 }
-// The same four values rounded to bf16 (round to nearest even), into a bf16 block.
-__device__ __forceinline__ void st_rows4_bf16(bufrsrc r, uint32_t vbase, uint32_t row_bytes, const f32x4& x) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) __builtin_amdgcn_raw_buffer_store_b16(f2bf(x[j]), r, vbase + j * row_bytes, 0, 0);
-}
-__device__ __forceinline__ bufrsrc rows_from_bf16(const void* p, int r0, int L, int D) {
-  return make_buf(reinterpret_cast<const bf16_t*>(p) + (int64_t)r0 * D, (uint32_t)(L > r0 ? (L - r0) * D * 2 : 0));
-}
 // Layout of a per-chunk state copy [K][V] (h, dh; only the chunk backward and the readout read them):
 // 16-column blocks, within one the 16-row tiles, within a tile the rows in the order
 // (i % 4, (i / 4) % 4), 16 columns each.  A state wave's lane (g4, c16) holds rows 16 ib + 4 g4 + j of
@@ -191,18 +183,6 @@ __device__ __forceinline__ void st_state4(void* p, int64_t e0, int ib, int g4, i
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[j]), r, hb_off<K>(16 * ib + 4 * g4 + j, col) * 4, 0, 0);
   }
 }
-// A lane's 4 D-layout values of 16-row tile `tile` (rows 4 g4 + j of column col) of the row-major
-// [rows][D] block whose element e0 is the block's first (fp32, or bf16 with B16; rows past L dropped).
-template <bool B16>
-__device__ __forceinline__ void st_tile4(void* p, int64_t e0, int tile, int L, int D, int g4, int col,
-                                         const f32x4& x) {
-  if constexpr (B16)
-    st_rows4_bf16(rows_from_bf16(reinterpret_cast<bf16_t*>(p) + e0, 16 * tile, L, D), (4 * g4 * D + col) * 2, D * 2,
-                  x);
-  else
-    st_rows4(rows_from(reinterpret_cast<float*>(p) + e0, 16 * tile, L, D), (4 * g4 * D + col) * 4, D * 4, x);
-}
-
 // A sequence of NS fragment-read + MFMA steps with the reads issued LA steps ahead, so the
 // LDS latency of step s+LA overlaps the MFMAs of step s.  rd(s, hi, lo) reads step s's A
 // fragment; mm(s, hi, lo) issues its MFMAs.  Both are fully unrolled (s is a constant).
@@ -214,6 +194,15 @@ __device__ __forceinline__ void mfma_pipe(Rd rd, Mm mm) {
     if (s < NS) rd(s, fh[s], fl[s]);
     if (s >= LA) mm(s - LA, fh[s - LA], fl[s - LA]);
   }
+}
+
+// Layout of the reverse pass's d delta copy of one chunk [C][V] (only the chunk backward reads it): 16-column
+// blocks, within one the four 16-row accumulator tiles, each as the pass's lanes hold it (lane r16 + 16 g4: the
+// rows 4 g4 .. + 3 of column r16).  A tile leaves in one 16-byte store per lane, whole 1 KB, and comes back the
+// same way as the MFMA operand d delta^T in permuted k order.  Row-major, the copy took 16 4-byte stores per
+// chunk step on the serial chain.
+__device__ __forceinline__ int dd_off(int c, int v) {
+  return (((v >> 4) * 4 + (c >> 4)) * 64 + (v & 15) + 16 * ((c >> 2) & 3)) * 4 + (c & 3);
 }
 
 // Block -> (bh, V-slice): the NV slices of one (b, h) go to one XCD (dispatch is round-robin
@@ -259,11 +248,10 @@ struct GroupPlan {
   int c0 = 0, c1 = 0;
 };
 
-// Precision of the per-chunk copies only the backward (and a separate readout) reads, as a bit mask
-// (kernel template argument): the forward pass's h (bit 0) and delta (bit 2), the reverse pass's dh
-// (bit 1) and d delta (bit 3); a set bit stores the copy in bf16 (rounded once), a clear bit in fp32.
-// The recurrences themselves stay fp32 on chip.
-enum : int { HB_H = 1, HB_DH = 2, HB_D = 4, HB_DD = 8 };
+// Precision of the per-chunk state copies only the backward (and a separate readout) reads, as a bit mask
+// (kernel template argument): the forward pass's h (bit 0), the reverse pass's dh (bit 1); a set bit stores the
+// copy in bf16 (rounded once), a clear bit in fp32.  The recurrences themselves stay fp32 on chip.
+enum : int { HB_H = 1, HB_DH = 2 };
 __device__ __forceinline__ void plan_range(const GroupPlan& P, int g, int NT, int& n0, int& n1) {
   if (P.NG == 1) {
     n0 = P.c0;
@@ -531,7 +519,7 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
         const int64_t e0 = row_bht(bh, t0, T, V);
 #pragma unroll
         for (int cb = 0; cb < 4; ++cb)
-          st_tile4<(HM & HB_D) != 0>(Dl, e0, cb, L, V, g4, col, D[cb]);  // rows past L dropped
+          st_rows4(rows_from(Dl + e0, 16 * cb, L, V), (4 * g4 * V + col) * 4, V * 4, D[cb]);  // rows past L dropped
       }
       if constexpr (RO) {  // publish the B fragments of h_n (multiplied with W above) and delta_n
 #pragma unroll
@@ -642,10 +630,9 @@ __global__ __launch_bounds__(256, 3) void readout_kernel(const float* __restrict
   // so a lane holds 4 consecutive rows of one column: 4 consecutive fragment slots of one lane,
   // written as 8 bytes of hi and 8 of lo
   {
-    constexpr int EH = (HM & HB_H) ? 2 : 4, ED = (HM & HB_D) ? 2 : 4;  // bytes per stored element
+    constexpr int EH = (HM & HB_H) ? 2 : 4;  // bytes per stored element
     const bufrsrc rh = make_buf(reinterpret_cast<const char*>(hbuf) + chunk * K * V * EH, K * V * EH);
-    const bufrsrc rd = make_buf(reinterpret_cast<const char*>(Dl) + ((int64_t)bh * T + t0) * V * ED,
-                                L * V * ED);  // rows past L read 0
+    const bufrsrc rd = make_buf(Dl + ((int64_t)bh * T + t0) * V, L * V * 4);  // rows past L read 0
     constexpr int HU = K / 16, DU = C / 16;  // 4-row blocks per wave
     const int qr = lane & 3, vq = 4 * (lane >> 2), vc = vq + qr;  // after the transpose: column vc
     float4 hx[HU], dx[DU];
@@ -665,7 +652,7 @@ __global__ __launch_bounds__(256, 3) void readout_kernel(const float* __restrict
     }
 #pragma unroll
     for (int u = 0; u < DU; ++u)
-      dx[u] = ld4h(rd, (4 * (w + 4 * u) + qr) * V + v0 + vq, std::integral_constant<bool, (HM & HB_D) != 0>{});
+      dx[u] = buf_ld4(rd, ((4 * (w + 4 * u) + qr) * V + v0 + vq) * 4);
     auto put = [&](bf16_t* buf, int nkb, int r0, const float4& x) {  // rows r0 .. r0+3 of column vc
       const float4 y = quad_transpose(x, qr);
       const int tile = (vc >> 4) * nkb + (r0 >> 5), ln = (vc & 15) + 16 * ((r0 & 31) >> 3);
@@ -1061,11 +1048,12 @@ __global__ __launch_bounds__(HW ? 2 * state_threads(V) : state_threads(V)) void 
               }
             });
       }
-      if (real) {
-        const int64_t e0 = row_bht(bh, t0, T, V);
+      if (real) {  // in the dd_off layout (rows past L are 0)
+        const bufrsrc rd = make_buf(dDl + ((int64_t)bh * NT + n) * C * V, C * V * 4);
 #pragma unroll
         for (int cb = 0; cb < 4; ++cb)
-          st_tile4<(HM & HB_DD) != 0>(dDl, e0, cb, L, V, g4, col, dD[cb]);  // rows past L dropped
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dD[cb]), rd,
+                                                 (uint32_t)(((col >> 4) * 4 + cb) * 64 + lane) * 16, 0, 0);
       }
     }
     __syncthreads();
