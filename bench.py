@@ -53,8 +53,7 @@ def kernel_counts(variant: str, B: int, T: int, H: int, K: int, V: int, infer: b
                   half_states: bool = False):
     """Algorithmic HBM bytes and FLOPs per launch of each kernel (inputs read once, outputs
     written once, no recompute).  N = B*T*H token-heads; per-token-head figures times N.  With
-    ``infer`` (no backward follows) the forward kernels skip what only the backward reads: A^T, and
-    h and delta of the fused state pass.  ``half_states``: the per-chunk state copies h and dh the
+    ``infer`` (no backward follows) the fused state pass skips what only the backward reads: h and delta.  ``half_states``: the per-chunk state copies h and dh the
     backward reads are bf16 (the isotropic scan with one chunk group)."""
     N = B * T * H
     kap_in = 4 * K if variant == "diag" else 4           # kappa fp32 [K] or beta fp32
@@ -63,27 +62,24 @@ def kernel_counts(variant: str, B: int, T: int, H: int, K: int, V: int, infer: b
     h_b = (2 if half_states else 4) * K * V / C           # one state copy per chunk
     mm = C * C / C * 4                                    # one fp32 C x C matrix per chunk
     per = {
-        # q,k,v bf16 + kappa + g fp32 -> U, W, Kf, Qg fp32 + M, A^T (the inverse, saved)
+        # q, k bf16 + kappa + g fp32 -> W, Kf, Qg fp32 + M, A (the inverse)
         # (iso: q, k raw, normalised in the kernel, and their rows' rstd written)
-        "mem_intra_fwd": (2 * 2 * K + 2 * V + kap_in + 4 * K + 4 * (V + 3 * K) + 2 * mm
-                          + (8 if variant == "iso" else 0),
-                          2 * (C * K + C * (V + K) / 2)),
-        # U, W, Kf, g_last, Qg, M -> h, delta, o  (one chunk group: the state pass does the readout)
-        "mem_state_readout_fwd": (4 * V + 8 * K + 4 * K / C + h_b + 4 * V + 4 * K + mm
+        "mem_intra_fwd": (2 * 2 * K + kap_in + 4 * K + 12 * K + 2 * mm + (8 if variant == "iso" else 0),
+                          2 * (C * K + C * K / 2)),
+        # v bf16, A, W, Kf, g_last, Qg, M -> h, delta, o  (one chunk group: the state pass does the readout)
+        "mem_state_readout_fwd": (2 * V + 12 * K + 2 * mm + 4 * K / C + h_b + 4 * V
                                   + (2 if variant == "iso" else 4) * V,
-                                  2 * 2 * K * V + 2 * (K * V + C * V / 2)),
-        # M, Kf, Qg, W, dO -> dh, d delta
-        "mem_state_bwd": (mm + 12 * K + do_b + h_b + 4 * V, 2 * (C * V / 2 + 3 * K * V)),
-        # h, dh, delta, d delta, dO, A^T, U, W, q, k, kappa, g (iso: and the q / k rstd of the in-op norm,
-        # whose backward it applies) -> dv, dq, dk, dkappa, dg (dQg, dW, dKf, dM, dKg and dN stay on chip);
-        # FLOPs: the state-gradient products, the solves and dN, the gradient contractions
-        "mem_bwd_chunk": (2 * h_b + 8 * V + do_b + mm + 4 * V + 4 * K + 2 * 2 * K + kap_in + 4 * K
+                                  2 * C * V / 2 + 2 * 2 * K * V + 2 * (K * V + C * V / 2)),
+        # M, A, Kf, Qg, W, dO -> dh, dX
+        "mem_state_bwd": (2 * mm + 12 * K + do_b + h_b + 4 * V, 2 * (2 * C * V / 2 + 3 * K * V)),
+        # h, dh, delta, dX, dO, q, k, kappa, g (iso: and the q / k rstd of the in-op norm, whose backward it
+        # applies) -> dv, dq, dk, dkappa, dg (dQg, dKg, dKf, dM and dN stay on chip);
+        # FLOPs: the products with h, dh and dX, dM and dN, the gradient contractions
+        "mem_bwd_chunk": (2 * h_b + 8 * V + do_b + 2 * 2 * K + kap_in + 4 * K
                           + 2 * V + 2 * 2 * K + dkap_out + 4 * K + (8 if variant == "iso" else 0),
-                          2 * (3 * K * V + C * V / 2) + 2 * (C * (V + K) / 2 + C * (V + K) / 2) + 2 * 2 * (C * K)),
+                          2 * (3 * K * V + C * V) + 2 * 2 * (C * K)),
     }
     if infer:
-        b, f = per["mem_intra_fwd"]
-        per["mem_intra_fwd"] = (b - mm, f)
         b, f = per["mem_state_readout_fwd"]
         per["mem_state_readout_fwd"] = (b - h_b - 4 * V, f)
     return {k: (b * N, f * N) for k, (b, f) in per.items()}
@@ -748,7 +744,7 @@ def main():
             "ms_per_step": {v: round(x, 4) for v, x in rec.items()},
             "tokens_per_s": {v: round(B * T / (x * 1e-3), 1) for v, x in rec.items()},
             "saved_bytes_save_mode": _lib_size("kdn_mem_saved_size", B, T, H, K, K),
-            "note": "forward keeps the op's inputs only (no WY factors, A^T or per-chunk states); identical gradients"}
+            "note": "forward keeps the op's inputs only (no WY factors, inverse or per-chunk states); identical gradients"}
     if not args.no_config3:
         line["also"]["config3"] = run_config3(min(args.steps, 10), args.warmup)
     if not args.no_config4:

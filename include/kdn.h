@@ -237,7 +237,8 @@ size_t kdn_mem_bwd_workspace_size(int B, int T, int H, int K, int V);
  * ranges in fp32 through `saved`, so every output is bit-identical to the stages in order.  Bits 1 and 2
  * in one call run the state pass with the readout fused.  Bit 3 (with stages >= 0) declares that
  * no backward follows (inference, as under torch.no_grad): the intermediates only the backward
- * reads are then not written, and `saved` is scratch for this call alone.  A caller that keeps no
+ * reads are then not written, and `saved` is scratch for this call alone.  v is read by the state
+ * pass (bit 1).  A caller that keeps no
  * `saved` from a training forward (the reference's policy: it re-runs recompute_w_u_fwd and the state
  * forward in its backward, iso_kdn_chunk.py:2101-2140, diag_kdn_chunk.py:3271-3277) rebuilds it for
  * kdn_mem_bwd with bit 0, then bit 1 alone (the state pass without the readout; o and final_state
@@ -259,11 +260,10 @@ int kdn_mem_fwd(const uint16_t* q, const uint16_t* k, const float* kappa_or_beta
  * inputs x the forward took, the kernels form the operand y = bf16(x rstd) again, and dq, dk are
  * returned for x: the norm's backward dx = rstd (dy - y (y . dy)) is applied to the fp32 dy in the
  * kernel (kdn_l2norm_bwd takes the bf16-rounded dy instead; the two agree to bf16 rounding).
- * `stages`: bit 0 reverse state pass, bit 1 the chunk-parallel backward, bits 2 and 3 the exact
- * path's solves and gradients for the chunks outside the factored range (-1 = all, in this order).
- * Bits 2 and 3 in one call run as one launch (each such chunk's solves, gradients and, with q_rstd, the
- * norm's backward of its rows in one workgroup), bit-identical to a call with bit 2 and then one with
- * bit 3.
+ * `stages`: bit 0 reverse state pass, bit 1 the chunk-parallel backward, bit 3 the exact path's
+ * gradients for the chunks outside the factored range (each such chunk's gradients and, with q_rstd, the
+ * norm's backward of its rows in one workgroup); -1 = all, in this order.  Bit 2 is accepted and has no
+ * work of its own (the exact path needs no separate solves).
  * Bits 0 and 1 in one call, with one chunk group (kdn_mem_state_groups == 1), at least 16 chunks
  * and at least 32 CUs the pass leaves idle (the overlapped schedule): the reverse pass runs in two
  * segments, and chunk-backward work of the first segment's chunks runs beside the second on a

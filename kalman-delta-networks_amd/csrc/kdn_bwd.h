@@ -1,11 +1,10 @@
 // Chunk-parallel backward of the KDN memory scan on bf16x3 MFMA (one kernel per chunk).
 //
-// Per chunk of C = 64 tokens (h = state entering the chunk, dh = gradient of the state leaving
-// it, delta / d delta = the chunk's delta and its gradient, A = (I + N)^{-1} saved by the forward):
-//   transposed solve         dX = A^T d delta, the gradient of X = V - Kg h (delta = A X), so dV = dX
-//   state-gradient products  dQg = dO h^T,  dKg = -dX h^T,  dKf = delta dh^T,
-//                            dM = lower(dO delta^T),  dgl_i = 2^{G_last,i} sum_v h_iv dh_iv
-//   inverse                  dN = -strict_lower(A^T (d delta X^T) A^T) = -strict_lower(dX delta^T)
+// Per chunk of C = 64 tokens (h = state entering the chunk, dh = gradient of the state leaving it,
+// delta = A X of the forward pass with X = V - Kg h and A = (I + N)^{-1}, dX = A^T d delta of the reverse pass):
+//   products                 dV = dX,  dQg = dO h^T,  dKg = -dX h^T,  dKf = delta dh^T,
+//                            dM = lower(dO delta^T),  dgl_i = 2^{G_last,i} sum_v h_iv dh_iv,
+//                            dN = -strict_lower(A^T (d delta X^T) A^T) = -strict_lower(dX delta^T)
 //   gradients                with block anchors m (below): e = 2^{G_c - m}, Lk = k e, Lq = q e,
 //                            R = kappa / e, eg = 2^{G_c}, f = 2^{G_last - G_c}
 //                            dLk = dN R,  dLq = scale dM R,  dR = dN^T Lk + scale dM^T Lq
@@ -17,6 +16,11 @@
 // m = (G_{16tl} + G_{16tl+15}) / 2 per channel (rows clamped to the chunk), for every factor it
 // contracts with, so each factor is <= 2^{span/2} on the diagonal block and <= 1 off it; the anchor
 // terms cancel exactly (N and M do not depend on the anchors) and are omitted.
+//
+// Bound by the CU's load path: per token-head (d = 128) h and dh 512 B each isotropic (1,024 diagonal), delta and
+// dX 512 each, dO, q, k 256 each and G 512.  A task's LDS (~140 KB) leaves one workgroup per CU, so nothing else
+// hides its loads.  Forming U, W, the solves' transposes and dX here as well (A^T, U, W read: 1,280 B more) it took
+// 609 us isotropic / 617 us diagonal at B4 T4096 H18, against 457 / 478.
 #pragma once
 #include "kdn_common.h"
 #include "kdn_intra.h"
@@ -73,23 +77,18 @@ __device__ __forceinline__ void upper_tile(int t, int& I, int& J) {
 // transposed solves and the gradients.  dQg, dW, dKf, dM, dKg, dN and the g_last dots never go to
 // HBM: each is produced in the register or LDS layout its consumer takes.
 // One chunk-head task of the order task = (NT - 1 - n) * B*H + bh (last chunks first, the order in
-// which the reverse state pass finishes them); block 512 (8 waves), one workgroup per CU (LDS 157 KB).
-//  * Staging.  The chunk rows of dO and delta are split into LDS fragments (rows c, k = v, natural
-//    order), all 64 rows at once; A^T goes to LDS as fp32.
-//  * Wave w owns V tile w (16 columns of V): its columns of d delta come from the reverse pass as the
-//    accumulator tiles that pass held (dd_off), two stacked tiles being a fragment in permuted k order, and
-//    give dX^T = d delta^T A (D tile: lane -> chunk row, 4 consecutive v), stored as dv and split into the
-//    row fragments of dX in LDS.
+// which the reverse state pass finishes them); block 512 (8 waves), one workgroup per CU (LDS 141 KB).
+//  * Staging.  The chunk rows of dO, delta and dX are split into LDS fragments (rows c, k = v, natural
+//    order), all 64 rows at once; delta and dX come as the state passes' accumulator tiles
+//    (kdn_state::st_tiles) and turn from columns to rows by a quad transpose, dX leaving as dv on the way.
 //  * Wave w owns channel tile it = w (16 channels of K).  It loads its 16 rows of h and of dh straight into
-//    split fragments (A operand, rows i, k = v) and forms, beside the solve,
-//      dQg^T = h dO^T,  dKf^T = dh delta^T    (D tile: lane -> chunk row, 4 consecutive channels:
-//                                              the layout of the gradient phase's elementwise terms)
-//      dgl_i = 2^{G_last,i} sum_v h_iv dh_iv,  and dM = lower(dO delta^T) for lower tiles w, w + 8;
-//    and from dX's fragments  dKg^T = -h dX^T  and  dN = -strict_lower(dX delta^T)  in the same forms.
-//    dX carries everything the inverse's gradient needs, so neither U nor W is read and no partial sum
-//    crosses the waves: as dN = -strict_lower(dV U^T + dKg W^T) the kernel read 1,024 B more per
-//    token-head (302 MB at B4 T4096 H18 d128) and summed eight waves' dN shares through LDS (step there
-//    1538 -> 1474 us isotropic, 2122 -> 2044 us diagonal).
+//    split fragments (A operand, rows i, k = v) and forms
+//      dQg^T = h dO^T,  dKg^T = -h dX^T,  dKf^T = dh delta^T    (D tile: lane -> chunk row, 4 consecutive
+//                                              channels: the layout of the gradient phase's elementwise terms)
+//      dgl_i = 2^{G_last,i} sum_v h_iv dh_iv,  and dM = lower(dO delta^T), dN = -strict_lower(dX delta^T)
+//    for lower tiles w, w + 8.  dX carries everything the inverse's gradient needs: with
+//    dN = -strict_lower(dV U^T + dKg W^T) the kernel read U, W and A^T (1,280 B more per token-head) and summed
+//    eight waves' dN shares through LDS.
 //  * Gradients.  dN, dM and their transposes are split once into LDS fragments (permuted k order:
 //    slot 4h + j of lane group g <-> k = 32 kb + 16 h + 4 g + j).  Per channel tile the factors R,
 //    Lk, Lq are built per lane for one channel and 16 chunk rows (rows outside the contraction's
@@ -97,19 +96,19 @@ __device__ __forceinline__ void upper_tile(int t, int& I, int& J) {
 //    fragments as B: the D tiles give each lane 4 consecutive channels of one chunk row, the layout
 //    of dQg, dKf and dKg, so the elementwise inputs and outputs move as 16-byte (fp32) and 8-byte
 //    (bf16) vectors.
-// Chunks flagged by the forward store the products (dQg, dW = -d delta h^T, dKf, dM, dgl) for the exact
-// kernels and stop after them.
+// Chunks flagged by the forward store the products (dQg, dKg, dKf, dM, dN, dgl) for the exact kernel and
+// stop after them.
 // ---------------------------------------------------------------------------------------------
 template <int K, int V, bool ISO, typename TDO, int HM>
 __device__ __forceinline__ void chunk_bwd_task(
     int task, const void* __restrict__ hbuf, const void* __restrict__ dhbuf, const float* __restrict__ Dl,
-    const float* __restrict__ dDl, const TDO* __restrict__ dO, const float* __restrict__ At,
-    const int* __restrict__ flags,
+    const float* __restrict__ dXl, const TDO* __restrict__ dO, const int* __restrict__ flags,
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, const float* __restrict__ q_rstd, const float* __restrict__ k_rstd, int T, int H,
     int NT, int BH, float scale, bf16_t* __restrict__ dv, bf16_t* __restrict__ dq, bf16_t* __restrict__ dk,
     float* __restrict__ dkap, float* __restrict__ dbeta, float* __restrict__ dg, float* __restrict__ xQg,
-    float* __restrict__ xW, float* __restrict__ xKf, float* __restrict__ xM, float* __restrict__ xgl) {
+    float* __restrict__ xKg, float* __restrict__ xKf, float* __restrict__ xM, float* __restrict__ xN,
+    float* __restrict__ xgl) {
   constexpr bool DO_BF16 = sizeof(TDO) == 2;
   // HM: which of h, dh were stored in bf16 (kdn_state::HB_*; the recurrences ran in fp32 and rounded
   // those copies once).  A bf16 operand enters a product without a lo half: one MFMA against another
@@ -120,16 +119,15 @@ __device__ __forceinline__ void chunk_bwd_task(
   constexpr int NW = 8;
   constexpr int VB = V / 32;        // k-blocks of the V contraction
   constexpr int NIT = K / 16;       // channel tiles (waves 0 .. NIT-1 own one each)
-  constexpr int NVT = V / 16;       // V tiles (waves 0 .. NVT-1)
   constexpr int RB = VB * TILE;     // one 16-row block of a [rows][V] operand as fragments
   constexpr int FR = 8 * TILE;      // one 64 x 64 operand as (4 row tiles x 2 k-blocks) fragments
-  constexpr int AP4 = C + 4;        // LDS row stride of A^T
-  constexpr int STAGE_BYTES = 3 * 4 * RB * 2 + C * AP4 * 4;
+  constexpr int STAGE_BYTES = 3 * 4 * RB * 2;
   constexpr int CONTRIB_BYTES = 4 * FR * 2;
   constexpr int LDS_BYTES = STAGE_BYTES > CONTRIB_BYTES ? STAGE_BYTES : CONTRIB_BYTES;
   constexpr int SU = C * V / 8 / 512;  // staging units (8 consecutive v of one row) per thread per operand
   static_assert(SU >= 1 && (C * V / 8) % 512 == 0, "staging units per thread");
-  static_assert(NIT <= NW && NVT <= NW, "K, V <= 128");
+  constexpr int TU = C * V / 4 / 512;  // tile units (4 rows of one column) of delta and of dX per thread
+  static_assert(NIT <= NW, "K <= 128");
   __shared__ __attribute__((aligned(16))) unsigned char smem[LDS_BYTES];
   __shared__ float sDgl[K];
   __shared__ float sBeta[NW * C];
@@ -139,14 +137,13 @@ __device__ __forceinline__ void chunk_bwd_task(
   bf16_t* sO = reinterpret_cast<bf16_t*>(smem);  // dO, delta, dX row fragments
   bf16_t* sD = sO + 4 * RB;
   bf16_t* sX = sD + 4 * RB;
-  float* sAt = reinterpret_cast<float*>(sX + 4 * RB);  // A^T [C][AP4]
   bf16_t* sF = reinterpret_cast<bf16_t*>(smem);  // gradients: dN, dM, dN^T, dM^T fragments
   const int n = NT - 1 - task / BH, bh = task % BH, b = bh / H, h = bh % H;
   const int t0 = n * C, L = min(C, T - t0);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
   const int64_t chunk = (int64_t)bh * NT + n;
   const bool flagged = flags[chunk] != 0;
-  const bool own_k = w < NIT, own_v = w < NVT;
+  const bool own_k = w < NIT;
   const int it = w;  // this wave's channel tile (when own_k)
   const int i0 = 16 * it + 4 * g4;
   if (q_rstd && tid < 2 * C) {  // read in the gradient phase, after phase 1's barriers
@@ -159,31 +156,19 @@ __device__ __forceinline__ void chunk_bwd_task(
   }
 
   // ================================ loads ================================
-  const int64_t row0 = ((int64_t)bh * T + t0) * V;
-  const bufrsrc rD = make_buf(Dl + row0, L * V * 4);  // rows past L read 0
   const bufrsrc rO = make_buf(dO + (((int64_t)b * T + t0) * H + h) * V, ((L - 1) * H + 1) * V * sizeof(TDO));
-  // d delta of this wave's V tile: accumulator tiles of 16 chunk rows (rows past L hold 0)
-  const float* dDn = dDl + chunk * C * V;
-  f32x4 xd[4];
+  // delta and dX: unit e = lane e % 64 of accumulator tile e / 64 (rows past L hold 0)
+  float4 td[TU], tx[TU];
 #pragma unroll
-  for (int J = 0; J < 4; ++J)
-    xd[J] = own_v ? *reinterpret_cast<const f32x4*>(dDn + ((w * 4 + J) * 64 + lane) * 4) : zero4();
-  // A^T of the chunk
-  constexpr int AU = C * C / 4 / 512;
-  float4 at_r[AU];
-  if (!flagged) {
-    const bufrsrc rA = make_buf(At + chunk * C * C, C * C * 4);
-#pragma unroll
-    for (int u = 0; u < AU; ++u) at_r[u] = buf_ld4(rA, (tid + 512 * u) * 16);
+  for (int u = 0; u < TU; ++u) {
+    td[u] = reinterpret_cast<const float4*>(Dl + chunk * C * V)[tid + 512 * u];
+    tx[u] = reinterpret_cast<const float4*>(dXl + chunk * C * V)[tid + 512 * u];
   }
-  float4 sr_D[SU][2];
   u32x4 sr_O[SU][DO_BF16 ? 1 : 2];
 #pragma unroll
   for (int u = 0; u < SU; ++u) {  // unit e: 16-row block, k-block, fragment lane
     const int e = tid + 512 * u, blk = e / (VB * 64), kb = (e / 64) % VB, sl = e & 63;
     const uint32_t c = (uint32_t)(16 * blk + (sl & 15)), v0 = (uint32_t)(32 * kb + 8 * (sl >> 4));
-    sr_D[u][0] = buf_ld4(rD, (c * V + v0) * 4);
-    sr_D[u][1] = buf_ld4(rD, (c * V + v0) * 4 + 16);
     if constexpr (DO_BF16) {
       sr_O[u][0] = __builtin_amdgcn_raw_buffer_load_b128(rO, (c * H * V + v0) * 2, 0, 0);
     } else {
@@ -274,81 +259,42 @@ __device__ __forceinline__ void chunk_bwd_task(
   for (int u = 0; u < SU; ++u) {
     const int e = tid + 512 * u, blk = e / (VB * 64), kb = (e / 64) % VB, sl = e & 63;
     const int off = blk * RB + kb * TILE + sl * 8;
-    auto put8 = [&](bf16_t* dst, const float4& x0, const float4& x1) {
+    if constexpr (DO_BF16) {  // exact in bf16: the lo half stays unused
+      *reinterpret_cast<uint4*>(sO + off) = uint4{sr_O[u][0].x, sr_O[u][0].y, sr_O[u][0].z, sr_O[u][0].w};
+    } else {
+      const float4 x0 = __builtin_bit_cast(float4, sr_O[u][0]), x1 = __builtin_bit_cast(float4, sr_O[u][1]);
       const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
       uint4 hi, lo;
       split8(x, hi, lo);
-      *reinterpret_cast<uint4*>(dst + off) = hi;
-      *reinterpret_cast<uint4*>(dst + off + 512) = lo;
-    };
-    put8(sD, sr_D[u][0], sr_D[u][1]);
-    if constexpr (DO_BF16)  // exact in bf16: the lo half stays unused
-      *reinterpret_cast<uint4*>(sO + off) = uint4{sr_O[u][0].x, sr_O[u][0].y, sr_O[u][0].z, sr_O[u][0].w};
-    else
-      put8(sO, __builtin_bit_cast(float4, sr_O[u][0]), __builtin_bit_cast(float4, sr_O[u][1]));
-  }
-  if (!flagged) {
-#pragma unroll
-    for (int u = 0; u < AU; ++u) {
-      const int e4 = tid + 512 * u, sr = e4 / (C / 4), c4 = e4 % (C / 4);
-      *reinterpret_cast<float4*>(sAt + sr * AP4 + 4 * c4) = at_r[u];
+      *reinterpret_cast<uint4*>(sO + off) = hi;
+      *reinterpret_cast<uint4*>(sO + off + 512) = lo;
     }
-  } else {  // the exact kernels take dW = -d delta h^T: the rows of d delta as fragments in dX's place
+  }
+  {
+    const bufrsrc rdv = make_buf(dv + (((int64_t)b * T + t0) * H + h) * V, ((L - 1) * H + 1) * V * 2);
 #pragma unroll
-    for (int u = 0; u < SU; ++u) {
-      const int e = tid + 512 * u, blk = e / (VB * 64), kb = (e / 64) % VB, sl = e & 63;
-      const int c = 16 * blk + (sl & 15), v0 = 32 * kb + 8 * (sl >> 4);
-      float x[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = dDn[kdn_state::dd_off(c, v0 + j)];
-      uint4 hi, lo;
-      split8(x, hi, lo);
-      *reinterpret_cast<uint4*>(sX + blk * RB + kb * TILE + sl * 8) = hi;
-      *reinterpret_cast<uint4*>(sX + blk * RB + kb * TILE + sl * 8 + 512) = lo;
+    for (int u = 0; u < TU; ++u) {  // after the transpose: row c, columns v0 .. v0 + 3
+      const int e = tid + 512 * u, tile = e >> 6, ln = e & 63;
+      const int c = 16 * (tile & 3) + 4 * (ln >> 4) + (ln & 3), v0 = 16 * (tile >> 2) + 4 * ((ln & 15) >> 2);
+      const int off = (c >> 4) * RB + (v0 >> 5) * TILE + ((c & 15) + 16 * ((v0 & 31) >> 3)) * 8 + (v0 & 7);
+      const float4 d4 = kdn_state::quad_transpose(td[u], ln & 3), x4 = kdn_state::quad_transpose(tx[u], ln & 3);
+      kdn_state::put_unit(sD, off, d4.x, d4.y, d4.z, d4.w);
+      kdn_state::put_unit(sX, off, x4.x, x4.y, x4.z, x4.w);
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2{(uint32_t)f2bf(x4.x) | ((uint32_t)f2bf(x4.y) << 16),
+                                                  (uint32_t)f2bf(x4.z) | ((uint32_t)f2bf(x4.w) << 16)},
+                                            rdv, ((uint32_t)(c * H) * V + v0) * 2, 0, 0);
     }
   }
   __syncthreads();
 
-  // ================================ phase 1: the solve, products with h, dh ================================
+  // ================================ phase 1: products with h, dh, dX ================================
   issue_qk();  // after phase 1's operands
   issue_g();
-  if (!flagged && own_v) {
-    // dX^T = d delta^T A (rows v of this wave's tile, cols s); k = chunk row c in permuted order: slot j of
-    // lane group g4 <-> c = 32 kb + 4 g4 + j (j < 4) or 32 kb + 16 + 4 g4 + (j - 4)
-    const bufrsrc rdv = make_buf(dv + (((int64_t)b * T + t0) * H + h) * V, ((L - 1) * H + 1) * V * 2);
-    f32x4 Y[4];
-#pragma unroll
-    for (int J = 0; J < 4; ++J) Y[J] = zero4();
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      uint4 xh, xl;
-      kdn_state::bfrag(xd[2 * kb], xd[2 * kb + 1], xh, xl);
-#pragma unroll
-      for (int J = 0; J < 4; ++J) {
-        if (J > 2 * kb + 1) continue;  // A[c][s] = 0 for c < s
-        const float* row = sAt + (16 * J + r16) * AP4 + 32 * kb + 4 * g4;
-        const float4 a0 = *reinterpret_cast<const float4*>(row), a1 = *reinterpret_cast<const float4*>(row + 16);
-        const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-        uint4 ah, al;
-        split8(av, ah, al);
-        Y[J] = mma3(xh, xl, ah, al, Y[J]);
-      }
-    }
-    const int v0 = 16 * w + 4 * g4;  // this lane's 4 columns of row s = 16 J + r16
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      const uint32_t lo = (uint32_t)f2bf(Y[J][0]) | ((uint32_t)f2bf(Y[J][1]) << 16);
-      const uint32_t hi = (uint32_t)f2bf(Y[J][2]) | ((uint32_t)f2bf(Y[J][3]) << 16);
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2{lo, hi}, rdv, ((uint32_t)((16 * J + r16) * H) * V + v0) * 2, 0, 0);
-      kdn_state::put_unit(sX, J * RB + (v0 >> 5) * TILE + (r16 + 16 * ((v0 & 31) >> 3)) * 8 + (v0 & 7), Y[J][0], Y[J][1],
-                          Y[J][2], Y[J][3]);
-    }
-  }
   f32x4 aQ[4], aK[4], kg[4];  // dQg^T, dKf^T, dKg^T (rows i, cols c): lane -> chunk row 16 J + r16, channels i0 ..
 #pragma unroll
   for (int tl = 0; tl < 4; ++tl) aQ[tl] = aK[tl] = kg[tl] = zero4();
-  uint4 fh[VB], fl[VB];  // h (split, or its bf16 values)
   if (own_k) {
+    uint4 fh[VB], fl[VB];  // h (split, or its bf16 values), then dh
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {
       if constexpr (LH) split8(hv[kb], fh[kb], fl[kb]);
@@ -361,9 +307,13 @@ __device__ __forceinline__ void chunk_bwd_task(
         uint4 oh, ol;
         afragx<LO_>(sO + tl * RB, kb, lane, oh, ol);
         aQ[tl] = mmx<LH, LO_>(fh[kb], fl[kb], oh, ol, aQ[tl]);
+        uint4 xh, xl;
+        afrag(sX + tl * RB, kb, lane, xh, xl);
+        kg[tl] = mmx<LH, true>(fh[kb], fl[kb], xh, xl, kg[tl]);
       }
+#pragma unroll
+    for (int tl = 0; tl < 4; ++tl) kg[tl] = -kg[tl];
     float dot = 0.f;
-    uint4 eh[VB], el[VB];  // dh
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {
       float hf[8], df[8];
@@ -373,8 +323,8 @@ __device__ __forceinline__ void chunk_bwd_task(
       if constexpr (!LDH) kdn_intra::unpack8(dhr[kb], df);
 #pragma unroll
       for (int j = 0; j < 8; ++j) dot += hf[j] * df[j];
-      if constexpr (LDH) split8(dhv[kb], eh[kb], el[kb]);
-      else eh[kb] = __builtin_bit_cast(uint4, dhr[kb]), el[kb] = uint4{0u, 0u, 0u, 0u};
+      if constexpr (LDH) split8(dhv[kb], fh[kb], fl[kb]);
+      else fh[kb] = __builtin_bit_cast(uint4, dhr[kb]), fl[kb] = uint4{0u, 0u, 0u, 0u};
     }
     dot += __shfl_xor(dot, 16, 64);
     dot += __shfl_xor(dot, 32, 64);
@@ -385,114 +335,70 @@ __device__ __forceinline__ void chunk_bwd_task(
       for (int tl = 0; tl < 4; ++tl) {
         uint4 xh, xl;
         afrag(sD + tl * RB, kb, lane, xh, xl);
-        aK[tl] = mmx<LDH, true>(eh[kb], el[kb], xh, xl, aK[tl]);
+        aK[tl] = mmx<LDH, true>(fh[kb], fl[kb], xh, xl, aK[tl]);
       }
   }
-  // dM tiles (c-block I, s-block J) = lower(dO delta^T) for lower tiles w and w + 8: mt lane -> column
-  // s = 16 J + r16, rows c = 16 I + 4 g4 + j; mtT the same tile transposed, lane -> row c = 16 I + r16,
-  // columns s = 16 J + 4 g4 + j.  Each gives one of the gradient phase's fragment forms directly.
-  f32x4 mt[2], mtT[2];
+  // dM = lower(dO delta^T) and dN = -strict_lower(dX delta^T), lower tiles (c-block I, s-block J) w and w + 8:
+  // mt, nt lane -> column s = 16 J + r16, rows c = 16 I + 4 g4 + j; mtT, ntT the same tiles transposed, lane ->
+  // row c = 16 I + r16, columns s = 16 J + 4 g4 + j.  Each gives one of the gradient phase's fragment forms.
+  f32x4 mt[2], mtT[2], nt[2], ntT[2];
 #pragma unroll
   for (int x = 0; x < 2; ++x) {
-    mt[x] = mtT[x] = zero4();
+    mt[x] = mtT[x] = nt[x] = ntT[x] = zero4();
     const int t = w + NW * x;
     if (t >= 10) continue;
     int I, J;
     lower_tile(t, I, J);
 #pragma unroll
     for (int kb = 0; kb < VB; ++kb) {
-      uint4 xh, xl, oh, ol;
+      uint4 xh, xl, oh, ol, yh, yl;
       afrag(sD + J * RB, kb, lane, xh, xl);
       afragx<LO_>(sO + I * RB, kb, lane, oh, ol);
       mt[x] = mmx<LO_, true>(oh, ol, xh, xl, mt[x]);
       mtT[x] = mmx<true, LO_>(xh, xl, oh, ol, mtT[x]);
-    }
-    if (I == J) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (r16 > 4 * g4 + j) mt[x][j] = 0.f;
-        if (4 * g4 + j > r16) mtT[x][j] = 0.f;
-      }
-    }
-  }
-
-  if (flagged) {  // the exact kernels take it from here: store the products in their layouts
-    __syncthreads();  // sDgl
-    if (own_k) {
-      const bufrsrc rQ = make_buf(xQg + ((int64_t)bh * T + t0) * K, L * K * 4);
-      const bufrsrc rW = make_buf(xW + ((int64_t)bh * T + t0) * K, L * K * 4);
-      const bufrsrc rKf = make_buf(xKf + ((int64_t)bh * T + t0) * K, L * K * 4);
-#pragma unroll
-      for (int tl = 0; tl < 4; ++tl) {
-        f32x4 aW = zero4();  // (d delta h^T)^T: rows i, cols c
-#pragma unroll
-        for (int kb = 0; kb < VB; ++kb) {
-          uint4 xh, xl;
-          afrag(sX + tl * RB, kb, lane, xh, xl);
-          aW = mmx<LH, true>(fh[kb], fl[kb], xh, xl, aW);
-        }
-        const uint32_t o = ((uint32_t)(16 * tl + r16) * K + i0) * 4;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, aQ[tl]), rQ, o, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, aK[tl]), rKf, o, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, -aW), rW, o, 0, 0);
-      }
-      if (g4 == 0) xgl[chunk * K + 16 * it + r16] = sDgl[16 * it + r16];
-    }
-    float* Mn = xM + chunk * C * C;
-#pragma unroll
-    for (int x = 0; x < 2; ++x) {
-      const int t = w + NW * x;
-      if (t >= 10) continue;
-      int I, J;
-      lower_tile(t, I, J);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) Mn[(16 * I + 4 * g4 + j) * C + 16 * J + r16] = mt[x][j];
-    }
-    if (w < 6) {  // upper tiles are zero
-      int I, J;
-      upper_tile(w, I, J);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) Mn[(16 * I + 4 * g4 + j) * C + 16 * J + r16] = 0.f;
-    }
-    return;
-  }
-  __syncthreads();  // dX's fragments are complete
-
-  // ================================ products with dX ================================
-  if (own_k) {
-#pragma unroll
-    for (int kb = 0; kb < VB; ++kb)
-#pragma unroll
-      for (int tl = 0; tl < 4; ++tl) {
-        uint4 xh, xl;
-        afrag(sX + tl * RB, kb, lane, xh, xl);
-        kg[tl] = mmx<LH, true>(fh[kb], fl[kb], xh, xl, kg[tl]);
-      }
-#pragma unroll
-    for (int tl = 0; tl < 4; ++tl) kg[tl] = -kg[tl];
-  }
-  // dN tiles = -strict_lower(dX delta^T), both forms as dM's
-  f32x4 nt[2], ntT[2];
-#pragma unroll
-  for (int x = 0; x < 2; ++x) {
-    nt[x] = ntT[x] = zero4();
-    const int t = w + NW * x;
-    if (t >= 10) continue;
-    int I, J;
-    lower_tile(t, I, J);
-#pragma unroll
-    for (int kb = 0; kb < VB; ++kb) {
-      uint4 xh, xl, yh, yl;
-      afrag(sD + J * RB, kb, lane, xh, xl);
       afrag(sX + I * RB, kb, lane, yh, yl);
       nt[x] = mma3(yh, yl, xh, xl, nt[x]);
       ntT[x] = mma3(xh, xl, yh, yl, ntT[x]);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      nt[x][j] = I == J && r16 >= 4 * g4 + j ? 0.f : -nt[x][j];
-      ntT[x][j] = I == J && 4 * g4 + j >= r16 ? 0.f : -ntT[x][j];
+      const int c = 4 * g4 + j;
+      if (I == J && r16 > c) mt[x][j] = 0.f;
+      if (I == J && c > r16) mtT[x][j] = 0.f;
+      nt[x][j] = I == J && r16 >= c ? 0.f : -nt[x][j];
+      ntT[x][j] = I == J && c >= r16 ? 0.f : -ntT[x][j];
     }
+  }
+
+  if (flagged) {  // the exact kernel takes it from here: store the products in its layouts
+    __syncthreads();  // sDgl
+    if (own_k) {
+      const bufrsrc rQ = make_buf(xQg + ((int64_t)bh * T + t0) * K, L * K * 4);
+      const bufrsrc rKg = make_buf(xKg + ((int64_t)bh * T + t0) * K, L * K * 4);
+      const bufrsrc rKf = make_buf(xKf + ((int64_t)bh * T + t0) * K, L * K * 4);
+#pragma unroll
+      for (int tl = 0; tl < 4; ++tl) {
+        const uint32_t o = ((uint32_t)(16 * tl + r16) * K + i0) * 4;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, aQ[tl]), rQ, o, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, kg[tl]), rKg, o, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, aK[tl]), rKf, o, 0, 0);
+      }
+      if (g4 == 0) xgl[chunk * K + 16 * it + r16] = sDgl[16 * it + r16];
+    }
+    float *Mn = xM + chunk * C * C, *Nn = xN + chunk * C * C;
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {  // tiles 10 .. 15: the upper ones, zero
+      const int t = w + NW * x;
+      int I, J;
+      if (t < 10) lower_tile(t, I, J);
+      else upper_tile(t - 10, I, J);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        Mn[(16 * I + 4 * g4 + j) * C + 16 * J + r16] = mt[x][j];
+        Nn[(16 * I + 4 * g4 + j) * C + 16 * J + r16] = nt[x][j];
+      }
+    }
+    return;
   }
   __syncthreads();  // every fragment read: the gradient phase's fragments may overwrite them
 
@@ -505,7 +411,6 @@ __device__ __forceinline__ void chunk_bwd_task(
 #pragma unroll
   for (int x = 0; x < 2; ++x) {  // rows form (row c, k = s) from the T tiles, transposed form (row s, k = c)
     const int t = w + NW * x;
-    if (t >= 16) continue;
     int I, J;  // tiles 10 .. 15: I < J, zero in both forms
     if (t < 10) lower_tile(t, I, J);
     else upper_tile(t - 10, I, J);
@@ -795,15 +700,15 @@ __device__ __forceinline__ void chunk_bwd_task(
 template <int K, int V, bool ISO, typename TDO, int HM>
 __global__ __launch_bounds__(512, 1) void chunk_bwd_kernel(
     const void* __restrict__ hbuf, const void* __restrict__ dhbuf, const float* __restrict__ Dl,
-    const float* __restrict__ dDl, const TDO* __restrict__ dO, const float* __restrict__ At,
-    const int* __restrict__ flags,
+    const float* __restrict__ dXl, const TDO* __restrict__ dO, const int* __restrict__ flags,
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, const float* __restrict__ q_rstd, const float* __restrict__ k_rstd, int T, int H,
     int NT, int BH, int task0, float scale, bf16_t* __restrict__ dv, bf16_t* __restrict__ dq, bf16_t* __restrict__ dk,
     float* __restrict__ dkap, float* __restrict__ dbeta, float* __restrict__ dg, float* __restrict__ xQg,
-    float* __restrict__ xW, float* __restrict__ xKf, float* __restrict__ xM, float* __restrict__ xgl) {
-  chunk_bwd_task<K, V, ISO, TDO, HM>(task0 + (int)blockIdx.x, hbuf, dhbuf, Dl, dDl, dO, At, flags, q, k, kap, gc, q_rstd,
-                                 k_rstd, T, H, NT, BH, scale, dv, dq, dk, dkap, dbeta, dg, xQg, xW, xKf, xM, xgl);
+    float* __restrict__ xKg, float* __restrict__ xKf, float* __restrict__ xM, float* __restrict__ xN,
+    float* __restrict__ xgl) {
+  chunk_bwd_task<K, V, ISO, TDO, HM>(task0 + (int)blockIdx.x, hbuf, dhbuf, Dl, dXl, dO, flags, q, k, kap, gc, q_rstd,
+                                 k_rstd, T, H, NT, BH, scale, dv, dq, dk, dkap, dbeta, dg, xQg, xKg, xKf, xM, xN, xgl);
 }
 
 }  // namespace kdn_bwd

@@ -4,9 +4,9 @@
 //   N[c,s] = sum_i k_ci kappa_si 2^{G_ci - G_si} (s < c),  M[c,s] = scale sum_i q_ci kappa_si 2^{G_ci - G_si} (s <= c)
 //   A = (I + N)^{-1}:  16x16 diagonal blocks by substitution, off-diagonal blocks level by level
 //                      A_IJ = -A_II sum_{J<=P<I} N_IP A_PJ           (fp32 MFMA)
-//   U = A V,  W = A (k 2^G),  Kf = kappa 2^{G_last - G},  Qg = scale q 2^G
+//   W = A (k 2^G),  Kf = kappa 2^{G_last - G},  Qg = scale q 2^G
 // N and M are K-contractions of factored operands (bf16x3 MFMA); the decay 2^{G_c - G_s} is split
-// at an anchor so neither factor overflows.  A^T is saved for the backward.
+// at an anchor so neither factor overflows.  The state pass forms U = A V beside its recurrence.
 //
 // intra_fwd_kernel (every chunk): one anchor per chunk and channel, the midpoint of the chunk's gate
 //   range m = (G_0 + G_{L-1}) / 2, so |G - m| <= span / 2 on every row:
@@ -24,8 +24,11 @@
 // token, spans ~370) takes the block kernel.
 //
 // Layout of work: wave w owns row block I = w (16 rows) for the N / M build, keeping its k / q
-// factors in registers and publishing its R fragments (and block anchors) to LDS; the U / W
-// products are split over the waves by output column tile.
+// factors in registers and publishing its R fragments (and block anchors) to LDS.
+//
+// HBM-bound: per token-head (d = 128) it reads q, k (512 B) and G (512), G and k again for W's operand (768, mostly
+// back from HBM), writes W, Kf, Qg (1,536), M and A (512); kappa adds 512 in the diagonal scan.  With U = A V
+// formed here too (v read, U written, 768 B more) it took 251 us at B4 T4096 H18 against 215.
 #pragma once
 #include <type_traits>
 #include "kdn_common.h"
@@ -49,7 +52,7 @@ using kdn_state::zero4;
 constexpr float kAnchorSpanMax = 200.f;
 constexpr float kBlockSpanMax = 120.f;   // base 2, per 16-token block: every product stays below 2^120
 constexpr int AP = C + 1;                // LDS row stride of the fp32 N and A tiles
-constexpr int XR = 128 + 4;              // LDS row stride of the staged [s][column] operands (<= 128 columns)
+constexpr int XR = 128 + 4;              // LDS row stride of the staged [s][channel] operand (<= 128 channels)
 
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -93,14 +96,13 @@ __device__ __forceinline__ void st8(bufrsrc r, uint32_t off, const float* f) {
                                          r, off + 16, 0, 0);
 }
 
-// Stages after the N / M build, shared by both kernels: the inverse A = (I + N)^{-1} from sN, A^T
-// saved to An, then U = A V and W = A (k 2^G) (rows past L dropped by the output descriptors).
-// The whole LDS buffer (sA / sN / sX) is free for this function's staging after the first barrier.
+// Stages after the N / M build, shared by both kernels: the inverse A = (I + N)^{-1} from sN, into sA and
+// then to An [c][s], and W = A (k 2^G) (rows past L dropped by the output descriptor).
+// The whole LDS buffer (sA / sN / sX) is free for this function's staging after A's fragments are read.
 // NORM (in-op L2 norm): k is raw in memory, sRk holds the rows' rstd.
-template <int K, int V, bool NORM>
-__device__ __forceinline__ void intra_solve_emit(float* sA, float* sN, float* sX, float* An, bufrsrc rv, bufrsrc rk,
-                                                 bufrsrc rG, bufrsrc rU, bufrsrc rW, int H, int tid,
-                                                 const float* sRk) {
+template <int K, bool NORM>
+__device__ __forceinline__ void intra_solve_emit(float* sA, const float* sN, float* sX, float* An, bufrsrc rk, bufrsrc rG,
+                                                 bufrsrc rW, int H, int tid, const float* sRk) {
   const int lane = tid & 63, w = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
   // ---- 3. diagonal blocks of A: X_I = (I + N_II)^{-1}, lane j < 16 of wave I owns column j
   if (lane < 16) {
@@ -147,18 +149,18 @@ __device__ __forceinline__ void intra_solve_emit(float* sA, float* sN, float* sX
     __syncthreads();
   }
 
-  // ---- 5. save A^T ([s][c], the orientation the backward contracts over) for the backward
+  // ---- 5. A to memory, whole rows
   {
-    const bufrsrc rA = make_buf(An, An ? C * C * 4 : 0u);  // no backward follows: nothing to save
+    const bufrsrc rA = make_buf(An, C * C * 4);
 #pragma unroll
     for (int u = 0; u < C * C / 4 / 256; ++u) {
-      const int e = 4 * (tid + 256 * u), sr = e / C, c0 = e % C;  // A^T[sr][c0 .. c0+3] = A[c0 + j][sr]
-      const float4 x = float4{sA[c0 * AP + sr], sA[(c0 + 1) * AP + sr], sA[(c0 + 2) * AP + sr], sA[(c0 + 3) * AP + sr]};
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rA, e * 4, 0, 0);
+      const int e = 4 * (tid + 256 * u);
+      const float* x = sA + (e / C) * AP + e % C;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, float4{x[0], x[1], x[2], x[3]}), rA, e * 4, 0, 0);
     }
   }
 
-  // ---- 6. U = A V, W = A (k 2^G) over output column tiles t (V/16 of U, then K/16 of W)
+  // ---- 6. W = A (k 2^G) over channel tiles t
   // A fragments in the permuted k order of the accumulator-layout B operands:
   // slots 0-3 <- s = 32 kb + 4 g4 + (0..3), slots 4-7 <- s = 32 kb + 16 + 4 g4 + (0..3)
   uint4 ah[4][2], al[4][2];
@@ -171,45 +173,35 @@ __device__ __forceinline__ void intra_solve_emit(float* sA, float* sN, float* sX
       const float x[8] = {row[0], row[1], row[2], row[3], row[16], row[17], row[18], row[19]};
       split8(x, ah[I][kb], al[I][kb]);
     }
-  // U = A V and W = A Kg (Kg = k 2^G) in transposed form: the operand (loaded coalesced as rows and
-  // staged in LDS row-major [s][col], read back by columns) is the A fragment and A's rows the B fragment, so the D
-  // tile gives each lane 4 consecutive output columns of one chunk row (16-byte stores).
+  // in transposed form: Kg = k 2^G (loaded coalesced as rows and staged in LDS row-major [s][channel], read back by
+  // columns) is the A fragment and A's rows the B fragment, so the D tile gives each lane 4 consecutive channels of
+  // one chunk row (16-byte stores).
   __syncthreads();  // every wave has its A fragments; the buffer is free
-  auto stage = [&](auto is_u) {
-    constexpr bool isU = decltype(is_u)::value;
-    constexpr int D = isU ? V : K, UNITS = C * D / 8 / 256;
 #pragma unroll
-    for (int u = 0; u < UNITS; ++u) {
-      const int e = tid + 256 * u, sr = e / (D / 8), c8 = 8 * (e % (D / 8));
-      const uint32_t o = (uint32_t)(sr * H) * D + c8;
-      float x[8];
-      if constexpr (isU) {
-        unpack8(__builtin_amdgcn_raw_buffer_load_b128(rv, o * 2, 0, 0), x);
-      } else {
-        float g[8];
-        unpack8(__builtin_amdgcn_raw_buffer_load_b128(rk, o * 2, 0, 0), x);
-        ld8(rG, o * 4, g);
-        if constexpr (NORM) {
-          const float rs = sRk[sr];
+  for (int u = 0; u < C * K / 8 / 256; ++u) {
+    const int e = tid + 256 * u, sr = e / (K / 8), c8 = 8 * (e % (K / 8));
+    const uint32_t o = (uint32_t)(sr * H) * K + c8;
+    float x[8], g[8];
+    unpack8(__builtin_amdgcn_raw_buffer_load_b128(rk, o * 2, 0, 0), x);
+    ld8(rG, o * 4, g);
+    if constexpr (NORM) {
+      const float rs = sRk[sr];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) x[j] = l2n(x[j], rs);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] *= fexp2(g[j]);
-      }
-      // row-major [s][col]: the 16 lanes of a row write consecutive 16-byte pieces (a column-major
-      // store here put 16 lanes on one bank)
-      *reinterpret_cast<float4*>(sX + sr * XR + c8) = float4{x[0], x[1], x[2], x[3]};
-      *reinterpret_cast<float4*>(sX + sr * XR + c8 + 4) = float4{x[4], x[5], x[6], x[7]};
+      for (int j = 0; j < 8; ++j) x[j] = l2n(x[j], rs);
     }
-  };
-  auto tile = [&](auto is_u, int t) {
-    constexpr bool isU = decltype(is_u)::value;
-    constexpr int D = isU ? V : K;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] *= fexp2(g[j]);
+    // row-major [s][channel]: the 16 lanes of a row write consecutive 16-byte pieces (a column-major
+    // store here put 16 lanes on one bank)
+    *reinterpret_cast<float4*>(sX + sr * XR + c8) = float4{x[0], x[1], x[2], x[3]};
+    *reinterpret_cast<float4*>(sX + sr * XR + c8 + 4) = float4{x[4], x[5], x[6], x[7]};
+  }
+  __syncthreads();
+  for (int t = w; t < K / 16; t += 4) {
     uint4 xh[2], xl[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
-      // column 16 t + r16, rows 32 kb + 4 g4 + (0..3) and + 16: with the row pitch XR = 4 (mod 64)
+      // channel 16 t + r16, rows 32 kb + 4 g4 + (0..3) and + 16: with the row pitch XR = 4 (mod 64)
       // the 64 lanes of each read fall on 64 different banks
       const float* colp = sX + (32 * kb + 4 * g4) * XR + 16 * t + r16;
       float x[8];
@@ -218,31 +210,20 @@ __device__ __forceinline__ void intra_solve_emit(float* sA, float* sN, float* sX
         x[jj] = colp[jj * XR];
         x[4 + jj] = colp[(16 + jj) * XR];
       }
-      split8(x, xh[kb], xl[kb]);  // exact for V (lo = 0)
+      split8(x, xh[kb], xl[kb]);
     }
-    const bufrsrc rO = isU ? rU : rW;
 #pragma unroll
     for (int I = 0; I < 4; ++I) {
       f32x4 acc = zero4();
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
         if (kb == 1 && I < 2) continue;  // A[c][s] = 0 for s > c
-        acc = mfma(xh[kb], ah[I][kb], acc);
-        acc = mfma(xh[kb], al[I][kb], acc);
-        if constexpr (!isU) acc = mfma(xl[kb], ah[I][kb], acc);
+        acc = mma3(xh[kb], xl[kb], ah[I][kb], al[I][kb], acc);
       }
       const uint32_t row = (uint32_t)(16 * I + r16);  // rows past L are dropped by the descriptor
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), rO,
-                                             (row * D + 16 * t + 4 * g4) * 4, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), rW, (row * K + 16 * t + 4 * g4) * 4, 0, 0);
     }
-  };
-  stage(std::true_type{});
-  __syncthreads();
-  for (int t = w; t < V / 16; t += 4) tile(std::true_type{}, t);
-  __syncthreads();
-  stage(std::false_type{});
-  __syncthreads();
-  for (int t = w; t < K / 16; t += 4) tile(std::false_type{}, t);
+  }
 }
 
 // In-op L2 norm of a chunk row held by the four lane groups of a wave (lane group g4 = lane >> 4
@@ -266,26 +247,25 @@ __device__ __forceinline__ float row_rstd(const u32x4 (&raw)[KB]) {
 }
 
 // grid (chunks, B*H), block 256: chunks n0 .. n0 + gridDim.x - 1 of every head.
-template <int K, int V, bool ISO, bool NORM = false>
+template <int K, bool ISO, bool NORM = false>
 __global__ __launch_bounds__(256, 3) void intra_fwd_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
-    const bf16_t* __restrict__ v, const float* __restrict__ gc, int T, int H, int NT, float scale,
-    float* __restrict__ U, float* __restrict__ W, float* __restrict__ Kf, float* __restrict__ Qg,
-    float* __restrict__ Mg, float* __restrict__ Ag, int* __restrict__ flags, float* __restrict__ q_rstd = nullptr,
+    const float* __restrict__ gc, int T, int H, int NT, float scale, float* __restrict__ W, float* __restrict__ Kf,
+    float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag, int* __restrict__ flags, float* __restrict__ q_rstd = nullptr,
     float* __restrict__ k_rstd = nullptr, int n0 = 0) {
   constexpr int KB = K / 32;
   // R fragments [s-tile][kb] until the N / M build, then A [c][s] in the same bytes
   constexpr int RBYTES = (C / 16) * KB * TILE * 2, ABYTES = C * AP * 4;
   constexpr int RABYTES = RBYTES > ABYTES ? RBYTES : ABYTES;
-  // [R fragments | A] then N [c][s]; the U/W stage reuses the whole buffer for its operand staging
+  // [R fragments | A] then N [c][s]; the W stage reuses the whole buffer for its operand staging
   constexpr int SBYTES = RABYTES + C * AP * 4 > C * XR * 4 ? RABYTES + C * AP * 4 : C * XR * 4;
-  static_assert(V <= 128 && K <= 128, "operand staging holds up to 128 columns");
+  static_assert(K <= 128, "operand staging holds up to 128 channels");
   __shared__ __attribute__((aligned(16))) unsigned char sbuf[SBYTES];
   __shared__ float sRk[C];  // in-op L2 norm: the rows' k rstd for the W stage
   bf16_t* sR = reinterpret_cast<bf16_t*>(sbuf);
   float* sA = reinterpret_cast<float*>(sbuf);
   float* sN = reinterpret_cast<float*>(sbuf + RABYTES);
-  float* sX = reinterpret_cast<float*>(sbuf);  // U/W stage: operand rows [s][col], pitch XR
+  float* sX = reinterpret_cast<float*>(sbuf);  // W stage: operand rows [s][channel], pitch XR
   const int n = n0 + blockIdx.x, bh = blockIdx.y, b = bh / H, h = bh % H;  // chunks n0 + gridDim.x
   const int t0 = n * C, L = min(C, T - t0);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
@@ -297,14 +277,12 @@ __global__ __launch_bounds__(256, 3) void intra_fwd_kernel(
   const bufrsrc rk = make_buf(k + in_row0 * K, rows_in * K * 2);
   const bufrsrc rq = make_buf(q + in_row0 * K, rows_in * K * 2);
   const bufrsrc rkap = ISO ? make_buf(kap + in_row0, rows_in * 4) : make_buf(kap + in_row0 * K, rows_in * K * 4);
-  const bufrsrc rv = make_buf(v + in_row0 * V, rows_in * V * 2);
   // [B*H, T, D] outputs
   const bufrsrc rKf = make_buf(Kf + ((int64_t)bh * T + t0) * K, L * K * 4);
   const bufrsrc rQg = make_buf(Qg + ((int64_t)bh * T + t0) * K, L * K * 4);
-  const bufrsrc rU = make_buf(U + ((int64_t)bh * T + t0) * V, L * V * 4);
   const bufrsrc rW = make_buf(W + ((int64_t)bh * T + t0) * K, L * K * 4);
   float* Mn = Mg + ((int64_t)bh * NT + n) * C * C;
-  float* An = Ag ? Ag + ((int64_t)bh * NT + n) * C * C : nullptr;
+  float* An = Ag + ((int64_t)bh * NT + n) * C * C;
 
   // ---- 0. the chunk's decay span max_i (G_0 - G_{L-1})_i, from rows 0 and L-1 alone, before any
   // other load or store: a chunk past the single anchor's range goes to the block-anchor kernel
@@ -336,8 +314,8 @@ __global__ __launch_bounds__(256, 3) void intra_fwd_kernel(
   const uint32_t crow = (uint32_t)(c * H), grow = (uint32_t)(min(c, L - 1) * H);
   uint4 lkh[KB], lkl[KB], lqh[KB], lql[KB];
   const float beta = ISO ? buf_ld(rkap, crow * 4) : 0.f;
-  // Kf and Qg leave through this wave's slice of the N tile's bytes (unused until stage 2): a lane's 8
-  // channels lie 32 bytes from the next lane's, so a direct store covers 16 rows in 16-byte pieces;
+  // Kf and Qg leave through this wave's slice of the N tile's bytes (unused until stage 2): a lane's
+  // 8 channels lie 32 bytes from the next lane's, so a direct store covers 16 rows in 16-byte pieces;
   // regrouped, each store writes 8 whole 128-byte row segments.  Slice: [Kf | Qg][16 rows][32 channels],
   // 16-byte quad q of row r at slot q ^ (r & 7).
   static_assert(4 * 2 * 16 * 32 * 4 <= C * AP * 4, "Kf / Qg staging fits the N tile");
@@ -409,23 +387,26 @@ __global__ __launch_bounds__(256, 3) void intra_fwd_kernel(
     *reinterpret_cast<uint4*>(sR + (w * KB + kb) * TILE + lane * 8) = rh;
     *reinterpret_cast<uint4*>(sR + (w * KB + kb) * TILE + 512 + lane * 8) = rl;
     wave_lds_sync();  // the previous column block's reads are issued before these writes
+    auto put_rows = [&](float* slice, const float* x) {  // this lane's 8 channels of row r16
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      float* slot = sKQ + r16 * 32 + (((2 * g4 + hf) ^ (r16 & 7)) * 4);
-      *reinterpret_cast<float4*>(slot) = float4{kf[4 * hf], kf[4 * hf + 1], kf[4 * hf + 2], kf[4 * hf + 3]};
-      *reinterpret_cast<float4*>(slot + 512) = float4{qg[4 * hf], qg[4 * hf + 1], qg[4 * hf + 2], qg[4 * hf + 3]};
-    }
+      for (int hf = 0; hf < 2; ++hf)
+        *reinterpret_cast<float4*>(slice + r16 * 32 + (((2 * g4 + hf) ^ (r16 & 7)) * 4)) =
+            float4{x[4 * hf], x[4 * hf + 1], x[4 * hf + 2], x[4 * hf + 3]};
+    };
+    auto st_rows = [&](const float* slice, bufrsrc r) {
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const int row = (lane >> 3) + 8 * hh, qd = lane & 7;
+        const float4 x = *reinterpret_cast<const float4*>(slice + row * 32 + ((qd ^ (row & 7)) * 4));
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r,
+                                               ((uint32_t)(16 * w + row) * K + 32 * kb + 4 * qd) * 4, 0, 0);
+      }
+    };
+    put_rows(sKQ, kf);
+    put_rows(sKQ + 512, qg);
     wave_lds_sync();
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int rr = (lane >> 3) + 8 * hh, qd = lane & 7;
-      const float* slot = sKQ + rr * 32 + ((qd ^ (rr & 7)) * 4);
-      const uint32_t off = ((uint32_t)(16 * w + rr) * K + 32 * kb + 4 * qd) * 4;
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, *reinterpret_cast<const float4*>(slot)),
-                                             rKf, off, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(
-          __builtin_bit_cast(u32x4, *reinterpret_cast<const float4*>(slot + 512)), rQg, off, 0, 0);
-    }
+    st_rows(sKQ, rKf);
+    st_rows(sKQ + 512, rQg);
   }
   __syncthreads();  // R fragments of every row block; the N tile's bytes are free again
 
@@ -456,13 +437,13 @@ __global__ __launch_bounds__(256, 3) void intra_fwd_kernel(
   }
   __syncthreads();
 
-  intra_solve_emit<K, V, NORM>(sA, sN, sX, An, rv, rk, rG, rU, rW, H, tid, sRk);
+  intra_solve_emit<K, NORM>(sA, sN, sX, An, rk, rG, rW, H, tid, sRk);
 }
 
 // LDS of the block-anchor path for one chunk (intra_fwd_block_chunk), carved from a caller's 16-byte aligned
-// pool: [R fragments | A] then N, the U/W stage reusing the whole buffer; the k rstd of the rows; the block
-// spans; the block anchors.
-template <int K, int V>
+// pool: [R fragments | A] then N, the W stage reusing the whole buffer; the k rstd of the rows; the block spans;
+// the block anchors.
+template <int K>
 struct BlockLds {
   static constexpr int KB = K / 32, RBYTES = (C / 16) * KB * TILE * 2, ABYTES = C * AP * 4;
   static constexpr int RABYTES = RBYTES > ABYTES ? RBYTES : ABYTES;
@@ -471,26 +452,24 @@ struct BlockLds {
   static_assert(SBYTES % 16 == 0, "16-byte arrays");
 };
 
-// The block-anchor path for one chunk intra_fwd_kernel flagged (block 256; lds: BlockLds<K, V>::bytes).
+// The block-anchor path for one chunk intra_fwd_kernel flagged (block 256; lds: BlockLds<K>::bytes).
 // Returns false, leaving the chunk flagged, when a 16-token block spans more than kBlockSpanMax (the exact
 // path takes it); otherwise writes the chunk's outputs and clears its flag.
-template <int K, int V, bool ISO, bool NORM>
+template <int K, bool ISO, bool NORM>
 __device__ __forceinline__ bool intra_fwd_block_chunk(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
-    const bf16_t* __restrict__ v, const float* __restrict__ gc, int T, int H, int NT, float scale,
-    float* __restrict__ U, float* __restrict__ W, float* __restrict__ Kf, float* __restrict__ Qg,
-    float* __restrict__ Mg, float* __restrict__ Ag, int* __restrict__ flags, float* __restrict__ q_rstd,
+    const float* __restrict__ gc, int T, int H, int NT, float scale, float* __restrict__ W, float* __restrict__ Kf,
+    float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag, int* __restrict__ flags, float* __restrict__ q_rstd,
     float* __restrict__ k_rstd, int n, int bh, unsigned char* lds) {
   constexpr int KB = K / 32;
-  using Lds = BlockLds<K, V>;
+  using Lds = BlockLds<K>;
   constexpr int RABYTES = Lds::RABYTES;
-  static_assert(V <= 128 && K <= 128, "operand staging holds up to 128 columns");
   unsigned char* sbuf = lds;
-  float* sRk = reinterpret_cast<float*>(lds + Lds::SBYTES);  // in-op L2 norm: the rows' k rstd for the W stage
   bf16_t* sR = reinterpret_cast<bf16_t*>(sbuf);
   float* sA = reinterpret_cast<float*>(sbuf);
   float* sN = reinterpret_cast<float*>(sbuf + RABYTES);
-  float* sX = reinterpret_cast<float*>(sbuf);  // U/W stage: operand rows [s][col], pitch XR
+  float* sX = reinterpret_cast<float*>(sbuf);  // W stage: operand rows [s][channel], pitch XR
+  float* sRk = reinterpret_cast<float*>(lds + Lds::SBYTES);  // in-op L2 norm: the rows' k rstd for the W stage
   float* sSpan = sRk + C;
   float* sMid = sSpan + 4;  // block anchors m_J per channel
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
@@ -505,14 +484,12 @@ __device__ __forceinline__ bool intra_fwd_block_chunk(
   const bufrsrc rk = make_buf(k + in_row0 * K, rows_in * K * 2);
   const bufrsrc rq = make_buf(q + in_row0 * K, rows_in * K * 2);
   const bufrsrc rkap = ISO ? make_buf(kap + in_row0, rows_in * 4) : make_buf(kap + in_row0 * K, rows_in * K * 4);
-  const bufrsrc rv = make_buf(v + in_row0 * V, rows_in * V * 2);
   // [B*H, T, D] outputs
   const bufrsrc rKf = make_buf(Kf + ((int64_t)bh * T + t0) * K, L * K * 4);
   const bufrsrc rQg = make_buf(Qg + ((int64_t)bh * T + t0) * K, L * K * 4);
-  const bufrsrc rU = make_buf(U + ((int64_t)bh * T + t0) * V, L * V * 4);
   const bufrsrc rW = make_buf(W + ((int64_t)bh * T + t0) * K, L * K * 4);
   float* Mn = Mg + ((int64_t)bh * NT + n) * C * C;
-  float* An = Ag ? Ag + ((int64_t)bh * NT + n) * C * C : nullptr;
+  float* An = Ag + ((int64_t)bh * NT + n) * C * C;
 
   // ---- 0. block anchors m_J = (G_{16J} + G_{16J+15}) / 2 per channel (rows clamped to the chunk)
   // and the block spans; a chunk with a span past kBlockSpanMax stays for the exact kernel
@@ -647,7 +624,7 @@ __device__ __forceinline__ bool intra_fwd_block_chunk(
   }
   __syncthreads();
 
-  intra_solve_emit<K, V, NORM>(sA, sN, sX, An, rv, rk, rG, rU, rW, H, tid, sRk);
+  intra_solve_emit<K, NORM>(sA, sN, sX, An, rk, rG, rW, H, tid, sRk);
   if (tid == 0) flags[lin] = 0;
   return true;
 }

@@ -9,20 +9,21 @@
 // the returned dg is the cotangent in these natural-log coordinates (not reverse-summed):
 //   N[c,s] = sum_i k_ci kappa_si e^{g_ci - g_si}   (s < c)       (write interactions)
 //   M[c,s] = scale sum_i q_ci kappa_si e^{g_ci - g_si}   (s <= c) (readout interactions)
-//   U = (I+N)^-1 V,  W = (I+N)^-1 (K e^g),  Kf = kappa e^{g_last - g},  Qg = scale Q e^g
+//   A = (I+N)^-1,  U = A V,  W = A (K e^g),  Kf = kappa e^{g_last - g},  Qg = scale Q e^g
 //   delta = U - W S_0,  O = Qg S_0 + M delta,  S_C = e^{g_last} S_0 + Kf^T delta
 //
 // Kernels (grid = one workgroup per chunk unless noted, 256 threads = 4 waves):
 //   intra_fwd    N/M (MFMA, one anchor per chunk, then one per 16-token block for the chunks
-//                that need it), forward substitution for U, W; Kf, Qg
+//                that need it), the inverse A; W, Kf, Qg
 //   state_fwd    serial over chunks, one workgroup per (V-slice, b, h): h per chunk, delta
 //   readout      chunk-parallel O = Qg h + M delta (kdn_state.h)
-//   state_bwd    serial reverse (kdn_state.h): d delta = M^T dO + Kf dS;  dS <- e dS + Qg^T dO - W^T d delta
-//   chunk_bwd    (kdn_bwd.h, 512 threads) per chunk: dV = (I+N)^-T d delta, dQg = dO h^T, dKg = -dV h^T,
-//                dKf = delta dh^T, dM = dO delta^T, dN = -dV delta^T, g_last terms; dq, dk, dkappa
-//                (or dbeta), dg from dN, dM and the elementwise factors
-//   *_exact      the chunks the forward flagged: the same backward by per-block anchors and scalar
-//                substitution (the products above come from chunk_bwd through HBM)
+//   state_bwd    serial reverse (kdn_state.h): d delta = M^T dO + Kf dS;  dX = A^T d delta;
+//                dS <- e dS + Qg^T dO - W^T d delta
+//   chunk_bwd    (kdn_bwd.h, 512 threads) per chunk: dV = dX, dQg = dO h^T, dKg = -dX h^T, dKf = delta dh^T,
+//                dM = dO delta^T, dN = -dX delta^T, g_last terms; dq, dk, dkappa (or dbeta), dg from dN, dM
+//                and the elementwise factors
+//   *_exact      the chunks the forward flagged: the same gradients by per-block anchors and per-element
+//                blocks (the products above come from chunk_bwd through HBM)
 //
 // g is kept in the base-2 units of g_cumsum, so e^{g_c - g_s} = exp2(G_c - G_s).
 // Decay factors (c >= s) are split at the start a of the row block (16 tokens):
@@ -283,24 +284,23 @@ __device__ void build_NM(const float* sQ, const float* sK, const float* sA, cons
 // Exact path for one chunk (per-block decay anchors, per-element diagonal blocks when a
 // block's span exceeds kSpanMax, scalar forward substitution).  Runs only for the chunks the
 // MFMA kernels (kdn_intra.h) leave flagged: a 16-token block spans more than their block-anchor range.
-// lds: ExactFwdLds<K, V>::bytes of a caller's 16-byte aligned pool.
-template <int K, int V>
+// lds: ExactFwdLds<K>::bytes of a caller's 16-byte aligned pool.
+template <int K>
 struct ExactFwdLds {
-  static constexpr int KP = K + 4, XP = V + K + 4;
+  static constexpr int KP = K + 4, XP = C + K + 4;
   static constexpr int OFF2 = (2 * C * KP > C * XP) ? 2 * C * KP : C * XP;
   static constexpr int bytes = (OFF2 + 2 * C * KP + C * NS + 4) * 4;
 };
-template <int K, int V, bool ISO>
+template <int K, bool ISO>
 __device__ void intra_fwd_exact_chunk(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
-    const bf16_t* __restrict__ v, const float* __restrict__ gc, int T, int H, int NT, float scale,
-    float* __restrict__ U, float* __restrict__ W, float* __restrict__ Kf, float* __restrict__ Qg,
-    float* __restrict__ Mg, float* __restrict__ Ag, int n, int bh, float* __restrict__ q_rstd,
+    const float* __restrict__ gc, int T, int H, int NT, float scale, float* __restrict__ W, float* __restrict__ Kf,
+    float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag, int n, int bh, float* __restrict__ q_rstd,
     float* __restrict__ k_rstd, unsigned char* lds) {
   constexpr int KP = K + 4;
-  constexpr int XP = V + K + 4;
+  constexpr int XP = ExactFwdLds<K>::XP;
   // sQ | sA are dead after Kf / Qg are written and are then reused for the solve's sX [C][XP]
-  constexpr int OFF2 = ExactFwdLds<K, V>::OFF2;
+  constexpr int OFF2 = ExactFwdLds<K>::OFF2;
   float* sBuf = reinterpret_cast<float*>(lds);
   float* sN = sBuf + OFF2 + 2 * C * KP;  // transposed: sN[s * NS + c] = N[c][s]
   float* sSpan = sN + C * NS;
@@ -327,22 +327,17 @@ __device__ void intra_fwd_exact_chunk(
     }
   }
   __syncthreads();
-  // forward substitution (I+N) X = [V | K e^g], thread = column; 16-row blocks
-  if (tid < V + K) {
-    const int j = tid;
-    const bool isV = j < V;
-    const int col = isV ? j : j - V;
-    float* dst = isV ? U : W;
-    const int D = isV ? V : K;
+  // forward substitution (I+N) X = [I | K e^g], thread = column (rows past L of N are zero); 16-row blocks
+  if (tid < C + K) {
+    const int j = tid, col = j - C;  // col < 0: column j of A
+    float* dA = Ag + ((int64_t)bh * NT + n) * C * C;
 #pragma unroll 1
     for (int I = 0; I < 4; ++I) {
       float acc[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int c = 16 * I + r;
-        float x = 0.f;
-        if (c < L) x = isV ? bf2f(v[bthk(b, t0 + c, h, col, T, H, V)]) : sK[c * KP + col] * exp2f(sG[c * KP + col]);
-        acc[r] = x;
+        acc[r] = col < 0 ? (c == j ? 1.f : 0.f) : c < L ? sK[c * KP + col] * exp2f(sG[c * KP + col]) : 0.f;
       }
 #pragma unroll 1
       for (int s = 0; s < 16 * I; ++s) {
@@ -366,7 +361,8 @@ __device__ void intra_fwd_exact_chunk(
       for (int r = 0; r < 16; ++r) {
         const int c = 16 * I + r;
         sX[c * XP + j] = acc[r];
-        if (c < L) dst[bht(bh, t0 + c, T, D) + col] = acc[r];
+        if (col < 0) dA[c * C + j] = acc[r];
+        else if (c < L) W[bht(bh, t0 + c, T, K) + col] = acc[r];
       }
     }
   }
@@ -387,14 +383,13 @@ __device__ __forceinline__ bool any_flagged(const int* __restrict__ flags, int N
 // Each flagged chunk takes the block-anchor path, and the exact path when that leaves it flagged, in the same
 // workgroup; the two paths' LDS arrays share one pool (one workgroup per CU).  A workgroup first loads all its
 // chunks' flags at once and exits when none is set.  One launch for both paths.
-template <int K, int V, bool ISO, bool NORM>
+template <int K, bool ISO, bool NORM>
 __global__ __launch_bounds__(256) void intra_fwd_flagged_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
-    const bf16_t* __restrict__ v, const float* __restrict__ gc, int T, int H, int NT, int BH, int n0, int n1,
-    float scale, float* __restrict__ U, float* __restrict__ W, float* __restrict__ Kf, float* __restrict__ Qg,
-    float* __restrict__ Mg, float* __restrict__ Ag, int* __restrict__ flags, float* __restrict__ q_rstd,
-    float* __restrict__ k_rstd) {
-  constexpr int LB = kdn_intra::BlockLds<K, V>::bytes, LE = ExactFwdLds<K, V>::bytes;
+    const float* __restrict__ gc, int T, int H, int NT, int BH, int n0, int n1, float scale, float* __restrict__ W,
+    float* __restrict__ Kf, float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag,
+    int* __restrict__ flags, float* __restrict__ q_rstd, float* __restrict__ k_rstd) {
+  constexpr int LB = kdn_intra::BlockLds<K>::bytes, LE = ExactFwdLds<K>::bytes;
   __shared__ __attribute__((aligned(16))) unsigned char lds[LB > LE ? LB : LE];
   const int len = n1 - n0, N = BH * len;
   int any = 0;
@@ -405,141 +400,21 @@ __global__ __launch_bounds__(256) void intra_fwd_flagged_kernel(
     const int bh = i / len, n = n0 + i % len;
     if (flags[(int64_t)bh * NT + n] == 0) continue;
     __syncthreads();  // LDS of the previous chunk is dead
-    if (!kdn_intra::intra_fwd_block_chunk<K, V, ISO, NORM>(q, k, kap, v, gc, T, H, NT, scale, U, W, Kf, Qg, Mg, Ag,
-                                                           flags, q_rstd, k_rstd, n, bh, lds)) {
+    if (!kdn_intra::intra_fwd_block_chunk<K, ISO, NORM>(q, k, kap, gc, T, H, NT, scale, W, Kf, Qg, Mg, Ag, flags,
+                                                        q_rstd, k_rstd, n, bh, lds)) {
       __syncthreads();  // the block path's span reads are done
-      intra_fwd_exact_chunk<K, V, ISO>(q, k, kap, v, gc, T, H, NT, scale, U, W, Kf, Qg, Mg, Ag, n, bh, q_rstd, k_rstd,
-                                       lds);
+      intra_fwd_exact_chunk<K, ISO>(q, k, kap, gc, T, H, NT, scale, W, Kf, Qg, Mg, Ag, n, bh, q_rstd, k_rstd, lds);
     }
   }
 }
 
-// ===========================================================================
-// Backward: transposed triangular solves and dN.
-// ===========================================================================
-// LDS bytes of the two exact backward steps (their arrays are carved from a caller's 16-byte aligned pool,
-// so one kernel can run both on the same bytes).  Every array size is a multiple of 4 floats.
-template <int K, int V>
+// LDS bytes of the exact backward (its arrays are carved from a caller's 16-byte aligned pool).
+template <int K>
 struct ExactLds {
-  static constexpr int KP = K + 4, XP = V + K + 4, P1 = 3 * C * KP, P2 = 2 * C * XP, R1 = P1 > P2 ? P1 : P2;
+  static constexpr int KP = K + 4;
   static constexpr int KQ = K + 8;  // QKStride<K, bf16_t>
-  static constexpr int solve = (R1 + C * NS + 4) * 4;
-  static constexpr int contrib = 2 * C * KQ * 2 + (2 * C * KP + 2 * C * NS + 4 + 5 * K + C * (K / 16)) * 4;
-  static constexpr int both = solve > contrib ? solve : contrib;
+  static constexpr int bytes = 2 * C * KQ * 2 + (2 * C * KP + 2 * C * NS + 4 + 5 * K + C * (K / 16)) * 4;
 };
-
-// Exact path for one chunk (rebuilds N with per-block anchors, scalar back substitution); runs
-// only for the chunks the forward flagged as outside the single-anchor range.  lds: ExactLds::solve bytes.
-template <int K, int V, bool ISO>
-__device__ void bwd_solve_exact_chunk(
-    const bf16_t* __restrict__ k, const float* __restrict__ kap, const float* __restrict__ gc,
-    const float* __restrict__ dDl, const float* __restrict__ dWg, const float* __restrict__ U,
-    const float* __restrict__ W, int T, int H, int NT, bf16_t* __restrict__ dv, float* __restrict__ dKg,
-    float* __restrict__ dNg, int n, int bh, const float* __restrict__ k_rstd, unsigned char* lds) {
-  constexpr int KP = K + 4;
-  constexpr int XP = V + K + 4;
-  // phase 1: sK | sA | sG (3 x C x KP); phase 2 (after the solve) reuses it as sX | sUW (2 x C x XP)
-  constexpr int R1 = ExactLds<K, V>::R1;
-  float* sBuf = reinterpret_cast<float*>(lds);
-  float* sN = sBuf + R1;
-  float* sSpan = sN + C * NS;
-  float* sK = sBuf;
-  float* sA = sBuf + C * KP;
-  float* sG = sBuf + 2 * C * KP;
-  const int b = bh / H, h = bh % H;
-  const int t0 = n * C, L = min(C, T - t0);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  stage_chunk<K, ISO, float>(nullptr, k, kap, gc, b, h, T, H, t0, L, (float*)nullptr, sK, sA, sG, sSpan, nullptr,
-                             k_rstd);
-  build_NM<K, false, false>(nullptr, sK, sA, sG, sSpan, 0.f, sN, nullptr);
-  __syncthreads();  // sK / sA / sG are dead from here on; sX reuses their space
-  float* sX = sBuf;
-  float* sUW = sBuf + C * XP;
-  // back substitution (I+N)^T X = [d delta | dW], thread = column; 16-row blocks, last first
-  if (tid < V + K) {
-    const int j = tid;
-    const bool isV = j < V;
-    const int col = isV ? j : j - V;
-#pragma unroll 1
-    for (int I = 3; I >= 0; --I) {
-      float acc[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int c = 16 * I + r;
-        float x = 0.f;
-        if (c < L)
-          x = isV ? dDl[((int64_t)bh * NT + n) * C * V + kdn_state::dd_off(c, col)] : dWg[bht(bh, t0 + c, T, K) + col];
-        acc[r] = x;
-      }
-#pragma unroll 1
-      for (int s = 16 * (I + 1); s < C; ++s) {
-        const float xs = sX[s * XP + j];
-        const float4* nrow = reinterpret_cast<const float4*>(sN + s * NS + 16 * I);
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          const float4 nv = nrow[r4];
-          acc[4 * r4 + 0] -= nv.x * xs;
-          acc[4 * r4 + 1] -= nv.y * xs;
-          acc[4 * r4 + 2] -= nv.z * xs;
-          acc[4 * r4 + 3] -= nv.w * xs;
-        }
-      }
-#pragma unroll
-      for (int r = 14; r >= 0; --r) {
-#pragma unroll
-        for (int r2 = r + 1; r2 < 16; ++r2) acc[r] -= sN[(16 * I + r2) * NS + 16 * I + r] * acc[r2];
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int c = 16 * I + r;
-        sX[c * XP + j] = acc[r];
-        if (c < L) {
-          if (isV) dv[bthk(b, t0 + c, h, col, T, H, V)] = f2bf(acc[r]);
-          else dKg[bht(bh, t0 + c, T, K) + col] = acc[r];
-        }
-      }
-    }
-  }
-  // stage [U | W] rows for dN
-  stage_f32<C, V, XP>(U + bht(bh, t0, T, V), V, L, sUW);
-  stage_f32<C, K, XP>(W + bht(bh, t0, T, K), K, L, sUW + V);
-  __syncthreads();
-  // dN = -(X [U|W]^T), strictly lower
-  float* dNn = dNg + ((int64_t)bh * NT + n) * C * C;
-  for (int tile = w; tile < 16; tile += 4) {
-    const int I = tile >> 2, J = tile & 3;
-    f32x4 acc = zero4();
-    if (J <= I) {
-      const int cA = 16 * I + (lane & 15), sB = 16 * J + (lane & 15);
-#pragma unroll 8
-      for (int st = 0; st < (V + K) / 4; ++st) {
-        const int jj = 4 * st + (lane >> 4);
-        acc = mfma4(sX[cA * XP + jj], sUW[sB * XP + jj], acc);
-      }
-    }
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int c = 16 * I + 4 * (lane >> 4) + jj, s = 16 * J + (lane & 15);
-      dNn[c * C + s] = (s < c) ? -acc[jj] : 0.f;
-    }
-  }
-}
-
-template <int K, int V, bool ISO>
-__global__ __launch_bounds__(256) void mem_bwd_solve_exact_kernel(
-    const bf16_t* __restrict__ k, const float* __restrict__ kap, const float* __restrict__ gc,
-    const float* __restrict__ dDl, const float* __restrict__ dWg, const float* __restrict__ U,
-    const float* __restrict__ W, int T, int H, int NT, int NB, const int* __restrict__ flags, bf16_t* __restrict__ dv,
-    float* __restrict__ dKg, float* __restrict__ dNg, const float* __restrict__ k_rstd) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[ExactLds<K, V>::solve];
-  if (!any_flagged(flags, NB)) return;
-  for (int lin = blockIdx.x; lin < NB; lin += gridDim.x) {
-    if (flags[lin] == 0) continue;
-    __syncthreads();
-    bwd_solve_exact_chunk<K, V, ISO>(k, kap, gc, dDl, dWg, U, W, T, H, NT, dv, dKg, dNg, lin % NT, lin / NT, k_rstd,
-                                     lds);
-  }
-}
 
 // ===========================================================================
 // Backward, exact path for one chunk: gradients of q, k, kappa (beta) and g from dN, dM and
@@ -547,7 +422,7 @@ __global__ __launch_bounds__(256) void mem_bwd_solve_exact_kernel(
 // for the chunks the forward flagged.  Output tile (row block I, 16 channels); lane holds
 // rows 16I + 4(lane/16) + j.
 // ===========================================================================
-template <int K, int V, bool ISO>
+template <int K, bool ISO>
 __device__ void bwd_contrib_exact_chunk(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, const float* __restrict__ dNg, const float* __restrict__ dMg,
@@ -558,8 +433,7 @@ __device__ void bwd_contrib_exact_chunk(
   constexpr int KP = K + 4;
   constexpr int NCT = K / 16;  // channel tiles
   constexpr int KQ = QKStride<K, bf16_t>::value;
-  static_assert(KQ == ExactLds<K, V>::KQ, "staged q / k stride");
-  // lds: ExactLds::contrib bytes
+  static_assert(KQ == ExactLds<K>::KQ, "staged q / k stride");
   bf16_t* sQ = reinterpret_cast<bf16_t*>(lds);  // bf16 inputs are exact in bf16
   bf16_t* sK = sQ + C * KQ;
   float* sA = reinterpret_cast<float*>(sK + C * KQ);
@@ -717,24 +591,6 @@ __device__ void bwd_contrib_exact_chunk(
   }
 }
 
-template <int K, int V, bool ISO>
-__global__ __launch_bounds__(256) void mem_bwd_contrib_exact_kernel(
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
-    const float* __restrict__ gc, const float* __restrict__ dNg, const float* __restrict__ dMg,
-    const float* __restrict__ dQg, const float* __restrict__ dKg, const float* __restrict__ dKf,
-    const float* __restrict__ dgl, int T, int H, int NT, int NB, const int* __restrict__ flags, float scale,
-    bf16_t* __restrict__ dq, bf16_t* __restrict__ dk, float* __restrict__ dkap, float* __restrict__ dbeta,
-    float* __restrict__ dg, const float* __restrict__ q_rstd, const float* __restrict__ k_rstd) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[ExactLds<K, V>::contrib];
-  if (!any_flagged(flags, NB)) return;
-  for (int lin = blockIdx.x; lin < NB; lin += gridDim.x) {
-    if (flags[lin] == 0) continue;
-    __syncthreads();
-    bwd_contrib_exact_chunk<K, V, ISO>(q, k, kap, gc, dNg, dMg, dQg, dKg, dKf, dgl, T, H, NT, scale, dq, dk, dkap,
-                                       dbeta, dg, lin % NT, lin / NT, q_rstd, k_rstd, lds);
-  }
-}
-
 // The in-op L2 norm's backward for the rows of the flagged chunks (whose dq, dk the exact kernel
 // above wrote for the normalised operands y = bf16(x rstd) of the raw q, k): dx = rstd (dy - y (y . dy)),
 // in place.
@@ -768,41 +624,25 @@ __device__ void l2norm_bwd_chunk_rows(const bf16_t* __restrict__ q, const bf16_t
     }
   }
 }
-template <int K>
-__global__ __launch_bounds__(256) void l2norm_bwd_flagged_kernel(
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ q_rstd,
-    const float* __restrict__ k_rstd, int T, int H, int NT, int NB, const int* __restrict__ flags,
-    bf16_t* __restrict__ dq, bf16_t* __restrict__ dk) {
-  if (!any_flagged(flags, NB)) return;
-  for (int lin = blockIdx.x; lin < NB; lin += gridDim.x)
-    if (flags[lin] != 0) l2norm_bwd_chunk_rows<K>(q, k, q_rstd, k_rstd, T, H, lin % NT, lin / NT, dq, dk);
-}
-
-// The whole exact backward of each flagged chunk in one workgroup: the solves (dv, dKg, dN), then the
-// gradients from them, then (in-op norm) the norm's backward of its q, k rows.  Each step reads only what
-// the previous ones wrote for the same chunk; the barrier between steps orders those global writes before
-// the next step's reads (the workgroup's waves share one CU's caches), and the steps' LDS arrays share one
-// pool.  One launch instead of the two or three a call with both exact stages would make.
-template <int K, int V, bool ISO>
+// The exact backward of each flagged chunk in one workgroup: the gradients from the products the chunk backward
+// left in HBM, then (in-op norm) the norm's backward of its q, k rows; the barrier between the two orders those
+// global writes before its reads (the workgroup's waves share one CU's caches).
+template <int K, bool ISO>
 __global__ __launch_bounds__(256) void mem_bwd_exact_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
-    const float* __restrict__ gc, const float* __restrict__ dDl, const float* __restrict__ dWg,
-    const float* __restrict__ U, const float* __restrict__ W, const float* __restrict__ dMg,
-    const float* __restrict__ dQg, const float* __restrict__ dKf, const float* __restrict__ dgl, int T, int H, int NT,
-    int NB, const int* __restrict__ flags, float scale, bf16_t* __restrict__ dv, float* __restrict__ dKg,
-    float* __restrict__ dNg, bf16_t* __restrict__ dq, bf16_t* __restrict__ dk, float* __restrict__ dkap,
-    float* __restrict__ dbeta, float* __restrict__ dg, const float* __restrict__ q_rstd,
-    const float* __restrict__ k_rstd) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[ExactLds<K, V>::both];
+    const float* __restrict__ gc, const float* __restrict__ dNg, const float* __restrict__ dMg,
+    const float* __restrict__ dQg, const float* __restrict__ dKg, const float* __restrict__ dKf,
+    const float* __restrict__ dgl, int T, int H, int NT, int NB, const int* __restrict__ flags, float scale,
+    bf16_t* __restrict__ dq, bf16_t* __restrict__ dk, float* __restrict__ dkap, float* __restrict__ dbeta,
+    float* __restrict__ dg, const float* __restrict__ q_rstd, const float* __restrict__ k_rstd) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[ExactLds<K>::bytes];
   if (!any_flagged(flags, NB)) return;
   for (int lin = blockIdx.x; lin < NB; lin += gridDim.x) {
     if (flags[lin] == 0) continue;
     const int n = lin % NT, bh = lin / NT;
     __syncthreads();
-    bwd_solve_exact_chunk<K, V, ISO>(k, kap, gc, dDl, dWg, U, W, T, H, NT, dv, dKg, dNg, n, bh, k_rstd, lds);
-    __syncthreads();
-    bwd_contrib_exact_chunk<K, V, ISO>(q, k, kap, gc, dNg, dMg, dQg, dKg, dKf, dgl, T, H, NT, scale, dq, dk, dkap,
-                                       dbeta, dg, n, bh, q_rstd, k_rstd, lds);
+    bwd_contrib_exact_chunk<K, ISO>(q, k, kap, gc, dNg, dMg, dQg, dKg, dKf, dgl, T, H, NT, scale, dq, dk, dkap, dbeta, dg,
+                                    n, bh, q_rstd, k_rstd, lds);
     if (q_rstd) {
       __syncthreads();
       l2norm_bwd_chunk_rows<K>(q, k, q_rstd, k_rstd, T, H, n, bh, dq, dk);
@@ -872,36 +712,34 @@ inline void with_copy_mask(int hm, F f) {
 
 // saved-buffer layout (floats), TT = B*H*T, NB = B*H*NT
 struct MemLayout {
-  int64_t U, W, Kf, Qg, M, A, h, D, flags, grp, mid, total;
+  int64_t W, Kf, Qg, M, A, h, D, flags, grp, mid, total;
   GroupCount gc;
   MemLayout(int B, int T, int H, int K, int V) {
     const int64_t TT = (int64_t)B * H * T, NB = (int64_t)B * H * cdiv(T, C);
     gc = plan_groups(B * H, cdiv(T, C), K, V);
-    U = 0;
-    W = U + TT * V;
+    W = 0;
     Kf = W + TT * K;
     Qg = Kf + TT * K;
     M = Qg + TT * K;
     A = M + NB * C * C;
     h = A + NB * C * C;
     D = h + NB * K * V;
-    flags = D + TT * V;  // NB ints: chunk taken by the exact intra-chunk path
+    flags = D + NB * C * V;  // (D: whole accumulator tiles, kdn_state::st_tiles)  NB ints: chunk taken by the exact intra-chunk path
     grp = round64(flags + NB);  // the forward state pass's group buffers (dead after the forward)
     mid = grp + group_floats((int64_t)B * H, gc, K, V);  // the overlapped forward's carried state
     total = mid + (int64_t)B * H * K * V;
   }
 };
 struct BwdLayout {
-  int64_t dh, dD, dQg, dW, dKf, dM, dgl, dKg, dN, carry, grp, total;
+  int64_t dh, dX, dQg, dKf, dM, dgl, dKg, dN, carry, grp, total;
   GroupCount gc;
   BwdLayout(int B, int T, int H, int K, int V) {
     const int64_t TT = (int64_t)B * H * T, NB = (int64_t)B * H * cdiv(T, C);
     gc = plan_groups(B * H, cdiv(T, C), K, V);
     dh = 0;
-    dD = dh + NB * K * V;
-    dQg = dD + NB * C * V;  // whole accumulator tiles (kdn_state::dd_off)
-    dW = dQg + TT * K;
-    dKf = dW + TT * K;
+    dX = dh + NB * K * V;
+    dQg = dX + NB * C * V;  // whole accumulator tiles (kdn_state::st_tiles)
+    dKf = dQg + TT * K;
     dM = dKf + TT * K;
     dgl = dM + NB * C * C;
     dKg = dgl + NB * K;
@@ -920,9 +758,11 @@ struct BwdLayout {
 // workgroups take the CUs the first one frees (the side launch starts a few microseconds later), and
 // the side launch's workgroups fill the idle CUs and backfill them as they finish.  The remaining
 // tasks run at full width after the pass.  A chunk-backward task lasts about kStepsPerTask chunk
-// steps of the pass running beside it (~36 us against ~5.7 us), which sizes the first segment so
-// that its tasks keep the idle CUs busy until the pass ends.
-constexpr float kStepsPerTask = 6.4f;
+// steps of the pass running beside it (~26 us against ~5.2 us), which sizes the first segment so
+// that its tasks keep the idle CUs busy until the pass ends and the remaining tasks fill the last
+// round of 256 CUs: at B4 T4096 H18 d128, 5.0 gives 1,120 side tasks and 13.6 main rounds (whole step
+// 1377 us isotropic, 1956 diagonal), 5.3 to 6.4 give 1,008 and 14.06 (1405 / 1980).
+constexpr float kStepsPerTask = 5.0f;
 constexpr unsigned kSideDelayTicks = 300;  // of the 100 MHz wall clock: 3 us
 struct BwdOverlap {
   int m1 = 0, side_tasks = 0;
@@ -1036,14 +876,12 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
                  float* q_rstd, float* k_rstd, int stages, hipStream_t stream) {
   const int NT = cdiv(T, C);
   MemLayout lay(B, T, H, K, V);
-  float *U = saved + lay.U, *W = saved + lay.W, *Kf = saved + lay.Kf, *Qg = saved + lay.Qg, *M = saved + lay.M,
-        *A = saved + lay.A, *hb = saved + lay.h, *D = saved + lay.D;
+  float *W = saved + lay.W, *Kf = saved + lay.Kf, *Qg = saved + lay.Qg, *M = saved + lay.M, *A = saved + lay.A,
+        *hb = saved + lay.h, *D = saved + lay.D;
   int* flags = reinterpret_cast<int*>(saved + lay.flags);
   const int hm = half_copies(iso, lay.gc);
-  // bit 3 (stages >= 0): no backward follows, so A^T and, where the readout is fused, h and delta
-  // are not written
+  // bit 3 (stages >= 0): no backward follows, so where the readout is fused h and delta are not written
   const bool infer = stages >= 0 && (stages & 8) != 0;
-  float* Asave = infer ? nullptr : A;
   // the intra-chunk build of chunks n0 .. n1 - 1 on stream s: the single-anchor kernel, then one launch for the
   // chunks it flagged (the block-anchor path, and the exact path for those it leaves flagged)
   auto launch_intra = [&](int n0, int n1, hipStream_t s) {
@@ -1053,10 +891,10 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
     // plain kernels registers
 #define KDN_INTRA(ISO_, NORM_)                                                                                         \
   do {                                                                                                                 \
-    hipLaunchKernelGGL((kdn_intra::intra_fwd_kernel<K, V, ISO_, NORM_>), gchunk, dim3(256), 0, s, q, k, kap, v, gc, T, \
-                       H, NT, scale, U, W, Kf, Qg, M, Asave, flags, q_rstd, k_rstd, n0);                               \
-    hipLaunchKernelGGL((intra_fwd_flagged_kernel<K, V, ISO_, NORM_>), dim3(gx), dim3(256), 0, s, q, k, kap, v, gc, T,  \
-                       H, NT, B * H, n0, n1, scale, U, W, Kf, Qg, M, Asave, flags, q_rstd, k_rstd);                  \
+    hipLaunchKernelGGL((kdn_intra::intra_fwd_kernel<K, ISO_, NORM_>), gchunk, dim3(256), 0, s, q, k, kap, gc, T, H,    \
+                       NT, scale, W, Kf, Qg, M, A, flags, q_rstd, k_rstd, n0);                                        \
+    hipLaunchKernelGGL((intra_fwd_flagged_kernel<K, ISO_, NORM_>), dim3(gx), dim3(256), 0, s, q, k, kap, gc, T, H, NT, \
+                       B * H, n0, n1, scale, W, Kf, Qg, M, A, flags, q_rstd, k_rstd);                                 \
   } while (0)
     if (iso && q_rstd) KDN_INTRA(true, true);
     else if (iso) KDN_INTRA(true, false);
@@ -1070,11 +908,11 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
     with_copy_mask(mask, [&](auto hmc) {
       constexpr int HM = decltype(hmc)::value;
       if (o_bf16)
-        hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, bf16_t, true, HM>), grid, bs, 0, stream, U, W, Kf, gc,
-                           hin, T, H, NT, B * H, hstore, dstore, hout, P, Qg, M, (bf16_t*)o);
+        hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, bf16_t, true, HM>), grid, bs, 0, stream, v, W, A, Kf,
+                           gc, hin, T, H, NT, B * H, hstore, dstore, hout, P, Qg, M, (bf16_t*)o);
       else
-        hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, true, HM>), grid, bs, 0, stream, U, W, Kf, gc,
-                           hin, T, H, NT, B * H, hstore, dstore, hout, P, Qg, M, (float*)o);
+        hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, true, HM>), grid, bs, 0, stream, v, W, A, Kf,
+                           gc, hin, T, H, NT, B * H, hstore, dstore, hout, P, Qg, M, (float*)o);
     });
   };
   // Overlapped schedule (bits 0, 1 and 2 in one call, one chunk group): the state pass (with the readout
@@ -1141,7 +979,7 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
     float* grp = saved + lay.grp;
     kdn_state::GroupPlan P{gcnt.NG, gcnt.m, 0, grp, grp + (int64_t)B * H * gcnt.NG * K * V};
     hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V>), dim3(B * H * (gcnt.NG - 1) * NS),
-                       dim3(kdn_state::state_threads(V)), 0, stream, U, W, Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P);
+                       dim3(kdn_state::state_threads(V)), 0, stream, v, W, A, Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P);
     KDN_CHECK_LAUNCH();
     if (gcnt.NG > 2) {
       hipLaunchKernelGGL((kdn_state::state_combine_kernel<K, V>), dim3(B * H * NV), dim3(kdn_state::state_threads(V)),
@@ -1161,7 +999,7 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
         B * H, lay.gc, saved + lay.grp, false, stream, [&](dim3 grid, const kdn_state::GroupPlan& P) {
           with_copy_mask(hm, [&](auto hmc) {
             hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, false, decltype(hmc)::value>), grid, bs, 0,
-                               stream, U, W, Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P);
+                               stream, v, W, A, Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P);
           });
         });
     if (rc) return rc;
@@ -1181,19 +1019,19 @@ int mem_bwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
   const int NT = cdiv(T, C);
   MemLayout lay(B, T, H, K, V);
   BwdLayout bl(B, T, H, K, V);
-  const float *U = saved + lay.U, *W = saved + lay.W, *Kf = saved + lay.Kf, *Qg = saved + lay.Qg,
-              *M = saved + lay.M, *A = saved + lay.A, *hb = saved + lay.h, *D = saved + lay.D;
+  const float *W = saved + lay.W, *Kf = saved + lay.Kf, *Qg = saved + lay.Qg, *M = saved + lay.M, *A = saved + lay.A,
+              *hb = saved + lay.h, *D = saved + lay.D;
   const int* flags = reinterpret_cast<const int*>(saved + lay.flags);
-  float *dh = work + bl.dh, *dD = work + bl.dD, *dQg = work + bl.dQg, *dW = work + bl.dW, *dKf = work + bl.dKf,
-        *dM = work + bl.dM, *dgl = work + bl.dgl, *dKg = work + bl.dKg, *dN = work + bl.dN;
+  float *dh = work + bl.dh, *dX = work + bl.dX, *dQg = work + bl.dQg, *dKf = work + bl.dKf, *dM = work + bl.dM,
+        *dgl = work + bl.dgl, *dKg = work + bl.dKg, *dN = work + bl.dN;
   const int hm = half_copies(iso, bl.gc);
   constexpr int NV = V / kdn_state::state_cols(V);
-  const dim3 bs(2 * kdn_state::state_threads(V));  // helper waves take M^T dO and Qg^T dO off the chain
+  const dim3 bs(2 * kdn_state::state_threads(V));  // state waves and helper waves
   auto launch_state = [&](dim3 grid, const kdn_state::GroupPlan& P, const float* dS_in, float* dS_out,
                           hipStream_t st) {
     with_copy_mask(hm, [&](auto hmc) {
-      hipLaunchKernelGGL((kdn_state::state_bwd_kernel<K, V, TDO, true, decltype(hmc)::value>), grid, bs, 0, st, M, Kf,
-                         Qg, W, gc, dO, dS_in, T, H, NT, B * H, dh, dD, dS_out, P);
+      hipLaunchKernelGGL((kdn_state::state_bwd_kernel<K, V, TDO, decltype(hmc)::value>), grid, bs, 0, st, M, Kf, Qg,
+                         W, A, gc, dO, dS_in, T, H, NT, B * H, dh, dX, dS_out, P);
     });
   };
   // every chunk's products with h / dh; the solves and gradients of the unflagged ones: the
@@ -1201,8 +1039,8 @@ int mem_bwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
   auto launch_chunk = [&](int task0, int task_end, hipStream_t st) {
 #define KDN_CHUNK_BWD(ISO_, HB_)                                                                                    \
   hipLaunchKernelGGL((kdn_bwd::chunk_bwd_kernel<K, V, ISO_, TDO, HB_>), dim3(task_end - task0), dim3(512), 0, st, hb, \
-                     dh, D, dD, dO, A, flags, q, k, kap, gc, q_rstd, k_rstd, T, H, NT, B * H, task0, scale, dv, dq, dk, \
-                     dkap, dbeta, dg, dQg, dW, dKf, dM, dgl)
+                     dh, D, dX, dO, flags, q, k, kap, gc, q_rstd, k_rstd, T, H, NT, B * H, task0, scale, dv, dq, dk,    \
+                     dkap, dbeta, dg, dQg, dKg, dKf, dM, dN, dgl)
     if (iso && hm == kIsoHalfCopies) KDN_CHUNK_BWD(true, kIsoHalfCopies);
     else if (iso) KDN_CHUNK_BWD(true, 0);
     else KDN_CHUNK_BWD(false, 0);
@@ -1251,42 +1089,15 @@ int mem_bwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
     launch_chunk(0, tasks, stream);
     KDN_CHECK_LAUNCH();
   }
-  if ((stages & 12) == 12) {  // both exact stages: one launch runs each flagged chunk's solves, gradients and norm
+  if (stages & 8) {  // the exact path's gradients (bit 2 has no work of its own)
     const int NB = B * H * NT, gx = min(NB, 256);  // one workgroup per CU fits (its LDS)
 #define KDN_EXACT(ISO_)                                                                                               \
-  hipLaunchKernelGGL((mem_bwd_exact_kernel<K, V, ISO_>), dim3(gx), dim3(256), 0, stream, q, k, kap, gc, dD, dW, U, W, \
-                     dM, dQg, dKf, dgl, T, H, NT, NB, flags, scale, dv, dKg, dN, dq, dk, dkap, dbeta, dg, q_rstd,      \
-                     k_rstd)
+  hipLaunchKernelGGL((mem_bwd_exact_kernel<K, ISO_>), dim3(gx), dim3(256), 0, stream, q, k, kap, gc, dN, dM, dQg, dKg, \
+                     dKf, dgl, T, H, NT, NB, flags, scale, dq, dk, dkap, dbeta, dg, q_rstd, k_rstd)
     if (iso) KDN_EXACT(true);
     else KDN_EXACT(false);
 #undef KDN_EXACT
     KDN_CHECK_LAUNCH();
-    return 0;
-  }
-  if (stages & 4) {  // the chunks left to the exact path: transposed solves into dv, dKg, dN
-    const int NB = B * H * NT, gx = min(NB, 512);
-    if (iso)
-      hipLaunchKernelGGL((mem_bwd_solve_exact_kernel<K, V, true>), dim3(gx), dim3(256), 0, stream, k, kap, gc, dD, dW,
-                         U, W, T, H, NT, NB, flags, dv, dKg, dN, k_rstd);
-    else
-      hipLaunchKernelGGL((mem_bwd_solve_exact_kernel<K, V, false>), dim3(gx), dim3(256), 0, stream, k, kap, gc, dD,
-                         dW, U, W, T, H, NT, NB, flags, dv, dKg, dN, k_rstd);
-    KDN_CHECK_LAUNCH();
-  }
-  if (stages & 8) {  // the exact path's gradients
-    const int NB = B * H * NT, gx = min(NB, 512);
-    if (iso)
-      hipLaunchKernelGGL((mem_bwd_contrib_exact_kernel<K, V, true>), dim3(gx), dim3(256), 0, stream, q, k, kap, gc, dN,
-                         dM, dQg, dKg, dKf, dgl, T, H, NT, NB, flags, scale, dq, dk, dkap, dbeta, dg, q_rstd, k_rstd);
-    else
-      hipLaunchKernelGGL((mem_bwd_contrib_exact_kernel<K, V, false>), dim3(gx), dim3(256), 0, stream, q, k, kap, gc,
-                         dN, dM, dQg, dKg, dKf, dgl, T, H, NT, NB, flags, scale, dq, dk, dkap, dbeta, dg, q_rstd, k_rstd);
-    KDN_CHECK_LAUNCH();
-    if (q_rstd) {  // the in-op norm's backward for the flagged chunks' rows
-      hipLaunchKernelGGL((l2norm_bwd_flagged_kernel<K>), dim3(gx), dim3(256), 0, stream, q, k, q_rstd, k_rstd, T, H,
-                         NT, NB, flags, dq, dk);
-      KDN_CHECK_LAUNCH();
-    }
   }
   return 0;
 }

@@ -1,9 +1,12 @@
 // Serial chunk-state passes of the KDN memory scan (forward and reverse).
 //
-//   forward  (per chunk n):  h_n = S;  delta = U - W S;  O = Qg S + M delta;
+//   forward  (per chunk n):  h_n = S;  U = A V;  delta = U - W S;  O = Qg S + M delta;
 //                            S = e^{g_last} S + Kf^T delta
-//   backward (reverse):      dh_n = dS;  d delta = M^T dO + Kf dS;
+//   backward (reverse):      dh_n = dS;  d delta = M^T dO + Kf dS;  dX = A^T d delta;
 //                            dS <- e^{g_last} dS + Qg^T dO - W^T d delta
+// (A = (I + N)^{-1} of the chunk, W = A Kg.)  U and dX are off the recurrence: the helper waves of each pass form
+// them.  On the recurrence instead (delta = A (V - Kg S), dS - Kg^T dX, which needs no W) the product with A
+// lengthened every chunk step of the forward pass by 0.5 us (376 -> 449 us at B4 T4096 H18 d128).
 //
 // Work split.  One workgroup per (b, h, 64-column slice of V), one wave per 16 state columns;
 // each wave keeps its columns for the whole sequence as K/16 MFMA accumulator tiles.  The
@@ -120,17 +123,25 @@ __device__ __forceinline__ void bfrag(f32x4 t0, f32x4 t1, uint4& hi, uint4& lo) 
   split2(t1[2], t1[3], hi.w, lo.w);
 }
 
-// Staging unit u of an A operand with contraction length KD: 4 consecutive k-slots of one lane
-// of one tile.  Consecutive u are consecutive lanes, so a wave's LDS stores are contiguous.
-struct Unit {
-  int row, k0, off;
+// The units of one of 256 staging threads (units t + 256 u) of a [16-row tiles] x [64 k] operand, with the thread's
+// part of every address in one register and the rest compile-time constants (as arithmetic on t + 256 u the
+// compiler, which does not know t < 256, keeps an address per unit): unit u is 4 k-slots from k0() of row r + 16 u.
+struct StageLane {
+  int r, k, kt, off;  // row in a tile, first k-slot within a k-block, k-block, LDS offset of unit 0
+  __device__ __forceinline__ explicit StageLane(int t)
+      : r(t & 15), k(16 * ((t >> 6) & 1) + 4 * ((t >> 4) & 3)), kt(t >> 7),
+        off((t >> 7) * TILE + (t & 63) * 8 + 4 * ((t >> 6) & 1)) {}
+  __device__ __forceinline__ int k0() const { return k + 32 * kt; }
+  static __device__ __forceinline__ constexpr int doff(int u) { return 2 * TILE * u; }
 };
-template <int KD>
-__device__ __forceinline__ Unit unit(int u) {
-  constexpr int KB = KD / 32;
-  const int tile = u >> 7, half = (u >> 6) & 1, L = u & 63;
-  return Unit{16 * (tile / KB) + (L & 15), 32 * (tile % KB) + 16 * half + 4 * (L >> 4), tile * TILE + L * 8 + 4 * half};
-}
+// Lower-triangular A (rows c, k = s) and A^T (rows s, k = c): only the 6 of 8 tiles that are not all zero are
+// staged, in the order (row tile, k-block) (0,0) (1,0) (2,0) (2,1) (3,0) (3,1) of A and (0,0) (0,1) (1,0) (1,1)
+// (2,1) (3,1) of A^T: tiles kt + 2 u of a staging thread, u < 3.
+constexpr int NTRI = 6;
+__device__ __forceinline__ int tri_row(const StageLane& l, int u) { return l.r + (u == 0 ? 16 * l.kt : 16 * (u + 1)); }
+__device__ __forceinline__ int tri_k0(const StageLane& l, int u) { return l.k + (u == 0 ? 0 : 32 * l.kt); }
+__device__ __forceinline__ int trit_row(const StageLane& l, int u) { return l.r + (u < 2 ? 16 * u : 32 + 16 * l.kt); }
+__device__ __forceinline__ int trit_k0(const StageLane& l, int u) { return l.k + (u < 2 ? 32 * l.kt : 32); }
 __device__ __forceinline__ void put_unit(bf16_t* buf, int off, float a, float b, float c, float d) {
   uint32_t h0, l0, h1, l1;
   split2(a, b, h0, l0);
@@ -143,19 +154,85 @@ __device__ __forceinline__ void afrag(const bf16_t* buf, int tile, int lane, uin
   lo = *reinterpret_cast<const uint4*>(buf + tile * TILE + 512 + lane * 8);
 }
 
-// Stores of one lane's 4 D-layout values (rows r0 + j of a column) with one voffset: the row
-// block goes into the descriptor base (rows past the end stay range-checked) and the row j
-// into the instruction's immediate offset, so no per-element address registers are kept.
-// (Quad-transposing the tile for 16-byte stores measured slower on the serial chain: the DPP
-// transposes cost more issue than the store instructions they save.)
-__device__ __forceinline__ void st_rows4(bufrsrc r, uint32_t vbase, uint32_t row_bytes, const f32x4& x) {
+// Staging of a [C][K] fp32 operand by 256 threads t, in units of 4 consecutive channels each, 8 lanes on
+// the 128 bytes of one row's 32 channels, so that a load instruction takes whole cache lines.  (By 16-row tiles, as
+// the fragments lie, an instruction takes 64-byte pieces of 16 rows; the passes are bound by the lines a CU loads.)
+// RowStage: as fragments with rows c, k = channel; ColStage: with rows i = channel, k = c, through a quad transpose
+// (the lanes of a quad hold 4 consecutive rows).  B4 T4096 H18 d128: RowStage took the reverse pass from 317 to 302
+// us, ColStage the forward pass from 363 to 358; in the reverse pass, whose state waves have less time to spare,
+// ColStage's transposes lost more than the lines saved (302 -> 315 us), so W^T stays with 4-byte gathers there.
+template <int K, int ROWS = C, int LD = K>
+struct RowStage {
+  static constexpr int NR = ROWS / 32, UN = NR * (K / 32), KB = K / 32;
+  int src, dst;  // byte offset of unit 0 in the operand (row stride LD), element offset in the LDS fragments
+  __device__ __forceinline__ explicit RowStage(int t) {
+    const int row = t >> 3, q = t & 7;
+    src = (row * LD + 4 * q) * 4;
+    dst = (row >> 4) * KB * TILE + ((row & 15) + 16 * (q & 3)) * 8 + 4 * (q >> 2);
+  }
+  __device__ __forceinline__ void load(bufrsrc r, float4 (&x)[UN]) const {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[j]), r, vbase + j * row_bytes, 0, 0);
-}
-// Descriptor over rows [r0, L) of a row-major [rows][D] fp32 block at p (row stride D).
-__device__ __forceinline__ bufrsrc rows_from(const float* p, int r0, int L, int D) {
-  return make_buf(p + (int64_t)r0 * D, (uint32_t)(L > r0 ? (L - r0) * D * 4 : 0));
-}
+    for (int u = 0; u < UN; ++u) x[u] = buf_ld4(r, src + (u % NR) * (32 * LD * 4) + (u / NR) * 128);
+  }
+  __device__ __forceinline__ void put(bf16_t* buf, const float4 (&x)[UN]) const {
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+      put_unit(buf, dst + (u % NR) * (2 * KB * TILE) + (u / NR) * TILE, x[u].x, x[u].y, x[u].z, x[u].w);
+  }
+};
+template <int K>
+struct ColStage {
+  static constexpr int UN = K / 16;
+  int src, dst, qr;
+  __device__ __forceinline__ explicit ColStage(int t) : qr(t & 3) {
+    const int p = (t >> 2) & 7, rb = t >> 5;
+    src = ((4 * rb + qr) * K + 4 * p) * 4;
+    dst = (p >> 2) * 2 * TILE + (4 * (p & 3) + qr + 16 * (rb & 3)) * 8 + 4 * (rb >> 2);
+  }
+  __device__ __forceinline__ void load(bufrsrc r, float4 (&x)[UN]) const {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) x[u] = buf_ld4(r, src + (u & 1) * (32 * K * 4) + (u >> 1) * 128);
+  }
+  __device__ __forceinline__ void put(bf16_t* buf, const float4 (&x)[UN]) const {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const float4 y = quad_transpose(x[u], qr);
+      put_unit(buf, dst + (u & 1) * TILE + (u >> 1) * (4 * TILE), y.x, y.y, y.z, y.w);
+    }
+  }
+};
+
+// A chunk's 64 rows x 64 columns of a bf16 tensor (V, dO) as B fragments (k = row, permuted order) of its four
+// 16-column groups, through 256 threads t: whole 128-byte row pieces are loaded, 8 columns of a row per lane and
+// unit; the 4 lanes of a quad hold 4 consecutive rows, so a transpose of their dwords gives each lane 4 rows of
+// 2 columns, two 8-byte halves of fragments.  frag: [group][kb], `pitch` uint4 apart, 64 lanes each.  (As 16
+// 2-byte loads per lane, 32-byte pieces of 4 rows each, V cost the forward state pass 65 us of 418 at B4 T4096
+// H18 d128: a CU's loads bound these passes.)
+struct Cols64 {
+  u32x4 x[2];
+  // p: the chunk's row 0, column 0 of the slice; row_bytes: from row to row; L rows (rows past them read 0)
+  __device__ __forceinline__ void load(const bf16_t* p, uint32_t row_bytes, int L, int t) {
+    const bufrsrc r = make_buf(p, L > 0 ? (uint32_t)(L - 1) * row_bytes + 128 : 0u);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      x[u] = __builtin_amdgcn_raw_buffer_load_b128(
+          r, (uint32_t)(4 * ((t >> 5) + 8 * u) + (t & 3)) * row_bytes + 16 * ((t >> 2) & 7), 0, 0);
+  }
+  __device__ __forceinline__ void publish(uint4* frag, int pitch, int t) const {
+    const int qr = t & 3, p = (t >> 2) & 7;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float4 y = quad_transpose(__builtin_bit_cast(float4, x[u]), qr);  // rows 0..3 of columns 2 qr, 2 qr + 1
+      const uint32_t a = __float_as_uint(y.x), b = __float_as_uint(y.y), c = __float_as_uint(y.z), d = __float_as_uint(y.w);
+      const int rb = (t >> 5) + 8 * u;  // 4-row block: k-block rb / 8, slots 4 (rb / 4 % 2) .., lane group rb % 4
+      uint2* dst = reinterpret_cast<uint2*>(frag + ((p >> 1) * 2 + (rb >> 3)) * pitch + 8 * (p & 1) + 2 * qr + 16 * (rb & 3)) +
+                   ((rb >> 2) & 1);
+      dst[0] = uint2{__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(d, c, 0x05040100u)};
+      dst[2] = uint2{__builtin_amdgcn_perm(b, a, 0x07060302u), __builtin_amdgcn_perm(d, c, 0x07060302u)};
+    }
+  }
+};
+
 // Layout of a per-chunk state copy [K][V] (h, dh; only the chunk backward and the readout read them):
 // 16-column blocks, within one the 16-row tiles, within a tile the rows in the order
 // (i % 4, (i / 4) % 4), 16 columns each.  A state wave's lane (g4, c16) holds rows 16 ib + 4 g4 + j of
@@ -196,13 +273,19 @@ __device__ __forceinline__ void mfma_pipe(Rd rd, Mm mm) {
   }
 }
 
-// Layout of the reverse pass's d delta copy of one chunk [C][V] (only the chunk backward reads it): 16-column
-// blocks, within one the four 16-row accumulator tiles, each as the pass's lanes hold it (lane r16 + 16 g4: the
-// rows 4 g4 .. + 3 of column r16).  A tile leaves in one 16-byte store per lane, whole 1 KB, and comes back the
-// same way as the MFMA operand d delta^T in permuted k order.  Row-major, the copy took 16 4-byte stores per
-// chunk step on the serial chain.
-__device__ __forceinline__ int dd_off(int c, int v) {
-  return (((v >> 4) * 4 + (c >> 4)) * 64 + (v & 15) + 16 * ((c >> 2) & 3)) * 4 + (c & 3);
+// Layout of the chunk copies [C][V] of delta (forward pass) and dX (reverse pass): 16-column blocks, within one
+// the four 16-row accumulator tiles, each as the pass's lanes hold it (lane r16 + 16 g4: the rows 4 g4 .. + 3 of
+// column r16).  A tile leaves in one 16-byte store per lane, 1 KB whole; row-major, the copy took 16 4-byte
+// stores per chunk step on the serial chain.  The readers turn 4 rows of a column into 4 columns of a row with a
+// quad transpose.  Rows past the sequence's end hold 0.  Element (c, v) of a chunk is at
+//   (((v / 16) * 4 + c / 16) * 64 + v % 16 + 16 ((c / 4) % 4)) * 4 + c % 4.
+template <int V>
+__device__ __forceinline__ void st_tiles(float* p, int64_t chunk, int col, int lane, const f32x4 (&x)[4]) {
+  const bufrsrc r = make_buf(p + chunk * C * V, C * V * 4);
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x[cb]), r,
+                                           (uint32_t)(((col >> 4) * 4 + cb) * 64 + lane) * 16, 0, 0);
 }
 
 // Block -> (bh, V-slice): the NV slices of one (b, h) go to one XCD (dispatch is round-robin
@@ -227,7 +310,7 @@ __device__ __forceinline__ int64_t row_bthk(int b, int t, int h, int T, int H, i
 // Chunk groups (two-level scan).  With NG > 1 groups of m chunks, each state pass runs as
 //   pass A  the first group in order (the true state), plus every middle group's affine map
 //           S_out = Phi S_in + Psi, taken by running the group from [0 | I] on V + K columns
-//           (the Psi columns see U / dO, the Phi columns start at the identity and see none);
+//           (the Psi columns see V / dO, the Phi columns start at the identity and see none);
 //   pass B  state_combine_kernel: the group-start states, serially, S_{g+1} = Phi_g S_g + Psi_g;
 //   pass C  every later group from its true incoming state (h / delta stores, final state).
 // Pass A's middle groups and pass C's groups all run in parallel, so the serial depth is about
@@ -299,7 +382,7 @@ __device__ __forceinline__ bool group_task(const GroupPlan& P, int BH, int& bh, 
 
 // ===========================================================================
 // Forward state pass.  grid: (B*H*V/COLS) for one group, or the pass's task count (GroupPlan);
-// block 4 COLS.  LDS 64.5 KB.
+// block 4 COLS.  LDS 76.5 KB.
 // The readout O = Qg h + M delta is left to readout_kernel: it is off the serial chain, and its
 // operands (Qg, M) would double the chunk operands staged on the chain's critical path.
 // ===========================================================================
@@ -313,8 +396,8 @@ __device__ __forceinline__ bool group_task(const GroupPlan& P, int BH, int& bh, 
 // pays for the fragment stores.  Both wave groups run the same barrier sequence.
 template <int K, int V, typename TO = float, bool RO = false, int HM = 0>
 __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 1 : 2) void state_fwd_kernel(
-    const float* __restrict__ U, const float* __restrict__ W, const float* __restrict__ Kf,
-    const float* __restrict__ gc, const float* __restrict__ h0, int T, int H, int NT, int BH,
+    const bf16_t* __restrict__ v, const float* __restrict__ W, const float* __restrict__ Ag,
+    const float* __restrict__ Kf, const float* __restrict__ gc, const float* __restrict__ h0, int T, int H, int NT, int BH,
     float* __restrict__ hbuf, float* __restrict__ Dl, float* __restrict__ ht, GroupPlan P,
     const float* __restrict__ Qg = nullptr, const float* __restrict__ Mg = nullptr, TO* __restrict__ out = nullptr) {
   constexpr int COLS = state_cols(V), NTHR = state_threads(V);
@@ -322,16 +405,20 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
   constexpr int ST = K / 16;           // state row tiles per wave
   static_assert((C * K / 4) % NTHR == 0, "staging units per thread");
   constexpr int UN = C * K / 4 / NTHR;  // staging units per thread of a C x K operand
+  constexpr int UA = NTRI * 128 / NTHR;  // ... of A
   __shared__ __attribute__((aligned(16))) bf16_t sW[(C / 16) * KB * TILE];        // W: rows c, k = i
+  __shared__ __attribute__((aligned(16))) bf16_t sA[NTRI * TILE];                  // A: rows c, k = s
   __shared__ __attribute__((aligned(16))) bf16_t sK[(K / 16) * (C / 32) * TILE];  // Kf^T: rows i, k = c
   __shared__ __attribute__((aligned(16))) float sE[K];
   // RO: B fragments of h_n ([wave][kb][hi, lo][lane], K / 32 k-blocks) then of delta_n (2 k-blocks)
   constexpr int NHF = 4 * KB * 2 * 64, NDF = 4 * 2 * 2 * 64;
   __shared__ __attribute__((aligned(16))) uint4 sHD[RO ? NHF + NDF : 1];
-  // RO: each readout wave's 16 output rows, regrouped so that every store writes whole row segments
-  constexpr int ROWB = COLS * (int)sizeof(TO), QPR = ROWB / 16, RPI = 1024 / ROWB;
-  static_assert(ROWB % 128 == 0 && RPI <= 16, "readout rows of 8 or more 16-byte quads");
-  __shared__ __attribute__((aligned(16))) uint4 sO[RO ? 4 * 16 * QPR : 1];
+  __shared__ f32x4 sU[RO ? 4 * 4 * 64 : 1];  // RO: U = A V of the next chunk: [state wave][row tile cb][lane]
+  __shared__ uint4 sV[RO ? 4 * 2 * 64 : 1];  // RO: V of the next chunk as B fragments: [column group][kb][lane]
+  // RO: a readout wave's output rows, RR at a time, regrouped so that every store writes whole row segments
+  constexpr int ROWB = COLS * (int)sizeof(TO), QPR = ROWB / 16, RPI = 1024 / ROWB, RR = 2048 / ROWB;
+  static_assert(ROWB % 128 == 0 && RPI <= 8 && RR <= 16, "readout rows of 8 or more 16-byte quads");
+  __shared__ __attribute__((aligned(16))) uint4 sO[RO ? 4 * RR * QPR : 1];
   int bh, vs, g;
   bool real, phi;
   if (!group_task<V, K, false>(P, BH, bh, vs, g, real, phi)) return;
@@ -341,6 +428,32 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
   int n0, n1;
   plan_range(P, g, NT, n0, n1);
 
+  static_assert(NTHR == 256, "StageLane");
+  const StageLane sl(tid & (NTHR - 1));
+  // A and V of a chunk (the readout waves of RO; the state waves otherwise): A is split into LDS; V, exact in
+  // bf16, gives the B fragments of U = A V
+  float4 rA[UA];
+  auto load_A = [&](int n) {
+    const bufrsrc ra = make_buf(Ag + ((int64_t)bh * NT + n) * C * C, C * C * 4);
+#pragma unroll
+    for (int u = 0; u < UA; ++u) rA[u] = buf_ld4(ra, (uint32_t)(tri_row(sl, u) * C + tri_k0(sl, u)) * 4);
+  };
+  auto stage_A = [&]() {
+#pragma unroll
+    for (int u = 0; u < UA; ++u) put_unit(sA, sl.off + sl.doff(u), rA[u].x, rA[u].y, rA[u].z, rA[u].w);
+  };
+  auto prod_U = [&](const uint4 (&vf)[2], f32x4 (&U)[4]) {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) U[cb] = zero4();
+    // step s: the tiles of k-block 0 (0, 1, 2, 4), then of k-block 1 (3, 5)
+    mfma_pipe<NTRI, 2>(
+        [&](int st, uint4& ah, uint4& al) { afrag(sA, st < 3 ? st : st == 3 ? 4 : 2 * st - 5, lane, ah, al); },
+        [&](int st, const uint4& ah, const uint4& al) {
+          const int cb = st < 4 ? st : st - 2, kb = st < 4 ? 0 : 1;
+          U[cb] = mma2(ah, al, vf[kb], U[cb]);
+        });
+  };
+
   if constexpr (RO) {
     if (tid >= NTHR) {  // readout waves: wave rw owns chunk rows 16 rw .. 16 rw + 15 of all COLS columns
       const int rw = w - 4, r16 = lane & 15;
@@ -349,7 +462,9 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
       auto load_QM = [&](int n) {  // this lane's A fragment slots of Qg and M rows (permuted k order)
         const int t0 = n * C, L = min(C, T - t0);
         const bufrsrc rq_ = make_buf(Qg + row_bht(bh, t0, T, K), L * K * 4);  // rows past L read 0
+        // (M[c][s] = 0 for s > c: the first two row tiles do without the second k-block)
         const bufrsrc rm_ = make_buf(Mg + ((int64_t)bh * NT + n) * C * C, C * C * 4);
+        const bufrsrc rm1 = make_buf(Mg + ((int64_t)bh * NT + n) * C * C, rw < 2 ? 0u : C * C * 4);
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -357,10 +472,32 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int hf = 0; hf < 2; ++hf) rm[kb][hf] = buf_ld4(rm_, (c * C + 32 * kb + 16 * hf + 4 * g4) * 4);
+          for (int hf = 0; hf < 2; ++hf) rm[kb][hf] = buf_ld4(kb ? rm1 : rm_, (c * C + 32 * kb + 16 * hf + 4 * g4) * 4);
       };
+      const int ht = tid - NTHR;
+      Cols64 rV;
+      auto load_AV = [&](int n) {
+        load_A(n);
+        rV.load(v + row_bthk(b, n * C, h, T, H, V) + vs * COLS, H * V * 2, min(C, T - n * C), ht);
+      };
+      auto stage_AV = [&]() {
+        stage_A();
+        rV.publish(sV, 64, ht);
+      };
+      auto publish_U = [&]() {
+        const uint4 vf[2] = {sV[(rw * 2) * 64 + lane], sV[(rw * 2 + 1) * 64 + lane]};
+        f32x4 U[4];
+        prod_U(vf, U);
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) sU[(rw * 4 + cb) * 64 + lane] = U[cb];
+      };
+      load_AV(n0);
       load_QM(n0);
-      __syncthreads();  // the state waves' prologue barrier
+      stage_AV();
+      __syncthreads();  // A, V of the first chunk staged
+      publish_U();
+      if (n0 + 1 < n1) load_AV(n0 + 1);
+      __syncthreads();  // U of the first chunk published
       for (int n = n0; n < n1; ++n) {
         const int t0 = n * C, L = min(C, T - t0);
         uint4 qh[KB], ql[KB], mh[2], ml[2];
@@ -376,12 +513,17 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
                               rm[kb][1].x, rm[kb][1].y, rm[kb][1].z, rm[kb][1].w};
           split8v(x, mh[kb], ml[kb]);
         }
-        if (n + 1 < n1) load_QM(n + 1);
-        __syncthreads();  // end of phase 1: h_n and delta_n fragments published
+        if (n + 1 < n1) {
+          load_QM(n + 1);
+          stage_AV();
+          if (n + 2 < n1) load_AV(n + 2);
+        }
+        __syncthreads();  // end of phase 1: h_n and delta_n fragments published, U_n read, A, V of chunk n + 1 staged
         const bufrsrc ro = make_buf(out + row_bthk(b, t0, h, T, H, V), (uint32_t)((L - 1) * H + 1) * V * sizeof(TO));
         const int qr = lane & 3;
         // this wave's rows; the barriers of each chunk separate the last chunk's reads from these writes
-        unsigned char* sOw = reinterpret_cast<unsigned char*>(sO) + rw * 16 * ROWB;
+        unsigned char* sOw = reinterpret_cast<unsigned char*>(sO) + rw * RR * ROWB;
+        float4 y[4];
 #pragma unroll
         for (int sw = 0; sw < 4; ++sw) {  // the 16 columns of state wave sw (four independent chains)
           f32x4 O = zero4();
@@ -396,70 +538,82 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
             const uint4 dh2 = sHD[NHF + ((sw * 2 + kb) * 2) * 64 + lane], dl2 = sHD[NHF + ((sw * 2 + kb) * 2 + 1) * 64 + lane];
             O = mma3(mh[kb], ml[kb], dh2, dl2, O);
           }
-          // lane (column 4 q + r, rows 4 g4 ..) -> quad transpose -> row 4 g4 + r, columns 4 q .. 4 q + 3,
-          // into this wave's LDS rows (16-byte quad j of row r at slot j ^ (r & 7))
-          const float4 y = quad_transpose(float4{O[0], O[1], O[2], O[3]}, qr);
-          const int r = 4 * g4 + qr, cb = (16 * sw + 4 * ((lane & 15) >> 2)) * (int)sizeof(TO);
-          unsigned char* dst = sOw + r * ROWB + (((cb >> 4) ^ (r & 7)) << 4) + (cb & 15);
-          if constexpr (sizeof(TO) == 2) {
-            *reinterpret_cast<u32x2*>(dst) =
-                u32x2{(uint32_t)f2bf(y.x) | ((uint32_t)f2bf(y.y) << 16), (uint32_t)f2bf(y.z) | ((uint32_t)f2bf(y.w) << 16)};
-          } else {
-            *reinterpret_cast<float4*>(dst) = y;
+          // lane (column 4 q + r, rows 4 g4 ..) -> quad transpose -> row 4 g4 + r, columns 4 q .. 4 q + 3
+          y[sw] = quad_transpose(float4{O[0], O[1], O[2], O[3]}, qr);
+        }
+#pragma unroll
+        for (int rd = 0; rd < 16 / RR; ++rd) {  // rows rd RR ..: 16-byte quad j of row r at slot j ^ (r & 7)
+          const int r = 4 * g4 + qr;
+          if (rd) wave_lds_sync();  // the previous round's reads are issued before these writes
+          if (RR == 16 || r / RR == rd) {
+#pragma unroll
+            for (int sw = 0; sw < 4; ++sw) {
+              const int cb = (16 * sw + 4 * ((lane & 15) >> 2)) * (int)sizeof(TO);
+              unsigned char* dst = sOw + (r % RR) * ROWB + (((cb >> 4) ^ (r & 7)) << 4) + (cb & 15);
+              if constexpr (sizeof(TO) == 2) {
+                *reinterpret_cast<u32x2*>(dst) = u32x2{(uint32_t)f2bf(y[sw].x) | ((uint32_t)f2bf(y[sw].y) << 16),
+                                                       (uint32_t)f2bf(y[sw].z) | ((uint32_t)f2bf(y[sw].w) << 16)};
+              } else {
+                *reinterpret_cast<float4*>(dst) = y[sw];
+              }
+            }
+          }
+          wave_lds_sync();
+#pragma unroll
+          for (int hh = 0; hh < RR / RPI; ++hh) {  // RPI whole rows of COLS columns per store
+            const int rr = lane / QPR + RPI * hh, qd = lane % QPR;
+            const u32x4 x = *reinterpret_cast<const u32x4*>(sOw + rr * ROWB + ((qd ^ (rr & 7)) << 4));
+            const uint32_t eb =
+                ((uint32_t)((16 * rw + rd * RR + rr) * H) * V + (uint32_t)(vs * COLS)) * (uint32_t)sizeof(TO) + 16 * qd;
+            __builtin_amdgcn_raw_buffer_store_b128(x, ro, eb, 0, 0);  // rows past L dropped
           }
         }
-        wave_lds_sync();
-#pragma unroll
-        for (int hh = 0; hh < 16 / RPI; ++hh) {  // RPI whole rows of COLS columns per store
-          const int rr = lane / QPR + RPI * hh, qd = lane % QPR;
-          const u32x4 x = *reinterpret_cast<const u32x4*>(sOw + rr * ROWB + ((qd ^ (rr & 7)) << 4));
-          const uint32_t eb =
-              ((uint32_t)((16 * rw + rr) * H) * V + (uint32_t)(vs * COLS)) * (uint32_t)sizeof(TO) + 16 * qd;
-          __builtin_amdgcn_raw_buffer_store_b128(x, ro, eb, 0, 0);  // rows past L dropped
-        }
-        __syncthreads();  // end of phase 2: the fragments may be overwritten
+        if (n + 1 < n1) publish_U();
+        __syncthreads();  // end of phase 2: the fragments may be overwritten, U of chunk n + 1 published
       }
       return;
     }
   }
 
-  float4 rW[UN];
-  float rK[UN][4], rU[4][4], rE = 0.f;
-  auto load_W = [&](int n) {  // W (rows c, k = i)
+  // without readout waves: V of this lane's column, U's B fragment (Phi columns: 0)
+  uint16_t rV[4][4];
+  auto load_V = [&](int n) {
     const int t0 = n * C, L = min(C, T - t0);
-    const bufrsrc rw = make_buf(W + row_bht(bh, t0, T, K), L * K * 4);  // rows past L read 0
-#pragma unroll
-    for (int u = 0; u < UN; ++u) {
-      const Unit x = unit<K>(tid + NTHR * u);
-      rW[u] = buf_ld4(rw, (x.row * K + x.k0) * 4);
-    }
-  };
-  auto load_K = [&](int n) {  // Kf^T (rows i, k = c), U rows of this lane, e^{g_last}
-    const int t0 = n * C, L = min(C, T - t0);
-    const bufrsrc rk = make_buf(Kf + row_bht(bh, t0, T, K), L * K * 4);
-    const bufrsrc ru = make_buf(U + row_bht(bh, t0, T, V), phi ? 0u : L * V * 4);  // Phi columns: U = 0
-#pragma unroll
-    for (int u = 0; u < UN; ++u) {
-      const Unit x = unit<C>(tid + NTHR * u);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) rK[u][j] = buf_ld(rk, ((x.k0 + j) * K + x.row) * 4);
-    }
+    const bufrsrc rv = make_buf(v + row_bthk(b, t0, h, T, H, V), phi ? 0u : ((L - 1) * H + 1) * V * 2);
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) rU[cb][j] = buf_ld(ru, ((16 * cb + 4 * g4 + j) * V + col) * 4);
-    {  // raw g_last of the chunk; the exponential is taken when staging, so no wait sits here
-      const bufrsrc rg = make_buf(gc + row_bthk(b, t0 + L - 1, h, T, H, K), K * 4);  // lanes >= K read 0
-      rE = buf_ld(rg, tid * 4);
+      for (int j = 0; j < 4; ++j)
+        rV[cb][j] = __builtin_amdgcn_raw_buffer_load_b16(rv, ((uint32_t)((16 * cb + 4 * g4 + j) * H) * V + col) * 2, 0, 0);
+  };
+  auto pack_V = [&](uint4 (&vf)[2]) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      auto p2 = [&](int cb, int j) { return (uint32_t)rV[cb][j] | ((uint32_t)rV[cb][j + 1] << 16); };
+      vf[kb] = uint4{p2(2 * kb, 0), p2(2 * kb, 2), p2(2 * kb + 1, 0), p2(2 * kb + 1, 2)};
     }
   };
+  const RowStage<K> stW(tid);
+  const ColStage<K> stK(tid);
+  float4 rW[UN], rK[UN];
+  float rE = 0.f;
+  auto load_W = [&](int n) {  // W (rows c, k = i)
+    const int t0 = n * C, L = min(C, T - t0);
+    stW.load(make_buf(W + row_bht(bh, t0, T, K), L * K * 4), rW);  // rows past L read 0
+  };
+  auto load_K = [&](int n) {  // Kf^T (rows i, k = c), g_last
+    const int t0 = n * C, L = min(C, T - t0);
+    stK.load(make_buf(Kf + row_bht(bh, t0, T, K), L * K * 4), rK);
+    // raw g_last of the chunk; the exponential is taken when staging, so no wait sits here
+    const bufrsrc rg = make_buf(gc + row_bthk(b, t0 + L - 1, h, T, H, K), K * 4);  // lanes >= K read 0
+    rE = buf_ld(rg, tid * 4);
+  };
   auto stage_W = [&]() {
-#pragma unroll
-    for (int u = 0; u < UN; ++u) put_unit(sW, unit<K>(tid + NTHR * u).off, rW[u].x, rW[u].y, rW[u].z, rW[u].w);
+    stW.put(sW, rW);
+    if constexpr (!RO) stage_A();
   };
   auto stage_K = [&]() {
-#pragma unroll
-    for (int u = 0; u < UN; ++u) put_unit(sK, unit<C>(tid + NTHR * u).off, rK[u][0], rK[u][1], rK[u][2], rK[u][3]);
+    stK.put(sK, rK);
     if (tid < K) sE[tid] = fexp2(rE);
   };
 
@@ -480,73 +634,71 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
   }
 
   load_W(n0);
+  if constexpr (!RO) load_A(n0), load_V(n0);
   stage_W();
   load_K(n0);
+  if constexpr (RO) __syncthreads();  // the helpers' first barrier
   __syncthreads();
   for (int n = n0; n < n1; ++n) {
-    const int t0 = n * C, L = min(C, T - t0);
     if (real && hbuf) {  // (no h, delta stores when the readout is fused and no backward follows)
       const int64_t e0 = ((int64_t)bh * NT + n) * K * V;
 #pragma unroll
       for (int ib = 0; ib < ST; ++ib) st_state4<K, V, (HM & HB_H) != 0>(hbuf, e0, ib, g4, col, S[ib]);
     }
 
-    // ---- phase 1: delta = U - W S   (reads sW; fills sK with chunk n; loads W of chunk n+1)
+    // ---- phase 1: delta = U - W S   (reads sW, sU; fills sK with chunk n; loads W of chunk n+1)
     stage_K();
-    float cU[4][4];
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) cU[cb][j] = rU[cb][j];
-    if (n + 1 < n1) load_W(n + 1);
-    f32x4 D[4];
+    f32x4 D[4];  // U, then delta
+    if constexpr (!RO) {
+      uint4 vf[2];
+      pack_V(vf);
+      prod_U(vf, D);
+    }
+    if (n + 1 < n1) {
+      load_W(n + 1);
+      if constexpr (!RO) load_A(n + 1), load_V(n + 1);
+    }
     {
       uint4 bh_[KB], bl_[KB];
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) bfrag(S[2 * kb], S[2 * kb + 1], bh_[kb], bl_[kb]);
+      f32x4 a[4];
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) D[cb] = zero4();
+      for (int cb = 0; cb < 4; ++cb) a[cb] = zero4();
       // step s: kb = s / 4, cb = s % 4
       mfma_pipe<4 * KB, 2>([&](int st, uint4& ah, uint4& al) { afrag(sW, (st & 3) * KB + (st >> 2), lane, ah, al); },
                            [&](int st, const uint4& ah, const uint4& al) {
-                             D[st & 3] = mma3(ah, al, bh_[st >> 2], bl_[st >> 2], D[st & 3]);
+                             a[st & 3] = mma3(ah, al, bh_[st >> 2], bl_[st >> 2], a[st & 3]);
                            });
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) D[cb][j] = cU[cb][j] - D[cb][j];
-      if (real && Dl) {
-        const int64_t e0 = row_bht(bh, t0, T, V);
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-          st_rows4(rows_from(Dl + e0, 16 * cb, L, V), (4 * g4 * V + col) * 4, V * 4, D[cb]);  // rows past L dropped
-      }
-      if constexpr (RO) {  // publish the B fragments of h_n (multiplied with W above) and delta_n
+      for (int cb = 0; cb < 4; ++cb) D[cb] = (RO ? sU[RO ? (w * 4 + cb) * 64 + lane : 0] : D[cb]) - a[cb];
+      if (real && Dl) st_tiles<V>(Dl, (int64_t)bh * NT + n, col, lane, D);
+      if constexpr (RO) {  // publish the B fragments of h_n (multiplied with W above)
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
           sHD[((w * KB + kb) * 2) * 64 + lane] = bh_[kb];
           sHD[((w * KB + kb) * 2 + 1) * 64 + lane] = bl_[kb];
         }
-        uint4 dh2, dl2;
-        bfrag(D[0], D[1], dh2, dl2);
-        sHD[NHF + ((w * 2) * 2) * 64 + lane] = dh2;
-        sHD[NHF + ((w * 2) * 2 + 1) * 64 + lane] = dl2;
-        bfrag(D[2], D[3], dh2, dl2);
-        sHD[NHF + ((w * 2 + 1) * 2) * 64 + lane] = dh2;
-        sHD[NHF + ((w * 2 + 1) * 2 + 1) * 64 + lane] = dl2;
+      }
+    }
+    uint4 dh_[2], dl_[2];  // the B fragments of delta
+    bfrag(D[0], D[1], dh_[0], dl_[0]);
+    bfrag(D[2], D[3], dh_[1], dl_[1]);
+    if constexpr (RO) {  // ... and of delta_n
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        sHD[NHF + ((w * 2 + kb) * 2) * 64 + lane] = dh_[kb];
+        sHD[NHF + ((w * 2 + kb) * 2 + 1) * 64 + lane] = dl_[kb];
       }
     }
     __syncthreads();
 
-    // ---- phase 2: S = e S + Kf^T delta   (reads sK; fills sW with chunk n+1; loads Kf, U, e of n+1)
+    // ---- phase 2: S = e S + Kf^T delta   (reads sK; fills sW (sA) with chunk n+1; loads Kf, e of n+1)
     if (n + 1 < n1) {
       stage_W();
       load_K(n + 1);
     }
     {
-      uint4 dh_[2], dl_[2];
-      bfrag(D[0], D[1], dh_[0], dl_[0]);
-      bfrag(D[2], D[3], dh_[1], dl_[1]);
 #pragma unroll
       for (int ib = 0; ib < ST; ++ib) {
         const float4 e = *reinterpret_cast<const float4*>(sE + 16 * ib + 4 * g4);
@@ -625,14 +777,14 @@ __global__ __launch_bounds__(256, 3) void readout_kernel(const float* __restrict
 #pragma unroll
     for (int p = 0; p < 2; ++p) m4[kb][p] = buf_ld4(rM, (c * C + 32 * kb + 8 * g4 + 4 * p) * 4);
 
-  // ---- stage h^T and delta^T.  A wave loads 4 rows x 64 columns per instruction (lane l: row
+  // ---- stage h^T and delta^T.  A wave loads 4 rows x 64 columns of h per instruction (lane l: row
   // 4 rb + l % 4, columns 4 (l / 4) .. +3), transposes each 4 x 4 block across its lane quad (DPP),
   // so a lane holds 4 consecutive rows of one column: 4 consecutive fragment slots of one lane,
   // written as 8 bytes of hi and 8 of lo
   {
     constexpr int EH = (HM & HB_H) ? 2 : 4;  // bytes per stored element
     const bufrsrc rh = make_buf(reinterpret_cast<const char*>(hbuf) + chunk * K * V * EH, K * V * EH);
-    const bufrsrc rd = make_buf(Dl + ((int64_t)bh * T + t0) * V, L * V * 4);  // rows past L read 0
+    const float* dn = Dl + chunk * C * V;
     constexpr int HU = K / 16, DU = C / 16;  // 4-row blocks per wave
     const int qr = lane & 3, vq = 4 * (lane >> 2), vc = vq + qr;  // after the transpose: column vc
     float4 hx[HU], dx[DU];
@@ -651,10 +803,11 @@ __global__ __launch_bounds__(256, 3) void readout_kernel(const float* __restrict
       hx[u] = ld4h(rh, hb_off<K>(hi, hv), std::integral_constant<bool, (HM & HB_H) != 0>{});
     }
 #pragma unroll
-    for (int u = 0; u < DU; ++u)
-      dx[u] = buf_ld4(rd, ((4 * (w + 4 * u) + qr) * V + v0 + vq) * 4);
-    auto put = [&](bf16_t* buf, int nkb, int r0, const float4& x) {  // rows r0 .. r0+3 of column vc
-      const float4 y = quad_transpose(x, qr);
+    for (int u = 0; u < DU; ++u) {  // delta comes as 4 rows of one column already (rows 4 (w + 4 u) .., column vc)
+      const int rb = w + 4 * u, vv = v0 + vc;
+      dx[u] = *reinterpret_cast<const float4*>(dn + (((vv >> 4) * 4 + (rb >> 2)) * 64 + (vv & 15) + 16 * (rb & 3)) * 4);
+    }
+    auto put = [&](bf16_t* buf, int nkb, int r0, const float4& y) {  // rows r0 .. r0+3 of column vc
       const int tile = (vc >> 4) * nkb + (r0 >> 5), ln = (vc & 15) + 16 * ((r0 & 31) >> 3);
       uint32_t h0, l0, h1, l1;
       split2(y.x, y.y, h0, l0);
@@ -664,7 +817,7 @@ __global__ __launch_bounds__(256, 3) void readout_kernel(const float* __restrict
       *reinterpret_cast<uint2*>(buf + off + 512) = uint2{l0, l1};
     };
 #pragma unroll
-    for (int u = 0; u < HU; ++u) put(sH, KB, 4 * (w + 4 * u), hx[u]);
+    for (int u = 0; u < HU; ++u) put(sH, KB, 4 * (w + 4 * u), quad_transpose(hx[u], qr));
 #pragma unroll
     for (int u = 0; u < DU; ++u) put(sD, 2, 4 * (w + 4 * u), dx[u]);
   }
@@ -717,42 +870,41 @@ __global__ __launch_bounds__(256, 3) void readout_kernel(const float* __restrict
 
 // ===========================================================================
 // Reverse state pass.  grid: (B*H*V/COLS) for one group, or the pass's task count (GroupPlan);
-// block 4 COLS.  LDS 112.5 KB.
-// With HW the block gets four helper waves (block 8 COLS, LDS 128.5 KB).  The products M^T dO and
-// Qg^T dO do not depend on the recurrence, so the helpers compute them one phase ahead of the state
-// waves and hand them over through LDS in the state waves' D layout: Qg^T dO of chunk n during
-// phase 1 of chunk n (added to dS in phase 2), M^T dO of chunk n - 1 during phase 2 of chunk n
+// block 8 COLS (four state waves and four helper waves), LDS 156.5 KB.
+// The products M^T dO and Qg^T dO do not depend on the recurrence, so the helpers compute them one phase
+// ahead of the state waves and hand them over through LDS in the state waves' D layout: Qg^T dO of chunk n
+// during phase 1 of chunk n (added to dS in phase 2), M^T dO of chunk n - 1 during phase 2 of chunk n
 // (added to d delta in phase 1 of chunk n - 1).  Helper wave hw owns the row tiles of those
 // products (Qg^T row tiles hw ST/4 .., M^T row tile hw) for all four column groups: their A
-// fragments (columns of Qg and M) are loaded straight into registers, one chunk ahead; each helper
-// loads dO of one column group and publishes its B fragments to the others through LDS.  The state
-// waves then stage only Kf and W^T and issue 32 split products per chunk instead of 56.  Both wave
-// groups run the same barrier sequence: two in the prologue, two per chunk.
+// fragments (columns of Qg and M) are loaded straight into registers, one chunk ahead; the helpers
+// publish dO's B fragments to each other through LDS, and each forms one column
+// group's dX = A^T d delta a phase after the state waves published d delta's fragments.  The state waves stage
+// Kf and W^T.  Both wave groups run the same barrier sequence: two in the
+// prologue, two per chunk.
 // ===========================================================================
-template <int K, int V, typename TDO, bool HW = false, int HM = 0>
-__global__ __launch_bounds__(HW ? 2 * state_threads(V) : state_threads(V)) void state_bwd_kernel(
+template <int K, int V, typename TDO, int HM = 0>
+__global__ __launch_bounds__(2 * state_threads(V)) void state_bwd_kernel(
     const float* __restrict__ Mg, const float* __restrict__ Kf, const float* __restrict__ Qg,
-    const float* __restrict__ W, const float* __restrict__ gc, const TDO* __restrict__ dO,
-    const float* __restrict__ dht, int T, int H, int NT, int BH, float* __restrict__ dhbuf,
-    float* __restrict__ dDl, float* __restrict__ dh0, GroupPlan P) {
+    const float* __restrict__ W, const float* __restrict__ Ag, const float* __restrict__ gc,
+    const TDO* __restrict__ dO, const float* __restrict__ dht, int T, int H, int NT, int BH,
+    float* __restrict__ dhbuf, float* __restrict__ dXl, float* __restrict__ dh0, GroupPlan P) {
   constexpr int COLS = state_cols(V), NTHR = state_threads(V);
   constexpr int KB = K / 32;
   constexpr int ST = K / 16;
   static_assert((C * K / 4) % NTHR == 0 && (C * C / 4) % NTHR == 0, "staging units per thread");
-  static_assert(!HW || (COLS == 64 && ST % 4 == 0), "helper waves: four state waves, K a multiple of 64");
+  static_assert(COLS == 64 && ST % 4 == 0, "helper waves: four state waves, K a multiple of 64");
   constexpr int UN = C * K / 4 / NTHR;  // staging units per thread of a C x K operand
-  constexpr int UM = C * C / 4 / NTHR;  // ... of M^T
+  constexpr int UA = NTRI * 128 / NTHR;  // ... of A^T
   constexpr bool DO_BF16 = sizeof(TDO) == 2;
-  // phase 1: M^T (rows c', k = c) and Kf (rows c, k = i);  phase 2: Qg^T, W^T (rows i, k = c).
-  // HW: M^T and Qg^T are not staged; the helpers' products and dO fragments take their place.
-  __shared__ __attribute__((aligned(16))) bf16_t sM[HW ? 8 : (C / 16) * (C / 32) * TILE];
+  // phase 1: Kf (rows c, k = i);  phase 2: W^T (rows i, k = c), the helpers' A^T (rows s, k = c)
   __shared__ __attribute__((aligned(16))) bf16_t sKn[(C / 16) * KB * TILE];
-  __shared__ __attribute__((aligned(16))) bf16_t sQ[HW ? 8 : (K / 16) * (C / 32) * TILE];
+  __shared__ __attribute__((aligned(16))) bf16_t sAt[NTRI * TILE];
   __shared__ __attribute__((aligned(16))) bf16_t sWt[(K / 16) * (C / 32) * TILE];
   __shared__ __attribute__((aligned(16))) float sE[K];
-  __shared__ f32x4 sPA[HW ? 4 * 4 * 64 : 1];   // M^T dO: [state wave][row tile cb][lane]
-  __shared__ f32x4 sPB[HW ? 4 * ST * 64 : 1];  // Qg^T dO: [state wave][row tile ib][lane]
-  __shared__ uint4 sO[HW ? 4 * 2 * 2 * 64 : 1];  // dO B fragments: [column group][kb][hi, lo][lane]
+  __shared__ f32x4 sPA[4 * 4 * 64];   // M^T dO: [state wave][row tile cb][lane]
+  __shared__ f32x4 sPB[4 * ST * 64];  // Qg^T dO: [state wave][row tile ib][lane]
+  __shared__ uint4 sO[4 * 2 * 2 * 64];  // dO B fragments: [column group][kb][hi, lo][lane]
+  __shared__ uint4 sDD[4 * 2 * 2 * 64];  // d delta B fragments: [state wave][kb][hi, lo][lane]
   int bh, vs, g;
   bool real, phi;
   if (!group_task<V, K, true>(P, BH, bh, vs, g, real, phi)) return;
@@ -761,216 +913,208 @@ __global__ __launch_bounds__(HW ? 2 * state_threads(V) : state_threads(V)) void 
   int n0, n1;
   plan_range(P, g, NT, n0, n1);
 
-  // dO as loaded (raw bf16 bits or fp32), widened only where the fragments are built, so the
-  // loads of a chunk are all issued before any of them is waited for
-  using RawO = std::conditional_t<DO_BF16, uint16_t, float>;
-  auto widen = [](RawO x) -> float {
-    if constexpr (DO_BF16) return bf2f(x);
-    else return x;
-  };
-  // dO rows 4 g4 + j (+ 16 cb) of column `col` of chunk n (rows past L and Phi columns read 0)
-  auto load_dO = [&](int n, int col, RawO (&rO)[4][4]) {
-    const int t0 = n * C, L = min(C, T - t0);
+  if (tid >= NTHR) {
+    constexpr int RT = ST / 4;  // Qg^T row tiles per helper wave
+    const int hw = w - 4, r16 = lane & 15;
+    // A fragment slot s of lane group g4 in k-block kb: chunk row c = 32 kb + 4 g4 + s (s < 4) or
+    // 32 kb + 16 + 4 g4 + s - 4
+    auto crow = [&](int kb, int s) { return (uint32_t)(32 * kb + 16 * (s >> 2) + 4 * g4 + (s & 3)); };
+    float rq[RT][2][8], rm[2][8], ra[UA][4];
+    const int ht = tid - NTHR;
+    // dO of the chunk as B fragments in sO: bf16 through all the helper waves together (the lo half is 0 and unused);
+    // fp32 by columns, helper hw the column group hw (rows 4 g4 + j (+ 16 cb)).  Phi columns read 0.
+    Cols64 rO16;
+    float rO[DO_BF16 ? 1 : 4][4];
+    auto load_dO = [&](int n) {
+      const int t0 = n * C, L = min(C, T - t0);
+      if constexpr (DO_BF16) {
+        rO16.load(reinterpret_cast<const bf16_t*>(dO) + row_bthk(b, t0, h, T, H, V) + (phi ? 0 : vs * COLS), H * V * 2,
+                  phi ? 0 : L, ht);
+      } else {
+        const bufrsrc ro = make_buf(dO + row_bthk(b, t0, h, T, H, V), phi ? 0u : ((L - 1) * H + 1) * V * 4);
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-      // dO rows 16 cb .. are H*V apart; the descriptor ends right after row L-1's head h
-      const int r0 = 16 * cb;
-      const bufrsrc ro = make_buf(dO + row_bthk(b, t0 + r0, h, T, H, V),
-                                  (!phi && L > r0) ? ((L - 1 - r0) * H + 1) * V * (uint32_t)sizeof(TDO) : 0u);
+        for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t e = (uint32_t)((4 * g4 + j) * H * V + col);
-        if constexpr (DO_BF16) rO[cb][j] = __builtin_amdgcn_raw_buffer_load_b16(ro, e * 2, 0, 0);
-        else rO[cb][j] = buf_ld(ro, e * 4);
+          for (int j = 0; j < 4; ++j)
+            rO[cb][j] = buf_ld(ro, ((uint32_t)((16 * cb + 4 * g4 + j) * H) * V + vs * COLS + 16 * hw + r16) * 4);
       }
-    }
-  };
-  // the B fragments (k = c) of those rows; a bf16 dO has ol = 0
-  auto dO_frags = [&](const RawO (&rO)[4][4], uint4 (&oh)[2], uint4 (&ol)[2]) {
+    };
+    auto load_Q = [&](int n) {  // Qg^T rows i = 16 (hw RT + t) + r16: Qg[c][i]
+      const int t0 = n * C, L = min(C, T - t0);
+      const bufrsrc r = make_buf(Qg + row_bht(bh, t0, T, K), L * K * 4);  // rows past L read 0
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-      bfrag(f32x4{widen(rO[2 * kb][0]), widen(rO[2 * kb][1]), widen(rO[2 * kb][2]), widen(rO[2 * kb][3])},
-            f32x4{widen(rO[2 * kb + 1][0]), widen(rO[2 * kb + 1][1]), widen(rO[2 * kb + 1][2]),
-                  widen(rO[2 * kb + 1][3])},
-            oh[kb], ol[kb]);
-  };
-
-  if constexpr (HW) {
-    if (tid >= NTHR) {
-      constexpr int RT = ST / 4;  // Qg^T row tiles per helper wave
-      const int hw = w - 4, r16 = lane & 15;
-      // A fragment slot s of lane group g4 in k-block kb: chunk row c = 32 kb + 4 g4 + s (s < 4) or
-      // 32 kb + 16 + 4 g4 + s - 4
-      auto crow = [&](int kb, int s) { return (uint32_t)(32 * kb + 16 * (s >> 2) + 4 * g4 + (s & 3)); };
-      float rq[RT][2][8], rm[2][8];
-      RawO rO[4][4];
-      auto load_Q = [&](int n) {  // Qg^T rows i = 16 (hw RT + t) + r16: Qg[c][i]
-        const int t0 = n * C, L = min(C, T - t0);
-        const bufrsrc r = make_buf(Qg + row_bht(bh, t0, T, K), L * K * 4);  // rows past L read 0
-#pragma unroll
-        for (int t = 0; t < RT; ++t)
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int s = 0; s < 8; ++s)
-              rq[t][kb][s] = buf_ld(r, (crow(kb, s) * K + (uint32_t)(16 * (hw * RT + t) + r16)) * 4);
-      };
-      auto load_M = [&](int n) {  // M^T rows c' = 16 hw + r16: M[c][c'] (k-block 0 is zero for hw >= 2)
-        const bufrsrc r = make_buf(Mg + ((int64_t)bh * NT + n) * C * C, C * C * 4);
+      for (int t = 0; t < RT; ++t)
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int s = 0; s < 8; ++s)
-            rm[kb][s] = (kb == 0 && hw >= 2) ? 0.f : buf_ld(r, (crow(kb, s) * C + (uint32_t)(16 * hw + r16)) * 4);
-      };
-      const int ocol = vs * COLS + 16 * hw + r16;  // the column group whose dO this wave loads
-      auto publish_O = [&]() {
-        uint4 oh[2], ol[2];
-        dO_frags(rO, oh, ol);
+            rq[t][kb][s] = buf_ld(r, (crow(kb, s) * K + (uint32_t)(16 * (hw * RT + t) + r16)) * 4);
+    };
+    auto load_M = [&](int n) {  // M^T rows c' = 16 hw + r16: M[c][c'] (k-block 0 is zero for hw >= 2)
+      const bufrsrc r = make_buf(Mg + ((int64_t)bh * NT + n) * C * C, C * C * 4);
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+          rm[kb][s] = (kb == 0 && hw >= 2) ? 0.f : buf_ld(r, (crow(kb, s) * C + (uint32_t)(16 * hw + r16)) * 4);
+    };
+    const int ocol = vs * COLS + 16 * hw + r16;  // this lane's column of the group whose dX this wave forms
+    const StageLane sl(tid - NTHR);
+    auto load_A = [&](int n) {  // A^T (rows s, k = c): A[c][s]
+      const bufrsrc r = make_buf(Ag + ((int64_t)bh * NT + n) * C * C, C * C * 4);
+#pragma unroll
+      for (int u = 0; u < UA; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ra[u][j] = buf_ld(r, (uint32_t)((trit_k0(sl, u) + j) * C + trit_row(sl, u)) * 4);
+    };
+    auto stage_A = [&]() {
+#pragma unroll
+      for (int u = 0; u < UA; ++u) put_unit(sAt, sl.off + sl.doff(u), ra[u][0], ra[u][1], ra[u][2], ra[u][3]);
+    };
+    // dX = A^T d delta of this wave's column group, from the state waves' published fragments (map groups: none)
+    auto product_X = [&](int n) {
+      f32x4 X[4];
+#pragma unroll
+      for (int sb = 0; sb < 4; ++sb) X[sb] = zero4();
+      uint4 dh_[2], dl_[2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        dh_[kb] = sDD[((hw * 2 + kb) * 2) * 64 + lane];
+        dl_[kb] = sDD[((hw * 2 + kb) * 2 + 1) * 64 + lane];
+      }
+      // step s: the tiles of k-block 0 (0, 2), then of k-block 1 (1, 3, 4, 5)
+      mfma_pipe<NTRI, 2>(
+          [&](int st, uint4& ah, uint4& al) { afrag(sAt, st < 2 ? 2 * st : st < 4 ? 2 * st - 3 : st, lane, ah, al); },
+          [&](int st, const uint4& ah, const uint4& al) {
+            const int sb = st < 2 ? st : st - 2, kb = st < 2 ? 0 : 1;
+            X[sb] = mma3(ah, al, dh_[kb], dl_[kb], X[sb]);
+          });
+      st_tiles<V>(dXl, (int64_t)bh * NT + n, ocol, lane, X);
+    };
+    auto publish_O = [&]() {
+      if constexpr (DO_BF16) {
+        rO16.publish(sO, 2 * 64, ht);
+      } else {
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-          sO[((hw * 2 + kb) * 2) * 64 + lane] = oh[kb];
-          if constexpr (!DO_BF16) sO[((hw * 2 + kb) * 2 + 1) * 64 + lane] = ol[kb];
+          uint4 oh, ol;
+          bfrag(f32x4{rO[2 * kb][0], rO[2 * kb][1], rO[2 * kb][2], rO[2 * kb][3]},
+                f32x4{rO[2 * kb + 1][0], rO[2 * kb + 1][1], rO[2 * kb + 1][2], rO[2 * kb + 1][3]}, oh, ol);
+          sO[((hw * 2 + kb) * 2) * 64 + lane] = oh;
+          sO[((hw * 2 + kb) * 2 + 1) * 64 + lane] = ol;
         }
-      };
-      uint4 foh[4][2], fol[4][2];  // dO fragments of all four column groups
-      auto read_O = [&]() {
+      }
+    };
+    uint4 foh[4][2], fol[4][2];  // dO fragments of all four column groups
+    auto read_O = [&]() {
 #pragma unroll
-        for (int sw = 0; sw < 4; ++sw)
+      for (int sw = 0; sw < 4; ++sw)
 #pragma unroll
-          for (int kb = 0; kb < 2; ++kb) {
-            foh[sw][kb] = sO[((sw * 2 + kb) * 2) * 64 + lane];
-            if constexpr (!DO_BF16) fol[sw][kb] = sO[((sw * 2 + kb) * 2 + 1) * 64 + lane];
-          }
-      };
-      auto prod = [&](const uint4& ah, const uint4& al, int sw, int kb, f32x4 acc) {
-        if constexpr (DO_BF16) return mma2(ah, al, foh[sw][kb], acc);
-        else return mma3(ah, al, foh[sw][kb], fol[sw][kb], acc);
-      };
-      auto product_A = [&]() {  // M^T dO (row tile hw) -> sPA
-        uint4 mh[2], ml[2];
+        for (int kb = 0; kb < 2; ++kb) {
+          foh[sw][kb] = sO[((sw * 2 + kb) * 2) * 64 + lane];
+          if constexpr (!DO_BF16) fol[sw][kb] = sO[((sw * 2 + kb) * 2 + 1) * 64 + lane];
+        }
+    };
+    auto prod = [&](const uint4& ah, const uint4& al, int sw, int kb, f32x4 acc) {
+      if constexpr (DO_BF16) return mma2(ah, al, foh[sw][kb], acc);
+      else return mma3(ah, al, foh[sw][kb], fol[sw][kb], acc);
+    };
+    auto product_A = [&]() {  // M^T dO (row tile hw) -> sPA
+      uint4 mh[2], ml[2];
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) split8v(rm[kb], mh[kb], ml[kb]);
+      for (int kb = 0; kb < 2; ++kb) split8v(rm[kb], mh[kb], ml[kb]);
+#pragma unroll
+      for (int sw = 0; sw < 4; ++sw) {
+        f32x4 acc = zero4();
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          if (kb == 0 && hw >= 2) continue;  // M^T[c'][c] = 0 for c < c'
+          acc = prod(mh[kb], ml[kb], sw, kb, acc);
+        }
+        sPA[(sw * 4 + hw) * 64 + lane] = acc;
+      }
+    };
+    auto product_B = [&]() {  // Qg^T dO (row tiles hw RT ..) -> sPB
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        uint4 qh[2], ql[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) split8v(rq[t][kb], qh[kb], ql[kb]);
 #pragma unroll
         for (int sw = 0; sw < 4; ++sw) {
           f32x4 acc = zero4();
 #pragma unroll
-          for (int kb = 0; kb < 2; ++kb) {
-            if (kb == 0 && hw >= 2) continue;  // M^T[c'][c] = 0 for c < c'
-            acc = prod(mh[kb], ml[kb], sw, kb, acc);
-          }
-          sPA[(sw * 4 + hw) * 64 + lane] = acc;
+          for (int kb = 0; kb < 2; ++kb) acc = prod(qh[kb], ql[kb], sw, kb, acc);
+          sPB[(sw * ST + hw * RT + t) * 64 + lane] = acc;
         }
-      };
-      auto product_B = [&]() {  // Qg^T dO (row tiles hw RT ..) -> sPB
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-          uint4 qh[2], ql[2];
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb) split8v(rq[t][kb], qh[kb], ql[kb]);
-#pragma unroll
-          for (int sw = 0; sw < 4; ++sw) {
-            f32x4 acc = zero4();
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) acc = prod(qh[kb], ql[kb], sw, kb, acc);
-            sPB[(sw * ST + hw * RT + t) * 64 + lane] = acc;
-          }
-        }
-      };
-      const int nl = n1 - 1;
-      load_dO(nl, ocol, rO);
-      load_M(nl);
-      load_Q(nl);
-      publish_O();
-      __syncthreads();  // prologue 1: dO fragments of chunk nl
-      read_O();
-      product_A();
-      if (nl > n0) {
-        load_dO(nl - 1, ocol, rO);
-        load_M(nl - 1);
       }
-      __syncthreads();  // prologue 2: M^T dO of chunk nl
-      for (int n = nl; n >= n0; --n) {
-        // phase 1: Qg^T dO of chunk n; dO fragments of chunk n - 1
-        product_B();
-        if (n > n0) {
-          load_Q(n - 1);
-          publish_O();
-        }
-        __syncthreads();
-        // phase 2: M^T dO of chunk n - 1
-        if (n > n0) {
-          read_O();
-          product_A();
-          if (n - 1 > n0) {
-            load_dO(n - 2, ocol, rO);
-            load_M(n - 2);
-          }
-        }
-        __syncthreads();
-      }
-      return;
+    };
+    const int nl = n1 - 1;
+    load_dO(nl);
+    load_M(nl);
+    load_A(nl);
+    load_Q(nl);
+    publish_O();
+    __syncthreads();  // prologue 1: dO fragments of chunk nl
+    read_O();
+    product_A();
+    if (nl > n0) {
+      load_dO(nl - 1);
+      load_M(nl - 1);
     }
+    __syncthreads();  // prologue 2: M^T dO of chunk nl
+    for (int n = nl; n >= n0; --n) {
+      // phase 1: A^T of chunk n staged; Qg^T dO of chunk n; dO fragments of chunk n - 1
+      stage_A();
+      if (n > n0) load_A(n - 1);
+      product_B();
+      if (n > n0) {
+        load_Q(n - 1);
+        publish_O();
+      }
+      __syncthreads();
+      // phase 2: dX of chunk n; M^T dO of chunk n - 1
+      if (real) product_X(n);
+      if (n > n0) {
+        read_O();
+        product_A();
+        if (n - 1 > n0) {
+          load_dO(n - 2);
+          load_M(n - 2);
+        }
+      }
+      __syncthreads();
+    }
+    return;
   }
 
   const int col = vs * COLS + 16 * w + (lane & 15);  // >= V: a Phi column (its dO is zero)
-  float rM[HW ? 1 : UM][4], rQ[HW ? 1 : UN][4], rWt[UN][4], rE = 0.f;
-  RawO rO[4][4];
+  const RowStage<K> stK(tid);
+  const StageLane sl(tid);
   float4 rKn[UN];
-  auto load_p1 = [&](int n) {  // M^T and Kf of chunk n
+  float rWt[UN][4], rE = 0.f;
+  auto load_p1 = [&](int n) {  // Kf of chunk n
     const int t0 = n * C, L = min(C, T - t0);
-    if constexpr (!HW) {
-      const bufrsrc rm = make_buf(Mg + ((int64_t)bh * NT + n) * C * C, C * C * 4);  // M[c][c'] row-major
-#pragma unroll
-      for (int u = 0; u < UM; ++u) {
-        const Unit x = unit<C>(tid + NTHR * u);  // row = c' (the d delta index), k = c
-#pragma unroll
-        for (int j = 0; j < 4; ++j) rM[u][j] = buf_ld(rm, ((x.k0 + j) * C + x.row) * 4);
-      }
-    }
-    const bufrsrc rk = make_buf(Kf + row_bht(bh, t0, T, K), L * K * 4);
-#pragma unroll
-    for (int u = 0; u < UN; ++u) {
-      const Unit x = unit<K>(tid + NTHR * u);
-      rKn[u] = buf_ld4(rk, (x.row * K + x.k0) * 4);
-    }
+    stK.load(make_buf(Kf + row_bht(bh, t0, T, K), L * K * 4), rKn);  // rows past L read 0
   };
-  auto load_p2 = [&](int n) {  // Qg^T, W^T, dO rows of this lane, e^{g_last} of chunk n
+  auto load_p2 = [&](int n) {  // W^T, g_last of chunk n
     const int t0 = n * C, L = min(C, T - t0);
-    const bufrsrc rq = make_buf(Qg + row_bht(bh, t0, T, K), L * K * 4);
     const bufrsrc rw = make_buf(W + row_bht(bh, t0, T, K), L * K * 4);
-#pragma unroll
-    for (int u = 0; u < UN; ++u) {
-      const Unit x = unit<C>(tid + NTHR * u);  // row = i, k = c
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t o = ((x.k0 + j) * K + x.row) * 4;
-        if constexpr (!HW) rQ[u][j] = buf_ld(rq, o);
-        rWt[u][j] = buf_ld(rw, o);
-      }
-    }
-    if constexpr (!HW) load_dO(n, col, rO);
-    {  // raw g_last of the chunk; the exponential is taken when staging, so no wait sits here
-      const bufrsrc rg = make_buf(gc + row_bthk(b, t0 + L - 1, h, T, H, K), K * 4);  // lanes >= K read 0
-      rE = buf_ld(rg, tid * 4);
-    }
-  };
-  auto stage_p1 = [&]() {
-    if constexpr (!HW) {
-#pragma unroll
-      for (int u = 0; u < UM; ++u) put_unit(sM, unit<C>(tid + NTHR * u).off, rM[u][0], rM[u][1], rM[u][2], rM[u][3]);
-    }
+    const uint32_t o = (uint32_t)(sl.k0() * K + sl.r) * 4;
 #pragma unroll
     for (int u = 0; u < UN; ++u)
-      put_unit(sKn, unit<K>(tid + NTHR * u).off, rKn[u].x, rKn[u].y, rKn[u].z, rKn[u].w);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) rWt[u][j] = buf_ld(rw, o + (j * K + 16 * u) * 4);
+    // raw g_last of the chunk; the exponential is taken when staging, so no wait sits here
+    const bufrsrc rg = make_buf(gc + row_bthk(b, t0 + L - 1, h, T, H, K), K * 4);  // lanes >= K read 0
+    rE = buf_ld(rg, tid * 4);
+  };
+  auto stage_p1 = [&]() {
+    stK.put(sKn, rKn);
   };
   auto stage_p2 = [&]() {
 #pragma unroll
-    for (int u = 0; u < UN; ++u) {
-      const int off = unit<C>(tid + NTHR * u).off;
-      if constexpr (!HW) put_unit(sQ, off, rQ[u][0], rQ[u][1], rQ[u][2], rQ[u][3]);
-      put_unit(sWt, off, rWt[u][0], rWt[u][1], rWt[u][2], rWt[u][3]);
-    }
+    for (int u = 0; u < UN; ++u) put_unit(sWt, sl.off + sl.doff(u), rWt[u][0], rWt[u][1], rWt[u][2], rWt[u][3]);
     if (tid < K) sE[tid] = fexp2(rE);
   };
 
@@ -993,21 +1137,16 @@ __global__ __launch_bounds__(HW ? 2 * state_threads(V) : state_threads(V)) void 
   load_p1(n1 - 1);
   stage_p1();
   load_p2(n1 - 1);
-  if constexpr (HW) __syncthreads();  // the helpers' first barrier
+  __syncthreads();  // the helpers' first barrier
   __syncthreads();
   for (int n = n1 - 1; n >= n0; --n) {
-    const int t0 = n * C, L = min(C, T - t0);
     if (real) {
       const int64_t e0 = ((int64_t)bh * NT + n) * K * V;
 #pragma unroll
       for (int ib = 0; ib < ST; ++ib) st_state4<K, V, (HM & HB_DH) != 0>(dhbuf, e0, ib, g4, col, dS[ib]);
     }
 
-    // dO of this chunk as B fragments (k = c), kept for both phases
-    uint4 oh[2], ol[2];
-    if constexpr (!HW) dO_frags(rO, oh, ol);
-
-    // ---- phase 1: d delta = M^T dO + Kf dS   (reads sM, sKn; fills sQ, sWt with chunk n)
+    // ---- phase 1: d delta = M^T dO + Kf dS   (reads sPA, sKn; fills sWt with chunk n)
     stage_p2();
     if (n > n0) load_p1(n - 1);
     f32x4 dD[4];
@@ -1015,83 +1154,46 @@ __global__ __launch_bounds__(HW ? 2 * state_threads(V) : state_threads(V)) void 
       uint4 bh_[KB], bl_[KB];
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) bfrag(dS[2 * kb], dS[2 * kb + 1], bh_[kb], bl_[kb]);
-      if constexpr (HW) {
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) dD[cb] = sPA[(w * 4 + cb) * 64 + lane];
-        // step m: Kf dS (kb = m / 4, cb = m % 4)
-        mfma_pipe<4 * KB, 2>([&](int st, uint4& ah, uint4& al) { afrag(sKn, (st & 3) * KB + (st >> 2), lane, ah, al); },
-                             [&](int st, const uint4& ah, const uint4& al) {
-                               dD[st & 3] = mma3(ah, al, bh_[st >> 2], bl_[st >> 2], dD[st & 3]);
-                             });
-      } else {
+      for (int cb = 0; cb < 4; ++cb) dD[cb] = sPA[(w * 4 + cb) * 64 + lane];
+      // step m: Kf dS (kb = m / 4, cb = m % 4)
+      mfma_pipe<4 * KB, 2>([&](int st, uint4& ah, uint4& al) { afrag(sKn, (st & 3) * KB + (st >> 2), lane, ah, al); },
+                           [&](int st, const uint4& ah, const uint4& al) {
+                             dD[st & 3] = mma3(ah, al, bh_[st >> 2], bl_[st >> 2], dD[st & 3]);
+                           });
+    }
+    uint4 dh_[2], dl_[2];  // the B fragments of d delta
+    bfrag(dD[0], dD[1], dh_[0], dl_[0]);
+    bfrag(dD[2], dD[3], dh_[1], dl_[1]);
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) dD[cb] = zero4();
-        // steps 0..5: M^T dO over the nonzero tiles (cb, kb): (0,0) (1,0) (0,1) (1,1) (2,1) (3,1)
-        // (M^T[c'][c] = M[c][c'] = 0 for c < c'); then Kf dS (kb = m / 4, cb = m % 4)
-        mfma_pipe<6 + 4 * KB, 2>(
-            [&](int st, uint4& ah, uint4& al) {
-              if (st < 6) {
-                const int cb = st < 2 ? st : st - 2, kb = st < 2 ? 0 : 1;
-                afrag(sM, cb * 2 + kb, lane, ah, al);
-              } else {
-                const int m = st - 6;
-                afrag(sKn, (m & 3) * KB + (m >> 2), lane, ah, al);
-              }
-            },
-            [&](int st, const uint4& ah, const uint4& al) {
-              if (st < 6) {
-                const int cb = st < 2 ? st : st - 2, kb = st < 2 ? 0 : 1;
-                dD[cb] = DO_BF16 ? mma2(ah, al, oh[kb], dD[cb]) : mma3(ah, al, oh[kb], ol[kb], dD[cb]);
-              } else {
-                const int m = st - 6, cb = m & 3, kb = m >> 2;
-                dD[cb] = mma3(ah, al, bh_[kb], bl_[kb], dD[cb]);
-              }
-            });
-      }
-      if (real) {  // in the dd_off layout (rows past L are 0)
-        const bufrsrc rd = make_buf(dDl + ((int64_t)bh * NT + n) * C * V, C * V * 4);
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dD[cb]), rd,
-                                                 (uint32_t)(((col >> 4) * 4 + cb) * 64 + lane) * 16, 0, 0);
-      }
+    for (int kb = 0; kb < 2; ++kb) {  // published for the helpers' dX
+      sDD[((w * 2 + kb) * 2) * 64 + lane] = dh_[kb];
+      sDD[((w * 2 + kb) * 2 + 1) * 64 + lane] = dl_[kb];
     }
     __syncthreads();
 
-    // ---- phase 2: dS <- e dS + Qg^T dO - W^T d delta   (reads sQ, sWt; fills sM, sKn with n-1)
+    // ---- phase 2: dS <- e dS + Qg^T dO - W^T d delta   (reads sPB, sWt; fills sKn with n-1)
     if (n > n0) {
       stage_p1();
       load_p2(n - 1);
     }
-    {
-      uint4 dh_[2], dl_[2];
-      bfrag(-dD[0], -dD[1], dh_[0], dl_[0]);
-      bfrag(-dD[2], -dD[3], dh_[1], dl_[1]);
 #pragma unroll
-      for (int ib = 0; ib < ST; ++ib) {
-        const float4 e = *reinterpret_cast<const float4*>(sE + 16 * ib + 4 * g4);
-        dS[ib] = f32x4{e.x * dS[ib][0], e.y * dS[ib][1], e.z * dS[ib][2], e.w * dS[ib][3]};
-        if constexpr (HW) dS[ib] += sPB[(w * ST + ib) * 64 + lane];
-      }
-      if constexpr (HW) {
-        // step s: dS[ib] -= W^T d delta (kb = s / ST, ib = s % ST)
-        mfma_pipe<2 * ST, 2>([&](int st, uint4& ah, uint4& al) { afrag(sWt, (st % ST) * 2 + st / ST, lane, ah, al); },
-                             [&](int st, const uint4& ah, const uint4& al) {
-                               dS[st % ST] = mma3(ah, al, dh_[st / ST], dl_[st / ST], dS[st % ST]);
-                             });
-      } else {
-        // step s: kb = s / (2 ST), ib = (s / 2) % ST, operand Qg^T (even s, B = dO) or W^T (odd s)
-        mfma_pipe<4 * ST, 2>(
-            [&](int st, uint4& ah, uint4& al) {
-              afrag((st & 1) ? sWt : sQ, ((st >> 1) % ST) * 2 + st / (2 * ST), lane, ah, al);
-            },
-            [&](int st, const uint4& ah, const uint4& al) {
-              const int kb = st / (2 * ST), ib = (st >> 1) % ST;
-              if (st & 1) dS[ib] = mma3(ah, al, dh_[kb], dl_[kb], dS[ib]);
-              else dS[ib] = DO_BF16 ? mma2(ah, al, oh[kb], dS[ib]) : mma3(ah, al, oh[kb], ol[kb], dS[ib]);
-            });
-      }
+    for (int kb = 0; kb < 2; ++kb) {  // rounding is symmetric: the fragments of -d delta
+      constexpr uint32_t sg = 0x80008000u;
+      dh_[kb] = uint4{dh_[kb].x ^ sg, dh_[kb].y ^ sg, dh_[kb].z ^ sg, dh_[kb].w ^ sg};
+      dl_[kb] = uint4{dl_[kb].x ^ sg, dl_[kb].y ^ sg, dl_[kb].z ^ sg, dl_[kb].w ^ sg};
     }
+#pragma unroll
+    for (int ib = 0; ib < ST; ++ib) {
+      const float4 e = *reinterpret_cast<const float4*>(sE + 16 * ib + 4 * g4);
+      dS[ib] = f32x4{e.x * dS[ib][0], e.y * dS[ib][1], e.z * dS[ib][2], e.w * dS[ib][3]};
+      dS[ib] += sPB[(w * ST + ib) * 64 + lane];
+    }
+    // step s: dS[ib] -= W^T d delta (kb = s / ST, ib = s % ST)
+    mfma_pipe<2 * ST, 2>([&](int st, uint4& ah, uint4& al) { afrag(sWt, (st % ST) * 2 + st / ST, lane, ah, al); },
+                         [&](int st, const uint4& ah, const uint4& al) {
+                           dS[st % ST] = mma3(ah, al, dh_[st / ST], dl_[st / ST], dS[st % ST]);
+                         });
     __syncthreads();
   }
   // the cotangent entering the group: d h0 (first group), the cotangent leaving group NG-2 (the last
@@ -1127,22 +1229,19 @@ __global__ __launch_bounds__(state_threads(V)) void state_combine_kernel(GroupPl
                                                                             int dir) {
   constexpr int COLS = state_cols(V), NTHR = state_threads(V), NV = V / COLS;
   constexpr int KB = K / 32, ST = K / 16, LD = V + K;
-  static_assert((K * K / 4) % NTHR == 0, "staging units per thread");
-  constexpr int UP = K * K / 4 / NTHR;  // staging units per thread of Phi
+  static_assert(NTHR == 256, "RowStage");
+  using PhiStage = RowStage<K, K, LD>;
+  const PhiStage stP(threadIdx.x);
   __shared__ __attribute__((aligned(16))) bf16_t sP[(K / 16) * KB * TILE];
   int bh, vs;
   xcd_map(blockIdx.x, NV, BH, bh, vs);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g4 = lane >> 4;
   const int col = vs * COLS + 16 * w + (lane & 15);
-  float4 rP[UP];
+  float4 rP[PhiStage::UN];
   float rPsi[ST][4];
   auto load = [&](int g) {
     const float* m = P.Mg + ((int64_t)bh * P.NG + g) * K * LD;
-#pragma unroll
-    for (int u = 0; u < UP; ++u) {
-      const Unit x = unit<K>(tid + NTHR * u);
-      rP[u] = *reinterpret_cast<const float4*>(m + x.row * LD + V + x.k0);
-    }
+    stP.load(make_buf(m + V, (uint32_t)((K - 1) * LD + K) * 4), rP);
 #pragma unroll
     for (int ib = 0; ib < ST; ++ib)
 #pragma unroll
@@ -1159,8 +1258,7 @@ __global__ __launch_bounds__(state_threads(V)) void state_combine_kernel(GroupPl
   load(g0);
   for (int i = 0; i < count; ++i) {
     const int g = g0 + i * dir;
-#pragma unroll
-    for (int u = 0; u < UP; ++u) put_unit(sP, unit<K>(tid + NTHR * u).off, rP[u].x, rP[u].y, rP[u].z, rP[u].w);
+    stP.put(sP, rP);
     f32x4 acc[ST];
 #pragma unroll
     for (int ib = 0; ib < ST; ++ib) acc[ib] = f32x4{rPsi[ib][0], rPsi[ib][1], rPsi[ib][2], rPsi[ib][3]};

@@ -23,8 +23,8 @@ NO_BACKWARD = 8  # stage bit: no backward follows, intermediates only the backwa
 def state_groups(B: int, T: int, H: int, K: int, V: int) -> int:
     """Chunk groups of the serial state passes at this shape (1: one pass, readout fused)."""
     return int(_lib.load().kdn_mem_state_groups(B, T, H, K, V))
-# bit 2: the chunk-parallel backward of every chunk (products with h and dh; solves and gradients of
-# the chunks the forward factored); bits 4 | 8: the exact path's solves and gradients (flagged chunks)
+# bit 2: the chunk-parallel backward of every chunk (products with h, dh and dX; gradients of the
+# chunks the forward factored); bits 4 | 8: the exact path's gradients (flagged chunks)
 BWD_STAGES = ((1, "mem_state_bwd"), (2, "mem_bwd_chunk"), (12, "mem_bwd_exact"))
 # bits 1 | 2 in one call: with one chunk group the reverse pass runs in segments and each finished
 # segment's chunk backward overlaps the next segment's pass on a second stream (same results)
@@ -35,8 +35,8 @@ DEFAULT_OVERLAP = True
 
 
 # What a training forward keeps for its backward; both give bit-identical gradients.
-#  "save"       the intra-chunk WY factors, A^T and the per-chunk states h, delta (kdn_mem_saved_size
-#               bytes, ~4.1 KB per token-head at K = V = 128: 1.21 GB at B4 T4096 H18), so the backward
+#  "save"       the intra-chunk WY factors and the per-chunk states h, delta (kdn_mem_saved_size
+#               bytes, ~3.6 KB per token-head at K = V = 128: 1.06 GB at B4 T4096 H18), so the backward
 #               starts at its own passes;
 #  "recompute"  only the op's inputs (and the in-op norm's rstd), as the reference's autograd functions
 #               keep them (iso_kdn_chunk.py:2206, diag_kdn_chunk.py:3253); the backward first rebuilds
