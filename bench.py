@@ -267,7 +267,7 @@ def run_layer_frontends(steps: int, warmup: int, B: int, T: int, H: int, K: int)
             step()
         torch.cuda.synchronize()
     N = B * T * D
-    nbytes = {"short_conv_fwd": 2 * N * 2, "short_conv_bwd": 3 * N * 2,  # per q|k|v group launch
+    nbytes = {"short_conv_fwd": 6 * N * 2, "short_conv_bwd": 9 * N * 2,  # one launch for the packed q|k|v
               "rms_norm_gated_fwd": 3 * N * 2 + B * T * H * 4, "rms_norm_gated_bwd": 5 * N * 2 + B * T * H * 4}
     out = {}
     for tag, nb in nbytes.items():

@@ -356,6 +356,11 @@ int kdn_xent_bwd(void* dlogits, int64_t dlogits_row_stride, const float* dlosses
 int kdn_short_conv_fwd(const void* x, int x_bf16, int64_t x_stride_b, int64_t x_stride_t, const void* weight,
                        int w_bf16, int B, int T, int D, int W, void* y, int64_t y_stride_b, int64_t y_stride_t,
                        hipStream_t stream);
+/* The packed q|k|v convolution (iso_kdn_chunk.py:47-478) in one launch: x [B,T,3D] and weight [3D,W]
+ * contiguous, q, k, v [B,T,D] contiguous, D the width of one of the three.  Equal to three calls of
+ * kdn_short_conv_fwd on the groups. */
+int kdn_qkv_conv_fwd(const void* x, int x_bf16, const void* weight, int w_bf16, int B, int T, int D, int W, void* q,
+                     void* k, void* v, hipStream_t stream);
 /* One token of the short convolution from carried inputs (decoding; no reference counterpart: the
  * reference refuses caching, model.py:104,184).  x [B,1,D] with batch stride x_stride_b, tail [B,3,D]
  * (the 3 earlier inputs, x's dtype, row stride D, batch stride tail_stride_b), y [B,1,D]:
@@ -364,7 +369,8 @@ int kdn_short_conv_fwd(const void* x, int x_bf16, int64_t x_stride_b, int64_t x_
 int kdn_short_conv_step(const void* x, int x_bf16, int64_t x_stride_b, void* tail, int64_t tail_stride_b,
                         const void* weight, int w_bf16, int B, int D, void* y, int64_t y_stride_b,
                         hipStream_t stream);
-/* Workspace of kdn_short_conv_bwd when dweight is requested: f32 partials per (b, 64-token block). */
+/* Workspace of kdn_short_conv_bwd when dweight is requested: f32 partials per
+ * (b, block of 32 to 128 tokens). */
 size_t kdn_short_conv_bwd_workspace_size(int B, int T, int D);
 /* Backward (iso_kdn_chunk.py:127-254, 379-437): g = dy * silu'(y) with the preactivation y recomputed
  * (rounded to x's dtype when round_preactivation, as the reference's raw_y buffer is),
@@ -374,6 +380,12 @@ int kdn_short_conv_bwd(const void* x, int x_bf16, int64_t x_stride_b, int64_t x_
                        int w_bf16, const void* dy, int64_t dy_stride_b, int64_t dy_stride_t, int B, int T, int D,
                        int W, int round_preactivation, void* dx, int64_t dx_stride_b, int64_t dx_stride_t,
                        void* dweight, void* workspace, size_t workspace_bytes, hipStream_t stream);
+/* Backward of kdn_qkv_conv_fwd (the preactivation rounded to x's dtype): dq, dk, dv [B,T,D] contiguous,
+ * each may be NULL (zero); dx [B,T,3D] and dweight [3D,W] contiguous, each may be NULL.  Workspace:
+ * kdn_short_conv_bwd_workspace_size(B, T, 3 D). */
+int kdn_qkv_conv_bwd(const void* x, int x_bf16, const void* weight, int w_bf16, const void* dq, const void* dk,
+                     const void* dv, int B, int T, int D, int W, void* dx, void* dweight, void* workspace,
+                     size_t workspace_bytes, hipStream_t stream);
 
 /* RMS norm over wide dense rows (the model's block norm FusedRMSNorm, reference
  * lit_gpt/rmsnorm.py:1182-1216, no residual / dropout): y = x rsqrt(mean(x^2) + eps) * weight, f32 math,

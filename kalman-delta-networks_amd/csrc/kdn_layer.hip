@@ -21,8 +21,6 @@
 namespace {
 
 constexpr int kConvW = 4;       // kernel width (the reference requires 4)
-constexpr int kConvRun = 8;     // tokens per inner run of a thread
-constexpr int kConvBlockT = 64; // tokens per backward thread (one dw partial per 64-token block)
 
 template <typename T>
 __device__ __forceinline__ void ld8v(const T* p, float* f);
@@ -82,53 +80,156 @@ __device__ __forceinline__ void ld_taps(const TW* p, float (&wt)[8][kConvW]) {
 #pragma unroll
     for (int j = 0; j < kConvW; ++j) wt[c][j] = f[c * kConvW + j];
 }
-// 8 channels of row t, or zeros outside [0, T): the load is unconditional (row clamped), so the
-// compiler issues every row's load before the first use
-template <typename TX>
-__device__ __forceinline__ void ld_row(const TX* base, int64_t st, int t, int T, float* f) {
-  const int tc = t < 0 ? 0 : (t >= T ? T - 1 : t);
-  ld8v(base + (int64_t)tc * st, f);
-  const bool ok = t >= 0 && t < T;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) f[c] = ok ? f[c] : 0.f;
+// ---------------------------------------------------------------------------
+// Short convolution over whole sequences.  Wave = 64 x 4 consecutive channels of one run of R tokens,
+// block = 4 consecutive runs.  A wave walks its run in groups of 4 rows: the next group's rows are in
+// flight while the current one is computed, the 3 earlier rows stay in registers, so every row is
+// loaded once (and 3 per run again) and rows outside the sequence are found by wave-uniform tests.
+// Held by the vector ALU and by the loads in flight rather than by the bytes: with one thread per 8
+// tokens x 8 channels (11 rows loaded and 11 gradients formed for 8, 248 registers in the backward) and an
+// IEEE reciprocal in the sigmoid, one group of B4 T4096 D2304 bf16 took 45.6 us forward and 91.6 backward; now
+// 35.6 / 61.3, and the packed q|k|v in one launch 87 / 143 (137 / 275 as three of the former; 95 / 142 at the
+// copy rate of 4.8 TB/s).
+// ---------------------------------------------------------------------------
+constexpr int kConvRuns = 4;   // runs per block
+constexpr int kConvC = 4;      // channels per lane
+// Tokens per run: 32 (9% of the backward's rows formed twice) while that leaves at least 8 waves per CU;
+// shorter sequences take shorter runs down to 8, for more waves.
+inline int conv_run(int B, int T, int D) {
+  int R = 32;
+  while (R > 8 && (int64_t)B * ((T + R - 1) / R) * ((D + 255) / 256) < 2048) R /= 2;
+  return R;
 }
-__device__ __forceinline__ float silu_grad(float y) {  // d/dy [y sigmoid(y)]
-  const float s = sigmoidf(y);
-  return s * (1.f + y * (1.f - s));
+inline int conv_blocks(int T, int R) { return (T + kConvRuns * R - 1) / (kConvRuns * R); }
+
+// a * sigmoid(a)'s sigmoid: the hardware reciprocal and one Newton step (as close to 1 / d as the IEEE
+// division, in about half its instructions); above 2^126 the raw reciprocal (0 at infinity) stands
+__device__ __forceinline__ float sigmoid_nr(float x) {
+  const float d = 1.f + __expf(-x), r = __builtin_amdgcn_rcpf(d);
+  const float rn = __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+  return d < 0x1p126f ? rn : r;
+}
+template <typename T>
+struct Row4;  // 4 channels of a row as loaded
+template <>
+struct Row4<bf16_t> {
+  uint2 v;
+  __device__ __forceinline__ void load(const bf16_t* p) { v = *reinterpret_cast<const uint2*>(p); }
+  __device__ __forceinline__ void get(float* f) const {
+    f[0] = __uint_as_float(v.x << 16), f[1] = __uint_as_float(v.x & 0xffff0000u);
+    f[2] = __uint_as_float(v.y << 16), f[3] = __uint_as_float(v.y & 0xffff0000u);
+  }
+};
+template <>
+struct Row4<float> {
+  float4 v;
+  __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const float4*>(p); }
+  __device__ __forceinline__ void get(float* f) const { f[0] = v.x, f[1] = v.y, f[2] = v.z, f[3] = v.w; }
+};
+// Nontemporal stores: an output is not read again by the kernel, and left in the caches it would push
+// out rows about to be read (B4 T4096 D2304 bf16: 36.3 -> 35.6 us forward, 67.8 -> 61.3 backward).
+__device__ __forceinline__ void st4v(bf16_t* p, const float* f) {
+  const u32x2 v = {(uint32_t)f2bf(f[0]) | ((uint32_t)f2bf(f[1]) << 16),
+                   (uint32_t)f2bf(f[2]) | ((uint32_t)f2bf(f[3]) << 16)};
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x2*>(p));
+}
+__device__ __forceinline__ void st4v(float* p, const float* f) {
+  const f32x4 v = {f[0], f[1], f[2], f[3]};
+  __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(p));
+}
+template <typename TW>
+__device__ __forceinline__ void ld_taps4(const TW* p, float (&wt)[kConvC][kConvW]) {
+#pragma unroll
+  for (int c = 0; c < kConvC; ++c) {
+    Row4<TW> r;
+    r.load(p + c * kConvW);
+    r.get(wt[c]);
+  }
+}
+// rows t .. t+3 of a wave's 4 channels; rows outside [0, T) are clamped (zeroed by get_rows)
+template <typename TX>
+__device__ __forceinline__ void load_rows(const TX* base, int64_t st, int t, int T, Row4<TX> (&r)[4]) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) r[u].load(base + (int64_t)min(max(t + u, 0), T - 1) * st);
+}
+template <typename TX>
+__device__ __forceinline__ void get_rows(const Row4<TX> (&r)[4], int t, int T, float (*f)[kConvC]) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) r[u].get(f[u]);
+  if (t >= 0 && t + 4 <= T) return;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (t + u < 0 || t + u >= T)
+#pragma unroll
+      for (int c = 0; c < kConvC; ++c) f[u][c] = 0.f;
+}
+// the preactivation of row u of a group, xw = the 3 rows before the group and its 4
+__device__ __forceinline__ float conv_pre(const float (&wt)[kConvC][kConvW], const float (*xw)[kConvC], int u, int c) {
+  float a = 0.f;
+#pragma unroll
+  for (int j = 0; j < kConvW; ++j) a += wt[c][j] * xw[u + j][c];
+  return a;
 }
 
-// ---------------------------------------------------------------------------
-// Short convolution forward.  Thread = (b, 8-token run, 8-channel group), channel groups
-// fastest.  y_t = silu(sum_j w_j x_{t-3+j}), x_{<0} = 0, fp32 then rounded to y's dtype.
-// ---------------------------------------------------------------------------
+// The 1 or 3 equal channel groups of a call: x, weight, dx and dweight hold them side by side (row of
+// n x D channels), y and dy are a tensor each.
+template <typename TX>
+struct ConvGroups {
+  TX* p[3];
+  int n;
+};
+// block -> (group, channel block of it, token block, batch row)
+struct ConvBlock {
+  int g, cb, blk, b, NB;
+  __device__ __forceinline__ ConvBlock(int n, int T, int D, int R) : NB((T + kConvRuns * R - 1) / (kConvRuns * R)) {
+    const int NCB = (D + 255) / 256, c = blockIdx.x % (n * NCB), r = blockIdx.x / (n * NCB);
+    g = c / NCB, cb = c % NCB, blk = r % NB, b = r / NB;
+  }
+};
+
+// y_t = silu(sum_j w_j x_{t-3+j}), x_{<0} = 0, fp32 then rounded to y's dtype.
 template <typename TX, typename TW>
 __global__ __launch_bounds__(256) void short_conv_fwd_kernel(const TX* __restrict__ x, int64_t xsb, int64_t xst,
-                                                             const TW* __restrict__ w, int B, int T, int D,
-                                                             TX* __restrict__ y, int64_t ysb, int64_t yst) {
-  const int CG = D / 8, NR = (T + kConvRun - 1) / kConvRun;
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= (int64_t)B * NR * CG) return;
-  const int cg = (int)(gid % CG), run = (int)((gid / CG) % NR), b = (int)(gid / ((int64_t)CG * NR));
-  const int d0 = 8 * cg, t0 = run * kConvRun;
-  float wt[8][kConvW];
-  ld_taps(w + (int64_t)d0 * kConvW, wt);
-  constexpr int NX = kConvRun + kConvW - 1;
-  float xr[NX][8];
+                                                             const TW* __restrict__ w, int T, int D, int R,
+                                                             ConvGroups<TX> y, int64_t ysb, int64_t yst) {
+  const ConvBlock cbk(y.n, T, D, R);
+  const int b = cbk.b, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int d0 = cbk.cb * 256 + kConvC * (threadIdx.x & 63), t0 = (cbk.blk * kConvRuns + wv) * R;
+  if (d0 >= D || t0 >= T) return;
+  float wt[kConvC][kConvW], xw[7][kConvC];
+  const TX* xb = x + (int64_t)b * xsb + cbk.g * D + d0;
+  TX* yb = y.p[cbk.g] + (int64_t)b * ysb + d0;
+  Row4<TX> nx[4];
+  load_rows(xb, xst, t0 - 4, T, nx);
+  ld_taps4(w + (int64_t)(cbk.g * D + d0) * kConvW, wt);
+  {
+    float f[4][kConvC];
+    get_rows(nx, t0 - 4, T, f);
 #pragma unroll
-  for (int r = 0; r < NX; ++r) ld_row(x + (int64_t)b * xsb + d0, xst, t0 - (kConvW - 1) + r, T, xr[r]);
+    for (int u = 0; u < 3; ++u)
 #pragma unroll
-  for (int u = 0; u < kConvRun; ++u) {
-    const int t = t0 + u;
-    if (t >= T) break;
-    float o[8];
+      for (int c = 0; c < kConvC; ++c) xw[u][c] = f[u + 1][c];
+  }
+  load_rows(xb, xst, t0, T, nx);
+  const int te = min(t0 + R, T);
+  for (int t = t0; t < te; t += 4) {
+    get_rows(nx, t, T, xw + 3);
+    load_rows(xb, xst, t + 4, T, nx);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      float a = 0.f;
+    for (int u = 0; u < 4; ++u) {
+      if (t + u >= te) break;
+      float o[kConvC];
 #pragma unroll
-      for (int j = 0; j < kConvW; ++j) a += wt[c][j] * xr[u + j][c];
-      o[c] = a * sigmoidf(a);
+      for (int c = 0; c < kConvC; ++c) {
+        const float a = conv_pre(wt, xw, u, c);
+        o[c] = a * sigmoid_nr(a);
+      }
+      st4v(yb + (int64_t)(t + u) * yst, o);
     }
-    st8v(y + (int64_t)b * ysb + (int64_t)t * yst + d0, o);
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int c = 0; c < kConvC; ++c) xw[u][c] = xw[u + 4][c];
   }
 }
 
@@ -161,7 +262,7 @@ __global__ __launch_bounds__(256) void short_conv_step_kernel(const TX* __restri
     float a = 0.f;
 #pragma unroll
     for (int j = 0; j < kConvW; ++j) a += wt[c][j] * xr[j][c];
-    o[c] = a * sigmoidf(a);
+    o[c] = a * sigmoid_nr(a);
   }
   st8v(y + (int64_t)b * ysb + d0, o);
 #pragma unroll
@@ -169,93 +270,100 @@ __global__ __launch_bounds__(256) void short_conv_step_kernel(const TX* __restri
 }
 
 // ---------------------------------------------------------------------------
-// Short convolution backward.  Block = 32 channel groups x 8 runs of 8 tokens (one 64-token
-// block of 256 channels); thread = (run, channel group), all its loads issued at once.
-// g_t = dy_t silu'(y_t) with y the recomputed preactivation (rounded to x's dtype when round_y,
-// as the reference's raw_y buffer is), dx_t = sum_j w_j g_{t+3-j}, and the dw_j partial
-// sum_t g_t x_{t-3+j} over the 64 tokens, reduced over the runs in LDS in a fixed order
-// -> part[b * NB + blk][d][j].
+// Short convolution backward, in the forward's walk.  g_t = dy_t silu'(y_t) with y the recomputed
+// preactivation (rounded to x's dtype when round_y, as the reference's raw_y buffer is),
+// dx_t = sum_j w_j g_{t+3-j} (so a group's dx rows come 3 rows late, and the run ends with 3 rows of
+// the next one), and the dw_j partial sum_t g_t x_{t-3+j} over the block's tokens, its runs added in
+// LDS in a fixed order -> part[b * NB + blk][d][j].
 // ---------------------------------------------------------------------------
-constexpr int kConvCG = 32;  // channel groups per backward block
 template <typename TX, typename TW>
 __global__ __launch_bounds__(256) void short_conv_bwd_kernel(const TX* __restrict__ x, int64_t xsb, int64_t xst,
-                                                             const TW* __restrict__ w, const TX* __restrict__ dy,
-                                                             int64_t dsb, int64_t dst, int B, int T, int D,
+                                                             const TW* __restrict__ w, ConvGroups<const TX> dys,
+                                                             int64_t dsb, int64_t dst, int T, int D, int R,
                                                              int round_y, TX* __restrict__ dx, int64_t gsb,
                                                              int64_t gst, float* __restrict__ part) {
-  __shared__ float s_dw[kConvBlockT / kConvRun][kConvCG * 8 * kConvW];
-  const int CG = D / 8, NB = (T + kConvBlockT - 1) / kConvBlockT, NCB = (CG + kConvCG - 1) / kConvCG;
-  const int cb = blockIdx.x % NCB, blk = (blockIdx.x / NCB) % NB, b = blockIdx.x / (NCB * NB);
-  const int lc = threadIdx.x % kConvCG, run = threadIdx.x / kConvCG;
-  const int cg = cb * kConvCG + lc, d0 = 8 * cg, t0 = blk * kConvBlockT + run * kConvRun;
-  const bool active = cg < CG && t0 < T;
-  float dw[8][kConvW];
+  __shared__ float4 s_dw[kConvRuns][kConvC][64];
+  const ConvBlock cbk(dys.n, T, D, R);
+  const int b = cbk.b, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int d0 = cbk.cb * 256 + kConvC * lane, t0 = (cbk.blk * kConvRuns + wv) * R;
+  const TX* dy = dys.p[cbk.g];
+  float dw[kConvC][kConvW] = {};
+  if (d0 < D && t0 < T) {
+    float wt[kConvC][kConvW], xw[7][kConvC], gw[7][kConvC];
+    const TX* xb = x + (int64_t)b * xsb + cbk.g * D + d0;
+    const TX* db = dy ? dy + (int64_t)b * dsb + d0 : xb;  // dy absent: zeros
+    if (!dy) dst = xst;
+    Row4<TX> nx[4], nd[4];
+    load_rows(xb, xst, t0 - 4, T, nx);
+    ld_taps4(w + (int64_t)(cbk.g * D + d0) * kConvW, wt);
+    {
+      float f[4][kConvC];
+      get_rows(nx, t0 - 4, T, f);
 #pragma unroll
-  for (int c = 0; c < 8; ++c)
+      for (int u = 0; u < 3; ++u)
 #pragma unroll
-    for (int j = 0; j < kConvW; ++j) dw[c][j] = 0.f;
-  if (active) {
-    float wt[8][kConvW];
-    ld_taps(w + (int64_t)d0 * kConvW, wt);
-    constexpr int NX = kConvRun + 2 * (kConvW - 1);  // x rows t0-3 .. t0+run+2
-    constexpr int NG = kConvRun + kConvW - 1;        // g at t0 .. t0+run+2
-    float xr[NX][8], dyr[NG][8];
-#pragma unroll
-    for (int r = 0; r < NX; ++r) ld_row(x + (int64_t)b * xsb + d0, xst, t0 - (kConvW - 1) + r, T, xr[r]);
-    if (dy) {
-#pragma unroll
-      for (int r = 0; r < NG; ++r) ld_row(dy + (int64_t)b * dsb + d0, dst, t0 + r, T, dyr[r]);
-    } else {
-#pragma unroll
-      for (int r = 0; r < NG; ++r)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) dyr[r][c] = 0.f;
+        for (int c = 0; c < kConvC; ++c) xw[u][c] = f[u + 1][c], gw[u][c] = 0.f;
     }
-    float gr[NG][8];
-#pragma unroll
-    for (int r = 0; r < NG; ++r)
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        float a = 0.f;
-#pragma unroll
-        for (int j = 0; j < kConvW; ++j) a += wt[c][j] * xr[r + j][c];
-        if (round_y) a = as_stored<TX>(a);
-        gr[r][c] = dyr[r][c] * silu_grad(a);
+    load_rows(xb, xst, t0, T, nx);
+    load_rows(db, dst, t0, T, nd);
+    const int te = min(t0 + R, T);
+    // groups of the run, then the 3 rows after it, of which only g is wanted
+    for (int t = t0; t < te + 3; t += 4) {
+      get_rows(nx, t, T, xw + 3);
+      get_rows(nd, t, dy ? T : 0, gw + 3);
+      const bool more = t + 4 < te + 3;
+      if (more) {
+        load_rows(xb, xst, t + 4, T, nx);
+        load_rows(db, dst, t + 4, T, nd);
       }
 #pragma unroll
-    for (int u = 0; u < kConvRun; ++u) {
-      const int t = t0 + u;
-      if (t >= T) break;
-      float o[8];
+      for (int u = 0; u < 4; ++u) {
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        float a = 0.f;
+        for (int c = 0; c < kConvC; ++c) {
+          float a = conv_pre(wt, xw, u, c);
+          if (round_y) a = as_stored<TX>(a);
+          const float s = sigmoid_nr(a);
+          gw[u + 3][c] *= s * (1.f + a * (1.f - s));
+        }
+        if (t + u < te) {
 #pragma unroll
-        for (int j = 0; j < kConvW; ++j) a += wt[c][j] * gr[u + kConvW - 1 - j][c];
-        o[c] = a;
+          for (int c = 0; c < kConvC; ++c)
 #pragma unroll
-        for (int j = 0; j < kConvW; ++j) dw[c][j] += gr[u][c] * xr[u + j][c];
+            for (int j = 0; j < kConvW; ++j) dw[c][j] += gw[u + 3][c] * xw[u + j][c];
+        }
+        const int r = t + u - 3;  // dx row
+        if (dx && r >= t0 && r < te) {
+          float o[kConvC];
+#pragma unroll
+          for (int c = 0; c < kConvC; ++c) {
+            float a = 0.f;
+#pragma unroll
+            for (int j = 0; j < kConvW; ++j) a += wt[c][j] * gw[u + 3 - j][c];
+            o[c] = a;
+          }
+          st4v(dx + (int64_t)b * gsb + (int64_t)r * gst + cbk.g * D + d0, o);
+        }
       }
-      if (dx) st8v(dx + (int64_t)b * gsb + (int64_t)t * gst + d0, o);
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+#pragma unroll
+        for (int c = 0; c < kConvC; ++c) xw[u][c] = xw[u + 4][c], gw[u][c] = gw[u + 4][c];
     }
   }
   if (!part) return;
-  // [run][tap][channel-in-group][group]: consecutive lanes (groups) hit consecutive banks
 #pragma unroll
-  for (int c = 0; c < 8; ++c)
-#pragma unroll
-    for (int j = 0; j < kConvW; ++j) s_dw[run][(j * 8 + c) * kConvCG + lc] = dw[c][j];
+  for (int c = 0; c < kConvC; ++c) s_dw[wv][c][lane] = float4{dw[c][0], dw[c][1], dw[c][2], dw[c][3]};
   __syncthreads();
-  // this block's 256 channels x 4 taps, summed over the 8 runs in order
-  for (int e = threadIdx.x; e < kConvCG * 8 * kConvW; e += 256) {
-    const int q = e / kConvW, j = e % kConvW;  // q = local channel (group-major), j = tap
-    const int lg = q / 8, c = q % 8, d = cb * kConvCG * 8 + q;
-    if (d >= D) continue;
-    float acc = 0.f;
+  // wave c sums channel c of every lane's 4 over the runs, in order
+  const int d = cbk.cb * 256 + kConvC * lane + wv;
+  if (d >= D) return;
+  float4 a = s_dw[0][wv][lane];
 #pragma unroll
-    for (int r = 0; r < kConvBlockT / kConvRun; ++r) acc += s_dw[r][(j * 8 + c) * kConvCG + lg];
-    part[((int64_t)b * NB + blk) * D * kConvW + (int64_t)d * kConvW + j] = acc;
+  for (int r = 1; r < kConvRuns; ++r) {
+    const float4 v = s_dw[r][wv][lane];
+    a.x += v.x, a.y += v.y, a.z += v.z, a.w += v.w;
   }
+  *reinterpret_cast<float4*>(part + (((int64_t)b * cbk.NB + cbk.blk) * dys.n * D + cbk.g * D + d) * kConvW) = a;
 }
 
 // out[j] = sum_p part[p * n + j] in a fixed order: block = 16 columns x 16 stripes of p, the
@@ -482,26 +590,45 @@ bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 extern "C" {
 
 // ---------------------------------------------------------------------------------- short conv
+static int conv_fwd(const void* x, int x_bf16, int64_t x_stride_b, int64_t x_stride_t, const void* weight, int w_bf16,
+                    int B, int T, int D, int W, int n, void* const* y, int64_t y_stride_b, int64_t y_stride_t,
+                    hipStream_t stream) {
+  if (B < 0 || T < 0 || D <= 0 || W != kConvW || D % 8 != 0 || !x || !weight) return KDN_ERR_ARG;
+  if (!al16(x) || !al16(weight) || x_stride_t % 8 != 0 || x_stride_b % 8 != 0 || y_stride_t % 8 != 0 ||
+      y_stride_b % 8 != 0)
+    return KDN_ERR_ARG;
+  for (int g = 0; g < n; ++g)
+    if (!y[g] || !al16(y[g])) return KDN_ERR_ARG;
+  if (B == 0 || T == 0) return 0;
+  const int R = conv_run(B, T, n * D);
+  const dim3 grid((unsigned)((int64_t)B * conv_blocks(T, R) * n * ((D + 255) / 256)));
+  auto launch = [&](auto tx, auto tw) {
+    using TX = decltype(tx);
+    using TW = decltype(tw);
+    ConvGroups<TX> yg{{}, n};
+    for (int g = 0; g < n; ++g) yg.p[g] = (TX*)y[g];
+    hipLaunchKernelGGL((short_conv_fwd_kernel<TX, TW>), grid, dim3(256), 0, stream, (const TX*)x, x_stride_b,
+                       x_stride_t, (const TW*)weight, T, D, R, yg, y_stride_b, y_stride_t);
+  };
+  if (x_bf16 && w_bf16) launch(bf16_t{}, bf16_t{});
+  else if (x_bf16) launch(bf16_t{}, float{});
+  else if (w_bf16) launch(float{}, bf16_t{});
+  else launch(float{}, float{});
+  KDN_CHECK_LAUNCH();
+  return 0;
+}
+
 int kdn_short_conv_fwd(const void* x, int x_bf16, int64_t x_stride_b, int64_t x_stride_t, const void* weight,
                        int w_bf16, int B, int T, int D, int W, void* y, int64_t y_stride_b, int64_t y_stride_t,
                        hipStream_t stream) {
-  if (B < 0 || T < 0 || D <= 0 || W != kConvW || D % 8 != 0 || !x || !weight || !y) return KDN_ERR_ARG;
-  if (!al16(x) || !al16(y) || !al16(weight) || x_stride_t % 8 != 0 || x_stride_b % 8 != 0 || y_stride_t % 8 != 0 ||
-      y_stride_b % 8 != 0)
-    return KDN_ERR_ARG;
-  if (B == 0 || T == 0) return 0;
-  const int64_t threads = (int64_t)B * ((T + kConvRun - 1) / kConvRun) * (D / 8);
-  const dim3 grid((unsigned)((threads + 255) / 256));
-#define KDN_CONV_FWD(TX, TW)                                                                                         \
-  hipLaunchKernelGGL((short_conv_fwd_kernel<TX, TW>), grid, dim3(256), 0, stream, (const TX*)x, x_stride_b,         \
-                     x_stride_t, (const TW*)weight, B, T, D, (TX*)y, y_stride_b, y_stride_t)
-  if (x_bf16 && w_bf16) KDN_CONV_FWD(bf16_t, bf16_t);
-  else if (x_bf16) KDN_CONV_FWD(bf16_t, float);
-  else if (w_bf16) KDN_CONV_FWD(float, bf16_t);
-  else KDN_CONV_FWD(float, float);
-#undef KDN_CONV_FWD
-  KDN_CHECK_LAUNCH();
-  return 0;
+  return conv_fwd(x, x_bf16, x_stride_b, x_stride_t, weight, w_bf16, B, T, D, W, 1, &y, y_stride_b, y_stride_t, stream);
+}
+
+int kdn_qkv_conv_fwd(const void* x, int x_bf16, const void* weight, int w_bf16, int B, int T, int D, int W, void* q,
+                     void* k, void* v, hipStream_t stream) {
+  void* const y[3] = {q, k, v};
+  return conv_fwd(x, x_bf16, (int64_t)T * 3 * D, 3 * (int64_t)D, weight, w_bf16, B, T, D, W, 3, y, (int64_t)T * D, D,
+                  stream);
 }
 
 int kdn_short_conv_step(const void* x, int x_bf16, int64_t x_stride_b, void* tail, int64_t tail_stride_b,
@@ -527,48 +654,70 @@ int kdn_short_conv_step(const void* x, int x_bf16, int64_t x_stride_b, void* tai
   return 0;
 }
 
+// (the packed q|k|v convolution: D = the packed width 3 x D)
 size_t kdn_short_conv_bwd_workspace_size(int B, int T, int D) {
   if (B <= 0 || T <= 0 || D <= 0) return 0;
-  const int64_t NB = (T + kConvBlockT - 1) / kConvBlockT;
-  return (size_t)((int64_t)B * NB * D * kConvW) * sizeof(float);
+  return (size_t)((int64_t)B * conv_blocks(T, conv_run(B, T, D)) * D * kConvW) * sizeof(float);
+}
+
+static int conv_bwd(const void* x, int x_bf16, int64_t x_stride_b, int64_t x_stride_t, const void* weight, int w_bf16,
+                    int n, const void* const* dy, int64_t dy_stride_b, int64_t dy_stride_t, int B, int T, int D, int W,
+                    int round_preactivation, void* dx, int64_t dx_stride_b, int64_t dx_stride_t, void* dweight,
+                    void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  if (B < 0 || T < 0 || D <= 0 || W != kConvW || D % 8 != 0 || !x || !weight) return KDN_ERR_ARG;
+  if (!al16(x) || !al16(weight) || (dx && !al16(dx)) || x_stride_t % 8 || x_stride_b % 8 ||
+      (dx && (dx_stride_t % 8 || dx_stride_b % 8)))
+    return KDN_ERR_ARG;
+  for (int g = 0; g < n; ++g)
+    if (dy[g] && (!al16(dy[g]) || dy_stride_t % 8 || dy_stride_b % 8)) return KDN_ERR_ARG;
+  if (B == 0 || T == 0) return 0;
+  if (dweight && (!workspace || workspace_bytes < kdn_short_conv_bwd_workspace_size(B, T, n * D) ||
+                  !al16(workspace)))
+    return KDN_ERR_ARG;
+  const int R = conv_run(B, T, n * D), NB = conv_blocks(T, R);
+  const dim3 grid((unsigned)((int64_t)B * NB * n * ((D + 255) / 256)));
+  float* part = dweight ? (float*)workspace : nullptr;
+  if (!dweight && !dx) return 0;
+  auto launch = [&](auto tx, auto tw) {
+    using TX = decltype(tx);
+    using TW = decltype(tw);
+    ConvGroups<const TX> dg{{}, n};
+    for (int g = 0; g < n; ++g) dg.p[g] = (const TX*)dy[g];
+    hipLaunchKernelGGL((short_conv_bwd_kernel<TX, TW>), grid, dim3(256), 0, stream, (const TX*)x, x_stride_b,
+                       x_stride_t, (const TW*)weight, dg, dy_stride_b, dy_stride_t, T, D, R, round_preactivation,
+                       (TX*)dx, dx_stride_b, dx_stride_t, part);
+  };
+  if (x_bf16 && w_bf16) launch(bf16_t{}, bf16_t{});
+  else if (x_bf16) launch(bf16_t{}, float{});
+  else if (w_bf16) launch(float{}, bf16_t{});
+  else launch(float{}, float{});
+  KDN_CHECK_LAUNCH();
+  if (dweight) {
+    const int64_t cols = (int64_t)n * D * kConvW;
+    const dim3 rg((unsigned)((cols + 15) / 16));
+    if (w_bf16)
+      hipLaunchKernelGGL((sum_partials_kernel<bf16_t>), rg, dim3(256), 0, stream, part, B * NB, cols, (bf16_t*)dweight);
+    else
+      hipLaunchKernelGGL((sum_partials_kernel<float>), rg, dim3(256), 0, stream, part, B * NB, cols, (float*)dweight);
+    KDN_CHECK_LAUNCH();
+  }
+  return 0;
 }
 
 int kdn_short_conv_bwd(const void* x, int x_bf16, int64_t x_stride_b, int64_t x_stride_t, const void* weight,
                        int w_bf16, const void* dy, int64_t dy_stride_b, int64_t dy_stride_t, int B, int T, int D,
                        int W, int round_preactivation, void* dx, int64_t dx_stride_b, int64_t dx_stride_t,
                        void* dweight, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-  if (B < 0 || T < 0 || D <= 0 || W != kConvW || D % 8 != 0 || !x || !weight) return KDN_ERR_ARG;
-  if (!al16(x) || !al16(weight) || (dy && !al16(dy)) || (dx && !al16(dx)) || x_stride_t % 8 || x_stride_b % 8 ||
-      (dy && (dy_stride_t % 8 || dy_stride_b % 8)) || (dx && (dx_stride_t % 8 || dx_stride_b % 8)))
-    return KDN_ERR_ARG;
-  if (B == 0 || T == 0) return 0;
-  if (dweight && (!workspace || workspace_bytes < kdn_short_conv_bwd_workspace_size(B, T, D) ||
-                  !al16(workspace)))
-    return KDN_ERR_ARG;
-  const int NB = (T + kConvBlockT - 1) / kConvBlockT, NCB = (D / 8 + kConvCG - 1) / kConvCG;
-  const dim3 grid((unsigned)((int64_t)B * NB * NCB));
-  float* part = dweight ? (float*)workspace : nullptr;
-  if (!dweight && !dx) return 0;
-#define KDN_CONV_BWD(TX, TW)                                                                                       \
-  hipLaunchKernelGGL((short_conv_bwd_kernel<TX, TW>), grid, dim3(256), 0, stream, (const TX*)x, x_stride_b,       \
-                     x_stride_t, (const TW*)weight, (const TX*)dy, dy_stride_b, dy_stride_t, B, T, D,             \
-                     round_preactivation, (TX*)dx, dx_stride_b, dx_stride_t, part)
-  if (x_bf16 && w_bf16) KDN_CONV_BWD(bf16_t, bf16_t);
-  else if (x_bf16) KDN_CONV_BWD(bf16_t, float);
-  else if (w_bf16) KDN_CONV_BWD(float, bf16_t);
-  else KDN_CONV_BWD(float, float);
-#undef KDN_CONV_BWD
-  KDN_CHECK_LAUNCH();
-  if (dweight) {
-    const int64_t n = (int64_t)D * kConvW;
-    const dim3 rg((unsigned)((n + 15) / 16));
-    if (w_bf16)
-      hipLaunchKernelGGL((sum_partials_kernel<bf16_t>), rg, dim3(256), 0, stream, part, B * NB, n, (bf16_t*)dweight);
-    else
-      hipLaunchKernelGGL((sum_partials_kernel<float>), rg, dim3(256), 0, stream, part, B * NB, n, (float*)dweight);
-    KDN_CHECK_LAUNCH();
-  }
-  return 0;
+  return conv_bwd(x, x_bf16, x_stride_b, x_stride_t, weight, w_bf16, 1, &dy, dy_stride_b, dy_stride_t, B, T, D, W,
+                  round_preactivation, dx, dx_stride_b, dx_stride_t, dweight, workspace, workspace_bytes, stream);
+}
+
+int kdn_qkv_conv_bwd(const void* x, int x_bf16, const void* weight, int w_bf16, const void* dq, const void* dk,
+                     const void* dv, int B, int T, int D, int W, void* dx, void* dweight, void* workspace,
+                     size_t workspace_bytes, hipStream_t stream) {
+  const void* const dy[3] = {dq, dk, dv};
+  return conv_bwd(x, x_bf16, (int64_t)T * 3 * D, 3 * (int64_t)D, weight, w_bf16, 3, dy, (int64_t)T * D, D, B, T, D, W, 1,
+                  dx, (int64_t)T * 3 * D, 3 * (int64_t)D, dweight, workspace, workspace_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------------- gated norm

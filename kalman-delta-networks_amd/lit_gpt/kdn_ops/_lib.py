@@ -55,6 +55,8 @@ _SIGS = {
     "kdn_short_conv_step": "pilplpiiipls",
     "kdn_short_conv_bwd_workspace_size": "iii",
     "kdn_short_conv_bwd": "pillpiplliiiiipllppzs",
+    "kdn_qkv_conv_fwd": "pipiiiiippps",
+    "kdn_qkv_conv_bwd": "pipipppiiiipppzs",
     "kdn_rms_norm_fwd": "pipilifpps",
     "kdn_rms_norm_bwd_workspace_size": "li",
     "kdn_rms_norm_bwd": "pipipplipppzs",

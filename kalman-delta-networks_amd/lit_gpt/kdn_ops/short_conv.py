@@ -13,7 +13,7 @@ Drop-in for the two fixed-length entry points the reference layers call
 Semantics: y[t] = silu(sum_j w[j] x[t-3+j]) per channel, zero history before t = 0, width 4,
 no bias, f32 arithmetic rounded to x's dtype.  The packed backward follows the reference's
 kernel (``iso_kdn_chunk.py:127-254``): the preactivation is recomputed into x's dtype before
-silu' is taken, and the weight gradient is a fixed-order sum of per-(batch, 64-token block)
+silu' is taken, and the weight gradient is a fixed-order sum of per-(batch, token block)
 partials.  The per-tensor backward keeps the recomputed preactivation in f32 (FLA's
 backward is not part of the reference tree).  All arithmetic runs in ``libkdn_hip.so``.
 """
@@ -158,6 +158,16 @@ def _prepare_gradient(name, gradient, *, B, T, D, device, dtype):
     return gradient
 
 
+def _qkv_conv_fwd(x, weight, D):
+    """All three groups in one launch (a third of the launches, and one ramp-up and tail instead of three)."""
+    B, T, _ = x.shape
+    ys = tuple(torch.empty((B, T, D), device=x.device, dtype=x.dtype) for _ in range(GROUPS))
+    with torch.cuda.device(x.device):
+        _lib.call("kdn_qkv_conv_fwd", _lib.ptr(x), _lib.is_bf16(x), _lib.ptr(weight), _lib.is_bf16(weight), B, T, D,
+                  KERNEL_WIDTH, *map(_lib.ptr, ys), _lib.stream_of(x), tag="short_conv_fwd")
+    return ys
+
+
 class _QKVCausalConv1d(torch.autograd.Function):
     """Reference iso_kdn_chunk.py:440-465."""
 
@@ -166,7 +176,7 @@ class _QKVCausalConv1d(torch.autograd.Function):
         D = _validate_qkv_conv_inputs(x, weight)
         ctx.save_for_backward(x, weight)
         ctx.set_materialize_grads(False)
-        return tuple(_conv_fwd(x[..., g * D:(g + 1) * D], weight[g * D:(g + 1) * D]) for g in range(GROUPS))
+        return _qkv_conv_fwd(x, weight, D)
 
     @staticmethod
     @once_differentiable
@@ -180,9 +190,12 @@ class _QKVCausalConv1d(torch.autograd.Function):
                  for n, g in (("dq", dq), ("dk", dk), ("dv", dv))]
         dx = torch.empty_like(x)
         dw = torch.empty_like(weight)
-        for g in range(GROUPS):
-            _conv_bwd(x[..., g * D:(g + 1) * D], weight[g * D:(g + 1) * D], grads[g], dx[..., g * D:(g + 1) * D],
-                      dw[g * D:(g + 1) * D], round_preactivation=True)
+        ws_bytes = _lib.size("kdn_short_conv_bwd_workspace_size", B, T, GROUPS * D)
+        ws = torch.empty(max(ws_bytes // 4, 1), device=x.device, dtype=torch.float32)
+        with torch.cuda.device(x.device):
+            _lib.call("kdn_qkv_conv_bwd", _lib.ptr(x), _lib.is_bf16(x), _lib.ptr(weight), _lib.is_bf16(weight),
+                      *map(_lib.ptr, grads), B, T, D, KERNEL_WIDTH, _lib.ptr(dx), _lib.ptr(dw), _lib.ptr(ws), ws_bytes,
+                      _lib.stream_of(x), tag="short_conv_bwd")
         return dx, dw
 
 
@@ -191,7 +204,7 @@ def qkv_causal_conv1d(x: torch.Tensor, weight: torch.Tensor):
     iso_kdn_chunk.py:468-478).  T = 1 equals the reference's one-token update with a zero cache."""
     d = _validate_qkv_conv_inputs(x, weight)
     if not torch.is_grad_enabled() or not (x.requires_grad or weight.requires_grad):
-        return tuple(_conv_fwd(x[..., g * d:(g + 1) * d], weight[g * d:(g + 1) * d]) for g in range(GROUPS))
+        return _qkv_conv_fwd(x, weight, d)
     return _QKVCausalConv1d.apply(x, weight)
 
 
