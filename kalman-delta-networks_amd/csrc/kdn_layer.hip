@@ -390,18 +390,32 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restri
 }
 
 // ---------------------------------------------------------------------------
-// Gated RMS norm.  D/8 lanes per row, 8 elements per lane, 256/(D/8) rows per block.
+// Gated RMS norm.  D/8 lanes per row, 8 elements per lane, 256/(D/8) rows per block.  HBM-bound: 3 tensors
+// forward, 5 backward.  Nontemporal stores keep the outputs from pushing out rows about to be read:
+// B4 T4096 H18 d128 bf16 (75.5 MB per tensor) 46.7 -> 38 us forward, 79 -> 73 backward (6.0 / 5.2 TB/s).
 // ---------------------------------------------------------------------------
+template <typename T>
+__device__ __forceinline__ void st8n(T* p, const float* f) {
+  st4v(p, f);
+  st4v(p + 4, f + 4);
+}
+template <>
+__device__ __forceinline__ void st8n<bf16_t>(bf16_t* p, const float* f) {
+  u32x4 v;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = (uint32_t)f2bf(f[2 * q]) | ((uint32_t)f2bf(f[2 * q + 1]) << 16);
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+}
 __device__ __forceinline__ float row_sum(float v, int lanes) {
   for (int o = 1; o < lanes; o <<= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
 __device__ __forceinline__ float gate_act(float g, int act) {  // 0: sigmoid(g), 1: g sigmoid(g)
-  const float s = sigmoidf(g);
+  const float s = sigmoid_nr(g);
   return act == 0 ? s : g * s;
 }
 __device__ __forceinline__ float gate_grad(float g, int act) {
-  const float s = sigmoidf(g);
+  const float s = sigmoid_nr(g);
   return act == 0 ? s * (1.f - s) : s * (1.f + g * (1.f - s));
 }
 
@@ -426,7 +440,7 @@ __global__ __launch_bounds__(256) void rms_gated_fwd_kernel(const TX* __restrict
 #pragma unroll
   for (int c = 0; c < 8; ++c) o[c] = xv[c] * rs * wv[c] * gate_act(gv[c], act);
   if (!ok) return;
-  st8v(y + row * D + d0, o);
+  st8n(y + row * D + d0, o);
   if (sub == 0 && rstd) rstd[row] = rs;
 }
 
@@ -473,8 +487,8 @@ __global__ __launch_bounds__(256) void rms_gated_bwd_kernel(const TX* __restrict
         og[c] = dyv[c] * n[c] * wv[c] * gate_grad(gv[c], act);
         dwv[c] += dyv[c] * n[c] * av[c];
       }
-      if (dx) st8v(dx + row * D + d0, o);
-      if (dg) st8v(dg + row * D + d0, og);
+      if (dx) st8n(dx + row * D + d0, o);
+      if (dg) st8n(dg + row * D + d0, og);
     }
   }
   if (!part) return;
