@@ -320,6 +320,34 @@ int kdn_gemv(const void* x, int x_bf16, int64_t x_row_stride, const uint16_t* W,
              int K, int gated, void* y, int64_t y_row_stride, hipStream_t stream);
 
 /* ---------------------------------------------------------------- language-model loss */
+/* Decode projection with its surroundings, M <= 64 rows: y[m,n] = sum_k xn[m,k] W[n,k] (+ bias[n]), then
+ * (+ res[m,n]), everything bf16 with fp32 accumulation and one rounding of the result.  xn = x [M,K] (row
+ * stride x_row_stride), or with norm_weight [K] the RMS-normed row x rsqrt(mean x^2 + eps) norm_weight.
+ * gated: W is [W1; W2] [2N,K] (bias [2N]) and the product is silu(xn W1^T + b1) * (xn W2^T + b2) (SwiGLU).
+ * bias, res, norm_weight may be NULL; workspace may be NULL where its size (norm: with norm_weight) is 0.
+ * K % 8 == 0; x, W, norm_weight 16-byte aligned, x_row_stride % 8 == 0.
+ * No reference counterpart (the reference refuses caching, model.py:104,184). */
+size_t kdn_decode_proj_workspace_size(int M, int N, int K, int norm, int gated);
+int kdn_decode_proj(const void* x, int64_t x_row_stride, const void* norm_weight, float eps, const void* W,
+                    const void* bias, const void* res, int64_t res_row_stride, int M, int N, int K, int gated, void* y,
+                    int64_t y_row_stride, void* workspace, size_t workspace_bytes, hipStream_t stream);
+/* One token through a KDN mixer between its input and output projections, all bf16 but the fp32 gate
+ * parameters, precision and memory.  p [B, p_row_stride]: the packed input projection's rows, q | k | v (H K
+ * each) from element 0, the hidden vectors (K each) of the retention (off_f), diagonal omega (off_w) and
+ * output (off_g) gates, and at off_r: isotropic omega_raw [H] then r_raw [H], diagonal r_raw [H].  tail_q/k/v:
+ * the 3 carried convolution inputs (row stride tail_row_stride, batch stride tail_stride_b), conv_q/k/v their
+ * taps [H K, 4].  Wf, Wo (diagonal; bias bo or NULL), Wg (bias bg or NULL): [H K, K].  Short convolution,
+ * gates, gain, memory update as kdn_short_conv_step, kdn_iso_gate_fwd / kdn_diag_norm_fwd +
+ * kdn_diag_frontend_fwd, kdn_kalman_step, then the sigmoid-gated RMS norm (norm_weight [K], eps) -> y [B, H K].
+ * The carried inputs, precision ([B,H] or [B,H,K]) and memory [B,H,K,K] advance in place.  K in {64, 128}; memory, Wf, Wo, Wg
+ * 16-byte aligned, taps and y 8-byte. */
+int kdn_decode_mixer(const void* p, int64_t p_row_stride, int off_f, int off_w, int off_r, int off_g, void* tail_q,
+                     void* tail_k, void* tail_v, int64_t tail_stride_b, int64_t tail_row_stride, const void* conv_q,
+                     const void* conv_k, const void* conv_v, const void* Wf, const void* Wo, const void* bo,
+                     const void* Wg, const void* bg, const float* omega_bias, const float* r_bias, const float* A_log,
+                     const float* dt_bias, float omega_min, float r_min, float info_scale, float scale,
+                     float* precision, float* memory, const void* norm_weight, float eps, int iso, int B, int H, int K,
+                     void* y, hipStream_t stream);
 /* Fused cross-entropy forward, one row of logits per token.  Replaces cross_entropy_fwd_kernel
  * (lit_gpt/fused_cross_entropy.py:29-100) as launched by CrossEntropyLoss.forward (:156-260).
  * logits [n_rows, n_cols] with row stride logits_row_stride elements, logits_dtype 0 f32, 1 bf16,

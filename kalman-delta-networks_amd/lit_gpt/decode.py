@@ -5,8 +5,8 @@ KDN layer's history is a fixed-size state (``KDNLayerState``), so a decode step 
 any context length: the chunked scan consumes the prompt (``prefill``), then each ``step`` runs
 one token through every block, the mixers through ``kdn_kalman_step``.
 
-One decode step launches a few hundred small kernels (about 20 per block), so at small batch
-the step is bound by launch overhead, not by the GPU.  With ``use_graph=True`` the step is
+One decode step is a chain of small dependent kernels (5 per block for a bf16 model, ``decode_block``; about
+20 otherwise), so at small batch the step is bound by launch overhead as much as by the GPU.  With ``use_graph=True`` the step is
 captured once as a HIP graph (``torch.cuda.CUDAGraph``) over fixed buffers -- the token ids, the
 logits and every layer's state -- and each later step is one graph replay.  The decoder's layer
 states are in-place states (``KDNLayerState.inplace``): each layer advances its own buffers, the
@@ -40,7 +40,6 @@ class KDNDecoder:
         if self.state is None:
             self.state = [KDNLayerState(tuple(c.clone() for c in s.conv), s.memory.clone(), s.precision.clone(),
                                         s.seen_tokens, inplace=True) for s in state]
-            self.logits = torch.empty_like(logits[:, -1])
         else:
             self._assign(state)
             for s, n in zip(self.state, state):
@@ -57,7 +56,8 @@ class KDNDecoder:
     def _eager_step(self):
         # the states are in-place states: the layers advance their buffers themselves
         logits, _ = self.model(self.tokens, state=self.state, return_state=True)
-        self.logits.copy_(logits[:, -1])
+        # (captured, this tensor is the graph's own output buffer, rewritten by every replay)
+        self.logits = logits[:, -1]
 
     def _capture(self):
         # warm up (library handles, allocator) on a side stream without advancing the state
@@ -84,7 +84,7 @@ class KDNDecoder:
     @torch.no_grad()
     def step(self, tokens: torch.Tensor) -> torch.Tensor:
         """Feed one token per sequence (``tokens`` [B] or [B,1]); returns the next-token logits [B,V]
-        (a view of this decoder's buffer, overwritten by the next step)."""
+        (with the graph a view of its output buffer, overwritten by the next step)."""
         if self.state is None:
             raise RuntimeError("call prefill() before step()")
         self.tokens.copy_(tokens.view(self.B, 1))

@@ -142,7 +142,7 @@ class DiagonalKalmanDeltaNetwork(nn.Module):
             D, d = self.key_dim, self.head_k_dim
             w_in = packed_weight(self, "in_proj", (self.q_proj.weight, self.k_proj.weight, self.v_proj.weight,
                                                    self.f_proj[0].weight, self.omega_proj[0].weight,
-                                                   self.g_proj[0].weight))
+                                                   self.g_proj[0].weight, self.r_proj.weight))[:-H]
             yq, yk, yv, f_hidden, w_hidden, g_hidden = linear(hidden_states, w_in).split(
                 (D, D, self.value_dim, d, d, d), dim=-1)
             projections = (yq, yk, yv)

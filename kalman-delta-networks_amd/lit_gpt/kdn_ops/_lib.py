@@ -49,6 +49,9 @@ _SIGS = {
     "kdn_mem_step": "pppipipiiiifppis",
     "kdn_kalman_step": "pppipppppppiiiiiffppis",
     "kdn_gemv": "pilppiiiipls",
+    "kdn_decode_proj_workspace_size": "iiiii",
+    "kdn_decode_proj": "plpfpppliiiiplpzs",
+    "kdn_decode_mixer": "pliiiipppllppppppppppppffffpppfiiiips",
     "kdn_xent_fwd": "pilpiiifffllliippps",
     "kdn_xent_bwd": "plplpilppiiifffllls",
     "kdn_short_conv_fwd": "pillpiiiiiplls",
@@ -69,7 +72,7 @@ _SIZE_FNS = {"kdn_iso_gate_bwd_workspace_size", "kdn_iso_gain_workspace_size", "
              "kdn_diag_gain_workspace_size", "kdn_diag_front_saved_size",
              "kdn_diag_front_workspace_size", "kdn_mem_saved_size", "kdn_mem_bwd_workspace_size",
              "kdn_short_conv_bwd_workspace_size", "kdn_rms_norm_gated_bwd_workspace_size",
-             "kdn_rms_norm_bwd_workspace_size"}
+             "kdn_rms_norm_bwd_workspace_size", "kdn_decode_proj_workspace_size"}
 _CT = {"p": ctypes.c_void_p, "i": ctypes.c_int, "l": ctypes.c_int64, "f": ctypes.c_float,
        "z": ctypes.c_size_t, "s": ctypes.c_void_p}
 

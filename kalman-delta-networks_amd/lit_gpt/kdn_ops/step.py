@@ -164,4 +164,86 @@ def kdn_gemv(x, weight, bias=None, *, gated=False):
     return y.view(*lead, N)
 
 
-__all__ = ("kdn_memory_step", "kdn_kalman_step", "kdn_gemv")
+def _rows(name, t, n):
+    if t.dtype != torch.bfloat16 or t.ndim != 2 or t.shape[1] != n or t.stride(1) != 1:
+        raise ValueError(f"{name} must be bf16 rows of {n} elements, got {t.dtype} {tuple(t.shape)}")
+
+
+def kdn_decode_proj(x, weight, *, norm_weight=None, eps=0.0, bias=None, residual=None, gated=False):
+    """One decode projection with what surrounds it: [residual +] (RMS-normed) ``x`` @ ``weight``^T [+ bias],
+    all bf16 [rows, features], at most 64 rows, one rounding.  ``gated``: ``weight`` = [w1; w2], SwiGLU."""
+    K = x.shape[-1]
+    R = weight.shape[0]
+    N = R // 2 if gated else R
+    _rows("x", x, K)
+    _rows("weight", weight, K)
+    M = x.shape[0]
+    if M > 64 or K % 8 or not weight.is_contiguous() or (gated and R % 2):
+        raise ValueError("kdn_decode_proj takes at most 64 rows, K % 8 == 0 and a contiguous weight")
+    for name, t, n in (("norm_weight", norm_weight, K), ("bias", bias, R)):
+        if t is not None and (t.dtype != torch.bfloat16 or t.shape != (n,) or not t.is_contiguous()):
+            raise ValueError(f"{name} must be a contiguous bf16 [{n}] or None")
+    if residual is not None:
+        _rows("residual", residual, N)
+        if residual.shape[0] != M:
+            raise ValueError(f"residual must have {M} rows, got {residual.shape[0]}")
+    _lib.require_device(x, weight, norm_weight, bias, residual)
+    y = torch.empty((M, N), device=x.device, dtype=torch.bfloat16)
+    ws_bytes = _lib.size("kdn_decode_proj_workspace_size", M, N, K, int(norm_weight is not None), int(bool(gated)))
+    ws = torch.empty(ws_bytes // 4, device=x.device, dtype=torch.float32) if ws_bytes else None
+    with torch.cuda.device(x.device):
+        _lib.call("kdn_decode_proj", _lib.ptr(x), x.stride(0), _lib.ptr(norm_weight), float(eps), _lib.ptr(weight),
+                  _lib.ptr(bias), _lib.ptr(residual), residual.stride(0) if residual is not None else 0, M, N, K,
+                  int(bool(gated)), _lib.ptr(y), N, _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
+    return y
+
+
+def kdn_decode_mixer(p, offsets, tails, taps, Wf, Wo, bo, Wg, bg, omega_bias, r_bias, A_log, dt_bias, *, omega_min,
+                     r_min, info_scale, precision, memory, norm_weight, eps, iso):
+    """One token of a mixer between its projections (``kdn_decode_mixer`` of the C ABI): ``p`` [B, n] the packed
+    input projection, ``offsets`` the elements (f, w, r, g) of its parts after q | k | v, ``tails`` the carried
+    convolution inputs (isotropic one [B,3,3HK], diagonal three [B,3,HK]; advanced in place, as are
+    ``precision`` and ``memory``).  Returns the gated, normed output [B, H K]."""
+    B, H, K, V = memory.shape
+    n = H * K
+    off_f, off_w, off_r, off_g = offsets
+    _rows("p", p, p.shape[1])
+    if K != V or K not in (64, 128) or p.shape[0] != B or memory.dtype != torch.float32 or not memory.is_contiguous():
+        raise ValueError(f"memory must be a contiguous fp32 [{B},H,K,K] with K in (64, 128), got {tuple(memory.shape)}")
+    if p.shape[1] < max(3 * n, off_f + K, off_w + K, off_g + K, off_r + (2 * H if iso else H)):
+        raise ValueError("p is narrower than its parts")
+    if precision.shape != ((B, H) if iso else (B, H, K)) or precision.dtype != torch.float32 or not precision.is_contiguous():
+        raise ValueError("precision must be a contiguous fp32 tensor of the layer's precision shape")
+    width = 3 * n if iso else n
+    if len(tails) != (1 if iso else 3) or any(t.shape != (B, 3, width) or t.dtype != torch.bfloat16
+                                              or not t.is_contiguous() for t in tails):
+        raise ValueError("carried convolution inputs must be contiguous bf16 [B,3,channels]")
+    if len(taps) != len(tails) or any(w.shape != (width, 4) or w.dtype != torch.bfloat16 or not w.is_contiguous()
+                                      for w in taps):
+        raise ValueError("convolution taps must be contiguous bf16 [channels,4]")
+    for name, w, shape in (("Wf", Wf, (n, K)), ("Wo", Wo, (n, K)), ("bo", bo, (n,)), ("Wg", Wg, (n, K)), ("bg", bg, (n,)),
+                           ("norm_weight", norm_weight, (K,))):
+        if w is None and (name in ("bo", "bg") or (iso and name == "Wo")):
+            continue
+        if w.shape != shape or w.dtype != torch.bfloat16 or not w.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous bf16 tensor of shape {shape}")
+    for name, w, m in (("omega_bias", omega_bias, H), ("r_bias", r_bias, H), ("A_log", A_log, H), ("dt_bias", dt_bias, n)):
+        if w is None and not iso and name in ("omega_bias", "r_bias"):
+            continue
+        if w.numel() != m or w.dtype != torch.float32 or not w.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous fp32 tensor of {m} elements")
+    _lib.require_device(p, *tails, *taps, Wf, Wo, bo, Wg, bg, omega_bias, r_bias, A_log, dt_bias, precision, memory, norm_weight)
+    y = torch.empty((B, n), device=p.device, dtype=torch.bfloat16)
+    step = n if iso else 0  # the isotropic layer's q, k, v parts sit side by side in one tensor
+    ptrs = [[t.data_ptr() + 2 * step * i * m for i, t in enumerate(ts if len(ts) == 3 else ts * 3)]
+            for ts, m in ((tails, 1), (taps, 4))]
+    with torch.cuda.device(p.device):
+        _lib.call("kdn_decode_mixer", _lib.ptr(p), p.stride(0), off_f, off_w, off_r, off_g, *ptrs[0], 3 * width, width,
+                  *ptrs[1], _lib.ptr(Wf), _lib.ptr(Wo), _lib.ptr(bo), _lib.ptr(Wg), _lib.ptr(bg), _lib.ptr(omega_bias),
+                  _lib.ptr(r_bias), _lib.ptr(A_log), _lib.ptr(dt_bias), float(omega_min), float(r_min), float(info_scale),
+                  K ** -0.5, _lib.ptr(precision), _lib.ptr(memory), _lib.ptr(norm_weight), float(eps), int(iso), B, H, K,
+                  _lib.ptr(y), _lib.stream_of(p))
+    return y
+
+
+__all__ = ("kdn_memory_step", "kdn_kalman_step", "kdn_gemv", "kdn_decode_proj", "kdn_decode_mixer")

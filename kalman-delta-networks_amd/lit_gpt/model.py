@@ -25,7 +25,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from ._inference import linear, packed_weight, swiglu_gate, use_packed
+from ._inference import decode_block, decode_head, linear, packed_weight, swiglu_gate, use_packed
 from .config import Config
 
 
@@ -104,8 +104,10 @@ class GPT(nn.Module):
         for i, block in enumerate(self.transformer.h):
             x, new = block(x, None, max_seq_length, kv_cache=states[i], use_state=stateful)
             states[i] = new
-        x = self.transformer.ln_f(x)
-        logits = linear(x, self.lm_head.weight)
+        logits = decode_head(x, self.transformer.ln_f, self.lm_head, self) if stateful else None
+        if logits is None:
+            x = self.transformer.ln_f(x)
+            logits = linear(x, self.lm_head.weight)
         return (logits, states) if return_state else logits
 
     @classmethod
@@ -144,6 +146,10 @@ class Block(nn.Module):
         the state after these tokens (None otherwise)."""
         if input_pos is not None:
             raise ValueError("KDN mixers do not support KV caching")
+        if use_state and mask is None:  # the decode step: one token on an in-place state
+            y = decode_block(self, x, kv_cache)
+            if y is not None:
+                return y, kv_cache
         n_1 = self.norm_1(x)
         h, _, new_kv_cache = self.attn(n_1, attention_mask=mask, past_key_values=kv_cache, use_cache=use_state)
         if self.config.parallel_residual:
