@@ -71,7 +71,7 @@ def xent_forward(logits, labels, *, smoothing=0.0, logit_scale=1.0, lse_square_s
         lse = torch.empty(n_rows, dtype=torch.float32, device=logits.device)
     z_losses = None if split else torch.empty(n_rows, dtype=torch.float32, device=logits.device)
     if n_rows:
-        with torch.cuda.device(logits.device):
+        with _lib.on(logits.device):
             _lib.call("kdn_xent_fwd", _lib.ptr(logits), _dtype_code(logits), logits.stride(0), _lib.ptr(labels), lab64,
                       n_rows, n_cols, float(smoothing), float(logit_scale), float(lse_square_scale), int(ignore_index),
                       total_classes, int(class_start_idx), int(bool(split)), int(precomputed_lse is not None),
@@ -94,7 +94,7 @@ def xent_backward(dlosses, logits, lse, labels, *, dlogits=None, smoothing=0.0, 
     lse = lse.float().contiguous()
     _lib.require_device(dlosses, logits, lse, labels, dlogits)
     if n_rows:
-        with torch.cuda.device(logits.device):
+        with _lib.on(logits.device):
             _lib.call("kdn_xent_bwd", _lib.ptr(dlogits), dlogits.stride(0), _lib.ptr(dlosses), dlosses.stride(0),
                       _lib.ptr(logits), _dtype_code(logits), logits.stride(0), _lib.ptr(lse), _lib.ptr(labels), lab64,
                       n_rows, n_cols, float(smoothing), float(logit_scale), float(lse_square_scale), int(ignore_index),

@@ -5,6 +5,7 @@ If the library is missing the first call raises RuntimeError.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import pathlib
@@ -96,23 +97,46 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = [_CT[c] for c in sig]
         fn.restype = ctypes.c_size_t if name in _SIZE_FNS else ctypes.c_int
+    _fns.clear()
     _lib = lib
     return lib
+
+
+_fns: dict = {}
+
+
+def _fn(name: str):
+    if _lib is None:
+        load()
+    fn = _fns[name] = getattr(_lib, name)
+    return fn
 
 
 def exported_symbols() -> tuple[str, ...]:
     return tuple(_SIGS)
 
 
+# A small pass is bound by the Python around its launches, so the binding adds little to each: pointers and
+# streams go to ctypes as plain integers, and the device is switched only when another one is current.  With
+# ctypes objects, torch.cuda.current_stream and a device context per call, the host took 138 us for the RMS
+# norm's forward and backward and 380 for the isotropic scan's at B1 T301 H4 d64 (autograd's hand-off to its
+# thread included); now 111 and 331.
 def ptr(t):
     """Device pointer of a tensor (or None -> NULL)."""
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def stream_of(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def stream_of(t: torch.Tensor) -> int:
+    """Handle of the current stream of ``t``'s device."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+_CURRENT = contextlib.nullcontext()
+
+
+def on(device: torch.device):
+    """Context in which ``device`` is current."""
+    return _CURRENT if device.index == torch._C._cuda_getDevice() else torch.cuda.device(device)
 
 
 class KernelTimer:
@@ -155,8 +179,7 @@ def timing() -> bool:
 def call(name: str, *args, tag: str | None = None):
     """Call entry point ``name``; under a KernelTimer the call is timed as ``tag`` (default: the
     entry name without its ``kdn_`` prefix)."""
-    lib = load()
-    fn = getattr(lib, name)
+    fn = _fns.get(name) or _fn(name)
     if _timer is not None:
         if tag is None:
             tag = name[4:] if name.startswith("kdn_") else name
@@ -173,7 +196,7 @@ def call(name: str, *args, tag: str | None = None):
 
 
 def size(name: str, *args) -> int:
-    return int(getattr(load(), name)(*args))
+    return (_fns.get(name) or _fn(name))(*args)
 
 
 def is_bf16(t: torch.Tensor) -> int:

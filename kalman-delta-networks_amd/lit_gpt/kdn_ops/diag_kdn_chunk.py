@@ -71,7 +71,7 @@ class _DiagKdnNormFunction(torch.autograd.Function):
         k_memory = torch.empty(q_raw.shape, device=dev, dtype=torch.bfloat16)
         q_norm = torch.empty(q_raw.shape[:-1], device=dev, dtype=torch.float32)
         k_norm = torch.empty_like(q_norm)
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.call("kdn_diag_norm_fwd", _lib.ptr(q_raw), _lib.ptr(k_raw), _lib.is_bf16(q_raw), rows, K,
                       _lib.ptr(q_memory), _lib.ptr(k_gain), _lib.ptr(k_memory), _lib.ptr(q_norm),
                       _lib.ptr(k_norm), _lib.stream_of(q_raw))
@@ -96,7 +96,7 @@ class _DiagKdnNormFunction(torch.autograd.Function):
         d_k_memory = d_k_memory.to(torch.bfloat16).contiguous() if d_k_memory is not None else None
         dq = torch.empty_like(q_raw) if d_q_memory is not None else None
         dk = torch.empty_like(k_raw) if (d_k_gain is not None or d_k_memory is not None) else None
-        with torch.cuda.device(q_raw.device):
+        with _lib.on(q_raw.device):
             _lib.call("kdn_diag_norm_bwd", _lib.ptr(q_raw), _lib.ptr(k_raw), _lib.is_bf16(q_raw), _lib.ptr(q_norm),
                       _lib.ptr(k_norm), _lib.ptr(d_q_memory), _lib.ptr(d_k_gain), _lib.ptr(d_k_memory), rows,
                       q_raw.shape[-1], _lib.ptr(dq), _lib.ptr(dk), _lib.stream_of(q_raw))
@@ -160,7 +160,7 @@ class _DiagKdnFrontendFunction(torch.autograd.Function):
         omega = torch.empty_like(g_cumsum)
         r = torch.empty((B, T, H), device=dev, dtype=torch.float32)
         mu = torch.empty((H,), device=dev, dtype=torch.float32)
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.call("kdn_diag_frontend_fwd", _lib.ptr(retention_raw), _lib.ptr(omega_raw), _lib.ptr(r_raw),
                       _lib.ptr(A_log), _lib.ptr(dt_bias), _lib.ptr(initial_precision_param), B, T, H, K,
                       _DIAG_KDN_MEMORY_CHUNK_SIZE, _lib.ptr(g_cumsum), _lib.ptr(alpha), _lib.ptr(omega),
@@ -188,7 +188,7 @@ class _DiagKdnFrontendFunction(torch.autograd.Function):
         dmu = torch.empty_like(mu_param) if (need_mu and d_initial_precision is not None) else None
         ws_bytes = _lib.size("kdn_diag_frontend_bwd_workspace_size", B, T, H, K, _DIAG_KDN_MEMORY_CHUNK_SIZE)
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.call("kdn_diag_frontend_bwd", _lib.ptr(retention_raw), _lib.ptr(omega_raw), _lib.ptr(r_raw),
                       _lib.ptr(A_log), _lib.ptr(dt_bias), _lib.ptr(mu_param), _lib.ptr(alpha),
                       _lib.ptr(d_g_cumsum), _lib.ptr(d_alpha), _lib.ptr(d_omega), _lib.ptr(d_r),
@@ -220,7 +220,7 @@ def _diag_kdn_gain_forward(k, alpha, omega, r, initial_precision, *, save_state,
     fprec = torch.empty((B, H, K), device=dev, dtype=torch.float32) if (output_final_state or save_state) else None
     ws_bytes = _lib.size("kdn_diag_gain_workspace_size", B, T, H, K)
     ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         _lib.call("kdn_diag_gain_fwd", _lib.ptr(k), _lib.ptr(alpha), _lib.ptr(omega), _lib.ptr(r),
                   _lib.ptr(initial_precision), prec_mode, B, T, H, K, float(K), _lib.ptr(kappa), _lib.ptr(p_prev),
                   _lib.ptr(D), _lib.ptr(fprec), _lib.ptr(ws), ws_bytes, _lib.stream_of(k))
@@ -259,7 +259,7 @@ class _DiagKdnGainFunction(torch.autograd.Function):
         G = torch.empty((B, T, H), device=dev, dtype=torch.float32)
         ws_bytes = _lib.size("kdn_diag_gain_workspace_size", B, T, H, K)
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.call("kdn_diag_gain_bwd", _lib.ptr(k), _lib.ptr(alpha), _lib.ptr(omega), _lib.ptr(r), _lib.ptr(mu),
                       prec_mode, _lib.ptr(dkappa), _lib.ptr(p_prev), _lib.ptr(D), _lib.ptr(fprec), _lib.ptr(dfp),
                       _lib.ptr(omega_raw), _lib.ptr(r_raw), B, T, H, K, float(K), _lib.ptr(dk), _lib.ptr(dalpha),
@@ -346,7 +346,7 @@ class _DiagKdnFrontFunction(torch.autograd.Function):
         ws_bytes = _lib.size("kdn_diag_front_workspace_size", B, T, H, K)
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
         prec_mode = 0 if initial_precision is None or initial_precision.ndim == 1 else 1
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             stream = _lib.stream_of(q_raw)
             _lib.call("kdn_diag_norm_fwd", _lib.ptr(q_raw), _lib.ptr(k_raw), _lib.is_bf16(q_raw), rows, K,
                       _lib.ptr(q_memory), None, _lib.ptr(k_memory), _lib.ptr(q_norm), _lib.ptr(k_norm), stream,
@@ -389,7 +389,7 @@ class _DiagKdnFrontFunction(torch.autograd.Function):
         ws_bytes = _lib.size("kdn_diag_front_workspace_size", B, T, H, K)
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
         dq = None
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             stream = _lib.stream_of(q_raw)
             _lib.call("kdn_diag_front_bwd", _lib.ptr(k_raw), _lib.is_bf16(k_raw), _lib.ptr(k_norm),
                       _lib.ptr(retention_raw), _lib.ptr(omega_raw), _lib.ptr(r_raw), _lib.ptr(A_log),
@@ -497,7 +497,7 @@ class _DiagKdnMemoryFunction(torch.autograd.Function):
         # only the backward reads are skipped (in that mode the backward rebuilds them from the inputs)
         need_backward = any(ctx.needs_input_grad)
         ctx.recompute = need_backward and _memscan.backward_mode() == "recompute"
-        with torch.cuda.device(q.device):
+        with _lib.on(q.device):
             o, saved, ht = _memscan.mem_fwd(q, k, kappa, False, v, g_cumsum, scale, initial_state=initial_state,
                                             output_final_state=output_final_state, out_dtype=out_dtype,
                                             need_backward=need_backward and not ctx.recompute)
@@ -527,7 +527,7 @@ class _DiagKdnMemoryFunction(torch.autograd.Function):
         else:
             do = do.contiguous()
         need_h0 = ctx.has_h0 and ctx.needs_input_grad[6]
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             if ctx.recompute:
                 saved = _memscan.rebuild_saved(q, k, kappa, False, v, g_cumsum, ctx.scale, initial_state=h0)
             dq, dk, dv, dkappa, dg, dh0 = _memscan.mem_bwd(q, k, kappa, False, v, g_cumsum, saved, ctx.scale, do,

@@ -84,7 +84,7 @@ def _iso_kdn_gate_precumsum_fwd(g_raw, omega_r_raw, omega_bias, r_bias, A_log, d
     omega = torch.empty_like(a)
     r = torch.empty_like(a)
     mu = torch.empty((H,), device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         _lib.call("kdn_iso_gate_fwd", _lib.ptr(g_raw), _lib.is_bf16(g_raw), _lib.ptr(omega_r_raw),
                   _lib.is_bf16(omega_r_raw), omega_r_raw.stride(0), omega_r_raw.stride(1),
                   _lib.ptr(omega_bias), _lib.ptr(r_bias), _lib.ptr(A_log), _lib.ptr(dt_bias),
@@ -139,7 +139,7 @@ def _iso_kdn_gate_precumsum_bwd(g_raw, omega_r_raw, omega_bias, r_bias, A_log, d
     dmu = torch.empty((H,), device=dev, dtype=torch.float32) if need_dmu else None
     ws_bytes = _lib.size("kdn_iso_gate_bwd_workspace_size", B, T, H, K, ISO_GATE_CHUNK_SIZE)
     ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         _lib.call("kdn_iso_gate_bwd", _lib.ptr(g_raw), _lib.is_bf16(g_raw), _lib.ptr(omega_r_raw),
                   _lib.is_bf16(omega_r_raw), omega_r_raw.stride(0), omega_r_raw.stride(1),
                   _lib.ptr(omega_bias), _lib.ptr(r_bias), _lib.ptr(A_log), _lib.ptr(dt_bias),
@@ -241,7 +241,7 @@ def _iso_kdn_gain_forward(a, omega, r, initial_precision, *, out_dtype, save_sta
     if T > 0 and B > 0:
         ws_bytes = _lib.size("kdn_iso_gain_workspace_size", B, T, H)
         ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=device)
-        with torch.cuda.device(device):
+        with _lib.on(device):
             _lib.call("kdn_iso_gain_fwd", _lib.ptr(a), _lib.ptr(omega), _lib.ptr(r),
                       _lib.ptr(initial_precision), prec_mode, B, T, H, float(posterior_scale), _lib.ptr(gain),
                       _lib.ptr(p_prev), _lib.ptr(fprec), _lib.ptr(ws), ws_bytes, _lib.stream_of(a))
@@ -264,7 +264,7 @@ def _iso_kdn_gain_backward(a, omega, r, initial_precision, dgain, p_prev, *, pos
         ws_bytes = _lib.size("kdn_iso_gain_workspace_size", B, T, H)
         ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=device)
         dfp = d_final_precision.float().contiguous() if d_final_precision is not None else None
-        with torch.cuda.device(device):
+        with _lib.on(device):
             _lib.call("kdn_iso_gain_bwd", _lib.ptr(a), _lib.ptr(omega), _lib.ptr(r), _lib.ptr(initial_precision),
                       prec_mode, _lib.ptr(dgain), _lib.ptr(p_prev), _lib.ptr(final_precision if dfp is not None
                                                                              else None),
@@ -370,7 +370,7 @@ class _IsoKDNFrontFunction(torch.autograd.Function):
         prec_mode = 0 if initial_precision is None or initial_precision.ndim == 1 else 1
         ws_bytes = _lib.size("kdn_iso_front_workspace_size", B, T, H, K)
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.call("kdn_iso_front_fwd", _lib.ptr(g_raw), _lib.is_bf16(g_raw), _lib.ptr(omega_r_raw),
                       _lib.is_bf16(omega_r_raw), omega_r_raw.stride(0), omega_r_raw.stride(1),
                       _lib.ptr(omega_bias), _lib.ptr(r_bias), _lib.ptr(A_log), _lib.ptr(dt_bias),
@@ -410,7 +410,7 @@ class _IsoKDNFrontFunction(torch.autograd.Function):
         dinit = (torch.empty_like(initial_precision) if initial_precision is not None and needs[7] else None)
         ws_bytes = _lib.size("kdn_iso_front_workspace_size", B, T, H, K)
         ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.call("kdn_iso_front_bwd", _lib.ptr(g_raw), _lib.is_bf16(g_raw), _lib.ptr(omega_r_raw),
                       _lib.is_bf16(omega_r_raw), omega_r_raw.stride(0), omega_r_raw.stride(1),
                       _lib.ptr(omega_bias), _lib.ptr(r_bias), _lib.ptr(A_log), _lib.ptr(dt_bias),
@@ -518,7 +518,7 @@ class _ChunkKDAPrecumsumFunction(torch.autograd.Function):
         need_backward = any(ctx.needs_input_grad)
         ctx.recompute = need_backward and _memscan.backward_mode() == "recompute"
         keep = need_backward and not ctx.recompute  # the forward's intermediates feed the backward
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             vb = v if v.dtype == torch.bfloat16 else v.to(torch.bfloat16)
             out_dtype = q.dtype if q.dtype == torch.float32 else torch.bfloat16
             if ctx.fused_norm:
@@ -551,7 +551,7 @@ class _ChunkKDAPrecumsumFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do, dht=None):
         need_h0 = ctx.h0_dtype is not None and ctx.needs_input_grad[6]
-        with torch.cuda.device(do.device):
+        with _lib.on(do.device):
             if ctx.fused_norm:
                 q, q_rstd, k, k_rstd, vb, g_cumsum, beta, saved, h0 = ctx.saved_tensors
                 if ctx.recompute:

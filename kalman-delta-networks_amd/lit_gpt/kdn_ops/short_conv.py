@@ -32,7 +32,7 @@ def _conv_fwd(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x [B,T,D] with unit channel stride (a packed-group view is fine), weight [D,4] dense."""
     B, T, D = x.shape
     y = torch.empty((B, T, D), device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         _lib.call("kdn_short_conv_fwd", _lib.ptr(x), _lib.is_bf16(x), x.stride(0), x.stride(1), _lib.ptr(weight),
                   _lib.is_bf16(weight), B, T, D, KERNEL_WIDTH, _lib.ptr(y), y.stride(0), y.stride(1),
                   _lib.stream_of(x), tag="short_conv_fwd")
@@ -44,7 +44,7 @@ def _conv_bwd(x, weight, dy, dx, dweight, *, round_preactivation: bool):
     B, T, D = x.shape
     ws_bytes = _lib.size("kdn_short_conv_bwd_workspace_size", B, T, D) if dweight is not None else 0
     ws = torch.empty(max(ws_bytes // 4, 1), device=x.device, dtype=torch.float32) if dweight is not None else None
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         _lib.call("kdn_short_conv_bwd", _lib.ptr(x), _lib.is_bf16(x), x.stride(0), x.stride(1), _lib.ptr(weight),
                   _lib.is_bf16(weight), _lib.ptr(dy), dy.stride(0) if dy is not None else 0,
                   dy.stride(1) if dy is not None else 0, B, T, D, KERNEL_WIDTH, int(round_preactivation),
@@ -162,7 +162,7 @@ def _qkv_conv_fwd(x, weight, D):
     """All three groups in one launch (a third of the launches, and one ramp-up and tail instead of three)."""
     B, T, _ = x.shape
     ys = tuple(torch.empty((B, T, D), device=x.device, dtype=x.dtype) for _ in range(GROUPS))
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         _lib.call("kdn_qkv_conv_fwd", _lib.ptr(x), _lib.is_bf16(x), _lib.ptr(weight), _lib.is_bf16(weight), B, T, D,
                   KERNEL_WIDTH, *map(_lib.ptr, ys), _lib.stream_of(x), tag="short_conv_fwd")
     return ys
@@ -192,7 +192,7 @@ class _QKVCausalConv1d(torch.autograd.Function):
         dw = torch.empty_like(weight)
         ws_bytes = _lib.size("kdn_short_conv_bwd_workspace_size", B, T, GROUPS * D)
         ws = torch.empty(max(ws_bytes // 4, 1), device=x.device, dtype=torch.float32)
-        with torch.cuda.device(x.device):
+        with _lib.on(x.device):
             _lib.call("kdn_qkv_conv_bwd", _lib.ptr(x), _lib.is_bf16(x), _lib.ptr(weight), _lib.is_bf16(weight),
                       *map(_lib.ptr, grads), B, T, D, KERNEL_WIDTH, _lib.ptr(dx), _lib.ptr(dw), _lib.ptr(ws), ws_bytes,
                       _lib.stream_of(x), tag="short_conv_bwd")
@@ -222,7 +222,7 @@ def short_conv_step(x: torch.Tensor, tail: torch.Tensor, weight: torch.Tensor) -
         raise ValueError(f"weight must be a contiguous [{D},{KERNEL_WIDTH}] tensor")
     _lib.require_device(x, tail, weight)
     y = torch.empty((B, 1, D), device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         _lib.call("kdn_short_conv_step", _lib.ptr(x), _lib.is_bf16(x), x.stride(0), _lib.ptr(tail), tail.stride(0),
                   _lib.ptr(weight), _lib.is_bf16(weight), B, D, _lib.ptr(y), y.stride(0), _lib.stream_of(x))
     return y

@@ -58,7 +58,7 @@ def kdn_memory_step(q, k, v, g_cumsum, *, state, beta=None, kappa=None, scale=No
     g_cumsum = g_cumsum.contiguous()
     o = torch.empty((B, 1, H, V), device=q.device, dtype=out_dtype)
     scale = K ** -0.5 if scale is None else float(scale)
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         _lib.call("kdn_mem_step", _lib.ptr(q), _lib.ptr(k), _lib.ptr(gate), int(iso), _lib.ptr(v),
                   _lib.is_bf16(q), _lib.ptr(g_cumsum), B, H, K, V, scale, _lib.ptr(state), _lib.ptr(o),
                   _lib.is_bf16(o), _lib.stream_of(q), tag="mem_step")
@@ -122,7 +122,7 @@ def kdn_kalman_step(q, k, v, g_cumsum, *, state, precision, omega, r, info_scale
         raise ValueError("precision_out must be a contiguous fp32 tensor of the precision's shape, distinct from it")
     o = torch.empty((B, 1, H, V), device=q.device, dtype=out_dtype)
     scale = K ** -0.5 if scale is None else float(scale)
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         _lib.call("kdn_kalman_step", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.is_bf16(q), _lib.ptr(g_cumsum.contiguous()),
                   _lib.ptr(gain_a), _lib.ptr(omega), _lib.ptr(r), _lib.ptr(kg), _lib.ptr(pin), _lib.ptr(precision_out),
                   int(iso), B, H, K, V, scale, float(info_scale), _lib.ptr(state), _lib.ptr(o), _lib.is_bf16(o),
@@ -158,7 +158,7 @@ def kdn_gemv(x, weight, bias=None, *, gated=False):
     _lib.require_device(x2, weight, bias)
     y = torch.empty((M, N), device=x.device, dtype=x.dtype)
     if M and N:
-        with torch.cuda.device(x.device):
+        with _lib.on(x.device):
             _lib.call("kdn_gemv", _lib.ptr(x2), _lib.is_bf16(x2), row_stride, _lib.ptr(weight), _lib.ptr(bias), M, N, K,
                       int(bool(gated)), _lib.ptr(y), y.stride(0), _lib.stream_of(x2))
     return y.view(*lead, N)
@@ -191,7 +191,7 @@ def kdn_decode_proj(x, weight, *, norm_weight=None, eps=0.0, bias=None, residual
     y = torch.empty((M, N), device=x.device, dtype=torch.bfloat16)
     ws_bytes = _lib.size("kdn_decode_proj_workspace_size", M, N, K, int(norm_weight is not None), int(bool(gated)))
     ws = torch.empty(ws_bytes // 4, device=x.device, dtype=torch.float32) if ws_bytes else None
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         _lib.call("kdn_decode_proj", _lib.ptr(x), x.stride(0), _lib.ptr(norm_weight), float(eps), _lib.ptr(weight),
                   _lib.ptr(bias), _lib.ptr(residual), residual.stride(0) if residual is not None else 0, M, N, K,
                   int(bool(gated)), _lib.ptr(y), N, _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
@@ -237,7 +237,7 @@ def kdn_decode_mixer(p, offsets, tails, taps, Wf, Wo, bo, Wg, bg, omega_bias, r_
     step = n if iso else 0  # the isotropic layer's q, k, v parts sit side by side in one tensor
     ptrs = [[t.data_ptr() + 2 * step * i * m for i, t in enumerate(ts if len(ts) == 3 else ts * 3)]
             for ts, m in ((tails, 1), (taps, 4))]
-    with torch.cuda.device(p.device):
+    with _lib.on(p.device):
         _lib.call("kdn_decode_mixer", _lib.ptr(p), p.stride(0), off_f, off_w, off_r, off_g, *ptrs[0], 3 * width, width,
                   *ptrs[1], _lib.ptr(Wf), _lib.ptr(Wo), _lib.ptr(bo), _lib.ptr(Wg), _lib.ptr(bg), _lib.ptr(omega_bias),
                   _lib.ptr(r_bias), _lib.ptr(A_log), _lib.ptr(dt_bias), float(omega_min), float(r_min), float(info_scale),

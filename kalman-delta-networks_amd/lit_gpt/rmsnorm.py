@@ -21,7 +21,7 @@ class _RMSNormFunction(torch.autograd.Function):
         rows = xf.shape[0]
         y = torch.empty_like(xf)
         rstd = torch.empty(rows, device=x.device, dtype=torch.float32)
-        with torch.cuda.device(x.device):
+        with _lib.on(x.device):
             _lib.call("kdn_rms_norm_fwd", _lib.ptr(xf), _lib.is_bf16(xf), _lib.ptr(weight), _lib.is_bf16(weight),
                       rows, D, float(eps), _lib.ptr(y), _lib.ptr(rstd), _lib.stream_of(x), tag="rms_norm_fwd")
         ctx.save_for_backward(xf, weight, rstd)
@@ -38,7 +38,7 @@ class _RMSNormFunction(torch.autograd.Function):
         dw = torch.empty_like(weight) if ctx.needs_input_grad[1] else None
         ws_bytes = _lib.size("kdn_rms_norm_bwd_workspace_size", rows, D) if dw is not None else 0
         ws = torch.empty(max(ws_bytes // 4, 1), device=xf.device, dtype=torch.float32) if dw is not None else None
-        with torch.cuda.device(xf.device):
+        with _lib.on(xf.device):
             _lib.call("kdn_rms_norm_bwd", _lib.ptr(xf), _lib.is_bf16(xf), _lib.ptr(weight), _lib.is_bf16(weight),
                       _lib.ptr(rstd), _lib.ptr(dyf), rows, D, _lib.ptr(dx), _lib.ptr(dw), _lib.ptr(ws), ws_bytes,
                       _lib.stream_of(xf), tag="rms_norm_bwd")
