@@ -362,6 +362,11 @@ int kdn_xent_fwd(const void* logits, int logits_dtype, int64_t logits_row_stride
                  int n_rows, int n_cols, float smoothing, float logit_scale, float lse_square_scale,
                  int64_t ignore_index, int64_t total_classes, int64_t class_start_idx, int split,
                  int precomputed_lse, float* losses, float* lse, float* z_losses, hipStream_t stream);
+/* The losses' and z-losses' sum, or with `mean` their mean over the rows not labelled ignore_index (0 / 0 = NaN
+ * when there are none), as FusedCrossEntropyLoss reduces them (fused_cross_entropy.py:336-414),
+ * and what they were divided by (f32 scalars).  One workgroup, summed in double precision in a fixed order. */
+int kdn_xent_reduce(const float* losses, const float* z_losses, const void* labels, int labels_i64, int n_rows,
+                    int64_t ignore_index, int mean, float* loss, float* z_loss, float* divisor, hipStream_t stream);
 /* Fused cross-entropy backward.  Replaces cross_entropy_bwd_kernel (fused_cross_entropy.py:103-150)
  * as launched by CrossEntropyLoss.backward (:262-294): dlogits[r, c] = dlosses[r] logit_scale
  * (p (1 + 2 lse_square_scale lse) - [c == label](1 - smoothing) - smoothing / total_classes),

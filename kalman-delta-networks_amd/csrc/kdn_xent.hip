@@ -78,7 +78,9 @@ template <typename T, int VEC> __device__ __forceinline__ void stv_buf(bufrsrc r
     T* e = reinterpret_cast<T*>(&u);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) e[i] = from_f<T>(f[i]);
-    __builtin_amdgcn_raw_buffer_store_b128(u, r, byte_off, 0, 0);
+    // nontemporal: left in the caches, the gradient pushes out the logits it is computed from (4096 x 32000
+    // bf16 in a loop: backward 87 -> 81 us, the next forward 76 -> 47)
+    __builtin_amdgcn_raw_buffer_store_b128(u, r, byte_off, 0, 2);
   }
 }
 
@@ -196,6 +198,38 @@ __global__ __launch_bounds__(kXentThreads) void xent_fwd_kernel(
   if (!split && z_losses) z_losses[row] = z;
 }
 
+// Sum (mean: over the rows that are not ignored) of the losses and z-losses in double precision, one
+// workgroup.  In place of a sum, a comparison, a count and a division, each a
+// launch of 4 us: loss of 4096 x 32000 bf16, forward and backward, 171 -> 133 us.
+constexpr int kReduceThreads = 1024;
+__global__ __launch_bounds__(kReduceThreads) void xent_reduce_kernel(const float* __restrict__ losses,
+                                                                     const float* __restrict__ z,
+                                                                     const void* __restrict__ labels, int labels_i64,
+                                                                     int n, int64_t ignore_index, int mean,
+                                                                     float* __restrict__ loss,
+                                                                     float* __restrict__ z_loss,
+                                                                     float* __restrict__ divisor) {
+  double a = 0., b = 0.;
+  int c = 0;
+  for (int i = threadIdx.x; i < n; i += kReduceThreads) {
+    a += (double)losses[i];
+    b += (double)z[i];
+    c += load_label(labels, labels_i64, i) != ignore_index;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64), c += __shfl_xor(c, o, 64);
+  __shared__ double s_a[kReduceThreads / 64], s_b[kReduceThreads / 64];
+  __shared__ int s_c[kReduceThreads / 64];
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) s_a[w] = a, s_b[w] = b, s_c[w] = c;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  a = 0., b = 0., c = 0;
+  for (int i = 0; i < kReduceThreads / 64; ++i) a += s_a[i], b += s_b[i], c += s_c[i];
+  const float d = mean ? (float)c : 1.f;
+  *loss = (float)(a / (double)d), *z_loss = (float)(b / (double)d), *divisor = d;
+}
+
 template <typename T, int VEC>
 void launch_fwd(const void* logits, int64_t ls, const void* labels, int labels_i64, int n_rows, int n_cols,
                 float smoothing, float logit_scale, float lse_sq, int64_t ignore_index, int64_t total, int64_t start,
@@ -291,6 +325,16 @@ bool args_ok(int dtype, int n_rows, int n_cols, int64_t total_classes, int64_t c
 }
 
 }  // namespace
+
+extern "C" int kdn_xent_reduce(const float* losses, const float* z_losses, const void* labels, int labels_i64, int n_rows,
+                               int64_t ignore_index, int mean, float* loss, float* z_loss, float* divisor,
+                               hipStream_t stream) {
+  if (n_rows <= 0 || !losses || !z_losses || !labels || !loss || !z_loss || !divisor) return KDN_ERR_ARG;
+  hipLaunchKernelGGL(xent_reduce_kernel, dim3(1), dim3(kReduceThreads), 0, stream, losses, z_losses, labels, labels_i64,
+                     n_rows, ignore_index, mean, loss, z_loss, divisor);
+  KDN_CHECK_LAUNCH();
+  return 0;
+}
 
 extern "C" int kdn_xent_fwd(const void* logits, int logits_dtype, int64_t logits_row_stride, const void* labels,
                             int labels_i64, int n_rows, int n_cols, float smoothing, float logit_scale,

@@ -102,50 +102,91 @@ def xent_backward(dlosses, logits, lse, labels, *, dlogits=None, smoothing=0.0, 
     return dlogits
 
 
+def _forward(ctx, logits, labels, precomputed_lse, smoothing, logit_scale, lse_square_scale, ignore_index,
+             inplace_backward, process_group):
+    """The Functions' shared forward: (losses, z_losses, tensors for ``_backward``)."""
+    if not logit_scale > 0.0:
+        raise ValueError(f"logit_scale must be positive, got {logit_scale}")
+    if logits.ndim != 2:
+        raise ValueError(f"logits must be [n_rows, n_cols], got {tuple(logits.shape)}")
+    n_rows, n_cols = logits.shape
+    if labels.shape != (n_rows,):
+        raise ValueError(f"labels must have shape ({n_rows},), got {tuple(labels.shape)}")
+    world_size = 1 if process_group is None else torch.distributed.get_world_size(process_group)
+    rank = 0 if process_group is None else torch.distributed.get_rank(process_group)
+    total_classes, class_start_idx = world_size * n_cols, rank * n_cols
+    if logits.stride(-1) != 1:
+        logits = logits.contiguous()
+    # as the reference, a precomputed lse is used only where it is the lse of the plain logits
+    use_lse = precomputed_lse if (precomputed_lse is not None and logit_scale == 1.0 and smoothing == 0.0) else None
+    split = world_size > 1
+    losses, lse, z_losses = xent_forward(logits, labels, smoothing=smoothing, logit_scale=logit_scale,
+                                         lse_square_scale=lse_square_scale, ignore_index=ignore_index,
+                                         total_classes=total_classes, class_start_idx=class_start_idx,
+                                         split=split, precomputed_lse=use_lse)
+    if split:
+        gathered = torch.empty(world_size, n_rows, dtype=lse.dtype, device=lse.device)
+        torch.distributed.all_gather_into_tensor(gathered, lse, group=process_group)
+        torch.distributed.all_reduce(losses, op=torch.distributed.ReduceOp.SUM, group=process_group)
+        losses, z_losses, lse = finish_split_losses(losses, gathered, labels, lse_square_scale, ignore_index)
+    ctx.smoothing, ctx.logit_scale, ctx.lse_square_scale = smoothing, logit_scale, lse_square_scale
+    ctx.ignore_index, ctx.inplace_backward = ignore_index, inplace_backward
+    ctx.total_classes, ctx.class_start_idx = total_classes, class_start_idx
+    return losses, z_losses, (logits, lse, labels)
+
+
+def _backward(ctx, dlosses, logits, lse, labels):
+    return xent_backward(dlosses, logits, lse, labels, dlogits=logits if ctx.inplace_backward else None,
+                         smoothing=ctx.smoothing, logit_scale=ctx.logit_scale, lse_square_scale=ctx.lse_square_scale,
+                         ignore_index=ctx.ignore_index, total_classes=ctx.total_classes,
+                         class_start_idx=ctx.class_start_idx)
+
+
 class CrossEntropyLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, labels, precomputed_lse=None, smoothing=0.0, logit_scale=1.0, lse_square_scale=0.0,
                 ignore_index=-100, inplace_backward=False, process_group=None):
-        if not logit_scale > 0.0:
-            raise ValueError(f"logit_scale must be positive, got {logit_scale}")
-        if logits.ndim != 2:
-            raise ValueError(f"logits must be [n_rows, n_cols], got {tuple(logits.shape)}")
-        n_rows, n_cols = logits.shape
-        if labels.shape != (n_rows,):
-            raise ValueError(f"labels must have shape ({n_rows},), got {tuple(labels.shape)}")
-        world_size = 1 if process_group is None else torch.distributed.get_world_size(process_group)
-        rank = 0 if process_group is None else torch.distributed.get_rank(process_group)
-        total_classes, class_start_idx = world_size * n_cols, rank * n_cols
-        if logits.stride(-1) != 1:
-            logits = logits.contiguous()
-        # as the reference, a precomputed lse is used only where it is the lse of the plain logits
-        use_lse = precomputed_lse if (precomputed_lse is not None and logit_scale == 1.0 and smoothing == 0.0) else None
-        split = world_size > 1
-        losses, lse, z_losses = xent_forward(logits, labels, smoothing=smoothing, logit_scale=logit_scale,
-                                             lse_square_scale=lse_square_scale, ignore_index=ignore_index,
-                                             total_classes=total_classes, class_start_idx=class_start_idx,
-                                             split=split, precomputed_lse=use_lse)
-        if split:
-            gathered = torch.empty(world_size, n_rows, dtype=lse.dtype, device=lse.device)
-            torch.distributed.all_gather_into_tensor(gathered, lse, group=process_group)
-            torch.distributed.all_reduce(losses, op=torch.distributed.ReduceOp.SUM, group=process_group)
-            losses, z_losses, lse = finish_split_losses(losses, gathered, labels, lse_square_scale, ignore_index)
-        ctx.save_for_backward(logits, lse, labels)
+        losses, z_losses, saved = _forward(ctx, logits, labels, precomputed_lse, smoothing, logit_scale,
+                                           lse_square_scale, ignore_index, inplace_backward, process_group)
+        ctx.save_for_backward(*saved)
         ctx.mark_non_differentiable(z_losses)
-        ctx.smoothing, ctx.logit_scale, ctx.lse_square_scale = smoothing, logit_scale, lse_square_scale
-        ctx.ignore_index, ctx.inplace_backward = ignore_index, inplace_backward
-        ctx.total_classes, ctx.class_start_idx = total_classes, class_start_idx
         return losses, z_losses
 
     @staticmethod
     def backward(ctx, grad_losses, grad_z_losses):
         del grad_z_losses  # the z-loss output is for logging; its term is inside the losses
-        logits, lse, labels = ctx.saved_tensors
-        dlogits = xent_backward(grad_losses, logits, lse, labels, dlogits=logits if ctx.inplace_backward else None,
-                                smoothing=ctx.smoothing, logit_scale=ctx.logit_scale,
-                                lse_square_scale=ctx.lse_square_scale, ignore_index=ctx.ignore_index,
-                                total_classes=ctx.total_classes, class_start_idx=ctx.class_start_idx)
-        return dlogits, None, None, None, None, None, None, None, None
+        return _backward(ctx, grad_losses, *ctx.saved_tensors), None, None, None, None, None, None, None, None
+
+
+# one workgroup reduces the rows: at most this many (64 a thread)
+_REDUCE_MAX_ROWS = 65536
+
+
+class _ReducedCrossEntropyLoss(torch.autograd.Function):
+    """``CrossEntropyLoss`` on one rank followed by the module's sum or mean: (loss, z_loss) scalars."""
+
+    @staticmethod
+    def forward(ctx, logits, labels, precomputed_lse, smoothing, logit_scale, lse_square_scale, ignore_index,
+                inplace_backward, mean):
+        losses, z_losses, saved = _forward(ctx, logits, labels, precomputed_lse, smoothing, logit_scale,
+                                           lse_square_scale, ignore_index, inplace_backward, None)
+        # three tensors: outputs that are views of one could not be modified in place
+        loss, z_loss, divisor = (torch.empty((), dtype=torch.float32, device=losses.device) for _ in range(3))
+        lab, lab64 = _labels_arg(labels)
+        with _lib.on(losses.device):
+            _lib.call("kdn_xent_reduce", _lib.ptr(losses), _lib.ptr(z_losses), _lib.ptr(lab), lab64, losses.numel(),
+                      int(ignore_index), int(mean), _lib.ptr(loss), _lib.ptr(z_loss), _lib.ptr(divisor),
+                      _lib.stream_of(losses))
+        ctx.save_for_backward(*saved, divisor)
+        ctx.mark_non_differentiable(z_loss)
+        return loss, z_loss
+
+    @staticmethod
+    def backward(ctx, grad_loss, grad_z_loss):
+        del grad_z_loss
+        logits, lse, labels, divisor = ctx.saved_tensors
+        dlosses = (grad_loss / divisor).expand(logits.shape[0])
+        return _backward(ctx, dlosses, logits, lse, labels), None, None, None, None, None, None, None, None
 
 
 def cross_entropy_loss(
@@ -197,6 +238,12 @@ class FusedCrossEntropyLoss(nn.Module):
         if input.ndim == 3:
             input = input.reshape(-1, input.size(-1))
             target = target.reshape(-1)
+        if (self.reduction != "none" and self.process_group is None and input.ndim == 2
+                and 0 < input.shape[0] <= _REDUCE_MAX_ROWS):
+            loss, z_loss = _ReducedCrossEntropyLoss.apply(input, target, precomputed_lse, self.label_smoothing,
+                                                          self.logit_scale, self.lse_square_scale, self.ignore_index,
+                                                          self.inplace_backward, self.reduction == "mean")
+            return (loss, z_loss) if self.return_z_loss else loss
         loss, z_loss = cross_entropy_loss(input, target, precomputed_lse=precomputed_lse,
                                           label_smoothing=self.label_smoothing, logit_scale=self.logit_scale,
                                           lse_square_scale=self.lse_square_scale, ignore_index=self.ignore_index,

@@ -54,6 +54,7 @@ _SIGS = {
     "kdn_decode_proj": "plpfpppliiiiplpzs",
     "kdn_decode_mixer": "pliiiipppllppppppppppppffffpppfiiiips",
     "kdn_xent_fwd": "pilpiiifffllliippps",
+    "kdn_xent_reduce": "pppiilippps",
     "kdn_xent_bwd": "plplpilppiiifffllls",
     "kdn_short_conv_fwd": "pillpiiiiiplls",
     "kdn_short_conv_step": "pilplpiiipls",
