@@ -20,7 +20,7 @@
 // Bound by the CU's load path: per token-head (d = 128) h and dh 512 B each isotropic (1,024 diagonal), delta and
 // dX 512 each, dO, q, k 256 each and G 512.  A task's LDS (~140 KB) leaves one workgroup per CU, so nothing else
 // hides its loads.  Forming U, W, the solves' transposes and dX here as well (A^T, U, W read: 1,280 B more) it took
-// 609 us isotropic / 617 us diagonal at B4 T4096 H18, against 457 / 478.
+// 609 us isotropic / 617 us diagonal at B4 T4096 H18, against 446 / 480.
 #pragma once
 #include "kdn_common.h"
 #include "kdn_intra.h"
@@ -669,9 +669,14 @@ __device__ __forceinline__ void chunk_bwd_task(
     sDot[tq][NW - 1][c] = dsum;  // each (tensor, row) is read and overwritten by this one thread
   }
   __syncthreads();
-  if (own_k) {  // dx = rstd (dy - y (y . dy)) for the raw q, k
-    const bufrsrc rdq = make_buf(dq + in_row0 * K, rows_in * K * 2);
-    const bufrsrc rdk = make_buf(dk + in_row0 * K, rows_in * K * 2);
+  // dx = rstd (dy - y (y . dy)) for the raw q, k, regrouped through LDS (the gradient phase's fragments are
+  // dead) so that a store writes whole rows: straight from the lanes it covered 16 rows in 32-byte pieces, at the
+  // end of the workgroup's life (chunk backward 462 -> 446 us isotropic at B4 T4096 H18).  Stores in
+  // mid-kernel overlap the arithmetic as they are: dg and the diagonal dq, dk gathered the same way lost 10 to 20 us
+  constexpr int XR = K + 8;  // row stride, bf16
+  bf16_t* sOut = reinterpret_cast<bf16_t*>(smem);  // [q, k][row][XR]
+  static_assert(2 * C * XR * 2 <= LDS_BYTES, "dq, dk rows");
+  if (own_k) {
 #pragma unroll
     for (int tl = 0; tl < 4; ++tl) {
       const int c = 16 * tl + r16;
@@ -685,14 +690,21 @@ __device__ __forceinline__ void chunk_bwd_task(
         xq[j] = rq_ * (dqs[tl][j] - yq[j] * dotq);
         xk[j] = rk_ * (dks[tl][j] - yk[j] * dotk);
       }
-      const uint32_t o = (uint32_t)(c * H) * K + i0;
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2{(uint32_t)f2bf(xq[0]) | ((uint32_t)f2bf(xq[1]) << 16),
-                                                  (uint32_t)f2bf(xq[2]) | ((uint32_t)f2bf(xq[3]) << 16)},
-                                            rdq, o * 2, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2{(uint32_t)f2bf(xk[0]) | ((uint32_t)f2bf(xk[1]) << 16),
-                                                  (uint32_t)f2bf(xk[2]) | ((uint32_t)f2bf(xk[3]) << 16)},
-                                            rdk, o * 2, 0, 0);
+      *reinterpret_cast<uint2*>(sOut + c * XR + i0) =
+          uint2{(uint32_t)f2bf(xq[0]) | ((uint32_t)f2bf(xq[1]) << 16), (uint32_t)f2bf(xq[2]) | ((uint32_t)f2bf(xq[3]) << 16)};
+      *reinterpret_cast<uint2*>(sOut + (C + c) * XR + i0) =
+          uint2{(uint32_t)f2bf(xk[0]) | ((uint32_t)f2bf(xk[1]) << 16), (uint32_t)f2bf(xk[2]) | ((uint32_t)f2bf(xk[3]) << 16)};
     }
+  }
+  __syncthreads();
+  const bufrsrc rdq = make_buf(dq + in_row0 * K, rows_in * K * 2), rdk = make_buf(dk + in_row0 * K, rows_in * K * 2);
+  constexpr int CH = K / 8;  // 16-byte pieces of a row
+#pragma unroll
+  for (int u = 0; u < C * CH / 512; ++u) {
+    const int e = tid + 512 * u, c = e / CH, i8 = 8 * (e % CH);
+    const uint32_t o = ((uint32_t)(c * H) * K + i8) * 2;  // rows past L dropped
+    __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4*>(sOut + c * XR + i8), rdq, o, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4*>(sOut + (C + c) * XR + i8), rdk, o, 0, 0);
   }
 }
 

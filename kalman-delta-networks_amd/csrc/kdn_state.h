@@ -252,12 +252,12 @@ __device__ __forceinline__ void st_state4(void* p, int64_t e0, int ib, int g4, i
     const bufrsrc r = make_buf(reinterpret_cast<bf16_t*>(p) + e0, K * V * 2);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      __builtin_amdgcn_raw_buffer_store_b16(f2bf(x[j]), r, hb_off<K>(16 * ib + 4 * g4 + j, col) * 2, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b16(f2bf(x[j]), r, hb_off<K>(16 * ib + 4 * g4 + j, col) * 2, 0, 2);
   } else {
     const bufrsrc r = make_buf(reinterpret_cast<float*>(p) + e0, K * V * 4);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[j]), r, hb_off<K>(16 * ib + 4 * g4 + j, col) * 4, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[j]), r, hb_off<K>(16 * ib + 4 * g4 + j, col) * 4, 0, 2);
   }
 }
 // A sequence of NS fragment-read + MFMA steps with the reads issued LA steps ahead, so the
@@ -277,7 +277,9 @@ __device__ __forceinline__ void mfma_pipe(Rd rd, Mm mm) {
 // the four 16-row accumulator tiles, each as the pass's lanes hold it (lane r16 + 16 g4: the rows 4 g4 .. + 3 of
 // column r16).  A tile leaves in one 16-byte store per lane, 1 KB whole; row-major, the copy took 16 4-byte
 // stores per chunk step on the serial chain.  The readers turn 4 rows of a column into 4 columns of a row with a
-// quad transpose.  Rows past the sequence's end hold 0.  Element (c, v) of a chunk is at
+// quad transpose.  Rows past the sequence's end hold 0.  These copies and the h, dh ones are stored nontemporal: the
+// pass never reads them back, and cached they pushed out the factors its next chunks load (state_bwd 301 -> 288 us
+// isotropic, 323 -> 303 diagonal at B4 T4096 H18 d128).  Element (c, v) of a chunk is at
 //   (((v / 16) * 4 + c / 16) * 64 + v % 16 + 16 ((c / 4) % 4)) * 4 + c % 4.
 template <int V>
 __device__ __forceinline__ void st_tiles(float* p, int64_t chunk, int col, int lane, const f32x4 (&x)[4]) {
@@ -285,7 +287,7 @@ __device__ __forceinline__ void st_tiles(float* p, int64_t chunk, int col, int l
 #pragma unroll
   for (int cb = 0; cb < 4; ++cb)
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x[cb]), r,
-                                           (uint32_t)(((col >> 4) * 4 + cb) * 64 + lane) * 16, 0, 0);
+                                           (uint32_t)(((col >> 4) * 4 + cb) * 64 + lane) * 16, 0, 2);
 }
 
 // Block -> (bh, V-slice): the NV slices of one (b, h) go to one XCD (dispatch is round-robin
