@@ -38,7 +38,7 @@ __device__ __forceinline__ uint4 pack8(const float* f) {
 // the other operand of the 16x16x32 products (MT tiles of 16, the columns past M unused: the matrix cores
 // are idle anyway).  K % 8 == 0: an 8-element segment past K is zero.
 //   resident (K <= 2304 = 8 waves x 9 steps of 32): a wave keeps its share of x in registers and the
-//     workgroup walks tiles of 16 rows of W (GATED: 16 of each half), a tile's loads all in flight at
+//     workgroup walks tiles of up to 16 rows of W (GATED: of each half), a tile's loads all in flight at
 //     once, the next tile's issued before the current one's sums meet.  Streaming x beside W instead halved
 //     the weight bytes in flight and read x once per tile from L2: M 1 / 32, N 32000 K 2304 took
 //     39.7 / 84.0 us, now 27.8 / 36.5 (5.3 / 4.0 TB/s); [2 x 6912, 2304] gated 21.0 / 27.2, now 17.3 / 22.5.
@@ -55,6 +55,7 @@ struct ProjArgs {
   bf16_t* y;
   int64_t ys;
   float* part;  // split: the partial products [split][M][N]
+  int tr;       // rows of W per tile, at most 16 (the 16-row operand repeats the last one)
 };
 constexpr int kResWaves = 8, kResSteps = 9, kStrWaves = 16;
 
@@ -63,8 +64,8 @@ template <int MT, int NA, int NW, bool NORM>
 __device__ __forceinline__ void proj_epilogue(const ProjArgs& A, const float (*acc)[NA * MT][256],
                                               const float (*ss)[MT * 16], int n0) {
   for (int e = threadIdx.x; e < MT * 256; e += 64 * NW) {
-    const int mt = e >> 8, l = (e >> 2) & 63, m = 16 * mt + (l & 15), n = n0 + 4 * (l >> 4) + (e & 3);
-    if (m >= A.M || n >= A.N) continue;
+    const int mt = e >> 8, l = (e >> 2) & 63, m = 16 * mt + (l & 15), nl = 4 * (l >> 4) + (e & 3), n = n0 + nl;
+    if (m >= A.M || nl >= A.tr || n >= A.N) continue;
     float v[NA];
 #pragma unroll
     for (int a = 0; a < NA; ++a) {
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(64 * kResWaves) void decode_proj_resident_kernel(co
   const int r = lane & 15, kg = lane >> 4, K = A.K, N = A.N;
   const int S = (K + 31) / 32, y0 = S * blockIdx.y / gridDim.y, y1 = S * (blockIdx.y + 1) / gridDim.y;
   const int s0 = y0 + (y1 - y0) * wv / NW, s1 = y0 + (y1 - y0) * (wv + 1) / NW;  // at most SW steps, possibly none
-  const int tiles = (N + 15) / 16;
+  const int tr = A.tr, tiles = (N + tr - 1) / tr;
   uint4 wf[SW][NA], xf[SW][MT], xl[LO ? SW : 1];
   // buffer loads: one offset per row and an immediate per step in place of 64-bit addresses.  A step past the
   // wave's share is loaded but not used; past the tensor's end the load returns 0.
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(64 * kResWaves) void decode_proj_resident_kernel(co
   auto ld = [](bufrsrc b, uint32_t v) { return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(b, v, 0, 0)); };
   const uint32_t vk = (uint32_t)s0 * 64 + 16 * kg;  // bytes into a row
   auto load_w = [&](int tile) {
-    const uint32_t vw = (uint32_t)min(16 * tile + r, N - 1) * (uint32_t)K * 2 + vk;
+    const uint32_t vw = (uint32_t)min(tr * tile + min(r, tr - 1), N - 1) * (uint32_t)K * 2 + vk;
 #pragma unroll
     for (int u = 0; u < SW; ++u)
 #pragma unroll
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(64 * kResWaves) void decode_proj_resident_kernel(co
         *reinterpret_cast<f32x4*>(&s_acc[buf][wv][a * MT + mt][4 * lane]) = acc[a][mt];
     if (tile + (int)gridDim.x < tiles) load_w(tile + gridDim.x);
     __syncthreads();  // s_acc[buf] is written again two tiles on, after the next barrier
-    proj_epilogue<MT, NA, NW, NORM>(A, s_acc[buf], s_ss, 16 * tile);
+    proj_epilogue<MT, NA, NW, NORM>(A, s_acc[buf], s_ss, tr * tile);
   }
 }
 
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(64 * kStrWaves) void decode_proj_stream_kernel(cons
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, kg = lane >> 4, K = A.K, N = A.N;
   const int S = (K + 31) / 32, s1 = S * (wv + 1) / NW;
-  const bf16_t* wr = A.W + (int64_t)min(16 * (int)blockIdx.x + r, N - 1) * K;
+  const bf16_t* wr = A.W + (int64_t)min(A.tr * (int)blockIdx.x + min(r, A.tr - 1), N - 1) * K;
   const bf16_t* xr[MT];
   f32x4 acc[NA][MT];
   float ss[MT] = {};
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(64 * kStrWaves) void decode_proj_stream_kernel(cons
     }
   }
   __syncthreads();
-  proj_epilogue<MT, NA, NW, NORM>(A, s_acc, s_ss, 16 * blockIdx.x);
+  proj_epilogue<MT, NA, NW, NORM>(A, s_acc, s_ss, A.tr * blockIdx.x);
 }
 
 // y = the splits' partial products in order, + bias, + res
@@ -277,17 +278,31 @@ __global__ __launch_bounds__(256) void decode_proj_sum_kernel(const ProjArgs A, 
 
 // Splits of K for more than 16 rows past the resident form's K: with x streamed beside W by one workgroup per tile,
 // the 144 workgroups of N 2304, K 6912 each loaded 442 KB of x and 221 KB of W at 32 rows (32.8 us); three
-// splits keep x resident over two tiles, on 216 CUs (17.5 us with the sum).  At most 16 rows stream: x is
-// small there and the sum's launch costs as much as it saves (15.2 us).
+// splits keep x resident over two tiles (16.6 us with the sum).  At most 16 rows stream: x is small there and
+// the sum's launch would cost more than it saves (12.4 us).
 inline int proj_splits(int M, int N, int K, bool norm, bool gated) {
   const int S = (K + 31) / 32, one = kResWaves * kResSteps;
   if (M <= 16 || norm || gated || S <= one || (int64_t)N * K >= (1ll << 31)) return 1;
   return (S + one - 1) / one;
 }
 
+// Tile height and count for `splits` products of N rows on 256 CUs: as few tiles per workgroup as 16-row tiles
+// allow, then the rows spread evenly (N 2304: 256 tiles of 9 rows, where 144 of 16 left 112 CUs idle; N 6912:
+// 494 of 14, two each, where 432 of 16 gave 216 workgroups 32 rows).  M 1: N 2304 K 6912 15.1 -> 12.4 us, K 2304
+// 5.9 -> 5.3.
+struct ProjShape {
+  int tr, tiles, grid;
+  ProjShape(int N, int splits) {
+    const int64_t rows = (int64_t)N * splits;
+    const int per = (int)((rows + 16 * 256 - 1) / (16 * 256));
+    tr = (int)((rows + 256 * per - 1) / (256 * per));
+    tiles = (N + tr - 1) / tr, grid = (tiles + per - 1) / per;
+  }
+};
+
 template <int MT, int NA, bool NORM>
-void launch_proj(const ProjArgs& A, hipStream_t stream) {
-  const int tiles = (A.N + 15) / 16, S = (A.K + 31) / 32;
+void launch_proj(ProjArgs A, hipStream_t stream) {
+  const int S = (A.K + 31) / 32;
   // (x of 64 rows fits the registers only without the norm and beside one weight tile)
   if constexpr (MT < 4 || (NA == 1 && !NORM)) {
     // (buffer offsets are 32 bits)
@@ -295,8 +310,9 @@ void launch_proj(const ProjArgs& A, hipStream_t stream) {
     const int splits = proj_splits(A.M, A.N, A.K, NORM, NA == 2);
     if (splits > 1 && fits) {
       if constexpr (MT > 1 && NA == 1 && !NORM) {
-        const int per = (tiles * splits + 255) / 256;
-        hipLaunchKernelGGL((decode_proj_resident_kernel<MT, NA, NORM, kResSteps>), dim3((tiles + per - 1) / per, splits),
+        const ProjShape p(A.N, splits);
+        A.tr = p.tr;
+        hipLaunchKernelGGL((decode_proj_resident_kernel<MT, NA, NORM, kResSteps>), dim3(p.grid, splits),
                            dim3(64 * kResWaves), 0, stream, A);
         hipLaunchKernelGGL(decode_proj_sum_kernel, dim3((unsigned)(((int64_t)A.M * A.N + 255) / 256)), dim3(256), 0, stream,
                            A, splits);
@@ -304,8 +320,9 @@ void launch_proj(const ProjArgs& A, hipStream_t stream) {
       }
     }
     if (S <= kResWaves * kResSteps && fits) {
-      // as many workgroups as fit at once (two per CU where the registers allow), with equal shares of tiles
-      const int slots = MT * NA == 1 && !NORM ? 512 : 256, per = (tiles + slots - 1) / slots, grid = (tiles + per - 1) / per;
+      const ProjShape p(A.N, 1);
+      A.tr = p.tr;
+      const int grid = p.grid;
       if (S <= kResWaves * 4)
         hipLaunchKernelGGL((decode_proj_resident_kernel<MT, NA, NORM, 4>), dim3(grid), dim3(64 * kResWaves), 0, stream, A);
       else
@@ -314,9 +331,11 @@ void launch_proj(const ProjArgs& A, hipStream_t stream) {
       return;
     }
   }
-  ProjArgs whole = A;
-  whole.part = nullptr;
-  hipLaunchKernelGGL((decode_proj_stream_kernel<MT, NA, NORM>), dim3(tiles), dim3(64 * kStrWaves), 0, stream, whole);
+  // (beyond 16 rows x is the larger stream, and a tile's rows share it)
+  A.part = nullptr;
+  A.tr = MT == 1 ? ProjShape(A.N, 1).tr : 16;
+  hipLaunchKernelGGL((decode_proj_stream_kernel<MT, NA, NORM>), dim3((A.N + A.tr - 1) / A.tr), dim3(64 * kStrWaves), 0,
+                     stream, A);
 }
 template <int MT>
 void launch_proj_m(const ProjArgs& A, int gated, hipStream_t stream) {
@@ -546,7 +565,7 @@ int kdn_decode_proj(const void* x, int64_t x_row_stride, const void* norm_weight
   const size_t need = kdn_decode_proj_workspace_size(M, N, K, norm_weight != nullptr, gated);
   if (need && (!workspace || workspace_bytes < need || !al(workspace, 4))) return KDN_ERR_ARG;
   const ProjArgs a{(const bf16_t*)x, x_row_stride, (const bf16_t*)norm_weight, eps, (const bf16_t*)W,
-                   (const bf16_t*)bias, (const bf16_t*)res, res_row_stride, M, N, K, (bf16_t*)y, y_row_stride, need ? (float*)workspace : nullptr};
+                   (const bf16_t*)bias, (const bf16_t*)res, res_row_stride, M, N, K, (bf16_t*)y, y_row_stride, need ? (float*)workspace : nullptr, 16};
   if (M <= 16) launch_proj_m<1>(a, gated, stream);
   else if (M <= 32) launch_proj_m<2>(a, gated, stream);
   else launch_proj_m<4>(a, gated, stream);
