@@ -130,22 +130,27 @@ def decode_block(block, x, state):
     """One token through ``block`` on an in-place ``state`` in five launches (``kdn_decode_proj`` and
     ``kdn_decode_mixer``), or None where the call is not of that form: bf16 parameters and activations,
     eval mode under no_grad, at most PACK_MAX_ROWS sequences, pre-norm RMS-norm blocks with an
-    (unbiased w1 | w2) SwiGLU, and no hooks that would miss the parts' calls.
+    (unbiased w1 | w2) SwiGLU, no parts of other types than the model's own, and no hooks that would miss the
+    parts' calls.
 
     At iso_kdn_1.3B width a two-layer step takes 152 us at one sequence and 221 at 32, against 201 and 327
     through the layers' own launches (16 per block)."""
-    from .diag_kdn import DiagonalKalmanDeltaNetwork
+    from .diag_kdn import DiagonalKalmanDeltaNetwork, ShortConvolution
     from .iso_kdn import IsotropicKalmanDeltaNetwork
     from .kdn_ops import step
+    from .kdn_ops.gated_norm import FusedRMSNormGated
     from .kdn_state import KDNLayerState, check_state
-    from .model import LLaMAMLP
+    from .model import LLaMAMLP, SwiGLU
     from .rmsnorm import FusedRMSNorm
     attn, mlp = block.attn, getattr(block, "mlp", None)
     iso = type(attn) is IsotropicKalmanDeltaNetwork
     if not (isinstance(state, KDNLayerState) and state.inplace and _decode_rows(x, block)
             and (iso or type(attn) is DiagonalKalmanDeltaNetwork) and type(mlp) is LLaMAMLP
             and not block.config.parallel_residual and type(block.norm_1) is FusedRMSNorm
-            and type(getattr(block, "norm_2", None)) is FusedRMSNorm and _plain(block)):
+            and type(getattr(block, "norm_2", None)) is FusedRMSNorm and type(mlp.swiglu) is SwiGLU
+            and type(attn.o_norm) is FusedRMSNormGated
+            and (iso or all(type(c) is ShortConvolution for c in (attn.q_conv1d, attn.k_conv1d, attn.v_conv1d)))
+            and _plain(block)):
         return None
     sw, on = mlp.swiglu, attn.o_norm
     if sw.w1.bias is not None or sw.w2.bias is not None or on.activation != "sigmoid" or on.weight is None:

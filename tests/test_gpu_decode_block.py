@@ -104,3 +104,23 @@ def test_decode_block_steps_aside():
         assert _inference.decode_block(block, x, live) is not None
     assert _inference.decode_block(block, x, live) is None  # autograd on
     assert copy.copy(live).seen_tokens == 5
+
+
+@pytest.mark.parametrize("mixer_type,part", [("iso_kdn", "mlp.swiglu"), ("iso_kdn", "attn.o_norm"),
+                                             ("diag_kdn", "attn.q_conv1d"), ("diag_kdn", "attn.v_conv1d")])
+def test_decode_block_keeps_a_replaced_parts_forward(mixer_type, part):
+    """A part that a user exchanged for one of a derived type answers through its own forward (here twice the
+    part's value), so the step goes through the layers' launches."""
+    dev = gpu_or_skip()
+    log(f"case decode_block replaced part {mixer_type} {part}")
+    cfg = model_mod.Config.from_name(("iso" if mixer_type == "iso_kdn" else "diag") + "_kdn_1.3B", n_layer=1, n_head=1,
+                                     n_embd=128, intermediate_size=256)
+    m = model_mod.GPT(cfg).to(dev).to(torch.bfloat16).eval()
+    block = m.transformer.h[0]
+    with torch.no_grad():
+        st = m(torch.zeros(1, 4, dtype=torch.long, device=dev), return_state=True)[1][0]
+        live = KDNLayerState(tuple(c.clone() for c in st.conv), st.memory.clone(), st.precision.clone(), 4, True)
+        module = block.get_submodule(part)
+        module.__class__ = type("Doubled", (type(module),), {"forward": lambda self, *a, **k: 2 * type(self).__base__.forward(self, *a, **k)})
+        assert _inference.decode_block(block, torch.randn(1, 1, 128, device=dev).bfloat16(), live) is None
+    assert live.seen_tokens == 4
