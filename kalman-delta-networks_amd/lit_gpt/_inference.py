@@ -196,13 +196,14 @@ def decode_block(block, x, state):
 
 
 def decode_head(x, norm, head, model):
-    """``head(norm(x))`` for the one-token step in one launch, or None (as ``decode_block``)."""
+    """The logits of ``norm(x)`` and ``head``'s weight (which is all that ``GPT.forward`` uses of it) for the one-token
+    step in one launch, or None (as ``decode_block``)."""
     from .kdn_ops import step
     from .rmsnorm import FusedRMSNorm
     if not (_decode_rows(x, model) and type(norm) is FusedRMSNorm and type(head) is torch.nn.Linear
-            and _bf16_dense(norm.weight, head.weight, head.bias) and _plain(norm) and _plain(head)):
+            and _bf16_dense(norm.weight, head.weight) and _plain(norm)):
         return None
-    y = step.kdn_decode_proj(x.view(x.shape[0], -1), head.weight, norm_weight=norm.weight, eps=norm.eps, bias=head.bias)
+    y = step.kdn_decode_proj(x.view(x.shape[0], -1), head.weight, norm_weight=norm.weight, eps=norm.eps)
     return y.view(x.shape[0], 1, -1)
 
 

@@ -124,3 +124,18 @@ def test_decode_block_keeps_a_replaced_parts_forward(mixer_type, part):
         module.__class__ = type("Doubled", (type(module),), {"forward": lambda self, *a, **k: 2 * type(self).__base__.forward(self, *a, **k)})
         assert _inference.decode_block(block, torch.randn(1, 1, 128, device=dev).bfloat16(), live) is None
     assert live.seen_tokens == 4
+
+
+def test_decode_head_takes_the_weight_alone():
+    """``GPT.forward`` multiplies by the head's weight and leaves a bias out, for one token as for many."""
+    dev = gpu_or_skip()
+    cfg = model_mod.Config.from_name("iso_kdn_1.3B", n_layer=1, n_head=1, n_embd=128, intermediate_size=256)
+    m = model_mod.GPT(cfg)
+    m.lm_head = torch.nn.Linear(128, m.lm_head.out_features, bias=True)
+    torch.nn.init.constant_(m.lm_head.bias, 3.0)
+    m = m.to(dev).to(torch.bfloat16).eval()
+    x = torch.randn(2, 1, 128, device=dev).bfloat16()
+    with torch.no_grad():
+        y = _inference.decode_head(x, m.transformer.ln_f, m.lm_head, m)
+        ref = m.transformer.ln_f(x).double() @ m.lm_head.weight.double().T
+    assert rel(y.float(), ref) < 6e-3  # two bf16 roundings
