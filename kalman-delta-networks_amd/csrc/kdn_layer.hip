@@ -102,12 +102,15 @@ inline int conv_run(int B, int T, int D) {
 }
 inline int conv_blocks(int T, int R) { return (T + kConvRuns * R - 1) / (kConvRuns * R); }
 
-// a * sigmoid(a)'s sigmoid: the hardware reciprocal and one Newton step (as close to 1 / d as the IEEE
-// division, in about half its instructions); above 2^126 the raw reciprocal (0 at infinity) stands
+// The sigmoid by the hardware reciprocal and one Newton step, about half the instructions of the IEEE division.  The
+// reciprocal is within an ulp, so the step leaves at most 2^-46 of the value beside its own rounding: within
+// 0.5000003 ulp of 1 / d where the division is within 0.5.  The exponential's error covers the difference: against float64 the
+// sigmoid's largest error is 3.9e-6 on [-85, -60], 1.0e-6 on [-20, -5] and 3.2e-7 on [-5, 5] with either.
+// The reciprocal flushes subnormal results, so it is taken of d / 4 = (1 + e^-x) / 4, at most 2^126 or infinite.
 __device__ __forceinline__ float sigmoid_nr(float x) {
-  const float d = 1.f + __expf(-x), r = __builtin_amdgcn_rcpf(d);
-  const float rn = __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
-  return d < 0x1p126f ? rn : r;
+  const float d4 = __builtin_fmaf(__expf(-x), 0.25f, 0.25f), r = __builtin_amdgcn_rcpf(d4);
+  const float rn = __builtin_fmaf(__builtin_fmaf(-d4, r, 1.f), r, r);
+  return 0.25f * (d4 < 0x1p127f ? rn : r);
 }
 template <typename T>
 struct Row4;  // 4 channels of a row as loaded
