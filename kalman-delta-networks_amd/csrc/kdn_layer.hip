@@ -83,8 +83,8 @@ __device__ __forceinline__ void ld_taps(const TW* p, float (&wt)[8][kConvW]) {
 // ---------------------------------------------------------------------------
 // Short convolution over whole sequences.  Wave = 64 x 4 consecutive channels of one run of R tokens,
 // block = 4 consecutive runs.  A wave walks its run in groups of 4 rows: the next group's rows are in
-// flight while the current one is computed, the 3 earlier rows stay in registers, so every row is
-// loaded once (and 3 per run again) and rows outside the sequence are found by wave-uniform tests.
+// flight while the current one is computed, the 3 earlier rows stay in registers, so a run loads its rows once
+// and the 4 before it (the backward also the 3 after it), and rows outside the sequence are found by wave-uniform tests.
 // Held by the vector ALU and by the loads in flight rather than by the bytes: with one thread per 8
 // tokens x 8 channels (11 rows loaded and 11 gradients formed for 8, 248 registers in the backward) and an
 // IEEE reciprocal in the sigmoid, one group of B4 T4096 D2304 bf16 took 45.6 us forward and 91.6 backward; now
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void short_conv_fwd_kernel(const TX* __restric
   const int te = min(t0 + R, T);
   for (int t = t0; t < te; t += 4) {
     get_rows(nx, t, T, xw + 3);
-    load_rows(xb, xst, t + 4, T, nx);
+    if (t + 4 < te) load_rows(xb, xst, t + 4, T, nx);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       if (t + u >= te) break;
