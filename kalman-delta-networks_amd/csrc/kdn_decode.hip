@@ -276,26 +276,28 @@ __global__ __launch_bounds__(256) void decode_proj_sum_kernel(const ProjArgs A, 
   A.y[(int64_t)m * A.ys + n] = f2bf(o);
 }
 
-// Splits of K for more than 16 rows past the resident form's K: with x streamed beside W by one workgroup per tile,
+// Splits of K for more than 8 rows past the resident form's K: with x streamed beside W by one workgroup per tile,
 // the 144 workgroups of N 2304, K 6912 each loaded 442 KB of x and 221 KB of W at 32 rows (32.8 us); three
-// splits keep x resident over two tiles (16.6 us with the sum).  At most 16 rows stream: x is small there and
-// the sum's launch would cost more than it saves (12.4 us).
+// splits keep x resident over two tiles (16.6 us with the sum; K 7208, four splits, M 9 / 16: 15.4 / 19.3 us streamed, 12.8 /
+// 13.8 split).  At most 8 rows stream: x is small there and the sum's launch costs what it saves (K 4608, N 1536,
+// M 8 / 9: 8.2 streamed, 8.0 split).
 inline int proj_splits(int M, int N, int K, bool norm, bool gated) {
   const int S = (K + 31) / 32, one = kResWaves * kResSteps;
-  if (M <= 16 || norm || gated || S <= one || (int64_t)N * K >= (1ll << 31)) return 1;
+  if (M <= 8 || norm || gated || S <= one || (int64_t)N * K >= (1ll << 31)) return 1;
   return (S + one - 1) / one;
 }
 
-// Tile height and count for `splits` products of N rows on 256 CUs: as few tiles per workgroup as 16-row tiles
-// allow, then the rows spread evenly (N 2304: 256 tiles of 9 rows, where 144 of 16 left 112 CUs idle; N 6912:
-// 494 of 14, two each, where 432 of 16 gave 216 workgroups 32 rows).  M 1: N 2304 K 6912 15.1 -> 12.4 us, K 2304
-// 5.9 -> 5.3.
+// Tile height and count for `splits` products of N rows on 256 CUs, one workgroup each: as few tiles per workgroup as
+// 16-row tiles allow within a split's share of the CUs, then the rows spread evenly (N 2304: 256 tiles of 9 rows,
+// where 144 of 16 left 112 CUs idle; N 6912: 494 of 14, two each, where 432 of 16 gave 216 workgroups 32 rows).
+// M 1: N 2304 K 6912 15.1 -> 12.4 us, K 2304 5.9 -> 5.3.  Shares: N 2048 in 3 splits runs 3 x 79 workgroups, where rows
+// spread over all the CUs alike gave 3 x 86, two too many (K 6144, M 17 / 64: 18.1 / 31.5 -> 13.7 / 20.3 us).
 struct ProjShape {
   int tr, tiles, grid;
   ProjShape(int N, int splits) {
-    const int64_t rows = (int64_t)N * splits;
-    const int per = (int)((rows + 16 * 256 - 1) / (16 * 256));
-    tr = (int)((rows + 256 * per - 1) / (256 * per));
+    const int cols = splits < 256 ? 256 / splits : 1;  // workgroups of one split, so that all splits run at once
+    const int per = (int)(((int64_t)N + 16 * cols - 1) / (16 * cols));
+    tr = (int)(((int64_t)N + (int64_t)cols * per - 1) / ((int64_t)cols * per));
     tiles = (N + tr - 1) / tr, grid = (tiles + per - 1) / per;
   }
 };
@@ -309,7 +311,7 @@ void launch_proj(ProjArgs A, hipStream_t stream) {
     const bool fits = (int64_t)A.N * A.K < (1ll << 31) && A.xs >= 0 && 64 * A.xs + A.K < (1ll << 31);
     const int splits = proj_splits(A.M, A.N, A.K, NORM, NA == 2);
     if (splits > 1 && fits) {
-      if constexpr (MT > 1 && NA == 1 && !NORM) {
+      if constexpr (NA == 1 && !NORM) {
         const ProjShape p(A.N, splits);
         A.tr = p.tr;
         hipLaunchKernelGGL((decode_proj_resident_kernel<MT, NA, NORM, kResSteps>), dim3(p.grid, splits),

@@ -139,3 +139,21 @@ def test_decode_head_takes_the_weight_alone():
         y = _inference.decode_head(x, m.transformer.ln_f, m.lm_head, m)
         ref = m.transformer.ln_f(x).double() @ m.lm_head.weight.double().T
     assert rel(y.float(), ref) < 6e-3  # two bf16 roundings
+
+
+# K past 2304 in splits from 9 rows on; each split's tiles fit its share of the CUs (2048 rows in 3: 79 workgroups)
+@pytest.mark.parametrize("M,N,K,bias,res", [(8, 100, 2312, True, True), (9, 100, 2312, True, True), (16, 2048, 6144, False, True),
+                                            (12, 3, 4616, True, False), (33, 5, 20744, False, True),
+                                            (64, 2048, 6144, True, False), (17, 4100, 2560, False, False)])
+def test_split_projection_matches_fp64(M, N, K, bias, res):
+    dev = gpu_or_skip()
+    log(f"case decode_proj split M={M} N={N} K={K} bias={bias} res={res}")
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).bfloat16()
+    W = (torch.randn(N, K, generator=g) / K ** 0.5).bfloat16()
+    b = torch.randn(N, generator=g).bfloat16() if bias else None
+    r = torch.randn(M, N, generator=g).bfloat16() if res else None
+    ref = x.double() @ W.double().T + (b.double() if bias else 0) + (r.double() if res else 0)
+    to = lambda t: t.to(dev) if t is not None else None  # noqa: E731
+    y = kdn_decode_proj(to(x), to(W), bias=to(b), residual=to(r))
+    assert float(((y.double().cpu() - ref).abs() / (ref.abs() + 1)).max()) < 2.0 ** -8  # one rounding (2^-9 of the value), fp32 sums
