@@ -42,7 +42,9 @@ __device__ __forceinline__ uint4 pack8(const float* f) {
 //     once, the next tile's issued before the current one's sums meet.  Streaming x beside W instead halved
 //     the weight bytes in flight and read x once per tile from L2: M 1 / 32, N 32000 K 2304 took
 //     39.7 / 84.0 us, now 27.8 / 36.5 (5.3 / 4.0 TB/s); [2 x 6912, 2304] gated 21.0 / 27.2, now 17.3 / 22.5.
-//   streaming (longer K): 16 waves, one tile per workgroup, x beside W.
+//   streaming (longer K, and more than 32 rows with the norm or the gate): 16 waves, one tile per workgroup, x beside
+//     W and so read once per tile.  Up to 8 rows that is little; beyond, x is the larger stream (M 64, N 32000 K 2304:
+//     590 MB of it for 147 MB of W, 152 us), and a caller with a choice takes the norm and the product apart.
 // ---------------------------------------------------------------------------------------------
 struct ProjArgs {
   const bf16_t* x;

@@ -126,14 +126,51 @@ def _bf16_dense(*params) -> bool:
                for p in params)
 
 
+# kdn_decode_proj keeps x in registers up to this K (8 waves x 9 steps of 32)
+_PROJ_RESIDENT_K = 2304
+
+
+def proj_fused(M: int, N: int, K: int, norm: bool, gated: bool) -> bool:
+    """Whether a decode projection of ``M`` rows runs as one ``kdn_decode_proj`` launch rather than apart (the norm
+    kernel, ``linear`` / ``swiglu_gate``, the addition).
+
+    * With x in registers (M <= 32, K <= 2304) one launch is the faster, K 512 to 2304: [2 x 7208, 2304] gated at M 1 /
+      32 takes 18.0 / 22.3 us, apart 19.7 / 27.2.  (Only the widest product, a head's, loses from 17 rows on: up to
+      5 us of 30.)
+    * A normed or gated product past either limit re-reads x for every tile of 16 output rows: [32000, 2304] at M 33 /
+      64 takes 112 / 152 us, apart 35; [2 x 7680, 2560] gated at M 1 / 32 takes 24 / 45, apart 21 / 30.  It stays one
+      launch for 5 to 8 rows, which the GEMV multiplies one by one (M 8: 26 us, apart 46), gated also for 9 to 16 up
+      to K 3072 (M 9 / 16: 26 / 29, apart 31), and beyond 32 rows where x is small and all tiles run at once (K <= 1024,
+      256 tiles; [2 x 3072, 1024] gated at M 64: 10.6, apart 18.6).
+    * A product by itself splits a longer K and stays one launch ([2560, 7680] at M 1 / 16 / 64: 14.7 / 15.7 / 23.9 us,
+      apart 14.9 / 16.2 / 26.1)."""
+    if not (norm or gated):
+        return True
+    if M <= 32:
+        return K <= _PROJ_RESIDENT_K or 5 <= M <= (16 if gated and K <= 3072 else 8)
+    return K <= 1024 and N <= 16 * 256
+
+
+def _decode_proj(x, weight, *, norm=None, bias=None, residual=None, gated=False):
+    """``kdn_decode_proj`` (``norm``: an RMS-norm module) by the rule of ``proj_fused``: in one launch, or apart."""
+    from .kdn_ops import step
+    N = weight.shape[0] // 2 if gated else weight.shape[0]
+    if proj_fused(x.shape[0], N, x.shape[1], norm is not None, gated):
+        return step.kdn_decode_proj(x, weight, norm_weight=None if norm is None else norm.weight,
+                                    eps=0.0 if norm is None else norm.eps, bias=bias, residual=residual, gated=gated)
+    h = x if norm is None else norm(x)
+    y = swiglu_gate(h, weight) if gated else linear(h, weight, bias)
+    return y if residual is None else residual + y
+
+
 def decode_block(block, x, state):
     """One token through ``block`` on an in-place ``state`` in five launches (``kdn_decode_proj`` and
-    ``kdn_decode_mixer``), or None where the call is not of that form: bf16 parameters and activations,
-    eval mode under no_grad, at most PACK_MAX_ROWS sequences, pre-norm RMS-norm blocks with an
-    (unbiased w1 | w2) SwiGLU, no parts of other types than the model's own, and no hooks that would miss the
-    parts' calls.
+    ``kdn_decode_mixer``; a few more where ``proj_fused`` takes a product apart), or None where the call is not
+    of that form: bf16 parameters and activations, eval mode under no_grad, at most PACK_MAX_ROWS sequences,
+    pre-norm RMS-norm blocks with an (unbiased w1 | w2) SwiGLU, no parts of other types than the model's own, and
+    no hooks that would miss the parts' calls.
 
-    At iso_kdn_1.3B width a two-layer step takes 152 us at one sequence and 221 at 32, against 201 and 327
+    At iso_kdn_1.3B width a two-layer step takes 144 us at one sequence and 216 at 32, against 199 and 325
     through the layers' own launches (16 per block)."""
     from .diag_kdn import DiagonalKalmanDeltaNetwork, ShortConvolution
     from .iso_kdn import IsotropicKalmanDeltaNetwork
@@ -180,27 +217,27 @@ def decode_block(block, x, state):
     w_in = packed_weight(attn, "in_proj", inputs, row_multiple=8 if iso else 1)  # the layers' own packing
     b_in = None if iso else packed_bias(attn, "in_proj_bias", (3 * n + 3 * K, attn.r_proj.bias))
     x0 = x.view(B, -1)
-    p = step.kdn_decode_proj(x0, w_in, norm_weight=block.norm_1.weight, eps=block.norm_1.eps, bias=b_in)
+    p = _decode_proj(x0, w_in, norm=block.norm_1, bias=b_in)
     o = step.kdn_decode_mixer(
         p, offsets, tuple(state.conv), taps, wf, wo, bo, wg, bg,
         as_f32(attn, "omega_bias", attn.omega_proj.bias) if iso else None,
         as_f32(attn, "r_bias", attn.r_proj.bias) if iso else None, as_f32(attn, "A_log", attn.A_log),
         as_f32(attn, "dt_bias", attn.dt_bias), omega_min=attn.omega_min, r_min=attn.r_min, info_scale=attn.info_scale,
         precision=state.precision, memory=state.memory, norm_weight=on.weight, eps=on.eps, iso=iso)
-    x1 = step.kdn_decode_proj(o, attn.o_proj.weight, residual=x0)
-    hid = step.kdn_decode_proj(x1, packed_weight(sw, "w12", (sw.w1.weight, sw.w2.weight)),
-                               norm_weight=block.norm_2.weight, eps=block.norm_2.eps, gated=True)
-    x2 = step.kdn_decode_proj(hid, sw.w3.weight, bias=sw.w3.bias, residual=x1)
+    x1 = _decode_proj(o, attn.o_proj.weight, residual=x0)
+    hid = _decode_proj(x1, packed_weight(sw, "w12", (sw.w1.weight, sw.w2.weight)), norm=block.norm_2, gated=True)
+    x2 = _decode_proj(hid, sw.w3.weight, bias=sw.w3.bias, residual=x1)
     state.seen_tokens += 1
     return x2.view(x.shape)
 
 
 def decode_head(x, norm, head, model):
     """The logits of ``norm(x)`` and ``head``'s weight (which is all that ``GPT.forward`` uses of it) for the one-token
-    step in one launch, or None (as ``decode_block``)."""
+    step in one launch, or None (as ``decode_block``, or where ``proj_fused`` takes them apart)."""
     from .kdn_ops import step
     from .rmsnorm import FusedRMSNorm
     if not (_decode_rows(x, model) and type(norm) is FusedRMSNorm and type(head) is torch.nn.Linear
+            and proj_fused(x.shape[0], head.out_features, x.shape[2], True, False)
             and _bf16_dense(norm.weight, head.weight) and _plain(norm)):
         return None
     y = step.kdn_decode_proj(x.view(x.shape[0], -1), head.weight, norm_weight=norm.weight, eps=norm.eps)

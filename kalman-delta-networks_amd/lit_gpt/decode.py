@@ -5,9 +5,9 @@ KDN layer's history is a fixed-size state (``KDNLayerState``), so a decode step 
 any context length: the chunked scan consumes the prompt (``prefill``), then each ``step`` runs
 one token through every block, the mixers through ``kdn_kalman_step``.
 
-One decode step is a chain of small dependent kernels (5 per block for a bf16 model, ``decode_block``; about
-20 otherwise), so at small batch the step is bound by launch overhead as much as by the GPU.  With ``use_graph=True`` the step is
-captured once as a HIP graph (``torch.cuda.CUDAGraph``) over fixed buffers -- the token ids, the
+One decode step is a chain of small dependent kernels (5 to 9 per block for a bf16 model, ``decode_block``;
+about 20 otherwise), so at small batch the step is bound by launch overhead as much as by the GPU.  With
+``use_graph=True`` the step is captured once as a HIP graph (``torch.cuda.CUDAGraph``) over fixed buffers -- the token ids, the
 logits and every layer's state -- and each later step is one graph replay.  The decoder's layer
 states are in-place states (``KDNLayerState.inplace``): each layer advances its own buffers, the
 mixers through ``kdn_kalman_step`` (the single-token gain and memory update in one launch).

@@ -157,3 +157,10 @@ def test_split_projection_matches_fp64(M, N, K, bias, res):
     to = lambda t: t.to(dev) if t is not None else None  # noqa: E731
     y = kdn_decode_proj(to(x), to(W), bias=to(b), residual=to(r))
     assert float(((y.double().cpu() - ref).abs() / (ref.abs() + 1)).max()) < 2.0 ** -8  # one rounding (2^-9 of the value), fp32 sums
+
+
+@pytest.mark.parametrize("mixer_type,B,H,d", [("iso_kdn", 33, 9, 128), ("diag_kdn", 33, 9, 128), ("iso_kdn", 2, 20, 128),
+                                              ("diag_kdn", 6, 38, 64), ("diag_kdn", 9, 20, 128)])
+def test_decode_block_with_projections_apart(mixer_type, B, H, d, monkeypatch):
+    """Beyond 32 rows and past K 2304 the normed and gated products leave the one launch (K 1152 and 2432, 2560)."""
+    test_decode_block_matches_the_layers_launches(mixer_type, B, H, d, monkeypatch)
