@@ -50,11 +50,13 @@ def mfma_peak(tag: str) -> float:
 
 
 def kernel_counts(variant: str, B: int, T: int, H: int, K: int, V: int, infer: bool = False,
-                  half_states: bool = False):
+                  half_states: bool = False, groups: bool = False):
     """Algorithmic HBM bytes and FLOPs per launch of each kernel (inputs read once, outputs
     written once, no recompute).  N = B*T*H token-heads; per-token-head figures times N.  With
-    ``infer`` (no backward follows) the fused state pass skips what only the backward reads: h and delta.  ``half_states``: the per-chunk state copies h and dh the
-    backward reads are bf16 (the isotropic scan with one chunk group)."""
+    ``groups`` (chunk groups) the intra-chunk build forms U = A v in place of the state passes; with ``infer`` (no
+    backward follows) the fused state pass skips what only the backward reads, h and delta, and the build of
+    groups A.  ``half_states``: the per-chunk state copies h and dh the backward reads are bf16 (the isotropic
+    scan with one chunk group)."""
     N = B * T * H
     kap_in = 4 * K if variant == "diag" else 4           # kappa fp32 [K] or beta fp32
     dkap_out = 4 * K if variant == "diag" else 4
@@ -79,6 +81,11 @@ def kernel_counts(variant: str, B: int, T: int, H: int, K: int, V: int, infer: b
                           + 2 * V + 2 * 2 * K + dkap_out + 4 * K + (8 if variant == "iso" else 0),
                           2 * (3 * K * V + C * V) + 2 * 2 * (C * K)),
     }
+    if groups:  # v read and U written by the build; U read in place of v and A by the state passes
+        b, f = per["mem_intra_fwd"]
+        per["mem_intra_fwd"] = (b + 6 * V - (mm if infer else 0), f + 2 * C * V / 2)
+        b, f = per["mem_state_readout_fwd"]
+        per["mem_state_readout_fwd"] = (b + 2 * V - mm, f - 2 * C * V / 2)
     if infer:
         b, f = per["mem_state_readout_fwd"]
         per["mem_state_readout_fwd"] = (b - h_b - 4 * V, f)
@@ -547,7 +554,7 @@ def run_config3(steps: int, warmup: int, B: int = 1, T: int = 32768, H: int = 18
             step()
         torch.cuda.synchronize()
     fwd_tags = ("diag_front_norm_fwd", "diag_front_fwd", "mem_intra_fwd", "mem_state_readout_fwd")
-    counts = kernel_counts("diag", B, T, H, K, K, infer=True)
+    counts = kernel_counts("diag", B, T, H, K, K, infer=True, groups=True)
     counts.update(frontend_counts("diag", B, T, H, K))
     kernels = {}
     for tag in fwd_tags:

@@ -238,7 +238,7 @@ size_t kdn_mem_bwd_workspace_size(int B, int T, int H, int K, int V);
  * in one call run the state pass with the readout fused.  Bit 3 (with stages >= 0) declares that
  * no backward follows (inference, as under torch.no_grad): the intermediates only the backward
  * reads are then not written, and `saved` is scratch for this call alone.  v is read by the state
- * pass (bit 1).  A caller that keeps no
+ * pass (bit 1), with several chunk groups (kdn_mem_state_groups) by the build (bit 0).  A caller that keeps no
  * `saved` from a training forward (the reference's policy: it re-runs recompute_w_u_fwd and the state
  * forward in its backward, iso_kdn_chunk.py:2101-2140, diag_kdn_chunk.py:3271-3277) rebuilds it for
  * kdn_mem_bwd with bit 0, then bit 1 alone (the state pass without the readout; o and final_state

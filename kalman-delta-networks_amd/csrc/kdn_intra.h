@@ -6,7 +6,8 @@
 //                      A_IJ = -A_II sum_{J<=P<I} N_IP A_PJ           (fp32 MFMA)
 //   W = A (k 2^G),  Kf = kappa 2^{G_last - G},  Qg = scale q 2^G
 // N and M are K-contractions of factored operands (bf16x3 MFMA); the decay 2^{G_c - G_s} is split
-// at an anchor so neither factor overflows.  The state pass forms U = A V beside its recurrence.
+// at an anchor so neither factor overflows.  The state pass forms U = A V beside its recurrence; with chunk groups,
+// whose first pass has no waves to spare, it is formed here (VU).
 //
 // intra_fwd_kernel (every chunk): one anchor per chunk and channel, the midpoint of the chunk's gate
 //   range m = (G_0 + G_{L-1}) / 2, so |G - m| <= span / 2 on every row:
@@ -100,9 +101,10 @@ __device__ __forceinline__ void st8(bufrsrc r, uint32_t off, const float* f) {
 // then to An [c][s], and W = A (k 2^G) (rows past L dropped by the output descriptor).
 // The whole LDS buffer (sA / sN / sX) is free for this function's staging after A's fragments are read.
 // NORM (in-op L2 norm): k is raw in memory, sRk holds the rows' rstd.
-template <int K, bool NORM>
+// VU > 0: U = A V too (V of VU columns through rv), to Un as accumulator tiles (kdn_state::st_tiles).
+template <int K, bool NORM, int VU>
 __device__ __forceinline__ void intra_solve_emit(float* sA, const float* sN, float* sX, float* An, bufrsrc rk, bufrsrc rG,
-                                                 bufrsrc rW, int H, int tid, const float* sRk) {
+                                                 bufrsrc rW, int H, int tid, const float* sRk, bufrsrc rv, float* Un) {
   const int lane = tid & 63, w = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
   // ---- 3. diagonal blocks of A: X_I = (I + N_II)^{-1}, lane j < 16 of wave I owns column j
   if (lane < 16) {
@@ -151,7 +153,7 @@ __device__ __forceinline__ void intra_solve_emit(float* sA, const float* sN, flo
 
   // ---- 5. A to memory, whole rows
   {
-    const bufrsrc rA = make_buf(An, C * C * 4);
+    const bufrsrc rA = make_buf(An, An ? C * C * 4 : 0u);  // (U formed here and no backward: nothing reads A)
 #pragma unroll
     for (int u = 0; u < C * C / 4 / 256; ++u) {
       const int e = 4 * (tid + 256 * u);
@@ -177,6 +179,44 @@ __device__ __forceinline__ void intra_solve_emit(float* sA, const float* sN, flo
   // columns) is the A fragment and A's rows the B fragment, so the D tile gives each lane 4 consecutive channels of
   // one chunk row (16-byte stores).
   __syncthreads();  // every wave has its A fragments; the buffer is free
+  if constexpr (VU > 0) {  // A the first operand: a lane holds 4 rows of one column; V is exact in bf16
+#pragma unroll
+    for (int u = 0; u < C * VU / 8 / 256; ++u) {
+      const int e = tid + 256 * u, sr = e / (VU / 8), c8 = 8 * (e % (VU / 8));
+      float x[8];
+      unpack8(__builtin_amdgcn_raw_buffer_load_b128(rv, ((uint32_t)(sr * H) * VU + c8) * 2, 0, 0), x);
+      *reinterpret_cast<float4*>(sX + sr * XR + c8) = float4{x[0], x[1], x[2], x[3]};
+      *reinterpret_cast<float4*>(sX + sr * XR + c8 + 4) = float4{x[4], x[5], x[6], x[7]};
+    }
+    __syncthreads();
+    const bufrsrc rU = make_buf(Un, C * VU * 4);
+    for (int t = w; t < VU / 16; t += 4) {
+      uint4 xh[2], xl[2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const float* colp = sX + (32 * kb + 4 * g4) * XR + 16 * t + r16;
+        float x[8];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          x[jj] = colp[jj * XR];
+          x[4 + jj] = colp[(16 + jj) * XR];
+        }
+        split8(x, xh[kb], xl[kb]);
+      }
+#pragma unroll
+      for (int I = 0; I < 4; ++I) {
+        f32x4 acc = zero4();
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          if (kb == 1 && I < 2) continue;  // A[c][s] = 0 for s > c
+          acc = kdn_state::mma2(ah[I][kb], al[I][kb], xh[kb], acc);
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), rU, (uint32_t)((t * 4 + I) * 64 + lane) * 16,
+                                               0, 0);
+      }
+    }
+    __syncthreads();
+  }
 #pragma unroll
   for (int u = 0; u < C * K / 8 / 256; ++u) {
     const int e = tid + 256 * u, sr = e / (K / 8), c8 = 8 * (e % (K / 8));
@@ -247,12 +287,13 @@ __device__ __forceinline__ float row_rstd(const u32x4 (&raw)[KB]) {
 }
 
 // grid (chunks, B*H), block 256: chunks n0 .. n0 + gridDim.x - 1 of every head.
-template <int K, bool ISO, bool NORM = false>
+// VU > 0 (chunk groups): U = A V is formed here, from V of VU columns.
+template <int K, bool ISO, bool NORM, int VU>
 __global__ __launch_bounds__(256, 3) void intra_fwd_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, int T, int H, int NT, float scale, float* __restrict__ W, float* __restrict__ Kf,
-    float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag, int* __restrict__ flags, float* __restrict__ q_rstd = nullptr,
-    float* __restrict__ k_rstd = nullptr, int n0 = 0) {
+    float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag, int* __restrict__ flags,
+    float* __restrict__ q_rstd, float* __restrict__ k_rstd, int n0, const bf16_t* __restrict__ v, float* __restrict__ Ug) {
   constexpr int KB = K / 32;
   // R fragments [s-tile][kb] until the N / M build, then A [c][s] in the same bytes
   constexpr int RBYTES = (C / 16) * KB * TILE * 2, ABYTES = C * AP * 4;
@@ -282,7 +323,7 @@ __global__ __launch_bounds__(256, 3) void intra_fwd_kernel(
   const bufrsrc rQg = make_buf(Qg + ((int64_t)bh * T + t0) * K, L * K * 4);
   const bufrsrc rW = make_buf(W + ((int64_t)bh * T + t0) * K, L * K * 4);
   float* Mn = Mg + ((int64_t)bh * NT + n) * C * C;
-  float* An = Ag + ((int64_t)bh * NT + n) * C * C;
+  float* An = Ag ? Ag + ((int64_t)bh * NT + n) * C * C : nullptr;
 
   // ---- 0. the chunk's decay span max_i (G_0 - G_{L-1})_i, from rows 0 and L-1 alone, before any
   // other load or store: a chunk past the single anchor's range goes to the block-anchor kernel
@@ -437,7 +478,8 @@ __global__ __launch_bounds__(256, 3) void intra_fwd_kernel(
   }
   __syncthreads();
 
-  intra_solve_emit<K, NORM>(sA, sN, sX, An, rk, rG, rW, H, tid, sRk);
+  const bufrsrc rv = make_buf(v + in_row0 * VU, rows_in * VU * 2);
+  intra_solve_emit<K, NORM, VU>(sA, sN, sX, An, rk, rG, rW, H, tid, sRk, rv, Ug + ((int64_t)bh * NT + n) * C * VU);
 }
 
 // LDS of the block-anchor path for one chunk (intra_fwd_block_chunk), carved from a caller's 16-byte aligned
@@ -455,12 +497,12 @@ struct BlockLds {
 // The block-anchor path for one chunk intra_fwd_kernel flagged (block 256; lds: BlockLds<K>::bytes).
 // Returns false, leaving the chunk flagged, when a 16-token block spans more than kBlockSpanMax (the exact
 // path takes it); otherwise writes the chunk's outputs and clears its flag.
-template <int K, bool ISO, bool NORM>
+template <int K, bool ISO, bool NORM, int VU>
 __device__ __forceinline__ bool intra_fwd_block_chunk(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, int T, int H, int NT, float scale, float* __restrict__ W, float* __restrict__ Kf,
     float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag, int* __restrict__ flags, float* __restrict__ q_rstd,
-    float* __restrict__ k_rstd, int n, int bh, unsigned char* lds) {
+    float* __restrict__ k_rstd, const bf16_t* __restrict__ v, float* __restrict__ Ug, int n, int bh, unsigned char* lds) {
   constexpr int KB = K / 32;
   using Lds = BlockLds<K>;
   constexpr int RABYTES = Lds::RABYTES;
@@ -489,7 +531,7 @@ __device__ __forceinline__ bool intra_fwd_block_chunk(
   const bufrsrc rQg = make_buf(Qg + ((int64_t)bh * T + t0) * K, L * K * 4);
   const bufrsrc rW = make_buf(W + ((int64_t)bh * T + t0) * K, L * K * 4);
   float* Mn = Mg + ((int64_t)bh * NT + n) * C * C;
-  float* An = Ag + ((int64_t)bh * NT + n) * C * C;
+  float* An = Ag ? Ag + ((int64_t)bh * NT + n) * C * C : nullptr;
 
   // ---- 0. block anchors m_J = (G_{16J} + G_{16J+15}) / 2 per channel (rows clamped to the chunk)
   // and the block spans; a chunk with a span past kBlockSpanMax stays for the exact kernel
@@ -624,7 +666,8 @@ __device__ __forceinline__ bool intra_fwd_block_chunk(
   }
   __syncthreads();
 
-  intra_solve_emit<K, NORM>(sA, sN, sX, An, rk, rG, rW, H, tid, sRk);
+  const bufrsrc rv = make_buf(v + in_row0 * VU, rows_in * VU * 2);
+  intra_solve_emit<K, NORM, VU>(sA, sN, sX, An, rk, rG, rW, H, tid, sRk, rv, Ug + ((int64_t)bh * NT + n) * C * VU);
   if (tid == 0) flags[lin] = 0;
   return true;
 }

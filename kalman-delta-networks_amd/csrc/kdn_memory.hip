@@ -14,7 +14,7 @@
 //
 // Kernels (grid = one workgroup per chunk unless noted, 256 threads = 4 waves):
 //   intra_fwd    N/M (MFMA, one anchor per chunk, then one per 16-token block for the chunks
-//                that need it), the inverse A; W, Kf, Qg
+//                that need it), the inverse A; W, Kf, Qg (with chunk groups U = A V)
 //   state_fwd    serial over chunks, one workgroup per (V-slice, b, h): h per chunk, delta
 //   readout      chunk-parallel O = Qg h + M delta (kdn_state.h)
 //   state_bwd    serial reverse (kdn_state.h): d delta = M^T dO + Kf dS;  dX = A^T d delta;
@@ -291,12 +291,13 @@ struct ExactFwdLds {
   static constexpr int OFF2 = (2 * C * KP > C * XP) ? 2 * C * KP : C * XP;
   static constexpr int bytes = (OFF2 + 2 * C * KP + C * NS + 4) * 4;
 };
-template <int K, bool ISO>
+// VU > 0: U = A V too, in fp32, to the chunk's accumulator tiles (kdn_state::st_tiles).
+template <int K, bool ISO, int VU>
 __device__ void intra_fwd_exact_chunk(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, int T, int H, int NT, float scale, float* __restrict__ W, float* __restrict__ Kf,
     float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag, int n, int bh, float* __restrict__ q_rstd,
-    float* __restrict__ k_rstd, unsigned char* lds) {
+    float* __restrict__ k_rstd, const bf16_t* __restrict__ v, float* __restrict__ Ug, unsigned char* lds) {
   constexpr int KP = K + 4;
   constexpr int XP = ExactFwdLds<K>::XP;
   // sQ | sA are dead after Kf / Qg are written and are then reused for the solve's sX [C][XP]
@@ -330,7 +331,7 @@ __device__ void intra_fwd_exact_chunk(
   // forward substitution (I+N) X = [I | K e^g], thread = column (rows past L of N are zero); 16-row blocks
   if (tid < C + K) {
     const int j = tid, col = j - C;  // col < 0: column j of A
-    float* dA = Ag + ((int64_t)bh * NT + n) * C * C;
+    float* dA = Ag ? Ag + ((int64_t)bh * NT + n) * C * C : nullptr;
 #pragma unroll 1
     for (int I = 0; I < 4; ++I) {
       float acc[16];
@@ -361,9 +362,25 @@ __device__ void intra_fwd_exact_chunk(
       for (int r = 0; r < 16; ++r) {
         const int c = 16 * I + r;
         sX[c * XP + j] = acc[r];
-        if (col < 0) dA[c * C + j] = acc[r];
-        else if (c < L) W[bht(bh, t0 + c, T, K) + col] = acc[r];
+        if (col < 0) {
+          if (dA) dA[c * C + j] = acc[r];
+        } else if (c < L) W[bht(bh, t0 + c, T, K) + col] = acc[r];
       }
+    }
+  }
+  if constexpr (VU > 0) {
+    __syncthreads();  // A: columns 0 .. C - 1 of sX
+    float* Un = Ug + ((int64_t)bh * NT + n) * C * VU;
+    for (int e = tid; e < (C / 4) * VU; e += 256) {  // rows 4 r4 .. + 3 of one column
+      const int col = e % VU, r4 = e / VU;
+      float acc[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < min(L, 4 * r4 + 4); ++s) {  // V is zero past L, A above its diagonal
+        const float x = bf2f(v[bthk(b, t0 + s, h, col, T, H, VU)]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = fmaf(sX[(4 * r4 + j) * XP + s], x, acc[j]);
+      }
+      const int tile = (col >> 4) * 4 + (r4 >> 2), ln = (col & 15) + 16 * (r4 & 3);
+      *reinterpret_cast<float4*>(Un + (tile * 64 + ln) * 4) = float4{acc[0], acc[1], acc[2], acc[3]};
     }
   }
 }
@@ -383,12 +400,13 @@ __device__ __forceinline__ bool any_flagged(const int* __restrict__ flags, int N
 // Each flagged chunk takes the block-anchor path, and the exact path when that leaves it flagged, in the same
 // workgroup; the two paths' LDS arrays share one pool (one workgroup per CU).  A workgroup first loads all its
 // chunks' flags at once and exits when none is set.  One launch for both paths.
-template <int K, bool ISO, bool NORM>
+template <int K, bool ISO, bool NORM, int VU>
 __global__ __launch_bounds__(256) void intra_fwd_flagged_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ kap,
     const float* __restrict__ gc, int T, int H, int NT, int BH, int n0, int n1, float scale, float* __restrict__ W,
     float* __restrict__ Kf, float* __restrict__ Qg, float* __restrict__ Mg, float* __restrict__ Ag,
-    int* __restrict__ flags, float* __restrict__ q_rstd, float* __restrict__ k_rstd) {
+    int* __restrict__ flags, float* __restrict__ q_rstd, float* __restrict__ k_rstd, const bf16_t* __restrict__ v,
+    float* __restrict__ Ug) {
   constexpr int LB = kdn_intra::BlockLds<K>::bytes, LE = ExactFwdLds<K>::bytes;
   __shared__ __attribute__((aligned(16))) unsigned char lds[LB > LE ? LB : LE];
   const int len = n1 - n0, N = BH * len;
@@ -400,10 +418,11 @@ __global__ __launch_bounds__(256) void intra_fwd_flagged_kernel(
     const int bh = i / len, n = n0 + i % len;
     if (flags[(int64_t)bh * NT + n] == 0) continue;
     __syncthreads();  // LDS of the previous chunk is dead
-    if (!kdn_intra::intra_fwd_block_chunk<K, ISO, NORM>(q, k, kap, gc, T, H, NT, scale, W, Kf, Qg, Mg, Ag, flags,
-                                                        q_rstd, k_rstd, n, bh, lds)) {
+    if (!kdn_intra::intra_fwd_block_chunk<K, ISO, NORM, VU>(q, k, kap, gc, T, H, NT, scale, W, Kf, Qg, Mg, Ag, flags,
+                                                            q_rstd, k_rstd, v, Ug, n, bh, lds)) {
       __syncthreads();  // the block path's span reads are done
-      intra_fwd_exact_chunk<K, ISO>(q, k, kap, gc, T, H, NT, scale, W, Kf, Qg, Mg, Ag, n, bh, q_rstd, k_rstd, lds);
+      intra_fwd_exact_chunk<K, ISO, VU>(q, k, kap, gc, T, H, NT, scale, W, Kf, Qg, Mg, Ag, n, bh, q_rstd, k_rstd, v, Ug,
+                                        lds);
     }
   }
 }
@@ -712,7 +731,7 @@ inline void with_copy_mask(int hm, F f) {
 
 // saved-buffer layout (floats), TT = B*H*T, NB = B*H*NT
 struct MemLayout {
-  int64_t W, Kf, Qg, M, A, h, D, flags, grp, mid, total;
+  int64_t W, Kf, Qg, M, A, h, D, flags, grp, mid, U, total;
   GroupCount gc;
   MemLayout(int B, int T, int H, int K, int V) {
     const int64_t TT = (int64_t)B * H * T, NB = (int64_t)B * H * cdiv(T, C);
@@ -727,7 +746,8 @@ struct MemLayout {
     flags = D + NB * C * V;  // (D: whole accumulator tiles, kdn_state::st_tiles)  NB ints: chunk taken by the exact intra-chunk path
     grp = round64(flags + NB);  // the forward state pass's group buffers (dead after the forward)
     mid = grp + group_floats((int64_t)B * H, gc, K, V);  // the overlapped forward's carried state
-    total = mid + (int64_t)B * H * K * V;
+    U = mid + (int64_t)B * H * K * V;  // chunk groups: U = A V in whole accumulator tiles, formed by the build
+    total = U + (gc.NG > 1 ? NB * C * V : 0);
   }
 };
 struct BwdLayout {
@@ -877,11 +897,15 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
   const int NT = cdiv(T, C);
   MemLayout lay(B, T, H, K, V);
   float *W = saved + lay.W, *Kf = saved + lay.Kf, *Qg = saved + lay.Qg, *M = saved + lay.M, *A = saved + lay.A,
-        *hb = saved + lay.h, *D = saved + lay.D;
+        *hb = saved + lay.h, *D = saved + lay.D, *U = saved + lay.U;
   int* flags = reinterpret_cast<int*>(saved + lay.flags);
   const int hm = half_copies(iso, lay.gc);
-  // bit 3 (stages >= 0): no backward follows, so where the readout is fused h and delta are not written
+  // chunk groups: the build forms U = A V and the state pass reads no A (state_fwd_kernel, UG)
+  const bool grouped = lay.gc.NG > 1;
+  // bit 3 (stages >= 0): no backward follows, so where the readout is fused h and delta are not written, nor A with
+  // chunk groups
   const bool infer = stages >= 0 && (stages & 8) != 0;
+  float* Ast = infer && grouped ? nullptr : A;
   // the intra-chunk build of chunks n0 .. n1 - 1 on stream s: the single-anchor kernel, then one launch for the
   // chunks it flagged (the block-anchor path, and the exact path for those it leaves flagged)
   auto launch_intra = [&](int n0, int n1, hipStream_t s) {
@@ -889,31 +913,40 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
     const int gx = min(B * H * (n1 - n0), 256);  // one workgroup per CU fits (its LDS)
     // the in-op L2 norm (q_rstd given) is a template variant: its row loads would otherwise cost the
     // plain kernels registers
-#define KDN_INTRA(ISO_, NORM_)                                                                                         \
+#define KDN_INTRA(ISO_, NORM_, VU_)                                                                                    \
   do {                                                                                                                 \
-    hipLaunchKernelGGL((kdn_intra::intra_fwd_kernel<K, ISO_, NORM_>), gchunk, dim3(256), 0, s, q, k, kap, gc, T, H,    \
-                       NT, scale, W, Kf, Qg, M, A, flags, q_rstd, k_rstd, n0);                                        \
-    hipLaunchKernelGGL((intra_fwd_flagged_kernel<K, ISO_, NORM_>), dim3(gx), dim3(256), 0, s, q, k, kap, gc, T, H, NT, \
-                       B * H, n0, n1, scale, W, Kf, Qg, M, A, flags, q_rstd, k_rstd);                                 \
+    hipLaunchKernelGGL((kdn_intra::intra_fwd_kernel<K, ISO_, NORM_, VU_>), gchunk, dim3(256), 0, s, q, k, kap, gc, T, H, \
+                       NT, scale, W, Kf, Qg, M, Ast, flags, q_rstd, k_rstd, n0, v, U);                                 \
+    hipLaunchKernelGGL((intra_fwd_flagged_kernel<K, ISO_, NORM_, VU_>), dim3(gx), dim3(256), 0, s, q, k, kap, gc, T, H, \
+                       NT, B * H, n0, n1, scale, W, Kf, Qg, M, Ast, flags, q_rstd, k_rstd, v, U);                      \
   } while (0)
-    if (iso && q_rstd) KDN_INTRA(true, true);
-    else if (iso) KDN_INTRA(true, false);
-    else if (q_rstd) KDN_INTRA(false, true);
-    else KDN_INTRA(false, false);
+#define KDN_INTRA_U(ISO_, NORM_)                                                                                       \
+  do {                                                                                                                 \
+    if (grouped) KDN_INTRA(ISO_, NORM_, V);                                                                            \
+    else KDN_INTRA(ISO_, NORM_, 0);                                                                                    \
+  } while (0)
+    if (iso && q_rstd) KDN_INTRA_U(true, true);
+    else if (iso) KDN_INTRA_U(true, false);
+    else if (q_rstd) KDN_INTRA_U(false, true);
+    else KDN_INTRA_U(false, false);
+#undef KDN_INTRA_U
 #undef KDN_INTRA
   };
   auto launch_ro = [&](dim3 grid, const kdn_state::GroupPlan& P, float* hstore, float* dstore, int mask,
                        const float* hin, float* hout) {
     const dim3 bs(2 * kdn_state::state_threads(V));
-    with_copy_mask(mask, [&](auto hmc) {
+    auto go = [&](auto hmc, auto ug) {
       constexpr int HM = decltype(hmc)::value;
+      constexpr bool UG = decltype(ug)::value;
       if (o_bf16)
-        hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, bf16_t, true, HM>), grid, bs, 0, stream, v, W, A, Kf,
-                           gc, hin, T, H, NT, B * H, hstore, dstore, hout, P, Qg, M, (bf16_t*)o);
+        hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, bf16_t, true, HM, UG>), grid, bs, 0, stream, v, W, A, Kf,
+                           gc, hin, T, H, NT, B * H, hstore, dstore, hout, P, U, Qg, M, (bf16_t*)o);
       else
-        hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, true, HM>), grid, bs, 0, stream, v, W, A, Kf,
-                           gc, hin, T, H, NT, B * H, hstore, dstore, hout, P, Qg, M, (float*)o);
-    });
+        hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, true, HM, UG>), grid, bs, 0, stream, v, W, A, Kf,
+                           gc, hin, T, H, NT, B * H, hstore, dstore, hout, P, U, Qg, M, (float*)o);
+    };
+    if (grouped) go(std::integral_constant<int, 0>{}, std::true_type{});  // (groups keep fp32 copies: half_copies)
+    else with_copy_mask(mask, [&](auto hmc) { go(hmc, std::false_type{}); });
   };
   // Overlapped schedule (bits 0, 1 and 2 in one call, one chunk group): the state pass (with the readout
   // fused) occupies B*H*V/64 CUs, one workgroup each, and leaves the rest idle.  The sequence runs in two
@@ -978,8 +1011,8 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
     constexpr int NV = V / kdn_state::state_cols(V), NS = NV + K / kdn_state::state_cols(V);
     float* grp = saved + lay.grp;
     kdn_state::GroupPlan P{gcnt.NG, gcnt.m, 0, grp, grp + (int64_t)B * H * gcnt.NG * K * V};
-    hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V>), dim3(B * H * (gcnt.NG - 1) * NS),
-                       dim3(kdn_state::state_threads(V)), 0, stream, v, W, A, Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P);
+    hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, false, 0, true>), dim3(B * H * (gcnt.NG - 1) * NS),
+                       dim3(kdn_state::state_threads(V)), 0, stream, v, W, A, Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P, U);
     KDN_CHECK_LAUNCH();
     if (gcnt.NG > 2) {
       hipLaunchKernelGGL((kdn_state::state_combine_kernel<K, V>), dim3(B * H * NV), dim3(kdn_state::state_threads(V)),
@@ -997,10 +1030,14 @@ int mem_fwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
     const dim3 bs(kdn_state::state_threads(V));
     const int rc = run_state_pass<K, V>(
         B * H, lay.gc, saved + lay.grp, false, stream, [&](dim3 grid, const kdn_state::GroupPlan& P) {
-          with_copy_mask(hm, [&](auto hmc) {
-            hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, false, decltype(hmc)::value>), grid, bs, 0,
-                               stream, v, W, A, Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P);
-          });
+          if (grouped)
+            hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, false, 0, true>), grid, bs, 0, stream, v, W, A,
+                               Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P, U);
+          else
+            with_copy_mask(hm, [&](auto hmc) {
+              hipLaunchKernelGGL((kdn_state::state_fwd_kernel<K, V, float, false, decltype(hmc)::value, false>), grid, bs,
+                                 0, stream, v, W, A, Kf, gc, h0, T, H, NT, B * H, hb, D, ht, P, U);
+            });
         });
     if (rc) return rc;
   }

@@ -5,7 +5,7 @@
 //   backward (reverse):      dh_n = dS;  d delta = M^T dO + Kf dS;  dX = A^T d delta;
 //                            dS <- e^{g_last} dS + Qg^T dO - W^T d delta
 // (A = (I + N)^{-1} of the chunk, W = A Kg.)  U and dX are off the recurrence: the helper waves of each pass form
-// them.  On the recurrence instead (delta = A (V - Kg S), dS - Kg^T dX, which needs no W) the product with A
+// them (with chunk groups the intra-chunk build forms U).  On the recurrence instead (delta = A (V - Kg S), dS - Kg^T dX, which needs no W) the product with A
 // lengthened every chunk step of the forward pass by 0.5 us (376 -> 449 us at B4 T4096 H18 d128).
 //
 // Work split.  One workgroup per (b, h, 64-column slice of V), one wave per 16 state columns;
@@ -396,11 +396,16 @@ __device__ __forceinline__ bool group_task(const GroupPlan& P, int BH, int& bh, 
 // HBM one chunk ahead, straight into registers) and store o.  That drops readout_kernel and its
 // re-reads of h and delta, and keeps the readout's MFMAs and stores off the serial chain, which only
 // pays for the fragment stores.  Both wave groups run the same barrier sequence.
-template <int K, int V, typename TO = float, bool RO = false, int HM = 0>
+// With UG (every pass of chunk groups) U = A V comes from the intra-chunk build (Ug, accumulator tiles) in place of A and
+// V: pass A has no helper waves to form it, on its chain the product and V's loads cost more than the copy, and pass
+// C would form it again.  No backward, isotropic, formed here / in the build (which then writes no A): B2 T2000 H9 d128 156.0 /
+// 147.0 us, B1 T8192 H18 d64 226.8 / 218.5, B1 T32768 H18 d128 1408 / 1388; training B2 T2000 H9 389.6 / 380.4, B1 T4096 H18
+// 625.5 / 632.3.
+template <int K, int V, typename TO, bool RO, int HM, bool UG>
 __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 1 : 2) void state_fwd_kernel(
     const bf16_t* __restrict__ v, const float* __restrict__ W, const float* __restrict__ Ag,
     const float* __restrict__ Kf, const float* __restrict__ gc, const float* __restrict__ h0, int T, int H, int NT, int BH,
-    float* __restrict__ hbuf, float* __restrict__ Dl, float* __restrict__ ht, GroupPlan P,
+    float* __restrict__ hbuf, float* __restrict__ Dl, float* __restrict__ ht, GroupPlan P, const float* __restrict__ Ug,
     const float* __restrict__ Qg = nullptr, const float* __restrict__ Mg = nullptr, TO* __restrict__ out = nullptr) {
   constexpr int COLS = state_cols(V), NTHR = state_threads(V);
   constexpr int KB = K / 32;           // k-blocks of a contraction over K
@@ -409,14 +414,14 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
   constexpr int UN = C * K / 4 / NTHR;  // staging units per thread of a C x K operand
   constexpr int UA = NTRI * 128 / NTHR;  // ... of A
   __shared__ __attribute__((aligned(16))) bf16_t sW[(C / 16) * KB * TILE];        // W: rows c, k = i
-  __shared__ __attribute__((aligned(16))) bf16_t sA[NTRI * TILE];                  // A: rows c, k = s
+  __shared__ __attribute__((aligned(16))) bf16_t sA[UG ? 8 : NTRI * TILE];         // A: rows c, k = s
   __shared__ __attribute__((aligned(16))) bf16_t sK[(K / 16) * (C / 32) * TILE];  // Kf^T: rows i, k = c
   __shared__ __attribute__((aligned(16))) float sE[K];
   // RO: B fragments of h_n ([wave][kb][hi, lo][lane], K / 32 k-blocks) then of delta_n (2 k-blocks)
   constexpr int NHF = 4 * KB * 2 * 64, NDF = 4 * 2 * 2 * 64;
   __shared__ __attribute__((aligned(16))) uint4 sHD[RO ? NHF + NDF : 1];
-  __shared__ f32x4 sU[RO ? 4 * 4 * 64 : 1];  // RO: U = A V of the next chunk: [state wave][row tile cb][lane]
-  __shared__ uint4 sV[RO ? 4 * 2 * 64 : 1];  // RO: V of the next chunk as B fragments: [column group][kb][lane]
+  __shared__ f32x4 sU[RO && !UG ? 4 * 4 * 64 : 1];  // RO: U = A V of the next chunk: [state wave][row tile cb][lane]
+  __shared__ uint4 sV[RO && !UG ? 4 * 2 * 64 : 1];  // RO: V of the next chunk as B fragments: [column group][kb][lane]
   // RO: a readout wave's output rows, RR at a time, regrouped so that every store writes whole row segments
   constexpr int ROWB = COLS * (int)sizeof(TO), QPR = ROWB / 16, RPI = 1024 / ROWB, RR = 2048 / ROWB;
   static_assert(ROWB % 128 == 0 && RPI <= 8 && RR <= 16, "readout rows of 8 or more 16-byte quads");
@@ -493,12 +498,14 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
 #pragma unroll
         for (int cb = 0; cb < 4; ++cb) sU[(rw * 4 + cb) * 64 + lane] = U[cb];
       };
-      load_AV(n0);
+      if constexpr (!UG) load_AV(n0);
       load_QM(n0);
-      stage_AV();
-      __syncthreads();  // A, V of the first chunk staged
-      publish_U();
-      if (n0 + 1 < n1) load_AV(n0 + 1);
+      if constexpr (!UG) {
+        stage_AV();
+        __syncthreads();  // A, V of the first chunk staged
+        publish_U();
+        if (n0 + 1 < n1) load_AV(n0 + 1);
+      }
       __syncthreads();  // U of the first chunk published
       for (int n = n0; n < n1; ++n) {
         const int t0 = n * C, L = min(C, T - t0);
@@ -517,8 +524,10 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
         }
         if (n + 1 < n1) {
           load_QM(n + 1);
-          stage_AV();
-          if (n + 2 < n1) load_AV(n + 2);
+          if constexpr (!UG) {
+            stage_AV();
+            if (n + 2 < n1) load_AV(n + 2);
+          }
         }
         __syncthreads();  // end of phase 1: h_n and delta_n fragments published, U_n read, A, V of chunk n + 1 staged
         const bufrsrc ro = make_buf(out + row_bthk(b, t0, h, T, H, V), (uint32_t)((L - 1) * H + 1) * V * sizeof(TO));
@@ -570,18 +579,18 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
             __builtin_amdgcn_raw_buffer_store_b128(x, ro, eb, 0, 0);  // rows past L dropped
           }
         }
-        if (n + 1 < n1) publish_U();
+        if (!UG && n + 1 < n1) publish_U();
         __syncthreads();  // end of phase 2: the fragments may be overwritten, U of chunk n + 1 published
       }
       return;
     }
   }
 
-  // without readout waves: V of this lane's column, U's B fragment (Phi columns: 0)
+  // without readout waves and groups: V of this lane's column, U's B fragment
   uint16_t rV[4][4];
   auto load_V = [&](int n) {
     const int t0 = n * C, L = min(C, T - t0);
-    const bufrsrc rv = make_buf(v + row_bthk(b, t0, h, T, H, V), phi ? 0u : ((L - 1) * H + 1) * V * 2);
+    const bufrsrc rv = make_buf(v + row_bthk(b, t0, h, T, H, V), ((L - 1) * H + 1) * V * 2);
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
@@ -594,6 +603,16 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
       auto p2 = [&](int cb, int j) { return (uint32_t)rV[cb][j] | ((uint32_t)rV[cb][j + 1] << 16); };
       vf[kb] = uint4{p2(2 * kb, 0), p2(2 * kb, 2), p2(2 * kb + 1, 0), p2(2 * kb + 1, 2)};
     }
+  };
+  float4 rU[UG ? 4 : 1];
+  auto load_U = [&](int n) {  // this lane's U (Phi columns have none: 0)
+    const bufrsrc r = make_buf(Ug + ((int64_t)bh * NT + n) * C * V, phi ? 0u : C * V * 4);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) rU[UG ? cb : 0] = buf_ld4(r, (uint32_t)(((col >> 4) * 4 + cb) * 64 + lane) * 16);
+  };
+  auto load_u = [&](int n) {  // what a state wave needs for U of chunk n
+    if constexpr (UG) load_U(n);
+    else if constexpr (!RO) load_A(n), load_V(n);
   };
   const RowStage<K> stW(tid);
   const ColStage<K> stK(tid);
@@ -612,7 +631,7 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
   };
   auto stage_W = [&]() {
     stW.put(sW, rW);
-    if constexpr (!RO) stage_A();
+    if constexpr (!RO && !UG) stage_A();
   };
   auto stage_K = [&]() {
     stK.put(sK, rK);
@@ -636,10 +655,10 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
   }
 
   load_W(n0);
-  if constexpr (!RO) load_A(n0), load_V(n0);
+  load_u(n0);
   stage_W();
   load_K(n0);
-  if constexpr (RO) __syncthreads();  // the helpers' first barrier
+  if constexpr (RO && !UG) __syncthreads();  // the helpers' first barrier
   __syncthreads();
   for (int n = n0; n < n1; ++n) {
     if (real && hbuf) {  // (no h, delta stores when the readout is fused and no backward follows)
@@ -651,14 +670,17 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
     // ---- phase 1: delta = U - W S   (reads sW, sU; fills sK with chunk n; loads W of chunk n+1)
     stage_K();
     f32x4 D[4];  // U, then delta
-    if constexpr (!RO) {
+    if constexpr (UG) {
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) D[cb] = __builtin_bit_cast(f32x4, rU[UG ? cb : 0]);
+    } else if constexpr (!RO) {
       uint4 vf[2];
       pack_V(vf);
       prod_U(vf, D);
     }
     if (n + 1 < n1) {
       load_W(n + 1);
-      if constexpr (!RO) load_A(n + 1), load_V(n + 1);
+      load_u(n + 1);
     }
     {
       uint4 bh_[KB], bl_[KB];
@@ -673,7 +695,7 @@ __global__ __launch_bounds__(RO ? 2 * state_threads(V) : state_threads(V), RO ? 
                              a[st & 3] = mma3(ah, al, bh_[st >> 2], bl_[st >> 2], a[st & 3]);
                            });
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) D[cb] = (RO ? sU[RO ? (w * 4 + cb) * 64 + lane : 0] : D[cb]) - a[cb];
+      for (int cb = 0; cb < 4; ++cb) D[cb] = (RO && !UG ? sU[RO && !UG ? (w * 4 + cb) * 64 + lane : 0] : D[cb]) - a[cb];
       if (real && Dl) st_tiles<V>(Dl, (int64_t)bh * NT + n, col, lane, D);
       if constexpr (RO) {  // publish the B fragments of h_n (multiplied with W above)
 #pragma unroll
