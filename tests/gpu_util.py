@@ -17,7 +17,7 @@ def gpu_or_skip():
 
 
 def rel(x, ref) -> float:
-    """max|x - ref| / max|ref| (the parity metric of the north star).
+    """max|x - ref| / max|ref|, the parity metric.
 
     When the reference is identically zero (e.g. the gate gradient of a single token,
     whose state does not depend on its own retention) the absolute error is returned."""
