@@ -38,12 +38,6 @@ using kdn_state::zero4;
 using kdn_state::afrag;
 using kdn_state::TILE;
 
-// a*b with a exact in bf16 (A operand) and b = bh + bl split (B operand)
-__device__ __forceinline__ f32x4 mma2b(uint4 a, uint4 bh, uint4 bl, f32x4 c) {
-  c = mfma(a, bh, c);
-  c = mfma(a, bl, c);
-  return c;
-}
 // a*b where each operand is split (hi + lo, AL / BL) or exact in bf16 (hi only): hi*hi, hi*lo, lo*hi
 // in the order of mma3, dropping the terms of an absent lo half.
 template <bool AL, bool BL>
@@ -73,9 +67,9 @@ __device__ __forceinline__ void upper_tile(int t, int& I, int& J) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// The whole chunk-parallel backward of one chunk in one kernel: the state-gradient products, the
-// transposed solves and the gradients.  dQg, dW, dKf, dM, dKg, dN and the g_last dots never go to
-// HBM: each is produced in the register or LDS layout its consumer takes.
+// The whole chunk-parallel backward of one chunk in one kernel: the products with h, dh and dX and the
+// gradients.  dQg, dKf, dM, dKg, dN and the g_last dots never go to HBM: each is produced in the register or
+// LDS layout its consumer takes.
 // One chunk-head task of the order task = (NT - 1 - n) * B*H + bh (last chunks first, the order in
 // which the reverse state pass finishes them); block 512 (8 waves), one workgroup per CU (LDS 141 KB).
 //  * Staging.  The chunk rows of dO, delta and dX are split into LDS fragments (rows c, k = v, natural
@@ -197,7 +191,7 @@ __device__ __forceinline__ void chunk_bwd_task(
   }
   // Diagonal variant, K = 128: the chunk's k and q rows for the gradient phase go straight from memory
   // into LDS (buffer loads with the LDS flag: no registers held), issued once phase 1's operands have
-  // arrived, so they land during phase 1 and the solve instead of as per-channel gathers in the gradient
+  // arrived, so they land during phase 1 instead of as per-channel gathers in the gradient
   // phase (diag step -30 us; the isotropic variant, whose gradient phase loads less, measured 7 us
   // slower with it and keeps the gathers).
   // One instruction moves 64 lanes x 16 B = 4 rows of 256 B; row c of tensor x sits at

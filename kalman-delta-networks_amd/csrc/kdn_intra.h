@@ -209,7 +209,7 @@ __device__ __forceinline__ void intra_solve_emit(float* sA, const float* sN, flo
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
           if (kb == 1 && I < 2) continue;  // A[c][s] = 0 for s > c
-          acc = kdn_state::mma2(ah[I][kb], al[I][kb], xh[kb], acc);
+          acc = mma2(ah[I][kb], al[I][kb], xh[kb], acc);
         }
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), rU, (uint32_t)((t * 4 + I) * 64 + lane) * 16,
                                                0, 0);

@@ -23,7 +23,12 @@
 //                dM = dO delta^T, dN = -dX delta^T, g_last terms; dq, dk, dkappa (or dbeta), dg from dN, dM
 //                and the elementwise factors
 //   *_exact      the chunks the forward flagged: the same gradients by per-block anchors and per-element
-//                blocks (the products above come from chunk_bwd through HBM)
+//                blocks (the products above come from chunk_bwd through HBM).  Their U, dV, dKg and dN take the bf16
+//                hi + lo products of the other chunks, with the exact path's A; with fp32 substitutions and
+//                products in their place the outputs were no nearer to float64, for the state passes' own hi + lo products
+//                bound them (B1 T201 H6 d128, bursts of e^-12 per token in 6 channels, mean of 12: o 5.111e-6 with fp32,
+//                5.116e-6; diagonal dkappa 5.058e-6, 5.057e-6, dg 5.380e-6, 5.372e-6; all channels at e^-6 +- 3: o
+//                4.4419e-6, 4.4416e-6).
 //
 // g is kept in the base-2 units of g_cumsum, so e^{g_c - g_s} = exp2(G_c - G_s).
 // Decay factors (c >= s) are split at the start a of the row block (16 tokens):
@@ -778,10 +783,11 @@ struct BwdLayout {
 // workgroups take the CUs the first one frees (the side launch starts a few microseconds later), and
 // the side launch's workgroups fill the idle CUs and backfill them as they finish.  The remaining
 // tasks run at full width after the pass.  A chunk-backward task lasts about kStepsPerTask chunk
-// steps of the pass running beside it (~26 us against ~5.2 us), which sizes the first segment so
-// that its tasks keep the idle CUs busy until the pass ends and the remaining tasks fill the last
-// round of 256 CUs: at B4 T4096 H18 d128, 5.0 gives 1,120 side tasks and 13.6 main rounds (whole step
-// 1377 us isotropic, 1956 diagonal), 5.3 to 6.4 give 1,008 and 14.06 (1405 / 1980).
+// steps of the pass running beside it (~26 us against ~5.2 us), which sizes the first segment so that its tasks
+// keep the idle CUs busy until the pass ends.  The training step over values of it, us: B4 T4096 H18 d128 isotropic
+// 1302 at 4.5 to 5.0, 1308 at 4.0, 1322 to 1328 at 5.2 to 6.4; T2048 711 to 713 up to 5.2, 737 to 742 from 5.5;
+// T3700 H17 1161 at 4.8 and 5.0, 1182 at 4.0, 1199 at 6.0; T1024 459 at 5.0 to 5.5, 463 below, 480 above; diagonal
+// T4096 1853 at 5.0, 1860 at 4.0, 1875 at 6.4 (where an end is worse, a last round of few tasks begins).
 constexpr float kStepsPerTask = 5.0f;
 constexpr unsigned kSideDelayTicks = 300;  // of the 100 MHz wall clock: 3 us
 struct BwdOverlap {
@@ -802,7 +808,9 @@ inline BwdOverlap plan_bwd_overlap(int BH, int NT, int NV, GroupCount gc, int cu
 // the rest's pass (see mem_fwd_impl).  The pass holds B*H*V/64 CUs; the side build's workgroups (three
 // per CU, each lasting about kBuildSteps chunk steps of the pass: the diagonal build is ~15% longer) take
 // the `idle` ones, so m1 balances the first range's pass against the second range's build there.
-// Measured at B4 T4096 H18 (m1 swept 30 .. 45): best at 39 (isotropic) and 42 (diagonal).
+// The forward over multiples 0.8 / 0.9 / 1 / 1.1 of the constants, us: B4 d128 isotropic T4096 H18 533 / 528 / 526 / 526, T2048
+// 303 / 294 / 290 / 290, T1024 175 / 175 / 163 / 163, T3700 H17 494 / 480 / 475 / 478; diagonal 706 / 711 / 712 / 719, 408 /
+// 397 / 396 / 403, 243 / 243 / 236 / 237, 649 / 638 / 636 / 645.
 constexpr float kBuildStepsIso = 7.3f, kBuildStepsDiag = 9.0f;
 inline int plan_fwd_overlap(int BH, int NT, int NV, int cus, bool iso) {
   const int idle = cus - BH * NV;
@@ -1071,7 +1079,7 @@ int mem_bwd_impl(const bf16_t* q, const bf16_t* k, const float* kap, int iso, co
                          W, A, gc, dO, dS_in, T, H, NT, B * H, dh, dX, dS_out, P);
     });
   };
-  // every chunk's products with h / dh; the solves and gradients of the unflagged ones: the
+  // every chunk's products with h, dh and dX and the gradients of the unflagged ones: the
   // chunk-head tasks task0 .. task_end - 1 (order of chunk_bwd_task: last chunks first)
   auto launch_chunk = [&](int task0, int task_end, hipStream_t st) {
 #define KDN_CHUNK_BWD(ISO_, HB_)                                                                                    \
