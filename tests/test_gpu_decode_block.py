@@ -164,3 +164,30 @@ def test_split_projection_matches_fp64(M, N, K, bias, res):
 def test_decode_block_with_projections_apart(mixer_type, B, H, d, monkeypatch):
     """Beyond 32 rows and past K 2304 the normed and gated products leave the one launch (K 1152 and 2432, 2560)."""
     test_decode_block_matches_the_layers_launches(mixer_type, B, H, d, monkeypatch)
+
+
+@pytest.mark.parametrize("mixer_type,B,H", [("iso_kdn", 9, 9), ("iso_kdn", 64, 18), ("diag_kdn", 33, 9), ("iso_kdn", 2, 20)])
+def test_captured_step_replays_as_the_eager_step(mixer_type, B, H):
+    """The decoder's graph where it holds split products (9 rows, w3 of K 3456) and where it holds library products
+    (33 and 64 rows, K 2560): every replay against the eager step, with eager work between the replays."""
+    dev = gpu_or_skip()
+    from lit_gpt.decode import KDNDecoder
+    log(f"case captured step {mixer_type} B={B} H={H}")
+    torch.manual_seed(B + H)
+    cfg = model_mod.Config.from_name(("iso" if mixer_type == "iso_kdn" else "diag") + "_kdn_1.3B", n_layer=1, n_head=H,
+                                     n_embd=128 * H, intermediate_size=3 * 128 * H, kdn_info_scale=128.0)
+    m = model_mod.GPT(cfg).to(dev).to(torch.bfloat16).eval()
+    idx = torch.randint(0, 200, (B, 9), device=dev)
+    eager, graph = KDNDecoder(m, B, use_graph=False), KDNDecoder(m, B, use_graph=True)
+    eager.prefill(idx[:, :4])
+    graph.prefill(idx[:, :4])
+    for t in range(4, 9):
+        a = eager.step(idx[:, t]).clone()
+        torch.cuda.synchronize()
+        b = graph.step(idx[:, t]).clone()
+        torch.cuda.synchronize()
+        # the same launches; a library product may take another order of its fp32 sum when captured (bf16 after it)
+        assert rel(b.float(), a.float()) < 2e-2
+    for s, p in zip(graph.state, eager.state):
+        assert s.seen_tokens == p.seen_tokens == 9
+        assert rel(s.memory, p.memory) < 2e-2 and rel(s.precision, p.precision) < 1e-2
